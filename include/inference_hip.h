@@ -56,7 +56,7 @@ void inference_state_refresh_from_sft(InferenceState *state);
 
 void inference_state_free(InferenceState *state);                    /* src/nn/fast_inference.h:21 */
 
-/* src/nn/fast_inference.h:26-28 (impl :612-675): greedy decoding.  Prefills the prompt token by token, then emits
+/* src/nn/fast_inference.h:26-28 (impl :612-675): greedy decoding.  Prefills the prompt (as inference_forward_tokens does), then emits
  * argmax tokens until an EOS token has been emitted, max_gen_len tokens are out or the cache is full.  Returns the
  * number of tokens written (the EOS token included, as in the reference). */
 int inference_generate(InferenceState *state, const uint32_t *prompt_tokens, int prompt_len,
@@ -80,8 +80,9 @@ int inference_generate_batch(InferenceState *state, const uint32_t *prompt_token
 int inference_step_batch(InferenceState *state, const int *tokens, int batch_size, int pos, float *logits);
 
 /* The next n tokens at the current position, which advances by n, and the logits [n_want][vocab] (host) at the places
- * want[0 .. n_want) among them, ascending; n_want may be 0.  A prompt may be cut into calls anywhere.  MODEL_NEVURAX and
- * MODEL_PAPOSUN run them as one step (long prompts: a few), the other models token by token.  No counterpart in the reference.  Returns 0,
+ * want[0 .. n_want) among them, ascending; n_want may be 0.  A prompt may be cut into calls anywhere.  They run as
+ * one step (long prompts: a few); the models that are not described layer by layer take portions of up to four tokens, and
+ * all tokens where head_dim is not 32, 64, 128 or 256 or memory for the products' operands is short, one by one.  No counterpart in the reference.  Returns 0,
  * -1 when the arguments do not fit. */
 int  inference_forward_tokens(InferenceState *state, const int *tokens, int n, const int *want, int n_want, float *logits);
 

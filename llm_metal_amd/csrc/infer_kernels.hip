@@ -11,6 +11,7 @@
 #include "backend.h"
 #include "devutil.h"
 #include "gemm.h"
+#include "prompt.h"
 #include <hip/hip_ext.h>
 
 using namespace lmhip;
@@ -80,6 +81,45 @@ const int8_t *q8_split_of(MetalBuf *W, int rows, int nb, const half_t **scales)
                (uint16_t *)(img + soff), n_blocks);
     *scales = (const half_t *)(img + soff);
     return (const int8_t *)img;
+}
+
+// One wave per 32 x 64 tile of two tiled F16 images of a Q8_0 matrix (prompt.h): hi = half(d q), lo = 2^11 (d q - hi), so that
+// hi + lo / 2^11 holds d q -- a half times an int8, 18 bits -- to 22.  A lane takes the 32 codes of one (row, block).
+__global__ __launch_bounds__(TB) void k_q8_tiled_pair(const int8_t *__restrict__ q, const half_t *__restrict__ d, half8 *__restrict__ hi,
+                                                      half8 *__restrict__ lo, int rows, int nb, int Kb, size_t tiles)
+{
+    const size_t tile = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile >= tiles) return;
+    const int lane = threadIdx.x & 63, row = (int)(tile / Kb) * 32 + (lane >> 1), blk = (int)(tile % Kb) * 2 + (lane & 1);
+    const bool live = row < rows && blk < nb;              // padding rows and columns hold zeros
+    const size_t b = live ? (size_t)row * nb + blk : 0;
+    const int4 *src = reinterpret_cast<const int4 *>(q + b * 32);
+    const int4 w[2] = {src[0], src[1]};
+    const float sc = live ? (float)d[b] : 0.f;
+    const size_t at = tile * 256 + (size_t)(lane & 1) * 32 + (lane >> 1);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int c[2] = {j & 1 ? w[j >> 1].z : w[j >> 1].x, j & 1 ? w[j >> 1].w : w[j >> 1].y};
+        half8 h, l;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float v = sc * (float)(int8_t)(c[e >> 2] >> (8 * (e & 3)));
+            h[e] = live ? f2h(v) : (half_t)0;
+            l[e] = live ? f2h((v - h2f(h[e])) * lmhip::Q8_RESIDUAL_SCALE) : (half_t)0;
+        }
+        hi[at + 64 * j] = h;
+        lo[at + 64 * j] = l;
+    }
+}
+
+// raises *out (a float's bits) to the largest |d|; a NaN is above every number
+__global__ __launch_bounds__(TB) void k_max_scale(const half_t *__restrict__ d, size_t n, unsigned *__restrict__ out)
+{
+    unsigned top = 0u;
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < n; i += (size_t)gridDim.x * TB) top = max(top, __float_as_uint(fabsf((float)d[i])));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = max(top, (unsigned)__shfl_xor((int)top, o, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(out, top);
 }
 
 // ---------------------------------------------------------------- matrix-vector products
@@ -1045,6 +1085,25 @@ void matvec_norm(MetalBuf *W, const NormIn &nin, MetalBuf *y, int rows, int cols
         launch_matvec_norm<0>(dptr(W), nullptr, nin, dptr_as<float>(y), rows, cols, glu);
     }
     mark_written(y);
+}
+
+void q8_to_tiled_pair(MetalBuf *W, int rows, int cols, half_t *hi, half_t *lo)
+{
+    if (rows <= 0 || cols <= 0 || (cols & 31)) { fprintf(stderr, "[fast_hip] q8_to_tiled_pair: unsupported shape %d x %d\n", rows, cols); abort(); }
+    REQUIRE_BYTES(W, (size_t)rows * (cols / 32) * 34, "q8_to_tiled_pair");
+    const half_t *d = nullptr;
+    const int8_t *q = q8_split_of(W, rows, cols / 32, &d);
+    const int Kb = tiled_kb(cols);
+    const size_t tiles = (size_t)tiled_rb(rows) * Kb;
+    LAUNCH(k_q8_tiled_pair, dim3((unsigned)((tiles + 3) / 4)), dim3(TB), 0, q, d, (half8 *)hi, (half8 *)lo, rows, cols / 32, Kb, tiles);
+}
+
+void q8_max_scale(MetalBuf *W, int rows, int cols, unsigned *out)
+{
+    REQUIRE_BYTES(W, (size_t)rows * (cols / 32) * 34, "q8_max_scale");
+    const half_t *d = nullptr;
+    q8_split_of(W, rows, cols / 32, &d);
+    LAUNCH(k_max_scale, dim3(128), dim3(TB), 0, d, (size_t)rows * (cols / 32), out);
 }
 
 void attention_decode_fused(const HeadPost &hp, MetalBuf *Kc, MetalBuf *Vc, float *out, int hd, int max_seq, int copies)

@@ -10,11 +10,13 @@
 #include "backend.h"
 #include "devutil.h"
 #include "fused.h"
+#include "prompt.h"
 #include "stack.h"
 #include "../../include/inference_hip.h"
 #include "../../include/loader_hip.h"
 
 #include <fstream>
+#include <functional>
 #include <math.h>
 #include <sstream>
 #include <string.h>
@@ -28,7 +30,9 @@ extern "C" MetalBuf *sft_get_token_emb_buf(SFTState *s);
 
 namespace {
 struct BatchRun;
+struct PromptRun;
 void batch_release(BatchRun *r);
+void prompt_release(PromptRun *r);
 // a state on a training state's tiles, or of a layer-by-layer model: one token through the lock-step path with a run of
 // one sequence
 void step_on_run(InferenceState *s, int token, int pos);
@@ -36,6 +40,10 @@ const float *logits_on_run(InferenceState *s);
 int argmax_on_run(InferenceState *s);
 void prefill_on_run(InferenceState *s, const uint32_t *tokens, int n, int pos);
 int forward_rows(InferenceState *s, const int *tokens, int n, const int *want, int n_want, float *logits);
+// the other models: n tokens of one sequence in steps of many rows, where the shape and memory allow that
+bool prompt_takes(InferenceState *s, int n);
+int prompt_forward(InferenceState *s, const int *tokens, int n, const int *want, int n_want, float *logits);
+void prompt_fill(InferenceState *s, const uint32_t *tokens, int n);
 }
 
 struct InferenceState {
@@ -73,6 +81,7 @@ struct InferenceState {
     int R;
     float scaling;
     MetalBuf *lora_t;                    // [2R]: A_q ln | A_v ln
+    PromptRun *prompt;                   // scratch of prompts taken many tokens at a time (NULL until used)
     BatchRun *batch;                     // scratch and caches of the lock-step batch path, kept from call to call (NULL until used)
 };
 
@@ -180,18 +189,6 @@ __global__ __launch_bounds__(64) void k_lora_down(const float *__restrict__ ln, 
     }
     s = wave_sum(s);
     if (threadIdx.x == 0) t[r] = s;
-}
-
-// A product of the batched step as the GEMM leaves it (gemm_f32a_exact without its last part): S planes of [2B, N], rows
-// b and B + b the value and residual images of sequence b, inv their factors.
-struct SplitPlanes {
-    const float *P, *inv;
-    size_t plane;
-    int S, N;
-};
-__device__ __forceinline__ float planes_at(const SplitPlanes &p, int B, int b, int n)
-{
-    return split_planes_value(p.P, p.S, p.plane, p.N, p.inv, B, b, n);
 }
 
 // act[b][i] = silu | gelu (gate) * up from the planes of the [gate | up] product of a batch
@@ -682,6 +679,7 @@ void inference_state_free(InferenceState *s)
     metal_flush();
     batch_release(s->batch);
     batch_release(s->single);
+    prompt_release(s->prompt);
     stack_free(s->stack);
     for (MetalBuf *b : {s->gate_v, s->up_v, s->x, s->x2, s->branch, s->ln, s->qkv, s->att, s->gu, s->logits, s->best, s->lora_t, s->rope_tabs})
         metal_buf_free(b);
@@ -752,6 +750,7 @@ int inference_forward_tokens(InferenceState *s, const int *tokens, int n, const 
     for (int i = 0; i < n_want; i++)
         if (want[i] < 0 || want[i] >= n || (i && want[i] <= want[i - 1])) { fprintf(stderr, "[FastGen] wanted places must ascend inside the portion\n"); return -1; }
     if (s->stack) return forward_rows(s, tokens, n, want, n_want, logits);
+    if (prompt_takes(s, n)) return prompt_forward(s, tokens, n, want, n_want, logits);
     for (int i = 0, w = 0; i < n; i++) {                                  // the other models take one token per step
         step_token(s, tokens[i], s->cur_len);
         s->cur_len++;
@@ -765,13 +764,17 @@ int inference_generate(InferenceState *s, const uint32_t *prompt_tokens, int pro
 {
     s->cur_len = 0;
     if (prompt_len <= 0 || max_gen_len <= 0 || prompt_len > s->max_seq) return 0;
-    for (int i = 0; i < prompt_len; i++) {
-        if (!token_ok(s, (int)prompt_tokens[i])) return 0;
-        if (s->stack) continue;                                       // takes the prompt at once, below
-        step_token(s, (int)prompt_tokens[i], i);                      // prefill: only the last logits are looked at
-        s->cur_len = i + 1;
+    int good = 0;                                                     // tokens ahead of one outside the vocabulary, if there is one
+    while (good < prompt_len && token_ok(s, (int)prompt_tokens[good])) good++;
+    // prefill: only the last logits are looked at
+    if (s->stack) {
+        if (good < prompt_len) return 0;
+        prefill_on_run(s, prompt_tokens, prompt_len, 0);
     }
-    if (s->stack) { prefill_on_run(s, prompt_tokens, prompt_len, 0); s->cur_len = prompt_len; }
+    else if (good == prompt_len && prompt_takes(s, prompt_len)) prompt_fill(s, prompt_tokens, prompt_len);
+    else for (int i = 0; i < good; i++) step_token(s, (int)prompt_tokens[i], i);
+    s->cur_len = good;
+    if (good < prompt_len) return 0;
     int next = argmax_host(s);
     output_tokens[0] = (uint32_t)next;
     int n_gen = 1;
@@ -997,6 +1000,269 @@ void step_on_run(InferenceState *s, int token, int pos)
     forward_token_batch(s, r, &token, pos);
     r.len = pos + 1;
 }
+// ---- prompts of the models that decode a token at a time, many tokens per step
+
+constexpr int PROMPT_ROWS = 1024;        // tokens of one step
+constexpr int PROMPT_WANT = 32;          // rows of logits formed together
+
+struct PromptRun {
+    int cap;                             // rows the buffers are sized for
+    MetalBuf *x, *ln, *q, *att, *act, *t, *a16, *inv_ln, *inv_br, *planes, *planes2, *ids, *sel, *sel_logits;
+    int *ids_host;                       // [max_seq], a token at its position: portions of one prompt do not overwrite each other
+};
+
+void prompt_release(PromptRun *r)
+{
+    if (!r) return;
+    for (MetalBuf *b : {r->x, r->ln, r->q, r->att, r->act, r->t, r->a16, r->inv_ln, r->inv_br, r->planes, r->planes2, r->ids, r->sel, r->sel_logits}) metal_buf_free(b);
+    if (r->ids_host) hipHostFree(r->ids_host);
+    delete r;
+}
+
+size_t free_memory()
+{
+    size_t f = 0, t = 0;
+    HIP_CHECK(hipMemGetInfo(&f, &t));
+    return f;
+}
+
+// Whether n tokens go many to a step: from five on.  A step of 2 to 32 rows takes 1.0 ms on F16 weights (nine layers of the 4B
+// shape; 1.8 tokens one by one) and 2.5 ms on Q8_0 ones (4.5 tokens: their tiled images are formed anew for every product), and
+// 500 tokens take 4.3 instead of 458 ms; portions of up to four stay bit for bit what single tokens give.
+// The first time: room for the tiled images of F16 weights (kept, as the batch path keeps them) besides 2 GB, and no Q8_0
+// weight beyond what a half holds; a state that does not qualify takes its tokens one by one.
+bool prompt_takes(InferenceState *s, int n)
+{
+    const bool q8 = !s->use_fp16 && !s->borrows_tiles;
+    if (s->stack || n < 5 || !prompt_attention_supported(s->hd) || s->D > 8192 || s->R > 64) return false;
+    if (s->prompt) return true;
+    if (!s->borrows_tiles) {
+        size_t need = (size_t)2 << 30;
+        MetalBuf *top = nullptr;
+        if (q8) {
+            top = metal_buf_create(sizeof(unsigned));
+            HIP_CHECK(hipMemsetAsync(dptr(top), 0, sizeof(unsigned), stream()));
+        }
+        const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
+        for (int L = 0; L < s->NL; L++) {
+            const InferenceState::Layer &lw = s->layers[L];
+            for (const WMat *w : {&lw.qkv, (const WMat *)lw.o, &lw.gu, (const WMat *)lw.down}) {
+                if (q8) q8_max_scale(w->mbuf, w->rows, w->cols, dptr_as<unsigned>(top));
+                else if (!w->mbuf->tiled[0].dev) need += tiled_elems(w->rows, w->cols) * sizeof(half_t);
+            }
+        }
+        bool fits = true;
+        if (q8) {
+            unsigned bits = 0;
+            HIP_CHECK(hipMemcpyAsync(&bits, dptr(top), sizeof bits, hipMemcpyDeviceToHost, stream()));
+            HIP_CHECK(hipStreamSynchronize(stream()));
+            metal_buf_free(top);
+            float d;
+            memcpy(&d, &bits, sizeof d);
+            fits = d * 128.f < 65504.f;                                   // (false for a NaN)
+            need += 2 * sizeof(half_t) * std::max({tiled_elems(qd + 2 * kd, s->D), tiled_elems(2 * s->IS, s->D), tiled_elems(s->D, s->IS), tiled_elems(s->D, qd)});
+        }
+        if (!fits || free_memory() < need) return false;
+    }
+    s->prompt = new PromptRun{};
+    PromptRun &r = *s->prompt;
+    const int qd = s->Hq * s->hd, cap = std::min(PROMPT_ROWS, s->max_seq);
+    r.cap = cap;
+    size_t a16 = 0;
+    for (int K : {s->D, qd, s->IS}) a16 = std::max(a16, tiled_elems(2 * cap, K));
+    r.x = fbuf((size_t)cap * s->D); r.ln = fbuf((size_t)cap * s->D);
+    r.q = fbuf((size_t)cap * qd); r.att = fbuf((size_t)cap * qd);
+    if (!prompt_glu_supported(s->IS)) r.act = fbuf((size_t)cap * s->IS);
+    r.a16 = metal_buf_create(a16 * sizeof(half_t));
+    r.inv_ln = fbuf((size_t)2 * cap); r.inv_br = fbuf((size_t)2 * cap);
+    r.ids = metal_buf_create((size_t)s->max_seq * sizeof(int));
+    r.sel = fbuf((size_t)PROMPT_WANT * s->D);
+    HIP_CHECK(hipHostMalloc((void **)&r.ids_host, (size_t)s->max_seq * sizeof(int), hipHostMallocDefault));
+    return true;
+}
+
+// a buffer of at least n floats (what it held is gone when it grows)
+float *at_least(MetalBuf *&b, size_t n)
+{
+    if (!b || b->size < n * sizeof(float)) { metal_buf_free(b); b = fbuf(n); }       // (the free waits for the stream)
+    return dptr_as<float>(b);
+}
+
+// planes of (the operand in r.a16, rows split by `inv`) x w^T: w the state's own matrix (its tiled F16 image, or for Q8_0 the
+// two images of d q and of what rounding that to F16 lost) or a training state's tiles
+SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv, int M)
+{
+    const half_t *a16 = dptr_as<half_t>(r.a16);
+    auto planes = [&](const WeightOp &op, int m, MetalBuf *&buf, size_t &stride) {
+        stride = (size_t)m * rows;
+        if (use_big_gemm(m, rows, cols, op.fmt)) {
+            const WeightOp f = f16_image_of(op, rows, cols);
+            const int chunks = big_gemm_chunks_for(m, rows, cols, f);
+            float *P = at_least(buf, stride * chunks);
+            return launch_gemm_big(a16, nullptr, f, P, rows, m, rows, cols, chunks, stride);
+        }
+        const GemmPlan p = plan_gemm(m, rows, cols, (op.fmt == 1 && op.nbq < tiled_rb(rows)) ? op.nbq : 0, op.fmt);
+        launch_gemm(a16, nullptr, op, at_least(buf, stride * p.S), rows, stride, m, rows, cols, p);
+        return p.S;
+    };
+    SplitPlanes out{};
+    out.inv = inv; out.N = rows;
+    if (tiles) out.S = planes(*tiles, 2 * M, r.planes, out.plane);
+    else if (s->use_fp16) out.S = planes(weight_f16(tiled_weight_of(w->mbuf, rows, cols)), 2 * M, r.planes, out.plane);
+    else {
+        const size_t n = tiled_elems(rows, cols);
+        half_t *hi = (half_t *)scratch(SCR_WF16, 2 * n * sizeof(half_t)), *lo = hi + n;
+        q8_to_tiled_pair(w->mbuf, rows, cols, hi, lo);
+        out.S = planes(weight_f16(hi), 2 * M, r.planes, out.plane);
+        out.S2 = planes(weight_f16(lo), M, r.planes2, out.plane2);
+        out.P2 = dptr_as<float>(r.planes2);
+    }
+    out.P = dptr_as<float>(r.planes);
+    return out;
+}
+
+// One step: the M tokens at positions pos .. pos + M - 1, their keys and values into kc and vc (the first sequence's part),
+// the final norm's rows into r.ln.  Per layer the launches of forward_token_batch, with the tokens as rows: ten, whatever M.
+void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, std::vector<MetalBuf *> &vc, int M, int pos)
+{
+    const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd, IS = s->IS, qd = Hq * hd, nqkv = qd + 2 * Hkv * hd;
+    const bool gemma = s->model_type == MODEL_GEMMA3, bt = s->borrows_tiles, adapters = !s->lora.empty();
+    const int *ids = dptr_as<int>(r.ids) + pos;
+    HIP_CHECK(hipMemcpyAsync((void *)ids, r.ids_host + pos, (size_t)M * sizeof(int), hipMemcpyHostToDevice, stream()));
+    launch_embed_ids(dptr_as<float>(s->emb), ids, s->emb_scale, dptr_as<float>(r.x), M, D);
+    half_t *a16 = dptr_as<half_t>(r.a16);
+    float *inv_ln = dptr_as<float>(r.inv_ln), *inv_br = dptr_as<float>(r.inv_br);
+    auto norm = [&](const SplitPlanes &br, MetalBuf *g_branch, MetalBuf *g, bool keep) {
+        float *ln = keep ? dptr_as<float>(r.ln) : nullptr;
+        const float *gb = g_branch ? dptr_as<float>(g_branch) : nullptr;
+        if (tiled_kb(D) * 64 <= 4096)
+            hipLaunchKernelGGL(k_add_norm_split<4>, dim3(M), dim3(1024), 0, stream(), dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, M, D, s->eps);
+        else
+            hipLaunchKernelGGL(k_add_norm_split<8>, dim3(M), dim3(1024), 0, stream(), dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, M, D, s->eps);
+    };
+    SplitPlanes pending{};
+    MetalBuf *pending_g = nullptr;
+    for (int L = 0; L < s->NL; L++) {
+        const InferenceState::Layer &lw = s->layers[L];
+        const BorrowedLayer *bl = bt ? &s->borrowed[L] : nullptr;
+        norm(pending, pending_g, lw.g_in, adapters && !bt);
+        PromptHeads h{};
+        // (a training state's fused matrix continues with the rows of A_q and A_v)
+        h.qkv = prompt_product(s, r, &lw.qkv, bt ? &bl->qkv : nullptr, nqkv + (bt && adapters ? 2 * s->R : 0), D, inv_ln, M);
+        h.g_q = lw.g_q ? dptr_as<float>(lw.g_q) : nullptr; h.g_k = lw.g_k ? dptr_as<float>(lw.g_k) : nullptr;
+        h.rope = dptr_as<float2>(s->rope_tabs) + ((size_t)s->theta_slot[L] * s->max_seq + pos) * (hd / 2);
+        h.q = dptr_as<float>(r.q); h.kc = dptr_as<float>(kc[L]); h.vc = dptr_as<float>(vc[L]);
+        h.M = M; h.Hq = Hq; h.Hkv = Hkv; h.hd = hd; h.pos = pos; h.max_seq = s->max_seq; h.eps = s->eps;
+        if (adapters) {
+            const InferenceState::Lora &lr = s->lora[L];
+            h.R = s->R; h.sc = s->scaling; h.Bq = dptr_as<float>(lr.Bq); h.Bv = dptr_as<float>(lr.Bv);
+            if (!bt) {
+                float *t = at_least(r.t, (size_t)r.cap * 2 * s->R);
+                hipLaunchKernelGGL(k_lora_down, dim3(2 * s->R, M), dim3(64), 0, stream(), dptr_as<float>(r.ln), dptr_as<float>(lr.Aq), dptr_as<float>(lr.Av), t, s->R, D);
+                h.t = t;
+            }
+        }
+        launch_prompt_heads(h);
+        launch_prompt_attention(h.q, h.kc, h.vc, dptr_as<float>(r.att), M, pos, Hq, Hkv, hd, s->max_seq);
+        mark_written(kc[L]); mark_written(vc[L]);
+        launch_rows_to_f16_split(dptr_as<float>(r.att), a16, inv_br, M, qd);
+        const SplitPlanes o = prompt_product(s, r, lw.o, bt ? &bl->o : nullptr, D, qd, inv_br, M);
+        norm(o, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, false);
+        const SplitPlanes gu = prompt_product(s, r, &lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln, M);
+        if (prompt_glu_supported(IS)) launch_prompt_glu(gu, a16, inv_br, M, IS, gemma ? 1 : 0);
+        else {
+            hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, M), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), M, IS, gemma ? 1 : 0);
+            launch_rows_to_f16_split(dptr_as<float>(r.act), a16, inv_br, M, IS);
+        }
+        pending = prompt_product(s, r, lw.down, bt ? &bl->down : nullptr, D, IS, inv_br, M);
+        pending_g = gemma ? lw.g_post_ff : nullptr;
+    }
+    norm(pending, pending_g, s->g_final, true);
+    HIP_CHECK(hipGetLastError());
+}
+
+// logits of rows m[0 .. count) of the step, count <= PROMPT_WANT, to out [count][V]: one by one through the matrix-vector
+// kernel while that reads the head a few times at most, else (and always on a training state's tiles) as one product
+void prompt_logits(InferenceState *s, PromptRun &r, const int *m, int count, float *out)
+{
+    const int D = s->D;
+    auto row = [&](int i, float *dst) {
+        HIP_CHECK(hipMemcpyAsync(dst, dptr_as<float>(r.ln) + (size_t)m[i] * D, (size_t)D * 4, hipMemcpyDeviceToDevice, stream()));
+    };
+    bool one_by_one = !s->borrows_tiles && (!s->use_fp16 || count < 4);
+    if (!s->borrows_tiles && !one_by_one && !s->lm_head->mbuf->tiled[0].dev)            // room for the head's tiled image
+        one_by_one = free_memory() < tiled_elems(s->V, D) * sizeof(half_t) + ((size_t)2 << 30);
+    if (one_by_one) {
+        for (int i = 0; i < count; i++) {
+            row(i, dptr_as<float>(s->ln));
+            mark_written(s->ln);
+            matvec(s, s->lm_head, s->ln, s->logits);
+            if (out != dptr_as<float>(s->logits))
+                HIP_CHECK(hipMemcpyAsync(out + (size_t)i * s->V, dptr(s->logits), (size_t)s->V * 4, hipMemcpyDeviceToDevice, stream()));
+        }
+        return;
+    }
+    for (int i = 0; i < count; i++) row(i, dptr_as<float>(r.sel) + (size_t)i * D);
+    launch_rows_to_f16_split(dptr_as<float>(r.sel), dptr_as<half_t>(r.a16), dptr_as<float>(r.inv_br), count, D);
+    const SplitPlanes lg = prompt_product(s, r, s->lm_head, s->borrows_tiles ? &s->borrowed_lm : nullptr, s->V, D, dptr_as<float>(r.inv_br), count);
+    launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, out, count, lg.N);
+}
+
+// n tokens from position pos on, in portions of equal size; after each, f(first token of the portion, its length)
+void prompt_portions(InferenceState *s, const int *tokens, int n, int pos, std::vector<MetalBuf *> &kc, std::vector<MetalBuf *> &vc,
+                     const std::function<void(int, int)> &f)
+{
+    PromptRun &r = *s->prompt;
+    const int portions = (n + r.cap - 1) / r.cap, each = (n + portions - 1) / portions;
+    for (int i = 0; i < n; i++) r.ids_host[pos + i] = tokens[i];
+    for (int at = 0; at < n; at += each) {
+        const int M = std::min(each, n - at);
+        prompt_step(s, r, kc, vc, M, pos + at);
+        f(at, M);
+    }
+}
+
+// a whole prompt from position 0 on; the last token's logits to `logits`
+void prompt_rows_all(InferenceState *s, const uint32_t *tokens, int n, std::vector<MetalBuf *> &kc, std::vector<MetalBuf *> &vc, MetalBuf *logits)
+{
+    prompt_portions(s, (const int *)tokens, n, 0, kc, vc, [&](int at, int M) {
+        const int last = M - 1;
+        if (at + M == n) prompt_logits(s, *s->prompt, &last, 1, dptr_as<float>(logits));
+    });
+}
+
+// the same on the sequence that the state itself holds
+void prompt_fill(InferenceState *s, const uint32_t *tokens, int n)
+{
+    if (!s->borrows_tiles) { prompt_rows_all(s, tokens, n, s->kc, s->vc, s->logits); return; }
+    BatchRun &r = batch_acquire(s, s->single, 1);
+    prompt_rows_all(s, tokens, n, r.kc, r.vc, r.logits);
+    r.len = n;
+}
+
+int prompt_forward(InferenceState *s, const int *tokens, int n, const int *want, int n_want, float *logits)
+{
+    BatchRun *run = s->borrows_tiles ? &batch_acquire(s, s->single, 1) : nullptr;
+    std::vector<MetalBuf *> &kc = run ? run->kc : s->kc, &vc = run ? run->vc : s->vc;
+    MetalBuf *row = run ? run->logits : s->logits;
+    int w = 0;
+    prompt_portions(s, tokens, n, s->cur_len, kc, vc, [&](int at, int M) {
+        while (w < n_want && want[w] < at + M) {
+            int m[PROMPT_WANT], k = 0;
+            while (w + k < n_want && k < PROMPT_WANT && want[w + k] < at + M) { m[k] = want[w + k] - at; k++; }
+            float *out = k == 1 ? dptr_as<float>(row) : at_least(s->prompt->sel_logits, (size_t)PROMPT_WANT * s->V);
+            prompt_logits(s, *s->prompt, m, k, out);
+            HIP_CHECK(hipMemcpyAsync(logits + (size_t)w * s->V, out, (size_t)k * s->V * sizeof(float), hipMemcpyDeviceToHost, stream()));
+            HIP_CHECK(hipStreamSynchronize(stream()));
+            w += k;
+        }
+    });
+    s->cur_len += n;
+    if (run) run->len = s->cur_len;
+    HIP_CHECK(hipStreamSynchronize(stream()));
+    return 0;
+}
+
 // A prompt, or a portion of one, for every sequence of the run, in as few steps as its scratch allows; the logits of the
 // last token stay in the run.
 void prefill_rows(InferenceState *s, BatchRun &r, const uint32_t *tokens, int n, int pos)
@@ -1075,6 +1341,13 @@ int inference_generate_batch(InferenceState *s, const uint32_t *prompt_tokens, i
     BatchRun &r = batch_acquire(s, s->batch, B);
     int tokens[32], next[32], active[32];
     if (s->stack) prefill_rows(s, r, prompt_tokens, prompt_len, 0);
+    else if (prompt_takes(s, prompt_len)) {                                   // once, into the first sequence's caches, and copied to the others
+        prompt_rows_all(s, prompt_tokens, prompt_len, r.kc, r.vc, r.logits);
+        for (int L = 0; L < s->NL; L++)
+            launch_copy_caches(dptr_as<float>(r.kc[L]), dptr_as<float>(r.vc[L]), B, s->Hkv, s->max_seq, s->hd, prompt_len);
+        for (int b = 1; b < B; b++)
+            HIP_CHECK(hipMemcpyAsync(dptr_as<float>(r.logits) + (size_t)b * s->V, dptr(r.logits), (size_t)s->V * 4, hipMemcpyDeviceToDevice, stream()));
+    }
     else for (int i = 0; i < prompt_len; i++) {                               // prefill: the same token for every sequence (:910-916)
         for (int b = 0; b < B; b++) tokens[b] = (int)prompt_tokens[i];
         forward_token_batch(s, r, tokens, i);

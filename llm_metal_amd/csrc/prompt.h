@@ -1,0 +1,62 @@
+// Many tokens of one sequence in one step, for the models whose decoding runs a token at a time (prompt.hip; the host side is
+// in inference.hip).  Every product reads its weight once for all of them on the matrix cores, with 22 bits of every fp32
+// activation kept (rows_to_f16_split); everything else is fp32.
+#pragma once
+#include "gemm.h"
+
+namespace lmhip {
+
+// A product as the GEMM leaves it: S planes of [2M, N], rows m and M + m the value and residual images of row m, inv their
+// factors.  P2 not null: S2 more planes of [M, N] of the value rows with what rounding the weights to fp16 lost, times 2^11.
+struct SplitPlanes {
+    const float *P, *inv;
+    size_t plane;
+    int S, N;
+    const float *P2;
+    size_t plane2;
+    int S2;
+};
+constexpr float Q8_RESIDUAL_SCALE = 2048.f;
+__device__ __forceinline__ float planes_at(const SplitPlanes &p, int M, int m, int n)
+{
+    float v = split_planes_value(p.P, p.S, p.plane, p.N, p.inv, M, m, n);
+    if (p.P2) {
+        float r = 0.f;
+        for (int s = 0; s < p.S2; s++) r += p.P2[s * p.plane2 + (size_t)m * p.N + n];
+        v = fmaf(r, p.inv[m] * (1.0f / Q8_RESIDUAL_SCALE), v);
+    }
+    return v;
+}
+
+// What follows the Q|K|V product for M tokens at positions pos .. pos + M - 1: adapter terms, per-head RMSNorm and RoPE; q to
+// [M][Hq * hd], k and v into the rows of the caches [Hkv, max_seq, hd].
+struct PromptHeads {
+    SplitPlanes qkv;                     // columns q | k | v, and the adapters' A_q x | A_v x behind them when t is null and R > 0
+    const float *g_q, *g_k;              // per-head norm gammas or null
+    const float *t, *Bq, *Bv;            // t [M][2R]
+    const float2 *rope;                  // (cos, sin) of position pos, hd / 2 pairs per position
+    float *q, *kc, *vc;
+    int M, Hq, Hkv, hd, R, pos, max_seq;
+    float eps, sc;
+};
+void launch_prompt_heads(const PromptHeads &a);
+
+// out [M][Hq * hd] = causal attention of the M queries at positions pos .. pos + M - 1 over the cache rows 0 .. pos + M - 1
+bool prompt_attention_supported(int hd);
+void launch_prompt_attention(const float *q, const float *kc, const float *vc, float *out, int M, int pos, int Hq, int Hkv, int hd, int max_seq);
+
+// rows m and M + m of the tiled operand a16 and their factors from act(gate) * up of the [gate | up] product
+bool prompt_glu_supported(int IS);
+void launch_prompt_glu(const SplitPlanes &gu, half_t *a16, float *inv, int M, int IS, int gelu);
+
+// x[m] = emb[ids[m]] * scale
+void launch_embed_ids(const float *emb, const int *ids, float scale, float *x, int M, int D);
+// positions 0 .. len - 1 of sequence 0's caches to sequences 1 .. B - 1; k, v: [B][Hkv, max_seq, hd]
+void launch_copy_caches(float *k, float *v, int B, int Hkv, int max_seq, int hd, int len);
+
+// infer_kernels.hip: a Q8_0 matrix as two tiled F16 images, half(d q) and 2^11 times what that rounding lost; 22 bits of d q
+void q8_to_tiled_pair(struct ::MetalBuf *W, int rows, int cols, half_t *hi, half_t *lo);
+// raises *out on the device, the bits of a float, to the largest |d| over the scales of a Q8_0 matrix (a NaN is above all)
+void q8_max_scale(struct ::MetalBuf *W, int rows, int cols, unsigned *out);
+
+}  // namespace lmhip

@@ -1,0 +1,372 @@
+// Kernels of a prompt's step: many tokens of one sequence at once (prompt.h).
+#include "backend.h"
+#include "devutil.h"
+#include "prompt.h"
+#include <stdio.h>
+
+using namespace lmhip;
+
+namespace {
+
+constexpr int TB = 256;
+
+__global__ __launch_bounds__(TB) void k_embed_ids(const float *__restrict__ emb, const int *__restrict__ ids, float scale, float *__restrict__ x, int D)
+{
+    const int i = blockIdx.x * TB + threadIdx.x, m = blockIdx.y;
+    if (i < D) x[(size_t)m * D + i] = emb[(size_t)ids[m] * D + i] * scale;
+}
+
+__global__ __launch_bounds__(TB) void k_copy_caches(float *__restrict__ k, float *__restrict__ v, size_t seq_step, size_t head_step, int n)
+{
+    const int i = blockIdx.x * TB + threadIdx.x;
+    if (i >= n) return;
+    float *c = blockIdx.z & 1 ? v : k;
+    const size_t at = (size_t)blockIdx.y * head_step + i;
+    c[(size_t)(1 + (blockIdx.z >> 1)) * seq_step + at] = c[at];
+}
+
+// One wave per (token, head); lane i owns the rotary pairs i and i + 64 of up to 256 values, as finish_head of the decoding
+// kernel does, with the same expressions.  Reads the product's planes (2 S loads per value) and writes each value once:
+// bound by those bytes, 25 MB at 500 tokens of the 4B shape.
+__global__ __launch_bounds__(TB) void k_prompt_heads(PromptHeads a)
+{
+    const int lane = threadIdx.x & 63, slot = blockIdx.x * 4 + (threadIdx.x >> 6), m = blockIdx.y;
+    if (slot >= a.Hq + 2 * a.Hkv) return;
+    const int kind = slot < a.Hq ? 0 : slot < a.Hq + a.Hkv ? 1 : 2;         // q, k, v
+    const int h = kind == 0 ? slot : kind == 1 ? slot - a.Hq : slot - a.Hq - a.Hkv;
+    const int hd = a.hd, half = hd / 2, nqkv = (a.Hq + 2 * a.Hkv) * hd;
+    float t = 0.f;                                                          // lane r < R: this token's A x, row r
+    const bool adapters = a.R > 0 && kind != 1;
+    if (adapters && lane < a.R) {
+        const int r = (kind == 0 ? 0 : a.R) + lane;
+        t = a.t ? a.t[(size_t)m * 2 * a.R + r] : planes_at(a.qkv, a.M, m, nqkv + r);
+    }
+    float x0[2] = {0.f, 0.f}, x1[2] = {0.f, 0.f};
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int i = lane + 64 * u;
+        if (i < half) { x0[u] = planes_at(a.qkv, a.M, m, slot * hd + i); x1[u] = planes_at(a.qkv, a.M, m, slot * hd + i + half); }
+        if (adapters) {
+            const float *B = (kind == 0 ? a.Bq : a.Bv) + (size_t)h * hd * a.R;
+            float d0 = 0.f, d1 = 0.f;
+            for (int r = 0; r < a.R; r++) {
+                const float tr = __shfl(t, r, 64);
+                if (i < half) { d0 = fmaf(B[(size_t)i * a.R + r], tr, d0); d1 = fmaf(B[(size_t)(i + half) * a.R + r], tr, d1); }
+            }
+            if (i < half) { x0[u] = fmaf(a.sc, d0, x0[u]); x1[u] = fmaf(a.sc, d1, x1[u]); }
+        }
+        ss += x0[u] * x0[u] + x1[u] * x1[u];
+    }
+    if (kind != 2) {
+        const float *g = kind == 0 ? a.g_q : a.g_k;
+        const float inv = g ? rsqrtf(wave_sum(ss) / (float)hd + a.eps) : 1.f;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int i = lane + 64 * u;
+            if (i >= half) continue;
+            if (g) { x0[u] *= inv * g[i]; x1[u] *= inv * g[i + half]; }
+            const float2 c = a.rope[(size_t)m * half + i];
+            const float r0 = x0[u] * c.x - x1[u] * c.y, r1 = x0[u] * c.y + x1[u] * c.x;
+            x0[u] = r0; x1[u] = r1;
+        }
+    }
+    float *dst = kind == 0 ? a.q + ((size_t)m * a.Hq + h) * hd : (kind == 1 ? a.kc : a.vc) + ((size_t)h * a.max_seq + a.pos + m) * hd;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int i = lane + 64 * u;
+        if (i < half) { dst[i] = x0[u]; dst[i + half] = x1[u]; }
+    }
+}
+
+// One (token, query head) by one wave, key by key, reading only what it sees: for rows beside which a later key's value is not
+// finite (below), where the tiles' zero probabilities would turn into NaN.
+template <int HD>
+__device__ __attribute__((noinline)) void attend_plain(const float *Q, const float *Kh, const float *Vh, float *out, int m, int head, int qpos, int Hq, float scale)
+{
+    constexpr int U = (HD + 63) / 64;
+    const int lane = threadIdx.x & 63;
+    const float *q = Q + ((size_t)m * Hq + head) * HD;
+    float o[U] = {}, mx = -3.0e38f, l = 0.f;
+    for (int j = 0; j <= qpos; j++) {
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; u++) if (lane + 64 * u < HD) s = fmaf(q[lane + 64 * u], Kh[(size_t)j * HD + lane + 64 * u], s);
+        s = wave_sum(s) * scale;
+        const float now = fmaxf(mx, s), keep = expf(mx - now), p = expf(s - now);
+        mx = now;
+        l = fmaf(l, keep, p);
+#pragma unroll
+        for (int u = 0; u < U; u++) if (lane + 64 * u < HD) o[u] = fmaf(o[u], keep, p * Vh[(size_t)j * HD + lane + 64 * u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) if (lane + 64 * u < HD) out[((size_t)m * Hq + head) * HD + lane + 64 * u] = o[u] / l;
+}
+
+// Attention in fp32 on the matrix cores (v_mfma_f32_32x32x2_f32: products and sums as exact as the decoding kernel's).
+// A workgroup serves 32 (token, query head) pairs of one key head -- row r of the key head is token r / G, head r % G of its
+// group, so a tile spans few positions whatever G is -- and its four waves take the key tiles in turn, 32 keys each, with a
+// running softmax of their own that the workgroup merges at the end: the chain of a wave is a quarter of the keys.  Scores are
+// formed transposed (keys x rows): a row is a lane, and the accumulator that holds a row's probabilities is, register by
+// register, the operand of the product with the values (the keys of a step are those the two lane halves hold), so nothing
+// passes through LDS until the merge.  Per tile 2 HD matrix instructions of 64 cycles: bound by them for long prompts
+// (a 2048-token one reads 17 MB of keys per 128 rows from L2), by the chain of one wave for short ones.
+template <int HD>
+__global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const float *__restrict__ Q, const float *__restrict__ Kc, const float *__restrict__ Vc,
+                                                                       float *__restrict__ out, int M, int pos, int Hq, int G, int max_seq, float scale)
+{
+    constexpr int CB = HD / 32, HH = HD / 2;
+    __shared__ float part[2][CB * 16][64];
+    __shared__ float st[4][2][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
+    const int kvh = blockIdx.y, rows = M * G, row0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 32;      // the longest first
+    const int r = min(row0 + col, rows - 1), m = r / G, head = kvh * G + r % G, qpos = pos + m;
+    const int first = pos + row0 / G, last = pos + min(row0 + 31, rows - 1) / G, tiles = last / 32 + 1;
+    const float *Kh = Kc + (size_t)kvh * max_seq * HD, *Vh = Vc + (size_t)kvh * max_seq * HD;
+
+    float4v q[HH / 4];                                     // columns half * HH .. of the lane's row
+    const float *qp = Q + ((size_t)m * Hq + head) * HD + half * HH;
+#pragma unroll
+    for (int i = 0; i < HH / 4; i++) q[i] = *reinterpret_cast<const float4v *>(qp + 4 * i);
+
+    float16v O[CB] = {};
+    float mx = -3.0e38f, l = 0.f, bad = 0.f;
+    for (int t = wave; t < tiles; t += 4) {
+        const float *kp = Kh + (size_t)min(t * 32 + col, last) * HD + half * HH;
+        float16v S = {};
+        float4v k[2][4];                                   // sixteen columns while the sixteen before are multiplied
+        auto keys = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) k[i & 1][e] = *reinterpret_cast<const float4v *>(kp + 16 * i + 4 * e);
+        };
+        keys(0);
+#pragma unroll
+        for (int i = 0; i < HH / 16; i++) {
+            if (i + 1 < HH / 16) keys(i + 1);
+            __builtin_amdgcn_sched_barrier(0);             // (all of a tile's loads together spill)
+#pragma unroll
+            for (int e = 0; e < 16; e++) S = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i & 1][e >> 2][e & 3], q[4 * i + (e >> 2)][e & 3], S, 0, 0, 0);
+        }
+        // value rows of four of the sixteen keys that the lane's half holds, keys 8 b + 4 half .. + 3 of the tile; the next
+        // four are requested while these are multiplied
+        float v[2][4][CB];
+        auto values = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float *vp = Vh + (size_t)min(t * 32 + 8 * b + 4 * half + e, last) * HD + col;
+#pragma unroll
+                for (int c = 0; c < CB; c++) v[b & 1][e][c] = vp[32 * c];
+            }
+        };
+        values(0);
+        float top = -3.0e38f;
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const bool seen = t * 32 + 8 * (j >> 2) + 4 * half + (j & 3) <= qpos;
+            S[j] = seen ? S[j] * scale : -INFINITY;
+            if (seen) top = fmaxf(top, S[j]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float now = fmaxf(mx, top), keep = expf(mx - now);
+        mx = now;
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; j++) { S[j] = expf(S[j] - now); sum += S[j]; }       // (a key that is not seen: 0)
+        l = fmaf(l, keep, sum);
+        if (__any(keep != 1.f)) {
+#pragma unroll
+            for (int c = 0; c < CB; c++)
+#pragma unroll
+                for (int j = 0; j < 16; j++) O[c][j] *= keep;
+        }
+        const bool partly = t * 32 + 31 > first;           // some rows do not see some keys of this tile
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            if (b < 3) values(b + 1);
+            if (partly) {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int c = 0; c < CB; c++) bad += v[b & 1][e][c] * 0.f;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int c = 0; c < CB; c++) O[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[b & 1][e][c], S[4 * b + e], O[c], 0, 0, 0);
+        }
+    }
+    if (__syncthreads_or(bad != 0.f)) {                    // a probability of zero has met an infinity or NaN
+        for (int i = wave; i < 32 && row0 + i < rows; i += 4) attend_plain<HD>(Q, Kh, Vh, out, (row0 + i) / G, kvh * G + (row0 + i) % G, pos + (row0 + i) / G, Hq, scale);
+        return;
+    }
+    l += __shfl_xor(l, 32, 64);
+    st[wave][0][lane] = mx; st[wave][1][lane] = l;
+    __syncthreads();
+    float all = st[0][0][lane];
+#pragma unroll
+    for (int w = 1; w < 4; w++) all = fmaxf(all, st[w][0][lane]);
+    float den = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) den = fmaf(st[w][1][lane], expf(st[w][0][lane] - all), den);
+    const float f = expf(mx - all);
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+#pragma unroll
+        for (int j = 0; j < 16; j++) O[c][j] *= f;
+    auto put = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CB; c++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) part[slot][c * 16 + j][lane] = O[c][j];
+    };
+    auto add = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CB; c++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) O[c][j] += part[slot][c * 16 + j][lane];
+    };
+    if (wave >= 2) put(wave - 2);
+    __syncthreads();
+    if (wave < 2) add(wave);
+    __syncthreads();
+    if (wave == 1) put(0);
+    __syncthreads();
+    if (wave != 0 || row0 + col >= rows) return;
+    add(0);
+    float *op = out + ((size_t)m * Hq + head) * HD + 4 * half;
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            float4v o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = O[c][4 * b + e] / den;
+            *reinterpret_cast<float4v *>(op + 32 * c + 8 * b) = o;
+        }
+}
+
+// One workgroup per token, the gated row in registers (C chunks of four columns per thread): the planes are read once and the
+// next product's operand leaves as two fp16 rows, where a gate kernel and a split kernel wrote and read the fp32 row between them.
+template <int C, int GELU>
+__global__ __launch_bounds__(1024) void k_prompt_glu(SplitPlanes gu, half_t *__restrict__ a16, float *__restrict__ inv, int M, int IS, int Kb)
+{
+    __shared__ float sm[16];
+    const int m = blockIdx.x;
+    float v[C][4];
+    float amax = 0.f;
+#pragma unroll
+    for (int u = 0; u < C; u++) {
+        const int n = (threadIdx.x + 1024 * u) * 4;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[u][e] = 0.f;
+        if (n < IS) {
+            auto four = [&](int at) __attribute__((always_inline)) {
+                const size_t ld = (size_t)gu.N;
+                const float *ph = gu.P + (size_t)m * ld + at, *pl = ph + (size_t)M * ld;
+                float4v hi = {}, lo = {};
+                for (int s = 0; s < gu.S; s++) {
+                    hi += *reinterpret_cast<const float4v *>(ph + s * gu.plane);
+                    lo += *reinterpret_cast<const float4v *>(pl + s * gu.plane);
+                }
+                const float ih = gu.inv[m], il = gu.inv[M + m];
+                float4v r;
+#pragma unroll
+                for (int e = 0; e < 4; e++) r[e] = fmaf(lo[e], il, hi[e] * ih);
+                if (gu.P2) {
+                    float4v z = {};
+                    for (int s = 0; s < gu.S2; s++) z += *reinterpret_cast<const float4v *>(gu.P2 + s * gu.plane2 + (size_t)m * ld + at);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) r[e] = fmaf(z[e], ih * (1.0f / Q8_RESIDUAL_SCALE), r[e]);
+                }
+                return r;
+            };
+            const float4v g = four(n), up = four(IS + n);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float act = GELU ? 0.5f * g[e] * (1.0f + tanhf(gelu_inner(g[e]))) : g[e] / (1.0f + expf(-g[e]));
+                v[u][e] = act * up[e];
+                amax = fmaxf(amax, fabsf(v[u][e]));
+            }
+        }
+    }
+    amax = block_max(amax, sm);
+    const float s = row_scale_for(amax), is = 1.0f / s;
+    float lmax = 0.f;
+#pragma unroll
+    for (int u = 0; u < C; u++) {
+        const int n = (threadIdx.x + 1024 * u) * 4;
+        half4 h;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            h[e] = f2h(v[u][e] * s);
+            v[u][e] -= h2f(h[e]) * is;
+            lmax = fmaxf(lmax, fabsf(v[u][e]));
+        }
+        if (n < Kb * 64) *reinterpret_cast<half4 *>(a16 + tiled_a_index(m, n, Kb)) = h;
+    }
+    lmax = block_max(lmax, sm);
+    const float s2 = row_scale_for(lmax);
+#pragma unroll
+    for (int u = 0; u < C; u++) {
+        const int n = (threadIdx.x + 1024 * u) * 4;
+        half4 h;
+#pragma unroll
+        for (int e = 0; e < 4; e++) h[e] = f2h(v[u][e] * s2);
+        if (n < Kb * 64) *reinterpret_cast<half4 *>(a16 + tiled_a_index(M + m, n, Kb)) = h;
+    }
+    if (threadIdx.x == 0) { inv[m] = is; inv[M + m] = 1.0f / s2; }
+}
+
+}  // namespace
+
+namespace lmhip {
+
+void launch_embed_ids(const float *emb, const int *ids, float scale, float *x, int M, int D)
+{
+    hipLaunchKernelGGL(k_embed_ids, dim3((D + TB - 1) / TB, M), dim3(TB), 0, stream(), emb, ids, scale, x, D);
+}
+
+void launch_copy_caches(float *k, float *v, int B, int Hkv, int max_seq, int hd, int len)
+{
+    if (B < 2) return;
+    const size_t head = (size_t)max_seq * hd;
+    hipLaunchKernelGGL(k_copy_caches, dim3((unsigned)(((size_t)len * hd + TB - 1) / TB), Hkv, 2 * (B - 1)), dim3(TB), 0, stream(), k, v, (size_t)Hkv * head, head, len * hd);
+}
+
+void launch_prompt_heads(const PromptHeads &a)
+{
+    if (a.M <= 0 || a.hd > 256 || (a.hd & 1) || a.R > 64 || a.pos < 0 || a.pos + a.M > a.max_seq) { fprintf(stderr, "[fast_hip] prompt_heads: unsupported shape\n"); abort(); }
+    hipLaunchKernelGGL(k_prompt_heads, dim3((a.Hq + 2 * a.Hkv + 3) / 4, a.M), dim3(TB), 0, stream(), a);
+}
+
+bool prompt_attention_supported(int hd) { return hd == 32 || hd == 64 || hd == 128 || hd == 256; }
+
+void launch_prompt_attention(const float *q, const float *kc, const float *vc, float *out, int M, int pos, int Hq, int Hkv, int hd, int max_seq)
+{
+    if (M <= 0 || pos < 0 || pos + M > max_seq || Hkv <= 0 || Hq % Hkv || (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)out) & 15)) {
+        fprintf(stderr, "[fast_hip] prompt_attention: unsupported shape\n"); abort();
+    }
+    const int G = Hq / Hkv;
+    const dim3 grid((M * G + 31) / 32, Hkv);
+    const float scale = 1.0f / sqrtf((float)hd);
+#define PA(HD_) hipLaunchKernelGGL(k_prompt_attn<HD_>, grid, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale)
+    if (hd == 32) PA(32); else if (hd == 64) PA(64); else if (hd == 128) PA(128); else if (hd == 256) PA(256);
+    else { fprintf(stderr, "[fast_hip] prompt_attention: unsupported head size %d\n", hd); abort(); }
+#undef PA
+}
+
+bool prompt_glu_supported(int IS) { return IS % 4 == 0 && tiled_kb(IS) * 64 <= 16384; }
+
+void launch_prompt_glu(const SplitPlanes &gu, half_t *a16, float *inv, int M, int IS, int gelu)
+{
+    if (!prompt_glu_supported(IS) || gu.N % 4 || gu.N < 2 * IS || (gu.plane | gu.plane2) % 4 || ((uintptr_t)gu.P | (uintptr_t)gu.P2) & 15) {
+        fprintf(stderr, "[fast_hip] prompt_glu: unsupported shape %d\n", IS); abort();
+    }
+    const int Kb = tiled_kb(IS), C = (Kb * 16 + 1023) / 1024;
+#define PG(C_) do { if (gelu) hipLaunchKernelGGL((k_prompt_glu<C_, 1>), dim3(M), dim3(1024), 0, stream(), gu, a16, inv, M, IS, Kb); \
+                    else hipLaunchKernelGGL((k_prompt_glu<C_, 0>), dim3(M), dim3(1024), 0, stream(), gu, a16, inv, M, IS, Kb); } while (0)
+    if (C == 1) PG(1); else if (C == 2) PG(2); else if (C == 3) PG(3); else PG(4);
+#undef PG
+}
+
+}  // namespace lmhip

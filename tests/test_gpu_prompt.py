@@ -1,0 +1,113 @@
+"""Prompts taken many tokens per step (inference_forward_tokens, the prefill of inference_generate and _generate_batch) against
+the same tokens one by one, which the other tests hold to the oracle.  Both keep fp32 (22 bits in the products' operands), so
+they agree to about sqrt(layers) ulps of the largest logit: 2e-5 leaves a factor of ten."""
+import numpy as np
+import pytest
+
+from llm_metal_amd.configs import C1, GEMMA3, QWEN3, SFTConfig
+from llm_metal_amd.sft import InferenceState, SFTState
+from llm_metal_amd.synth import make_batch, make_model
+from tests.gpu_util import maxrel
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-5
+SHAPES = [
+    SFTConfig("hd32_group4", QWEN3, NL=2, D=160, Hq=8, Hkv=2, hd=32, IS=416, V=512),
+    SFTConfig("hd64_group3", QWEN3, NL=2, D=192, Hq=3, Hkv=1, hd=64, IS=352, V=516),
+    SFTConfig("hd128_group1", QWEN3, NL=2, D=288, Hq=2, Hkv=2, hd=128, IS=608, V=512),
+    SFTConfig("hd128_group16", QWEN3, NL=1, D=256, Hq=16, Hkv=1, hd=128, IS=4224, V=512),
+    SFTConfig("hd256_gemma", GEMMA3, NL=7, D=128, Hq=4, Hkv=1, hd=256, IS=256, V=512, tied=True),
+    SFTConfig("hd16_one_by_one", QWEN3, NL=1, D=128, Hq=4, Hkv=2, hd=16, IS=256, V=512),
+]
+
+
+def tokens(c, n, seed):
+    return [int(t) for t in np.random.default_rng(seed).integers(0, c.V, n)]
+
+
+def one_by_one(inf, toks):
+    inf.reset()
+    return np.stack([inf.forward_token(t) for t in toks])
+
+
+@pytest.mark.parametrize("n", [2, 7, 31, 33, 65, 130, 300])
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+@pytest.mark.parametrize("c", SHAPES, ids=lambda c: c.name)
+def test_prompt_equals_tokens_one_by_one(c, fmt, n):
+    print(c.name, fmt, n, flush=True)
+    model, toks = make_model(c, seed=3, gamma_jitter=0.1), tokens(c, n + 3, n)
+    with InferenceState(c, model, max_seq=n + 3, use_fp16=fmt == "f16") as inf:
+        want = one_by_one(inf, toks)
+        inf.reset()
+        got = inf.forward_tokens(toks[:n], range(n))
+        assert inf.position() == n and maxrel(got, want[:n]) < TOL
+        # decoding goes on from the caches the prompt left, and so does a further portion
+        assert maxrel(inf.forward_token(toks[n]), want[n]) < TOL
+        assert maxrel(inf.forward_tokens(toks[n + 1:], [1]), want[-1:]) < TOL
+        cut = max(1, n // 3)
+        inf.reset()
+        inf.forward_tokens(toks[:cut])
+        assert maxrel(inf.forward_tokens(toks[cut:n], [n - cut - 1]), want[n - 1:n]) < TOL
+
+
+def test_prompt_of_several_steps():
+    c = C1.with_(name="long", NL=1, V=256)
+    model, toks = make_model(c, seed=4), tokens(c, 2500, 5)
+    at = [0, 832, 833, 1024, 1666, 1667, 2499]
+    with InferenceState(c, model, max_seq=2500) as inf:
+        want = one_by_one(inf, toks)[at]
+        inf.reset()
+        assert maxrel(inf.forward_tokens(toks, at), want) < TOL
+
+
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+def test_prompt_with_adapters(fmt):
+    """On a training state's tiles (adapter rows inside the fused matrix) and on own weights with its adapters attached."""
+    c = C1.with_(weight_format=fmt)
+    model, toks = make_model(c, seed=6, gamma_jitter=0.1), tokens(c, 70, 7)
+    with SFTState(c, model) as sft:
+        sft.train_step(*make_batch(c, seed=8), 1e-3)
+        with InferenceState(sft=sft, max_seq=80) as shared, InferenceState(c, model, max_seq=80, use_fp16=fmt == "f16") as own:
+            own.attach_lora(sft)
+            for inf in (shared, own):
+                want = one_by_one(inf, toks)
+                inf.reset()
+                assert maxrel(inf.forward_tokens(toks, range(70)), want) < TOL
+                assert maxrel(inf.forward_token(toks[0]), inf.forward_token(toks[0])) < 1.0     # goes on
+
+
+def test_generation_from_prompts():
+    c = C1
+    model, prompt = make_model(c, seed=9, gamma_jitter=0.1), tokens(C1, 45, 10)
+    with InferenceState(c, model, max_seq=64) as inf:
+        inf.set_eos([c.V - 1])
+        nxt, want = int(one_by_one(inf, prompt)[-1].argmax()), []
+        for _ in range(10):
+            want.append(nxt)
+            nxt = inf.forward_token_argmax(nxt)
+        assert list(inf.generate(prompt, 10)) == want
+        assert [list(r) for r in inf.generate_batch(prompt, 10, 3)] == [want] * 3
+        assert list(inf.generate(prompt[:5] + [c.V], 4)) == [] and inf.position() == 5
+
+
+def test_infinite_values_stay_with_later_tokens():
+    c = SHAPES[2].with_(NL=1)
+    model, toks = make_model(c, seed=11), list(range(50))
+    with InferenceState(c, model, max_seq=50) as inf:
+        want = inf.forward_tokens(toks, range(50))
+    model["token_emb"][20] = np.inf
+    with InferenceState(c, model, max_seq=50) as inf:
+        got = inf.forward_tokens(toks, range(50))
+    assert maxrel(got[:20], want[:20]) < TOL and np.isfinite(got[:20]).all()
+    assert not np.isfinite(got[20:]).any()
+
+
+def test_q8_weights_beyond_a_half_take_tokens_one_by_one():
+    c = SHAPES[2].with_(NL=1)
+    model = make_model(c, seed=12)
+    model["wd"][0] *= 1e7                                  # code times scale beyond 65504
+    toks = tokens(c, 40, 13)
+    with InferenceState(c, model, max_seq=40, use_fp16=False) as inf:
+        want = one_by_one(inf, toks)
+        inf.reset()
+        assert np.isfinite(want).all() and np.array_equal(inf.forward_tokens(toks, range(40)), want)
