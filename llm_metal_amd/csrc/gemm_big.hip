@@ -232,19 +232,22 @@ __global__ __launch_bounds__(256) void gemm_big(GemmKArgs g)
             }
         return;
     }
+    // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
+    const EdgeStore edge(g.P + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
+    uint32_t col[NW];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int k = 0; k < NW; k++) { const int n = (nb0 + NW * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int m = (mb0 + 2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m >= g.M) continue;
-            const float sc = g.a_inv_scale ? g.a_inv_scale[m] : 1.0f;
+    for (int i = 0; i < 2; i++) {
+        float sc[16];
 #pragma unroll
-            for (int k = 0; k < NW; k++) {
-                const int n = (nb0 + NW * wn + k) * 32 + r;
-                if (n < g.N) g.P[(size_t)m * g.ldp + n] = acc[i][k][v] * sc;
-            }
-        }
+        for (int v = 0; v < 16; v++)
+            sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+#pragma unroll
+            for (int k = 0; k < NW; k++) edge.f32((2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+    }
 }
 
 
@@ -394,19 +397,22 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
             }
         return;
     }
+    // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
+    const EdgeStore edge(Cp + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
+    uint32_t col[4];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int m = (mb0 + 2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m >= g.M) continue;
-            const float sc = g.a_inv_scale ? g.a_inv_scale[m] : 1.0f;
+    for (int i = 0; i < 2; i++) {
+        float sc[16];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int n = (nb0 + 4 * wn + k) * 32 + r;
-                if (n < g.N) Cp[(size_t)m * g.ldp + n] = acc[i][k][v] * sc;
-            }
-        }
+        for (int v = 0; v < 16; v++)
+            sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) edge.f32((2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+    }
 }
 
 
@@ -545,19 +551,22 @@ __global__ __launch_bounds__(256) void gemm_big_f16_256(GemmKArgs g)
             }
         return;
     }
+    // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
+    const EdgeStore edge(Cp + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
+    uint32_t col[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int m = (mb0 + 4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m >= g.M) continue;
-            const float sc = g.a_inv_scale ? g.a_inv_scale[m] : 1.0f;
+    for (int i = 0; i < 4; i++) {
+        float sc[16];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int n = (nb0 + 4 * wn + k) * 32 + r;
-                if (n < g.N) Cp[(size_t)m * g.ldp + n] = acc[i][k][v] * sc;
-            }
-        }
+        for (int v = 0; v < 16; v++)
+            sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) edge.f32((4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+    }
 }
 
 // The 256 x 256 block over Q8_0 weight tiles that stay quantised all the way into LDS: the dequant-fused product for
@@ -761,19 +770,22 @@ __global__ __launch_bounds__(256) void gemm_big_q8(GemmKArgs g)
             }
         return;
     }
+    // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
+    const EdgeStore edge(Cp + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
+    uint32_t col[4];
 #pragma unroll
-    for (int i = 0; i < MI; i++)
+    for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int m = (mb0 + MI * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m >= g.M) continue;
-            const float sc = g.a_inv_scale ? g.a_inv_scale[m] : 1.0f;
+    for (int i = 0; i < MI; i++) {
+        float sc[16];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int n = (nb0 + 4 * wn + k) * 32 + r;
-                if (n < g.N) Cp[(size_t)m * g.ldp + n] = acc[i][k][v] * sc;
-            }
-        }
+        for (int v = 0; v < 16; v++)
+            sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + MI * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) edge.f32((MI * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+    }
 }
 
 }  // namespace

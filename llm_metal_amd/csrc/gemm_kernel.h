@@ -89,6 +89,31 @@ __device__ __forceinline__ void load_w_q8_cols(half8 (&w)[4], const WeightOp &W,
     w[3] = q8_unpack8(r1[2], r1[3]) * s3;
 }
 
+// Stores of a tile that reaches past the matrix.  Under a test per element the compiler branches around every store and drains
+// the queue before it -- 12 to 15 us per launch of the large-M kernels (250 rows: 33 us on 6176 x 2560 against 18 at 256,
+// whose tiles lie inside).  Here nothing branches: the stores go through a buffer descriptor that ends with the matrix's last
+// row, and an element in a column past the end gets an offset past that end; the hardware drops what lies outside.
+struct EdgeStore {
+    __amdgpu_buffer_rsrc_t window;
+    int row_bytes;
+    // base: the tile's first row; rows: of the matrix from there on (a tile has at most 256); ld: row stride
+    template <typename T> __device__ __forceinline__ EdgeStore(T *base, int rows, int ld)
+    {
+        row_bytes = ld * (int)sizeof(T);
+        const size_t n = (size_t)min(rows, 256) * (size_t)row_bytes;
+        window = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(n < 0x7fffffff ? n : 0x7fffffff), 0x00020000);
+    }
+    static __device__ __forceinline__ uint32_t column(bool in, int bytes) { return in ? (uint32_t)bytes : 0x80000000u; }
+    __device__ __forceinline__ void f32(int row, uint32_t col, float v) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), window, (uint32_t)(row * row_bytes) + col, 0, 0);
+    }
+    __device__ __forceinline__ void f16(int row, uint32_t col, half_t v) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, v), window, (uint32_t)(row * row_bytes) + col, 0, 0);
+    }
+};
+
 // First register of the segment that wave w of nw still holds after `rounds` rounds of the accumulator exchange (see the
 // end of gemm_tiled): every round halves the segment, the wave whose bit nw >> (round + 1) is set keeps the upper half.
 __host__ __device__ constexpr int exchange_seg_lo(int regs, int nw, int w, int rounds)
@@ -243,10 +268,10 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_tiled(GemmKArgs g)
                 Pp[(size_t)m * g.ldp + n] = sres[k]; \
             } \
         } else { \
+            const EdgeStore edge(Pp + (size_t)mb0 * 32 * g.ldp, M - mb0 * 32, g.ldp); \
             _Pragma("unroll") for (int k = 0; k < Q; k++) { \
-                const int i = i0 + k, mb = i / (NB * 16), b = (i / 16) % NB, v = i % 16; \
-                const int m = (mb0 + mb) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), n = (nb0 + b) * 32 + r; \
-                if (m < M && n < N) Pp[(size_t)m * g.ldp + n] = sres[k]; \
+                const int i = i0 + k, mb = i / (NB * 16), b = (i / 16) % NB, v = i % 16, n = (nb0 + b) * 32 + r; \
+                edge.f32(mb * 32 + 8 * (v >> 2) + 4 * h + (v & 3), EdgeStore::column(n < N, n * 4), sres[k]); \
             } \
         } } }
     ALL_WAVES(PART_STORE, 0)
@@ -421,10 +446,14 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
     const bool inside = 64 <= g.M && (tile + 1) * 64 <= g.N;
     if constexpr (HALFP) {
         half_t *Ph = reinterpret_cast<half_t *>(g.P) + (size_t)chunk * g.plane_stride;
+        if (inside) {
 #pragma unroll
-        for (int k = 0; k < Q; k++) {
-            const int v = kg * Q + k, m = qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (inside || (m < g.M && n < g.N)) Ph[(size_t)m * g.ldp + n] = f2h(res[k] * g.half_scale);
+            for (int k = 0; k < Q; k++) { const int v = kg * Q + k; Ph[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = f2h(res[k] * g.half_scale); }
+        } else {
+            const EdgeStore edge(Ph, g.M, g.ldp);
+            const uint32_t col = EdgeStore::column(n < g.N, n * 2);
+#pragma unroll
+            for (int k = 0; k < Q; k++) { const int v = kg * Q + k; edge.f16(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, f2h(res[k] * g.half_scale)); }
         }
         return;
     }
@@ -440,11 +469,10 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
 #pragma unroll
         for (int k = 0; k < Q; k++) { const int v = kg * Q + k; Pp[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = res[k]; }
     } else {
+        const EdgeStore edge(Pp, g.M, g.ldp);
+        const uint32_t col = EdgeStore::column(n < g.N, n * 4);
 #pragma unroll
-        for (int k = 0; k < Q; k++) {
-            const int v = kg * Q + k, m = qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (m < g.M && n < g.N) Pp[(size_t)m * g.ldp + n] = res[k];
-        }
+        for (int k = 0; k < Q; k++) { const int v = kg * Q + k; edge.f32(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, res[k]); }
     }
 }
 
@@ -582,20 +610,30 @@ __global__ __launch_bounds__(512) void gemm_ring_wide(KARGS24)
     const bool inside = 64 <= g.M && (tile + 1) * 32 * WB <= g.N;
     if constexpr (HALFP) {
         half_t *Ph = reinterpret_cast<half_t *>(g.P) + (size_t)chunk * g.plane_stride;
+        if (inside) {
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int m = qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (inside || (m < g.M && n < g.N)) Ph[(size_t)m * g.ldp + n] = f2h(acc[v] * g.half_scale);
+            for (int v = 0; v < 16; v++) Ph[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = f2h(acc[v] * g.half_scale);
+        } else {
+            const EdgeStore edge(Ph, g.M, g.ldp);
+            const uint32_t col = EdgeStore::column(n < g.N, n * 2);
+#pragma unroll
+            for (int v = 0; v < 16; v++) edge.f16(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, f2h(acc[v] * g.half_scale));
         }
         return;
     }
     float *Pp = g.P + (size_t)chunk * g.plane_stride;
+    if (SCALE) {
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int m = qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        float o = acc[v];
-        if (SCALE) o *= g.a_inv_scale[min(m, g.M - 1)];
-        if (inside || (m < g.M && n < g.N)) Pp[(size_t)m * g.ldp + n] = o;
+        for (int v = 0; v < 16; v++) acc[v] *= g.a_inv_scale[min(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)];
+    }
+    if (inside) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) Pp[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = acc[v];
+    } else {
+        const EdgeStore edge(Pp, g.M, g.ldp);
+        const uint32_t col = EdgeStore::column(n < g.N, n * 4);
+#pragma unroll
+        for (int v = 0; v < 16; v++) edge.f32(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, acc[v]);
     }
 }
 
