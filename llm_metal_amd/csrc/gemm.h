@@ -134,8 +134,9 @@ int launch_gemm_big(const half_t *A_tiled, const float *a_inv_scale, const Weigh
 // first group_of[M / 128] blocks have rows (the rest of C is not written).  M is a multiple of 128; `groups`: how many weights.
 void launch_gemm_groups(const half_t *A_tiled, const float *a_inv_scale, const half_t *W_tiled, size_t group_stride, const int *group_of,
                         float *C, int ldc, int M, int N, int K, int groups);
-// true when the large-M kernel is the faster one for this product
-bool use_big_gemm(int M, int N, int K, int fmt);
+// true when the large-M kernel is the faster one for this product; one_plane: its result is wanted in one plane
+bool use_big_gemm(int M, int N, int K, int fmt, bool one_plane = false);
+bool mid_takes_big(int M, int N, int K, bool one_plane);   // the part of that rule for 65 to 1023 rows on F16 tiles (gemm_big.hip)
 // Q8_0 blocks in the reference's row-major layout ([rows][cols/32] blocks of 34 bytes) -> kernel tiles.
 // Element (r, c) goes to tiled (row_off + r, k_off + c) with row scales (fmt 1), or, transposed, to
 // (row_off + c, k_off + r) with column scales (fmt 2).  Kb_dst = K blocks per row block of the destination.

@@ -280,6 +280,12 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
         const int total = group.of[MT] * NT, share = (total + 7) >> 3, seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * share + seq;
         if (seq >= share || t >= total) return;
         mt = t / NT; nt = t % NT;
+    } else if (g.m_tiles) {
+        // few row blocks: those of one (column block, chunk) are consecutive workgroups of one XCD, so a weight tile comes
+        // from memory once; the pairs are dealt to the XCDs in turn
+        const int slot = blockIdx.x >> 3, pair = (slot / MT) * 8 + (blockIdx.x & 7);
+        if (pair >= NT * g.S) return;
+        mt = slot % MT; nt = pair % NT; chunk = pair / NT;
     } else if (g.S > 1) {
         const int t = blockIdx.x % (MT * NT);
         chunk = blockIdx.x / (MT * NT); mt = t % MT; nt = t / MT;
@@ -435,7 +441,13 @@ __global__ __launch_bounds__(256) void gemm_big_f16_256(GemmKArgs g)
     const int MT = (g.M + 255) >> 8, NT = (g.N + 255) >> 8;
     const int m_patches = (MT + 7) >> 3;
     int mt, nt, chunk = 0;
-    if (g.S > 1) {
+    if (g.m_tiles) {
+        // few row blocks: those of one (column block, chunk) are consecutive workgroups of one XCD, so a weight tile comes
+        // from memory once; the pairs are dealt to the XCDs in turn
+        const int slot = blockIdx.x >> 3, pair = (slot / MT) * 8 + (blockIdx.x & 7);
+        if (pair >= NT * g.S) return;
+        mt = slot % MT; nt = pair % NT; chunk = pair / NT;
+    } else if (g.S > 1) {
         const int t = blockIdx.x % (MT * NT);
         chunk = blockIdx.x / (MT * NT); mt = t % MT; nt = t / MT;
     } else {
@@ -790,6 +802,43 @@ __global__ __launch_bounds__(256) void gemm_big_q8(GemmKArgs g)
 
 }  // namespace
 
+// Products of 65 to 1023 rows on F16 tiles: which of the three kernels, and how many K chunks.  None of them wins over the
+// whole range -- the streaming kernel pulls every activation tile through each CU's registers (1.65 us per GFLOP), the large-M
+// blocks pay for their prologue, for CUs without a block and for rows a block does not have -- so the planner adds up what each
+// would take and picks the least.  Microseconds, fitted on MI355X to 16 shapes (1152 .. 32768 columns, K 1024 .. 32768; Qwen3-4B and
+// Gemma3-1B layers forward and backward) at 72 .. 1000 rows with cold weights, 5 to 8 % rms; a plane's bytes count once more for
+// the consumer that reads them.  The choice is within 2 % of the best of all measured ones over these shapes, 34 % below the
+// streaming kernel alone: 6176 x 2560 at 250 rows 26.7 -> 19.5 us, 19456 x 2560 64 -> 36, 2560 x 19456 at 500 rows 102 -> 56.
+namespace {
+struct MidPlan { int big, wide, chunks; };
+double mid_big_us(int wide, int M, int N, int K, int S, int cus)
+{
+    const int bm = wide ? 256 : 128, Kb = tiled_kb(K), steps = (Kb + S - 1) / S;
+    S = (Kb + steps - 1) / steps;
+    const long mt = (M + bm - 1) / bm, nt = (N + 255) / 256, per_xcd = ((nt * S + 7) / 8) * mt;    // (the dealing of m_tiles below)
+    const long rounds = (per_xcd + cus / 8 - 1) / (cus / 8);
+    const double busy = (double)(mt * nt * S) / ((double)rounds * cus), plane_mb = (double)S * M * N * 4e-6;
+    if (wide) return 1.6 + rounds * (7.5 + steps * (1.04 + 0.65 * busy)) + (0.144 + 0.2) * plane_mb;
+    return 3.9 + rounds * (2.6 + steps * (0.73 + 0.23 * busy)) + (0.23 + 0.2) * plane_mb;
+}
+MidPlan mid_plan(int M, int N, int K, bool one_plane)
+{
+    const int cus = num_cus() > 0 ? num_cus() : 256, Kb = tiled_kb(K);
+    const GemmPlan t = plan_gemm(M, N, K);
+    // (a single plane from a streaming product that leaves several: one more pass over them)
+    double best = 5.1 + 0.152 * (2e-6 * N * K) + 1.65 * (2e-9 * M * N * K) + (0.115 + (one_plane && t.S == 1 ? 0.0 : 0.2)) * (4e-6 * t.S * M * N);
+    MidPlan p{0, 0, 1};
+    for (int wide = 0; wide < 2; wide++)
+        for (int S = 1; S <= (one_plane ? 1 : 20) && S * 4 <= Kb; S++) {
+            const double us = mid_big_us(wide, M, N, K, S, cus) - (one_plane ? 0.2 * (4e-6 * M * N) : 0.0);
+            if (us < best) { best = us; p = MidPlan{1, wide, S}; }
+        }
+    return p;
+}
+bool mid_rows(int M, int fmt) { return fmt == 0 && M > 64 && M < 1024; }
+}  // namespace
+bool mid_takes_big(int M, int N, int K, bool one_plane) { return mid_plan(M, N, K, one_plane).big != 0; }
+
 // How many K chunks the large-M kernel should cut a product with F16 tiles into: three when its 128 x 256 output blocks
 // would leave a third of the CUs or more without work and K is at least 4096, else one.  Measured on MI355X at 2048
 // rows: the products with 2560 output columns (160 blocks for 256 CUs) go from 66 / 140 / 281 / 93 us to 54 / 103 /
@@ -799,6 +848,7 @@ int big_gemm_chunks(int M, int N, int K, int fmt)
 {
     if (fmt != 0 || g_big_split == 0) return 1;
     if (g_big_split > 1) return g_big_split;
+    if (mid_rows(M, fmt)) return mid_plan(M, N, K, false).chunks;
     const long blocks = (long)((M + 127) / 128) * ((N + 128 * WPW - 1) / (128 * WPW));
     const int cus = num_cus() > 0 ? num_cus() : 256;
     // a handful of blocks over a very long K (the LM head's backward at a few hundred rows: 25 blocks, K = 262 144): as
@@ -853,6 +903,7 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
     g.M = M; g.N = N; g.Mb = Mb; g.Nb = Nb; g.Kb = Kb;
     g.steps_per_chunk = (Kb + chunks - 1) / chunks;
     g.S = (Kb + g.steps_per_chunk - 1) / g.steps_per_chunk;
+    g.m_tiles = mid_rows(M, W.fmt) || (W.fmt == 0 && M <= 64);
     const dim3 block(256);
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     const bool prof = gemm_prof_begin(weight_stream_bytes(W, N, K), 2.0 * M * N * K, &ev_a, &ev_b);
@@ -860,6 +911,7 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
     // the kernels), the ids past the matrix returning at once
     auto grid_of = [&](const GemmKArgs &a, int bm, int bn) {
         const int mt = (a.M + bm - 1) / bm, nt = (a.N + bn - 1) / bn;
+        if (a.m_tiles) return dim3(8 * mt * ((nt * a.S + 7) / 8));
         return dim3(a.S > 1 ? mt * nt * a.S : 8 * 32 * ((mt + 7) / 8) * (((nt + 7) / 8 + 3) / 4));
     };
     if (W.fmt == 0 || q8_wide) {
@@ -875,7 +927,9 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
         };
         const bool deep = g.steps_per_chunk >= 20;
         // (Q8_0 tiles: the wide block only, see gemm_big_q8)
-        const bool wide = W.fmt != 0 || g_big_block == 2 || (g_big_block == 0 && deep && share(256, 256) >= 0.9 * share(128, 128 * WPW));
+        const bool mid = mid_rows(M, W.fmt);
+        const bool wide = W.fmt != 0 || g_big_block == 2 || (g_big_block == 0 && mid && mid_big_us(1, M, N, K, g.S, cus) < mid_big_us(0, M, N, K, g.S, cus)) ||
+                          (g_big_block == 0 && !mid && deep && share(256, 256) >= 0.9 * share(128, 128 * WPW));
         // A product of at least one full round of wide blocks whose last round would be half empty or less: the columns
         // of the full rounds go to wide blocks, the rest to 128 x 256 blocks in a launch of their own
         const int MX = (M + 255) / 256, NX = (N + 255) / 256, full = MX * NX / cus, rest = MX * NX % cus;
@@ -893,7 +947,7 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
             else BIG_LAUNCH((gemm_big_q8<2, 256>));
 #undef BIG_LAUNCH
         };
-        if (g_big_block == 0 && !wide && deep && g.S == 1 && full >= 1 && rest > 0 && rest * 2 <= cus && wide_cols < N) {
+        if (g_big_block == 0 && !wide && !mid && deep && g.S == 1 && full >= 1 && rest > 0 && rest * 2 <= cus && wide_cols < N) {
             GemmKArgs g1 = g, g2 = g;
             const int rb = wide_cols / 32;                 // weight row blocks that go to the wide launch
             g1.N = wide_cols; g1.Nb = rb;

@@ -200,7 +200,8 @@ size_t max_planes_elems(SFTState *s)
         // whichever kernel the product takes (the choice can be forced at run time): the planes of the streaming kernel, or
         // up to four K chunks of the large-M one; the LM head writes the logits directly unless the streaming kernel splits K
         const bool head = sh.N == s->V && sh.K == s->D;
-        const size_t e = (size_t)(head ? (p.S > 1 ? p.S : 0) : std::max({p.S, 4, big_gemm_chunks(s->BN, sh.N, sh.K, 0)})) * s->BN * sh.N;
+        const int chunks = big_gemm_chunks(s->BN, sh.N, sh.K, 0), most = std::max(p.S, chunks);
+        const size_t e = (size_t)(head ? (most > 1 ? most : 0) : std::max(most, 4)) * s->BN * sh.N;
         if (e > mx) mx = e;
     }
     set_gemm_ring(ring_was);
@@ -216,8 +217,14 @@ constexpr int MAX_SCALE_GROUPS = 64;                      // group_inv holds thi
 ScaleGroups scale_groups_for(SFTState *s, const WeightOp &W, int N, int K)
 {
     ScaleGroups none{0, 1, 0};
-    if (s->full_param || use_big_gemm(s->BN, N, K, W.fmt)) return none;      // weight gradients take one factor per row
-    const GemmPlan p = plan_gemm(s->BN, N, K, (W.fmt == 1 && W.nbq < tiled_rb(N)) ? W.nbq : 0, W.fmt);
+    if (s->full_param) return none;                       // weight gradients take one factor per row
+    GemmPlan p{};
+    if (use_big_gemm(s->BN, N, K, W.fmt)) {
+        if (s->BN >= 1024) return none;
+        const int chunks = big_gemm_chunks(s->BN, N, K, W.fmt), Kb = tiled_kb(K);
+        p.steps = (Kb + chunks - 1) / chunks;
+        p.S = (Kb + p.steps - 1) / p.steps;
+    } else p = plan_gemm(s->BN, N, K, (W.fmt == 1 && W.nbq < tiled_rb(N)) ? W.nbq : 0, W.fmt);
     const int plane_cols = p.steps * 64, cus = num_cus() > 0 ? num_cus() : 256;
     const int want = (2 * cus + s->BN - 1) / s->BN;
     if (p.S <= 1 || want <= 1 || plane_cols > 4096) return none;
@@ -320,14 +327,20 @@ float half_scale_for(SFTState *s, int kind, int L, bool T)
 Planes gemm(SFTState *s, const half_t *A, const float *inv, const WeightOp &W, int N, int K, float *out = nullptr,
             const ScaleGroups *sg = nullptr, float hscale = 0.f)
 {
-    if (use_big_gemm(s->BN, N, K, W.fmt)) {                 // one launch; final output, or a few K chunks as planes
+    if (use_big_gemm(s->BN, N, K, W.fmt, out != nullptr)) { // one launch; final output, or a few K chunks as planes
         float *C = out ? out : at<float>(s->planes);
         const WeightOp Wf = resident_image(s, W, N, K);
         const int chunks = out ? 1 : big_gemm_chunks_for(s->BN, N, K, Wf);
         const size_t stride = (size_t)s->BN * N;
         if (!out && chunks * stride > s->planes_cap) { fprintf(stderr, "[fast_sft] plane buffer too small\n"); abort(); }
-        const int planes = launch_gemm_big(A, inv, Wf, C, N, s->BN, N, K, chunks, stride);
-        return make_planes(C, planes, stride, N, nullptr);
+        const bool groups = sg && sg->cols;
+        const int planes = launch_gemm_big(A, groups ? nullptr : inv, Wf, C, N, s->BN, N, K, chunks, stride);
+        if (!groups) return make_planes(C, planes, stride, N, nullptr);
+        const int steps = (tiled_kb(K) + chunks - 1) / chunks;
+        if (out || sg->cols != (steps * 64) << sg->shift || sg->groups != (planes + (1 << sg->shift) - 1) >> sg->shift) {
+            fprintf(stderr, "[fast_sft] column groups of the operand do not match the K chunks of the product\n"); abort();
+        }
+        return make_planes(C, planes, stride, N, inv, sg->shift, sg->groups);
     }
     GemmPlan p = plan_gemm(s->BN, N, K, (W.fmt == 1 && W.nbq < tiled_rb(N)) ? W.nbq : 0, W.fmt);
     float *P = out ? out : at<float>(s->planes);
@@ -437,7 +450,8 @@ void forward_impl(SFTState *s, bool gather, bool zero_rows = false)
         // layout: the large-M kernel writes it there, the streaming kernel's planes are summed into it by the GLU kernel
         float *gu_keep = at<float>(s->gu_sav, (size_t)L * BN * 2 * IS);
         const WeightOp wgu = wop(s, W_GU, L, false);
-        const bool direct = use_big_gemm(BN, 2 * IS, D, wgu.fmt);
+        // (below 1024 rows only where one K chunk is the best plan: the planes of several cost less than idle CUs do)
+        const bool direct = use_big_gemm(BN, 2 * IS, D, wgu.fmt, true) && (BN >= 1024 || big_gemm_chunks(BN, 2 * IS, D, wgu.fmt) == 1);
         Planes pg = gemm(s, ln2, ln2inv, wgu, 2 * IS, D, direct ? gu_keep : nullptr, nullptr, half_scale_for(s, W_GU, L, false));
         GluArgs ga{};
         ga.in = pg; ga.IS = IS; ga.gelu = gemma;
@@ -464,7 +478,7 @@ void forward_impl(SFTState *s, bool gather, bool zero_rows = false)
     nf.pf = prefetch_for(s, wop(s, W_LM, 0, false), s->V, D, 1024);
     launch_norm_rows(nf, BN);
     GemmPlan pl = plan_gemm(BN, s->V, D, 0, s->q8_native ? 1 : 0);
-    if (pl.S == 1 || use_big_gemm(BN, s->V, D, s->q8_native ? 1 : 0)) {
+    if (pl.S == 1 || use_big_gemm(BN, s->V, D, s->q8_native ? 1 : 0, true)) {
         gemm(s, lnf, lnfinv, wop(s, W_LM, 0, false), s->V, D, at<float>(s->logits));
     } else {
         Planes p = gemm(s, lnf, lnfinv, wop(s, W_LM, 0, false), s->V, D);
