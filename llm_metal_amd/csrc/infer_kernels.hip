@@ -669,6 +669,163 @@ __global__ __launch_bounds__(TB) void k_attn_decode(const float *__restrict__ Q,
     }
 }
 
+// The same for a context of one slice and no adapters, head sizes 64, 128 and 256: the launch is a chain of latencies (at 64 keys it
+// moves 64 KB per head), so nothing in it waits for more than one trip to memory.  A key belongs to 16 lanes, each with HD / 16 of
+// its columns; the 16 groups of a workgroup take keys in turn and keep a running softmax of their own, so keys, values, the
+// product's row and the norm weights are all requested at the start, a score is a sum over 16 lanes (four DPP adds, no LDS), and
+// one barrier comes before the groups are merged.  Every group finishes the query head and the newest key in its own registers
+// (columns d and d + HD / 2 of a rotary pair are in the same lane from HD = 128 on); the newest key and value do not take the
+// way through the cache, which the first head of a key head's group writes for the launches to come.
+// Against k_attn_decode<4, true> at up to 129 keys: 16.4 -> 5.8 us (four heads of 256), 9.6 -> 4.2 (8 x 32 heads of 128),
+// 11.1 -> 7.0 where 128 more workgroups request the next weights.
+constexpr int SHORT_KEYS = 256;
+template <int HD>
+__global__ __launch_bounds__(TB) void k_attn_short(float *__restrict__ out, int hd, int max_seq, int G, float scale, HeadPost hp)
+{
+    constexpr int C = HD / 64, U = 4;                      // 16-byte pieces per lane and key; keys a group has in flight
+    __shared__ float po[16][HD], pm[16], pl[16];
+    const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 4, sub = tid & 15;
+    const int heads = (int)gridDim.x - hp.pf_wgs;
+    if ((int)blockIdx.x >= heads) {                        // a workgroup that only asks for the next product's weights
+        if (blockIdx.z == 0) request_bytes_ahead(hp.pf_base, hp.pf_bytes, blockIdx.x - heads, hp.pf_wgs);
+        return;
+    }
+    const int hq = blockIdx.x, hk = hq / G, z = blockIdx.z, pos = hp.pos;
+    const float *row = hp.qkv + (size_t)z * hp.qkv_step;
+    const size_t cache = (size_t)z * hp.cache_step + (size_t)hk * max_seq * HD;
+    float *Kh = hp.kc + cache, *Vh = hp.vc + cache;
+
+    auto sum16 = [](float v) __attribute__((always_inline)) {
+        v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));     // lane ^ 1
+        v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));     // lane ^ 2
+        v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));    // 7 - lane of eight
+        v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, false));    // 15 - lane of sixteen
+        return v;
+    };
+    float4v q[C], kn[C], vn[C], gq[C], gk[C], k[U][C], v[U][C];
+    float2 rot[C][4];
+    auto keys = [&](int j0) __attribute__((always_inline)) {               // (past the newest cached key: the last one again)
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const size_t at = (size_t)max(min(j0 + 16 * u, pos - 1), 0) * HD + 4 * sub;
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                k[u][c] = *reinterpret_cast<const float4v *>(Kh + at + 64 * c);
+                v[u][c] = *reinterpret_cast<const float4v *>(Vh + at + 64 * c);
+            }
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int d = 4 * sub + 64 * c;
+        q[c] = *reinterpret_cast<const float4v *>(row + (size_t)hq * HD + d);
+        kn[c] = *reinterpret_cast<const float4v *>(row + (size_t)(hp.Hq + hk) * HD + d);
+        vn[c] = *reinterpret_cast<const float4v *>(row + (size_t)(hp.Hq + hp.Hkv + hk) * HD + d);
+        gq[c] = gk[c] = float4v{1.f, 1.f, 1.f, 1.f};
+        if (hp.g_q) gq[c] = *reinterpret_cast<const float4v *>(hp.g_q + d);
+        if (hp.g_k) gk[c] = *reinterpret_cast<const float4v *>(hp.g_k + d);
+#pragma unroll
+        for (int e = 0; e < 4; e++) rot[c][e] = hp.rope[(d + e) % (HD / 2)];
+    }
+    keys(grp);
+    // RMSNorm and RoPE of a head in the group's lanes
+    auto finish = [&](float4v (&x)[C], const float4v (&g)[C], bool normed) __attribute__((always_inline)) {
+        if (normed) {
+            float ss = 0.f;
+#pragma unroll
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss += x[c][e] * x[c][e];
+            const float inv = rsqrtf(sum16(ss) / (float)HD + hp.eps);
+#pragma unroll
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[c][e] *= inv * g[c][e];
+        }
+        if (C == 1) {                                      // the pair's other column is eight lanes away
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float o = __shfl_xor(x[0][e], 8, 64);
+                x[0][e] = sub < 8 ? x[0][e] * rot[0][e].x - o * rot[0][e].y : o * rot[0][e].y + x[0][e] * rot[0][e].x;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < C / 2; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float a = x[c][e], b = x[c + C / 2][e], cs = rot[c][e].x, sn = rot[c][e].y;
+                    x[c][e] = a * cs - b * sn; x[c + C / 2][e] = a * sn + b * cs;
+                }
+        }
+    };
+    finish(q, gq, hp.g_q != nullptr);
+    finish(kn, gk, hp.g_k != nullptr);
+    if (grp == 0 && hq % G == 0) {
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            *reinterpret_cast<float4v *>(Kh + (size_t)pos * HD + 4 * sub + 64 * c) = kn[c];
+            *reinterpret_cast<float4v *>(Vh + (size_t)pos * HD + 4 * sub + 64 * c) = vn[c];
+        }
+    }
+    auto dot = [&](const float4v (&x)[C]) __attribute__((always_inline)) {
+        float s = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = fmaf(q[c][e], x[c][e], s);
+        return sum16(s) * scale;
+    };
+    // the newest key belongs to group 0
+    const float s0 = dot(kn);
+    float m = grp == 0 ? s0 : -3.0e38f, l = grp == 0 ? 1.f : 0.f;
+    if (grp == 0 && !(s0 > -3.0e38f)) { m = -3.0e38f; l = __expf(s0 - m); }           // (not a number, or minus infinity)
+    float4v o[C];
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[c][e] = grp == 0 ? l * vn[c][e] : 0.f;
+    for (int j0 = grp; j0 < pos; j0 += 16 * U) {
+        float s[U], top = m;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            s[u] = dot(k[u]);
+            if (j0 + 16 * u < pos) top = fmaxf(top, s[u]);
+        }
+        const float keep = __expf(m - top);
+        m = top;
+        l *= keep;
+#pragma unroll
+        for (int c = 0; c < C; c++) o[c] *= keep;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool in = j0 + 16 * u < pos;
+            const float p = in ? __expf(s[u] - m) : 0.f;
+            l += p;
+#pragma unroll
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[c][e] = fmaf(p, in ? v[u][c][e] : 0.f, o[c][e]);
+        }
+        if (j0 + 16 * U < pos) keys(j0 + 16 * U);
+    }
+#pragma unroll
+    for (int c = 0; c < C; c++) *reinterpret_cast<float4v *>(&po[grp][4 * sub + 64 * c]) = o[c];
+    if (sub == 0) { pm[grp] = m; pl[grp] = l; }
+    __syncthreads();
+    if (tid >= HD) return;
+    float all = pm[0];
+#pragma unroll
+    for (int g = 1; g < 16; g++) all = fmaxf(all, pm[g]);
+    float den = 0.f, num = 0.f;
+#pragma unroll
+    for (int g = 0; g < 16; g++) {
+        const float w = __expf(pm[g] - all);
+        den = fmaf(pl[g], w, den);
+        num = fmaf(po[g][tid], w, num);
+    }
+    out[((size_t)z * hp.Hq + hq) * HD + tid] = num / den;
+}
+
 // merge of the slices of one query head: grid = Hq (times the sequences of a batch), block = hd threads (<= 256)
 __global__ __launch_bounds__(TB) void k_attn_combine(const float *__restrict__ part_o, const float *__restrict__ part_ml,
                                                      float *__restrict__ out, int hd, int nsplit)
@@ -746,6 +903,16 @@ void attention_launch(const float *Q, const float *Kc, const float *Vc, float *o
     HeadPost post{};
     if (hp) post = *hp;
     if ((Hq / gpw) * nsplit * copies > 128 || !post.pf_base || !post.pf_bytes) post.pf_wgs = 0;      // no spare CUs, or nothing to ask for
+    // (the row's steps and the caches keep 16-byte alignment: hd is a multiple of 64)
+    if (hp && n_attend <= SHORT_KEYS && !hp->R && (hd == 64 || hd == 128 || hd == 256) && hp->qkv_step % 4 == 0 &&
+        !(((uintptr_t)hp->qkv | (uintptr_t)hp->kc | (uintptr_t)hp->vc | (uintptr_t)hp->g_q | (uintptr_t)hp->g_k) & 15)) {
+        post.pf_wgs = Hq * copies > 128 || !hp->pf_base || !hp->pf_bytes ? 0 : hp->pf_wgs;
+        const dim3 heads(Hq + post.pf_wgs, 1, copies);
+#define SHORT_LAUNCH(HD_) LAUNCH((k_attn_short<HD_>), heads, dim3(TB), 0, out, hd, max_seq, G, scale, post)
+        if (hd == 64) SHORT_LAUNCH(64); else if (hd == 128) SHORT_LAUNCH(128); else SHORT_LAUNCH(256);
+#undef SHORT_LAUNCH
+        return;
+    }
     const dim3 grid(Hq / gpw + post.pf_wgs, nsplit, copies);
     const HeadPost none{};
 #define ATTN_LAUNCH(V_, F_) LAUNCH((k_attn_decode<V_, F_>), grid, dim3(TB), lds, Q, Kc, Vc, out, po, pml, \
