@@ -77,8 +77,9 @@ void matvec_norm(MetalBuf *W, const NormIn &nin, MetalBuf *y, int rows, int cols
 void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, float eps, float *y, int rows, int cols);
 
 // infer_kernels.hip: y = W . RMSNorm(v; g) with v = xr + RMSNorm(br + b_br; g_br) (br may be null) over the first dim of cols
-// entries, v also to x_out (F16 rows); gelu: y = tanh-GELU of it
-void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int cols, int gelu);
+// entries, v also to x_out; F16 rows or Q8_0 blocks.  act 0: as it is; 1, 2: the gated pairs of matvec_glu (SiLU, GELU); 3: its
+// tanh-GELU (F16 rows)
+void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int cols, int q8, int act);
 // infer_kernels.hip: y = W . x (F16 rows, cols a multiple of 8)
 void matvec_rows(MetalBuf *W, const float *x, float *y, int rows, int cols);
 

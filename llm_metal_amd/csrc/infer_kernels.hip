@@ -160,14 +160,14 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
     int row0 = ((blockIdx.x * REPS) * 4 + wave) * (GLU ? 1 : R);
     size_t roff[R];                                             // element offset of each row (clamped: extra rows are not stored)
     float acc[R];
-    auto set_rows = [&]() __attribute__((always_inline)) {
+    auto set_rows = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            roff[r] = GLU ? ((size_t)r * rows + min(row0, rows - 1)) * cols : (size_t)min(row0 + r, rows - 1) * cols;
-            acc[r] = 0.f;
-        }
+        for (int r = 0; r < R; r++)
+            roff[r] = GLU ? ((size_t)r * rows + min(first, rows - 1)) * cols : (size_t)min(first + r, rows - 1) * cols;
     };
-    set_rows();
+    set_rows(row0);
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.f;
 
     auto load = [&](Stage &g, int c) __attribute__((always_inline)) {
 #pragma unroll
@@ -224,10 +224,49 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
         }
     };
 
+    // The vector's parts are requested ahead of the first weights: loads return in order, so behind the weights the sums and the
+    // norm would wait for memory as well.  A thread has up to four pieces of 1024 columns in registers at a time.
+    constexpr int VG = 4;
+    float4v rv[NORM ? VG : 1], rg[NORM ? VG : 1], rb[NORM == 1 || NORM == 3 ? VG : 1], rgb[NORM == 3 ? VG : 1];
+    auto load_vector = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < VG; u++) {
+            // a wave whose piece lies behind the vector asks for nothing (a load of one address by all lanes takes the CU's
+            // address unit as long as any other)
+            if (__builtin_amdgcn_readfirstlane(i0 + u * TB * 4) >= cols) break;
+            const int i = min(i0 + u * TB * 4, cols - 4);
+            rv[u] = *reinterpret_cast<const float4v *>(&nin.xr[i]);
+            rg[u] = *reinterpret_cast<const float4v *>(&nin.g[i]);
+            if ((NORM == 1 || NORM == 3) && nin.br) {
+                rb[u] = *reinterpret_cast<const float4v *>(&nin.br[i]);
+                if (NORM == 3) rgb[u] = *reinterpret_cast<const float4v *>(&nin.g_br[i]);
+                if (NORM == 3 && nin.b_br) rb[u] += *reinterpret_cast<const float4v *>(&nin.b_br[i]);
+            }
+        }
+    };
+    const bool in_registers = cols <= VG * TB * 4;
+    if (NORM == 1 || (NORM && in_registers)) { load_vector(tid * 4); __builtin_amdgcn_sched_barrier(0); }
     Stage cur;
     load(cur, lane * 8);
+    if (NORM) __builtin_amdgcn_sched_barrier(0);
     float norm_inv = 1.f;
-    if (NORM == 2) {
+    if (NORM == 2 && in_registers) {
+        float sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < VG; u++)
+            if (tid * 4 + u * TB * 4 < cols) sum += (rv[u][0] + rv[u][1]) + (rv[u][2] + rv[u][3]);
+        const float mean = block_sum(sum, red) / (float)nin.dim;
+        float ss = 0.f;
+#pragma unroll
+        for (int u = 0; u < VG; u++) {
+            const int i = tid * 4 + u * TB * 4;
+            if (i >= cols) break;
+#pragma unroll
+            for (int e = 0; e < 4; e++) { rv[u][e] = i + e < nin.dim ? rv[u][e] - mean : 0.f; ss += rv[u][e] * rv[u][e]; }
+            *reinterpret_cast<float4v *>(&xs[i]) = rv[u] * rg[u];
+        }
+        norm_inv = 1.f / sqrtf(block_sum(ss, red) / (float)nin.dim + nin.eps);
+    } else if (NORM == 2) {
         float sum = 0.f;
         for (int i = tid * 4; i < cols; i += TB * 4) {
             const float4v v = *reinterpret_cast<const float4v *>(&nin.xr[i]);
@@ -242,6 +281,34 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
 #pragma unroll
             for (int e = 0; e < 4; e++) { v[e] = i + e < nin.dim ? v[e] - mean : 0.f; ss += v[e] * v[e]; }
             *reinterpret_cast<float4v *>(&xs[i]) = v * gg;
+        }
+        norm_inv = 1.f / sqrtf(block_sum(ss, red) / (float)nin.dim + nin.eps);
+    } else if (NORM == 3 && in_registers) {
+        float post = 0.f;
+        if (nin.br) {
+            float ss = 0.f;
+#pragma unroll
+            for (int u = 0; u < VG; u++) {
+                const int i = tid * 4 + u * TB * 4;
+                if (i >= cols) break;
+#pragma unroll
+                for (int e = 0; e < 4; e++) { rb[u][e] = i + e < nin.dim ? rb[u][e] : 0.f; ss += rb[u][e] * rb[u][e]; }
+            }
+            post = 1.f / sqrtf(block_sum(ss, red) / (float)nin.dim + nin.eps);
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int u = 0; u < VG; u++) {
+            const int i = tid * 4 + u * TB * 4;
+            if (i >= cols) break;
+            if (nin.br) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) rv[u][e] = fmaf(rb[u][e] * post, rgb[u][e], rv[u][e]);
+                if (blockIdx.x == 0 && nin.x_out) *reinterpret_cast<float4v *>(&nin.x_out[i]) = rv[u];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) ss += rv[u][e] * rv[u][e];        // (zeros behind dim)
+            *reinterpret_cast<float4v *>(&xs[i]) = rv[u] * rg[u];
         }
         norm_inv = 1.f / sqrtf(block_sum(ss, red) / (float)nin.dim + nin.eps);
     } else if (NORM == 3) {
@@ -274,24 +341,19 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
         norm_inv = 1.f / sqrtf(block_sum(ss, red) / (float)nin.dim + nin.eps);
     } else if (NORM) {
         float ss = 0.f;
-        for (int i0 = tid * 4; i0 < cols; i0 += TB * 16) {      // four groups of a thread requested together
-            float4v v[4], b[4], gg[4];
+        for (int i0 = tid * 4;;) {                              // four groups of a thread requested together
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int i = min(i0 + u * TB * 4, cols - 4);
-                v[u] = *reinterpret_cast<const float4v *>(&nin.xr[i]);
-                if (nin.br) b[u] = *reinterpret_cast<const float4v *>(&nin.br[i]);
-                gg[u] = *reinterpret_cast<const float4v *>(&nin.g[i]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
+            for (int u = 0; u < VG; u++) {
                 const int i = i0 + u * TB * 4;
                 if (i >= cols) break;
-                if (nin.br) v[u] += b[u];
-                ss += v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
-                *reinterpret_cast<float4v *>(&xs[i]) = v[u] * gg[u];
-                if (blockIdx.x == 0 && nin.x_out) *reinterpret_cast<float4v *>(&nin.x_out[i]) = v[u];
+                if (nin.br) rv[u] += rb[u];
+                ss += rv[u][0] * rv[u][0] + rv[u][1] * rv[u][1] + rv[u][2] * rv[u][2] + rv[u][3] * rv[u][3];
+                *reinterpret_cast<float4v *>(&xs[i]) = rv[u] * rg[u];
+                if (blockIdx.x == 0 && nin.x_out) *reinterpret_cast<float4v *>(&nin.x_out[i]) = rv[u];
             }
+            i0 += TB * 4 * VG;
+            if (i0 - tid * 4 >= cols) break;
+            load_vector(i0);
         }
         norm_inv = rsqrtf(block_sum(ss, red) / (float)cols + nin.eps);      // its barriers also publish xs
     } else if (XLDS) {
@@ -299,30 +361,38 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
             *reinterpret_cast<float4v *>(&xs[i]) = *reinterpret_cast<const float4v *>(&x[i]);
         __syncthreads();
     }
+    // stage after stage, across the row groups: the first stage of the next group is requested under the last of this one
+    int c = lane * 8, rep = 0;
 #pragma unroll 1
-    for (int rep = 0; rep < REPS; rep++) {
-        if (rep) {                                              // the next group of rows, with the same vector
-            row0 += 4 * (GLU ? 1 : R);
-            set_rows();
-            load(cur, lane * 8);
+    for (;;) {
+        const bool done = c - lane * 8 + 512 * U >= cols;       // the group's last stage (uniform)
+        int cn = c + 512 * U;
+        if (REPS > 1 && done && rep + 1 < REPS) {
+            set_rows(row0 + 4 * (GLU ? 1 : R));
+            cn = lane * 8;
         }
-        for (int c = lane * 8; c < cols; c += 512 * U) {
-            Stage nxt;
-            load(nxt, c + 512 * U);
-            use(cur, c);
-            cur = nxt;
-        }
-        if (GLU) {
-            const float g = wave_sum(acc[0]) * norm_inv, u = wave_sum(acc[R - 1]) * norm_inv;
-            if (lane == 0 && row0 < rows)                       // the expressions of silu_mul / gelu_mul
-                y[row0] = (GLU == 1 ? g / (1.0f + expf(-g)) : 0.5f * g * (1.0f + tanhf(gelu_inner(g)))) * u;
-        } else {
+        Stage nxt;
+        load(nxt, cn);
+        use(cur, c);
+        if (done) {
+            if (GLU) {
+                const float g = wave_sum(acc[0]) * norm_inv, u = wave_sum(acc[R - 1]) * norm_inv;
+                if (lane == 0 && row0 < rows)                   // the expressions of silu_mul / gelu_mul
+                    y[row0] = (GLU == 1 ? g / (1.0f + expf(-g)) : 0.5f * g * (1.0f + tanhf(gelu_inner(g)))) * u;
+            } else {
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float s = wave_sum(acc[r]) * norm_inv;
-                if (lane == 0 && row0 + r < rows) y[row0 + r] = ACT ? 0.5f * s * (1.0f + tanhf(gelu_inner(s))) : s;
+                for (int r = 0; r < R; r++) {
+                    const float s = wave_sum(acc[r]) * norm_inv;
+                    if (lane == 0 && row0 + r < rows) y[row0 + r] = ACT ? 0.5f * s * (1.0f + tanhf(gelu_inner(s))) : s;
+                }
             }
+            if (++rep >= REPS) break;
+            row0 += 4 * (GLU ? 1 : R);
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] = 0.f;
         }
+        cur = nxt;
+        c = cn;
     }
 }
 
@@ -1203,24 +1273,41 @@ void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, floa
 #undef LN_LAUNCH
 }
 
-void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int cols, int gelu)
+// glu 0: y = W . v; 1, 2: the gated pairs of matvec_glu (W has 2 * rows rows; 1 SiLU, 2 GELU); 3: tanh-GELU of it
+void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int cols, int q8, int act)
 {
-    bool ok = rows > 0 && nin.dim > 0 && nin.dim <= cols && !(cols & 7) && cols <= 15360 && aligned16(dptr(W)) && nin.xr && nin.g && nin.x_out != nin.xr;
+    bool ok = rows > 0 && nin.dim > 0 && nin.dim <= cols && !(cols & (q8 ? 31 : 7)) && cols <= 15360 && aligned16(dptr(W)) && nin.xr && nin.g && nin.x_out != nin.xr;
     for (const void *p : {(const void *)nin.xr, (const void *)nin.g, (const void *)nin.br, (const void *)nin.g_br, (const void *)nin.b_br, (const void *)nin.x_out})
         ok = ok && aligned16(p);
-    if (!ok || (nin.br && !nin.g_br)) { fprintf(stderr, "[fast_hip] matvec_norms_around: unsupported shape %d x %d or operands\n", rows, cols); abort(); }
-    REQUIRE_BYTES(W, (size_t)rows * cols * 2, "matvec_norms_around");
-    hipEvent_t ev_a = nullptr, ev_b = nullptr;
-    const bool prof = gemm_prof_begin(2.0 * rows * cols, 2.0 * rows * cols, &ev_a, &ev_b);
-    const size_t lds = (size_t)cols * 4;
+    if (!ok || (nin.br && !nin.g_br) || (q8 && act == 3)) { fprintf(stderr, "[fast_hip] matvec_norms_around: unsupported shape %d x %d or operands\n", rows, cols); abort(); }
+    const int wrows = act == 1 || act == 2 ? 2 * rows : rows;
     const half_t *scales = nullptr;
-#define AROUND_LAUNCH(REPS_, ACT_) do { \
-    const dim3 grid((rows + 8 * REPS_ - 1) / (8 * REPS_)); \
-    if (prof) hipExtLaunchKernelGGL((k_matvec<0, 2, 2, 1, 0, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), ev_a, ev_b, 0, dptr(W), scales, nullptr, y, rows, cols, nin); \
-    else hipLaunchKernelGGL((k_matvec<0, 2, 2, 1, 0, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), dptr(W), scales, nullptr, y, rows, cols, nin); \
+    const void *w = dptr(W);
+    if (q8) {
+        REQUIRE_BYTES(W, (size_t)wrows * (cols / 32) * 34, "matvec_norms_around");
+        w = q8_split_of(W, wrows, cols / 32, &scales);
+    } else REQUIRE_BYTES(W, (size_t)wrows * cols * 2, "matvec_norms_around");
+    hipEvent_t ev_a = nullptr, ev_b = nullptr;
+    const bool prof = gemm_prof_begin((q8 ? 34.0 / 32.0 : 2.0) * wrows * cols, 2.0 * wrows * cols, &ev_a, &ev_b);
+    const size_t lds = (size_t)cols * 4;
+    // columns of up to three steps of 512: a wave asks for whole rows at once (1152 columns, gated Q8_0 pairs: 14.3 us with two
+    // steps, the second stage of which is all but empty, 13.7 with three)
+#define AROUND_LAUNCH_U(FMT_, U_, GLU_, RPW_, REPS_, ACT_) do { \
+    const dim3 grid((rows + RPW_ * REPS_ - 1) / (RPW_ * REPS_)); \
+    if (prof) hipExtLaunchKernelGGL((k_matvec<FMT_, 2, U_, 1, GLU_, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), ev_a, ev_b, 0, w, scales, nullptr, y, rows, cols, nin); \
+    else hipLaunchKernelGGL((k_matvec<FMT_, 2, U_, 1, GLU_, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), w, scales, nullptr, y, rows, cols, nin); \
     HIP_CHECK(hipGetLastError()); } while (0)
-    if (gelu) { if (rows >= 16384) AROUND_LAUNCH(4, 1); else AROUND_LAUNCH(1, 1); }
-    else { if (rows >= 16384) AROUND_LAUNCH(4, 0); else AROUND_LAUNCH(1, 0); }
+#define AROUND_LAUNCH(FMT_, GLU_, RPW_, REPS_, ACT_) do { \
+    if (cols > 1024 && cols <= 1536) AROUND_LAUNCH_U(FMT_, 3, GLU_, RPW_, REPS_, ACT_); else AROUND_LAUNCH_U(FMT_, 2, GLU_, RPW_, REPS_, ACT_); } while (0)
+    if (act == 3) { if (rows >= 16384) AROUND_LAUNCH(0, 0, 8, 4, 1); else AROUND_LAUNCH(0, 0, 8, 1, 1); }
+    else if (act == 0) {
+        if (q8) AROUND_LAUNCH(1, 0, 8, 1, 0);
+        else if (rows >= 16384) AROUND_LAUNCH(0, 0, 8, 4, 0);
+        else AROUND_LAUNCH(0, 0, 8, 1, 0);
+    }
+    else if (q8) { if (act == 1) AROUND_LAUNCH(1, 1, 4, 2, 0); else AROUND_LAUNCH(1, 2, 4, 2, 0); }
+    else { if (act == 1) AROUND_LAUNCH(0, 1, 4, 2, 0); else AROUND_LAUNCH(0, 2, 4, 2, 0); }
+#undef AROUND_LAUNCH_U
 #undef AROUND_LAUNCH
 }
 

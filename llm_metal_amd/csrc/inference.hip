@@ -308,17 +308,19 @@ void forward_token(InferenceState *s, int token, int pos)
     // (matvec_norm) and the sum goes to the other of two residual buffers; the Q|K|V product only without adapters,
     // whose down-projection reads the normed vector too.
     MetalBuf *x = s->x, *x_other = s->x2;
-    const bool fuse_ffn = !gemma && D <= 12288, fuse_qkv = fuse_ffn && s->lora.empty();
+    // (Gemma3's branch is normed on its way into the sum: matvec_norms_around does that too)
+    const bool fuse_ffn = D <= 12288, fuse_qkv = fuse_ffn && s->lora.empty();
     const int q8 = s->use_fp16 ? 0 : 1;
-    auto normed_product = [&](MetalBuf *W, MetalBuf *branch, MetalBuf *g, MetalBuf *y, int rows, int glu) {
+    auto normed_product = [&](MetalBuf *W, MetalBuf *branch, MetalBuf *g_branch, MetalBuf *g, MetalBuf *y, int rows, int glu) {
         NormIn n{dptr_as<float>(x), branch ? dptr_as<float>(branch) : nullptr, dptr_as<float>(g), branch ? dptr_as<float>(x_other) : nullptr,
-                 s->eps};
-        matvec_norm(W, n, y, rows, D, q8, glu);
+                 s->eps, D, g_branch ? dptr_as<float>(g_branch) : nullptr, nullptr};
+        if (gemma) { matvec_norms_around(W, n, dptr_as<float>(y), rows, D, q8, glu); mark_written(y); }
+        else matvec_norm(W, n, y, rows, D, q8, glu);
         if (branch) std::swap(x, x_other);
     };
     for (int L = 0; L < s->NL; L++) {
         const InferenceState::Layer &lw = s->layers[L];
-        if (fuse_qkv) normed_product(lw.qkv.mbuf, pending, lw.g_in, s->qkv, lw.qkv.rows, 0);
+        if (fuse_qkv) normed_product(lw.qkv.mbuf, pending, pending_g, lw.g_in, s->qkv, lw.qkv.rows, 0);
         else {
             add_norm(s, x, pending, pending_g, lw.g_in);
             matvec(s, &lw.qkv, s->ln, s->qkv);
@@ -346,7 +348,7 @@ void forward_token(InferenceState *s, int token, int pos)
         matvec(s, lw.o, s->att, s->branch);
         // x += o (Gemma3: RMSNorm(o; g_post_attn)); ln = RMSNorm(x; g_pre_ff | g_post_attn);
         // act = silu | gelu (gate) * up, formed in the epilogue of the [gate; up] product
-        if (fuse_ffn) normed_product(lw.gu.mbuf, s->branch, lw.g_post_attn, s->gate_v, s->IS, 1);
+        if (fuse_ffn) normed_product(lw.gu.mbuf, s->branch, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, s->gate_v, s->IS, gemma ? 2 : 1);
         else {
             add_norm(s, x, s->branch, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn);
             matvec_glu(lw.gu.mbuf, s->ln, s->gate_v, s->IS, D, q8, gemma ? 1 : 0);

@@ -631,7 +631,7 @@ void decode_layers_around(LayerStack *st, StackRun *r, int pos)
     in.eps = st->cfg.eps; in.dim = st->D;
     auto product_of = [&](const StackMat &w, MetalBuf *g, float *y, int gelu) {
         in.xr = at; in.g = ptr<float>(g); in.x_out = in.br ? next : nullptr;
-        matvec_norms_around(w.buf, in, y, w.rows, w.cols, gelu);
+        matvec_norms_around(w.buf, in, y, w.rows, w.cols, 0, gelu ? 3 : 0);
         if (in.br) std::swap(at, next);
     };
     auto leave = [&](MetalBuf *g, MetalBuf *b) { in.br = cout; in.g_br = ptr<float>(g); in.b_br = ptr<float>(b); };
@@ -769,7 +769,7 @@ void stack_logits(LayerStack *st, StackRun *r, const int *want, int n, float *lo
     if (r->one) {                                         // whatever `want` says, it is the one row
         if (st->cfg.norms == NORMS_AROUND)
             matvec_norms_around(st->head.buf, NormIn{r->xr, ptr<float>(r->cout), ptr<float>(st->g_final), nullptr, st->cfg.eps, st->D, r->post_g, r->post_b},
-                                logits, st->head.rows, st->head.cols, 0);
+                                logits, st->head.rows, st->head.cols, 0, 0);
         else matvec_layernorm(st->head.buf, ptr<float>(r->x), ptr<float>(st->g_final), st->D, st->cfg.eps, logits, st->head.rows, st->head.cols);
         return;
     }
