@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_qkv_post_tile(QkvPostArgs a, uint4 *q_r
             float ss = 0.f;
 #pragma unroll
             for (int c = 0; c < HD / 32; c++) { const float4 v = ld4(Xs + rr * LDS_LD + 32 * c + 4 * part); ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; }
-            ss += __shfl_xor(ss, 1, WAVE); ss += __shfl_xor(ss, 2, WAVE); ss += __shfl_xor(ss, 4, WAVE);
+            ss = xor_add<4>(xor_add<2>(xor_add<1>(ss)));
             if (part == 0) Inv[rr] = rsqrtf(ss / (float)HD + a.eps);
         }
         __syncthreads();
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(256) void k_fa_fwd(FaArgs a)
             for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[v]);
         }
         mx = fmaxf(mx * a.scale_log2, -1e30f);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        mx = xor_max<32>(mx);
         if (__any(mx > m + 8.0f)) {
             const float m_new = fmaxf(m, mx);
             const float alpha = __builtin_amdgcn_exp2f(m - m_new);
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(256) void k_fa_fwd(FaArgs a)
         if (kb + 1 <= kb_hi) step(kb + 1, buf1, buf0);
     }
     if (!active) return;
-    l += __shfl_xor(l, 32, WAVE);
+    l = xor_add<32>(l);
     const float inv = 1.0f / l;
     if (hh == 0) a.lse[((size_t)b * a.Hq + h) * nblk * 32 + i] = i < N ? m + log2f(l) : 0.f;
     const int qd = a.Hq * HD, Kb = tiled_kb(qd);

@@ -248,8 +248,8 @@ __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int l
             for (int c = 0; c < 4; c++) { e[c] = (j + c <= i && j + c < nk && j + c >= lo) ? e[c] * a.scale : -1e30f; red = fmaxf(red, e[c]); }
         }
     }
-    if (BWD) { red += __shfl_xor(red, 1, WAVE); red += __shfl_xor(red, 2, WAVE); red += __shfl_xor(red, 4, WAVE); }
-    else { red = fmaxf(red, __shfl_xor(red, 1, WAVE)); red = fmaxf(red, __shfl_xor(red, 2, WAVE)); red = fmaxf(red, __shfl_xor(red, 4, WAVE)); }
+    if (BWD) { red = xor_add<4>(xor_add<2>(xor_add<1>(red))); }
+    else { red = xor_max<4>(xor_max<2>(xor_max<1>(red))); }
     float inv = 1.0f;
     if (!BWD) {
         float sum = 0.f;
@@ -260,7 +260,7 @@ __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int l
 #pragma unroll
             for (int c = 0; c < 4; c++) { e[c] = (j + c <= i && j + c < nk && j + c >= lo) ? expf(e[c] - red) : 0.f; sum += e[c]; }
         }
-        sum += __shfl_xor(sum, 1, WAVE); sum += __shfl_xor(sum, 2, WAVE); sum += __shfl_xor(sum, 4, WAVE);
+        sum = xor_add<4>(xor_add<2>(xor_add<1>(sum)));
         inv = 1.0f / sum;
     }
     float *gdst = (BWD ? a.dscore : a.probs) + goff;

@@ -13,18 +13,41 @@ typedef float    float4v __attribute__((ext_vector_type(4)));
 
 #define WAVE 64
 
+// v + (or max with) the value of lane ^ O, without the trip through LDS that __shfl_xor takes: DPP inside rows of sixteen lanes,
+// gfx950's row and half swaps across them.  Every lane of the wave active.  The same operands meet as with __shfl_xor, so the
+// results are the same bit for bit; six dependent steps take some 50 cycles instead of 700 (Q8_0 head of
+// 262 144 rows, one reduction per row: 86 -> 77 us; k_qkv_bwd_rows at 64 rows 9.6 -> 8.0; gated product with its norms 12.9 -> 11.7).
+template <int CTRL, int BANKS = 0xF> __device__ __forceinline__ float dpp_move(float old, float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v), CTRL, 0xF, BANKS, false));
+}
+struct LanePair { float a, b; };                           // v of this lane and of lane ^ O, in either order
+template <int O> __device__ __forceinline__ LanePair lane_pair(float v)
+{
+    static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "a power of two below 64");
+    if constexpr (O == 1) return {v, dpp_move<0xB1>(v, v)};                          // quad_perm [1, 0, 3, 2]
+    else if constexpr (O == 2) return {v, dpp_move<0x4E>(v, v)};                     // quad_perm [2, 3, 0, 1]
+    else if constexpr (O == 4) return {v, dpp_move<0x114, 0xA>(dpp_move<0x104, 0x5>(v, v), v)};   // four up in the even quads, four down in the odd ones
+    else if constexpr (O == 8) return {v, dpp_move<0x128>(v, v)};                    // rotated by eight of sixteen
+    else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        unsigned x, y;                                     // (copies: a bit cast of a vector's element reads the first one)
+        if constexpr (O == 16) { const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false); x = r[0]; y = r[1]; }
+        else { const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false); x = r[0]; y = r[1]; }
+        return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
+    }
+}
+template <int O> __device__ __forceinline__ float xor_add(float v) { const LanePair p = lane_pair<O>(v); return p.a + p.b; }
+template <int O> __device__ __forceinline__ float xor_max(float v) { const LanePair p = lane_pair<O>(v); return fmaxf(p.a, p.b); }
+
 __device__ __forceinline__ float wave_sum(float v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+    return xor_add<1>(xor_add<2>(xor_add<4>(xor_add<8>(xor_add<16>(xor_add<32>(v))))));
 }
 
 __device__ __forceinline__ float wave_max(float v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-    return v;
+    return xor_max<1>(xor_max<2>(xor_max<4>(xor_max<8>(xor_max<16>(xor_max<32>(v))))));
 }
 
 // Workgroup reductions for blocks of up to 1024 threads (16 waves).  `smem`

@@ -669,8 +669,8 @@ __global__ __launch_bounds__(NT) void k_qkv_bwd_rows(QkvBwdArgs a)
                 }
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-#pragma unroll
-                    for (int o = 4; o < 64; o <<= 1) { aq[e] += __shfl_xor(aq[e], o, WAVE); av[e] += __shfl_xor(av[e], o, WAVE); }
+                    aq[e] = xor_add<32>(xor_add<16>(xor_add<8>(xor_add<4>(aq[e]))));
+                    av[e] = xor_add<32>(xor_add<16>(xor_add<8>(xor_add<4>(av[e]))));
                 }
                 if (lane < 4) {
 #pragma unroll
@@ -699,8 +699,8 @@ __global__ __launch_bounds__(NT) void k_qkv_bwd_rows(QkvBwdArgs a)
                 }
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-#pragma unroll
-                    for (int o = 2; o < 64; o <<= 1) { q8s[e] += __shfl_xor(q8s[e], o, WAVE); v8s[e] += __shfl_xor(v8s[e], o, WAVE); }
+                    q8s[e] = xor_add<32>(xor_add<16>(xor_add<8>(xor_add<4>(xor_add<2>(q8s[e])))));
+                    v8s[e] = xor_add<32>(xor_add<16>(xor_add<8>(xor_add<4>(xor_add<2>(v8s[e])))));
                 }
                 if (lane < 2) {
 #pragma unroll
@@ -721,8 +721,8 @@ __global__ __launch_bounds__(NT) void k_qkv_bwd_rows(QkvBwdArgs a)
                 }
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-#pragma unroll
-                    for (int o = 4; o < 64; o <<= 1) { aq[e] += __shfl_xor(aq[e], o, WAVE); av[e] += __shfl_xor(av[e], o, WAVE); }
+                    aq[e] = xor_add<32>(xor_add<16>(xor_add<8>(xor_add<4>(aq[e]))));
+                    av[e] = xor_add<32>(xor_add<16>(xor_add<8>(xor_add<4>(av[e]))));
                 }
                 if (lane < 4) {
 #pragma unroll

@@ -166,7 +166,7 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
             S[j] = seen ? S[j] * scale : -INFINITY;
             if (seen) top = fmaxf(top, S[j]);
         }
-        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        top = xor_max<32>(top);
         const float now = fmaxf(mx, top), keep = expf(mx - now);
         mx = now;
         float sum = 0.f;
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
         for (int i = wave; i < 32 && row0 + i < rows; i += 4) attend_plain<HD>(Q, Kh, Vh, out, (row0 + i) / G, kvh * G + (row0 + i) % G, pos + (row0 + i) / G, Hq, scale);
         return;
     }
-    l += __shfl_xor(l, 32, 64);
+    l = xor_add<32>(l);
     st[wave][0][lane] = mx; st[wave][1][lane] = l;
     __syncthreads();
     float all = st[0][0][lane];

@@ -57,7 +57,7 @@ __device__ __forceinline__ void prompt_attend(const half8 (&qf)[NJ], const uint4
         float mx = s[0];
 #pragma unroll
         for (int v = 1; v < 16; v++) mx = fmaxf(mx, s[v]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        mx = xor_max<32>(mx);
         const float m_new = fmaxf(m_run, mx);
         if (__any(m_new > m_run)) {
             const float alpha = exp2f(m_run - m_new);
@@ -92,7 +92,7 @@ __device__ __forceinline__ void prompt_attend(const half8 (&qf)[NJ], const uint4
         step(kb + 1, buf1);
         FA_WAIT_AND_BARRIER();
     }
-    l_run += __shfl_xor(l_run, 32, WAVE);
+    l_run = xor_add<32>(l_run);
 }
 
 // a lane's query row divided by its weight sum, columns below vdim
