@@ -191,6 +191,26 @@ __global__ __launch_bounds__(256) void q8_operand_to_f16(lmhip::WeightOp W, int 
     for (int j = 0; j < 4; j++) out[tile * 256 + j * 64 + lane] = w[j];
 }
 
+// dst (tiled, from row block rb0 on) <- src row-major F16 [rows, cols], cols a multiple of 8: a wave turns one 32 x 64 tile, read as
+// 128 bytes of each row and written, through LDS, 1 KB at a time.  Pieces of eight that lie past the matrix are not written.
+__global__ __launch_bounds__(256) void tile_f16_rows(const half_t *__restrict__ src, int rows, int cols, half8 *__restrict__ dst, int Kb, int rb0)
+{
+    __shared__ half8 t[4][32][9];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = blockIdx.x * 4 + wave, rb = blockIdx.y;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int r = rb * 32 + 8 * i + (lane >> 3), c = kb * 64 + 8 * (lane & 7);
+        if (r < rows && c < cols) t[wave][8 * i + (lane >> 3)][lane & 7] = *reinterpret_cast<const half8 *>(src + (size_t)r * cols + c);
+    }
+    __syncthreads();
+    half8 *p = dst + ((size_t)(rb0 + rb) * Kb + kb) * 256 + lane;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int r = rb * 32 + (lane & 31), c = kb * 64 + (lane >> 5) * 32 + 8 * j;
+        if (r < rows && c < cols) p[j * 64] = t[wave][lane & 31][(lane >> 5) * 4 + j];
+    }
+}
+
 // Row-major F16 [rows, cols] -> tiled layout, optionally transposed; 64x64 element tiles via LDS
 // so that both the reads (along cols) and the writes (16-byte groups along the destination K) coalesce.
 __global__ __launch_bounds__(256) void tile_f16(const half_t *__restrict__ src, int rows, int cols,
@@ -493,6 +513,12 @@ void launch_tile_f16(const half_t *src, int rows, int cols, half_t *dst_tiled, i
                      int row_off, int k_off, int transpose)
 {
     if (rows <= 0 || cols <= 0) return;
+    if (!transpose && k_off == 0 && row_off % 32 == 0 && cols % 8 == 0 && !((uintptr_t)src & 15)) {
+        hipLaunchKernelGGL(tile_f16_rows, dim3((tiled_kb(cols) + 3) / 4, tiled_rb(rows)), dim3(256), 0, stream(), src, rows, cols,
+                           reinterpret_cast<half8 *>(dst_tiled), Kb_dst, row_off / 32);
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
     hipLaunchKernelGGL(tile_f16, dim3((cols + 63) / 64, (rows + 63) / 64), dim3(256), 0, stream(),
                        src, rows, cols, dst_tiled, Kb_dst, row_off, k_off, transpose);
     HIP_CHECK(hipGetLastError());
