@@ -28,6 +28,37 @@ __device__ __forceinline__ float planes_at(const SplitPlanes &p, int M, int m, i
     return v;
 }
 
+// Four neighbouring elements (n, N and the plane strides multiples of four, P and P2 16-byte aligned); the planes are requested
+// four at a time and added in their order.
+__device__ __forceinline__ float4v planes4_at(const SplitPlanes &p, int M, int m, int n)
+{
+    const float *ph = p.P + (size_t)m * p.N + n, *pl = ph + (size_t)M * p.N;
+    float4v hi = *reinterpret_cast<const float4v *>(ph), lo = *reinterpret_cast<const float4v *>(pl);
+    for (int s0 = 1; s0 < p.S; s0 += 4) {
+        float4v h[4], l[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const size_t o = (size_t)min(s0 + q, p.S - 1) * p.plane;
+            h[q] = *reinterpret_cast<const float4v *>(ph + o);
+            l[q] = *reinterpret_cast<const float4v *>(pl + o);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (s0 + q < p.S) { hi += h[q]; lo += l[q]; }
+    }
+    const float ih = p.inv[m], il = p.inv[M + m];
+    float4v r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = fmaf(lo[e], il, hi[e] * ih);
+    if (p.P2) {
+        float4v z = {};
+        for (int s = 0; s < p.S2; s++) z += *reinterpret_cast<const float4v *>(p.P2 + s * p.plane2 + (size_t)m * p.N + n);
+#pragma unroll
+        for (int e = 0; e < 4; e++) r[e] = fmaf(z[e], ih * (1.0f / Q8_RESIDUAL_SCALE), r[e]);
+    }
+    return r;
+}
+
 // What follows the Q|K|V product for M tokens at positions pos .. pos + M - 1: adapter terms, per-head RMSNorm and RoPE; q to
 // [M][Hq * hd], k and v into the rows of the caches [Hkv, max_seq, hd].
 struct PromptHeads {

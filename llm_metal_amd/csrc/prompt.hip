@@ -260,27 +260,7 @@ __global__ __launch_bounds__(1024) void k_prompt_glu(SplitPlanes gu, half_t *__r
 #pragma unroll
         for (int e = 0; e < 4; e++) v[u][e] = 0.f;
         if (n < IS) {
-            auto four = [&](int at) __attribute__((always_inline)) {
-                const size_t ld = (size_t)gu.N;
-                const float *ph = gu.P + (size_t)m * ld + at, *pl = ph + (size_t)M * ld;
-                float4v hi = {}, lo = {};
-                for (int s = 0; s < gu.S; s++) {
-                    hi += *reinterpret_cast<const float4v *>(ph + s * gu.plane);
-                    lo += *reinterpret_cast<const float4v *>(pl + s * gu.plane);
-                }
-                const float ih = gu.inv[m], il = gu.inv[M + m];
-                float4v r;
-#pragma unroll
-                for (int e = 0; e < 4; e++) r[e] = fmaf(lo[e], il, hi[e] * ih);
-                if (gu.P2) {
-                    float4v z = {};
-                    for (int s = 0; s < gu.S2; s++) z += *reinterpret_cast<const float4v *>(gu.P2 + s * gu.plane2 + (size_t)m * ld + at);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) r[e] = fmaf(z[e], ih * (1.0f / Q8_RESIDUAL_SCALE), r[e]);
-                }
-                return r;
-            };
-            const float4v g = four(n), up = four(IS + n);
+            const float4v g = planes4_at(gu, M, m, n), up = planes4_at(gu, M, m, IS + n);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float act = GELU ? 0.5f * g[e] * (1.0f + tanhf(gelu_inner(g[e]))) : g[e] / (1.0f + expf(-g[e]));

@@ -111,3 +111,17 @@ def test_q8_weights_beyond_a_half_take_tokens_one_by_one():
         want = one_by_one(inf, toks)
         inf.reset()
         assert np.isfinite(want).all() and np.array_equal(inf.forward_tokens(toks, range(40)), want)
+
+
+@pytest.mark.parametrize("D,IS", [(32, 260), (1184, 352), (4128, 416)])
+def test_norms_of_a_batch(D, IS):
+    """The norm between a batch's products in pieces of four columns: a row shorter than its padding, one piece and two per
+    thread.  Single sequences go another way."""
+    print(D, IS, flush=True)
+    c = SFTConfig("odd", QWEN3, NL=2, D=D, Hq=2, Hkv=1, hd=64, IS=IS, V=512)
+    model = make_model(c, seed=13, gamma_jitter=0.1)
+    seqs = np.random.default_rng(5).integers(0, c.V, (3, 4))
+    with InferenceState(c, model, max_seq=8) as inf:
+        got = np.stack([inf.step_batch(seqs[:, i], i) for i in range(4)], axis=1)
+        for b in range(3):
+            assert maxrel(got[b], one_by_one(inf, [int(t) for t in seqs[b]])) < TOL
