@@ -219,18 +219,63 @@ __global__ __launch_bounds__(256) void k_delta_prepare(DeltaRows a, int DP)
     }
 }
 
-// grid (ceil(vdim / 16), H, B); a workgroup owns sixteen columns of a head's state, each of its waves TPW tiles of sixteen
+// grid (ceil(vdim / 16), H, B); a workgroup owns sixteen columns of a head's state, each of NW waves TPW tiles of sixteen
 // rows, held as the accumulators of v_mfma_f32_16x16x4_f32 (fp32 operands and sums).  The register order of an accumulator
 // -- column lane & 15, rows 4 (lane >> 4) + 0 .. 3 -- is also a legal order of the reduction index of an operand, so S, U
-// and V - P go from one product into the next as they are.  Per chunk the waves add their parts of P and W through LDS (one
-// barrier); everything from memory is asked for SETS chunks ahead.
+// and V - P go from one product into the next as they are.  Per chunk the waves add their parts of P through LDS (one
+// barrier).  One chunk's chain bounds the kernel -- P, its sum over the waves, U, S, 1.1 us a chunk when everything a chunk
+// needs stood in it -- so what the next chunk does not wait for is taken out of it:
+//   - the products with the queries run while the parts of P come back from LDS;
+//   - a wave of its own, one chunk behind, adds up the waves' parts of W, applies B U and writes the outputs;
+//   - operands are asked for SETS chunks ahead, a few between each group of matrix instructions: in one go they hold the
+//     waves up at the CU's address unit.
+// 2000 tokens, 8 heads of 128 x 128: 137 us with all of it in the chain, 102 now (which XCD a
+// head's workgroups share makes no difference).
 template <int TPW, int SETS, int NW>
-__global__ __launch_bounds__(64 * NW) void k_delta_chunks(DeltaRows a, int DP, int chunks)
+__global__ __launch_bounds__(64 * (NW + 1)) void k_delta_chunks(DeltaRows a, int DP, int chunks)
 {
-    __shared__ float4v red[2][NW][2][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, r4 = lane >> 4;
+    __shared__ float4v red[2][NW][64], part[2][NW + 1][64];   // parts of P; parts of W and, behind them, U
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, r4 = lane >> 4;
     const int h = blockIdx.y, b = blockIdx.z, T = a.r.T, j = blockIdx.x * 16 + c, jc = min(j, a.vdim - 1);
     const int vd = a.H * a.vdim;
+    const size_t chunk0 = (size_t)b * chunks;
+    const uint32_t mb0 = (uint32_t)(c * CT + 4 * r4);
+    auto at4 = [](const float *base, uint32_t i) __attribute__((always_inline)) {
+        return *reinterpret_cast<const float4v *>(reinterpret_cast<const char *>(base) + 4u * i);
+    };
+    auto at1 = [](const float *base, uint32_t i) __attribute__((always_inline)) {
+        return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + 4u * i);
+    };
+
+    if (wave == NW) {                                     // the outputs; as many barriers as the other waves meet
+        constexpr int AHEAD = 4;
+        float *const o = a.o + (size_t)b * T * vd;
+        auto bm = [&](int ck) __attribute__((always_inline)) { return at4(a.mb + ((chunk0 + min(ck, chunks - 1)) * a.H + h) * (2 * CT * CT) + CT * CT, mb0); };
+        float4v bs[AHEAD];
+#pragma unroll
+        for (int n = 0; n < AHEAD; n++) bs[n] = bm(n);
+        __syncthreads();
+        for (int c0 = 0; c0 < chunks; c0 += AHEAD)
+#pragma unroll
+            for (int n = 0; n < AHEAD; n++) {
+                const int ck = c0 + n;
+                if (ck >= chunks) break;                  // uniform
+                __syncthreads();
+                float4v w = part[ck & 1][0][lane];
+#pragma unroll
+                for (int i = 1; i < NW; i++) w += part[ck & 1][i][lane];
+                const float4v u = part[ck & 1][NW][lane];
+#pragma unroll
+                for (int v = 0; v < 4; v++) w = __builtin_amdgcn_mfma_f32_16x16x4f32(bs[n][v], u[v], w, 0, 0, 0);
+                bs[n] = bm(ck + AHEAD);
+                float *to = o + (size_t)(ck * CT + 4 * r4) * vd + h * a.vdim + jc;
+                const int last = T - ck * CT - 4 * r4;
+#pragma unroll
+                for (int v = 0; v < 4; v++) if (j < a.vdim && v < last) to[(size_t)v * vd] = w[v];
+            }
+        return;
+    }
+
     float *Sg = a.S + (((size_t)b * a.H + h) * a.vdim + jc) * a.dim;
     const int d0 = wave * TPW * 16 + 4 * r4;              // rows d0 + 16 tile + 0 .. 3
     float4v S[TPW];
@@ -241,82 +286,82 @@ __global__ __launch_bounds__(64 * NW) void k_delta_chunks(DeltaRows a, int DP, i
             const int d = d0 + 16 * i + v;
             S[i][v] = (a.r.pos > 0 && d < a.dim) ? Sg[d] : 0.f;
         }
-    auto at4 = [](const float *base, uint32_t i) __attribute__((always_inline)) {
-        return *reinterpret_cast<const float4v *>(reinterpret_cast<const char *>(base) + 4u * i);
+    const uint32_t frag = (uint32_t)(wave * TPW * 256 + lane * 4);
+    struct Set { float4v k[TPW], q[TPW], u[TPW], g[TPW], m, v; };
+    struct From { const float *k, *q, *u, *g, *m, *v; int last; };     // (a chunk's own part of every address is scalar)
+    auto from = [&](int ck) __attribute__((always_inline)) {
+        const int cc = min(ck, chunks - 1);
+        const size_t chunk = (chunk0 + cc) * a.H + h, f = chunk * (size_t)(DP * CT);
+        return From{a.kd + f, a.qd + f, a.ku + f, a.gc + chunk * DP, a.mb + chunk * (2 * CT * CT), a.v + ((size_t)b * T + (size_t)cc * CT) * vd, T - 1 - cc * CT};
     };
-    auto at1 = [](const float *base, uint32_t i) __attribute__((always_inline)) {
-        return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + 4u * i);
+    auto fetch_k = [&](Set &x, const From &y, int i) __attribute__((always_inline)) { x.k[i] = at4(y.k, frag + 256 * i); x.u[i] = at4(y.u, frag + 256 * i); };
+    auto fetch_q = [&](Set &x, const From &y, int i) __attribute__((always_inline)) { x.q[i] = at4(y.q, frag + 256 * i); x.g[i] = at4(y.g, (uint32_t)(d0 + 16 * i)); };
+    auto fetch_v = [&](Set &x, const From &y, int v) __attribute__((always_inline)) {
+        if (v == 0) x.m = at4(y.m, mb0);
+        x.v[v] = at1(y.v, (uint32_t)min(4 * r4 + v, y.last) * (uint32_t)vd + (uint32_t)(h * a.vdim + jc));
     };
-    const uint32_t out0 = (uint32_t)((b * T + 4 * r4) * vd + h * a.vdim + jc);
-    struct Set { float4v k[TPW], q[TPW], u[TPW], g[TPW], m, b, v; };
-    auto fetch = [&](Set &x, int ck) __attribute__((always_inline)) {
-        const uint32_t chunk = (uint32_t)((b * chunks + min(ck, chunks - 1)) * a.H + h);
-        const uint32_t f = chunk * (uint32_t)(DP * CT) + (uint32_t)(wave * TPW * 256 + lane * 4);
-#pragma unroll
-        for (int i = 0; i < TPW; i++) {
-            x.k[i] = at4(a.kd, f + 256 * i); x.q[i] = at4(a.qd, f + 256 * i); x.u[i] = at4(a.ku, f + 256 * i);
-            x.g[i] = at4(a.gc, chunk * (uint32_t)DP + (uint32_t)(d0 + 16 * i));
-        }
-        const uint32_t mb = chunk * (uint32_t)(2 * CT * CT) + (uint32_t)(c * CT + 4 * r4);
-        x.m = at4(a.mb, mb); x.b = at4(a.mb, mb + CT * CT);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            x.v[v] = at1(a.v, (uint32_t)(b * T + min(min(ck, chunks - 1) * CT + 4 * r4 + v, T - 1)) * (uint32_t)vd + (uint32_t)(h * a.vdim + jc));
-    };
-    auto take = [&](const Set &x, int ck) __attribute__((always_inline)) {
+    auto take = [&](const Set &x, int ck, Set &next, const From &y) __attribute__((always_inline)) {
         float4v p = {0.f, 0.f, 0.f, 0.f}, w = p;
 #pragma unroll
-        for (int i = 0; i < TPW; i++)
+        for (int i = 0; i < TPW; i++) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                p = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][v], S[i][v], p, 0, 0, 0);
-                w = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][v], S[i][v], w, 0, 0, 0);
-            }
-        float4v(&rd)[NW][2][64] = red[ck & 1];
-        rd[wave][0][lane] = p; rd[wave][1][lane] = w;
+            for (int v = 0; v < 4; v++) p = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][v], S[i][v], p, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_q(next, y, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        red[ck & 1][wave][lane] = p;
         __syncthreads();
-        float4v pn[NW], wn[NW];
+        float4v pn[NW];
 #pragma unroll
-        for (int n = 0; n < NW; n++) pn[n] = rd[n][0][lane];
+        for (int n = 0; n < NW; n++) pn[n] = red[ck & 1][n][lane];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int n = 0; n < NW; n++) wn[n] = rd[n][1][lane];
-        p = pn[0]; w = wn[0];
+        for (int i = 0; i < TPW; i++) {
 #pragma unroll
-        for (int n = 1; n < NW; n++) { p += pn[n]; w += wn[n]; }
+            for (int v = 0; v < 4; v++) w = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][v], S[i][v], w, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_k(next, y, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < TPW; i++) S[i] *= x.g[i];
+        p = pn[0];
+#pragma unroll
+        for (int n = 1; n < NW; n++) p += pn[n];
         const float4v z = x.v - p;
         float4v u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int v = 0; v < 4; v++) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[v], z[v], u, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < TPW; i++) {
-            S[i] *= x.g[i];
+        for (int v = 0; v < 4; v++) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.u[i][v], u[v], S[i], 0, 0, 0);
-        }
-        if (ck % NW == wave) {                            // the waves take the outputs in turn
-#pragma unroll
-            for (int v = 0; v < 4; v++) w = __builtin_amdgcn_mfma_f32_16x16x4f32(x.b[v], u[v], w, 0, 0, 0);
-            char *to = reinterpret_cast<char *>(a.o) + 4u * (out0 + (uint32_t)(ck * CT) * (uint32_t)vd);
-            if (j < a.vdim) {
-                if (ck * CT + CT <= T) {
-#pragma unroll
-                    for (int v = 0; v < 4; v++) *reinterpret_cast<float *>(to + 4u * (uint32_t)(v * vd)) = w[v];
-                } else
-#pragma unroll
-                    for (int v = 0; v < 4; v++) if (ck * CT + 4 * r4 + v < T) *reinterpret_cast<float *>(to + 4u * (uint32_t)(v * vd)) = w[v];
+            for (int i = 0; i < TPW; i++) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.u[i][v], u[v], S[i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_v(next, y, v);
+            if (v == 0) {                                 // (read behind the next barrier, written again behind the one after)
+                part[ck & 1][wave][lane] = w;
+                if (wave == 0) part[ck & 1][NW][lane] = u;
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     Set x[SETS];
 #pragma unroll
-    for (int n = 0; n < SETS - 1; n++) fetch(x[n], n);
+    for (int n = 0; n < SETS - 1; n++) {
+        const From y = from(n);
+#pragma unroll
+        for (int i = 0; i < TPW; i++) { fetch_k(x[n], y, i); fetch_q(x[n], y, i); }
+#pragma unroll
+        for (int v = 0; v < 4; v++) fetch_v(x[n], y, v);
+    }
     for (int ck = 0; ck < chunks; ck += SETS)
 #pragma unroll
         for (int n = 0; n < SETS; n++) {
             if (ck + n >= chunks) break;                  // uniform
-            fetch(x[(n + SETS - 1) % SETS], ck + n + SETS - 1);
-            take(x[n], ck + n);
+            take(x[n], ck + n, x[(n + SETS - 1) % SETS], from(ck + n + SETS - 1));
         }
+    __syncthreads();
     if (j < a.vdim)
 #pragma unroll
         for (int i = 0; i < TPW; i++)
@@ -402,7 +447,7 @@ __global__ __launch_bounds__(256) void k_cat_rows(CatRows a)
 
 }  // namespace
 
-// waves of a workgroup of k_delta_chunks and tiles of each
+// waves of a workgroup of k_delta_chunks that hold the state, and tiles of each
 struct ChunkShape { int nw, tpw; int dp() const { return nw * tpw * 16; } };
 static ChunkShape chunk_shape(int dim)
 {
@@ -425,7 +470,7 @@ void launch_delta_inputs(const DeltaRows &a)
 void launch_delta_scan(const DeltaRows &a)
 {
     const ChunkShape cs = chunk_shape(a.dim);
-    const dim3 grid((a.vdim + 15) / 16, a.H, a.r.B), block(64 * cs.nw);
+    const dim3 grid((a.vdim + 15) / 16, a.H, a.r.B), block(64 * (cs.nw + 1));
     const int chunks = delta_chunks(a.r.T);
 #define CHUNKS(T_, S_, N_) LAUNCH((k_delta_chunks<T_, S_, N_>), grid, block, 0, a, cs.dp(), chunks)
     if (cs.tpw == 2) CHUNKS(2, 4, 4); else if (cs.tpw == 4) CHUNKS(4, 2, 4);

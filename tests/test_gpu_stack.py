@@ -111,6 +111,22 @@ def test_lock_step_batches_against_each_alone(fmt, mixed, tmp_path):
         assert logit_error(inf.forward_tokens(list(seqs[0]), range(45)), want[0]) < TOL[fmt]
 
 
+@pytest.mark.parametrize("dim", [16, 32, 48, 64, 128, 200])
+def test_chunks_of_a_recurrence(dim, tmp_path):
+    """Prompts of one chunk of sixteen tokens to nine, full and not (operands are asked for, and outputs written, chunks apart), for
+    each number of waves that hold the state; decoding goes on from it."""
+    say("chunks", dim)
+    cfg = config([(delta(2, 1, dim, 40, 3), None)], width=64)
+    m = Model(cfg, tmp_path)
+    toks = m.tokens(146, seed=9)
+    want = so.run(cfg, m.W, toks)
+    with state(m, "f32", 160) as inf:
+        for n in (2, 15, 16, 17, 33, 48, 64, 65, 80, 97, 144):
+            inf.reset()
+            assert logit_error(inf.forward_tokens(toks[:n], range(n)), want[:n]) < TOL["f32"], n
+            assert logit_error(inf.forward_token(toks[n])[None], want[n:n + 1]) < TOL["f32"], n
+
+
 @pytest.mark.parametrize("window", [1, 2, 15, 16, 17, 63, 64, 65, 100])
 def test_window_edges(window, tmp_path):
     """One attention layer: a token just outside the window must not matter at all, one just inside must, in a prompt and in
