@@ -13,7 +13,7 @@ from llm_metal_amd.configs import C1
 from llm_metal_amd.sft import InferenceState
 from llm_metal_amd.synth import make_model, write_stack_checkpoint
 from oracle import stack_oracle as so
-from tests.stack_models import MODELS, Model, config, channel, delta, latent, logit_error, moe
+from tests.stack_models import MODELS, Model, around, channel, config, delta, dense, grouped, latent, logit_error, mlstm, moe
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -125,6 +125,19 @@ def test_chunks_of_a_recurrence(dim, tmp_path):
             inf.reset()
             assert logit_error(inf.forward_tokens(toks[:n], range(n)), want[:n]) < TOL["f32"], n
             assert logit_error(inf.forward_token(toks[n])[None], want[n:n + 1]) < TOL["f32"], n
+
+
+@pytest.mark.parametrize("width", [1024, 1088, 1536, 1600, 2048, 2112])
+def test_widths_of_decoded_rows(width, tmp_path):
+    """Decoding with the norms formed inside the products: rows of two, three and four steps of 512 columns, the last one full and
+    not, asked for ahead of the norm, and longer ones."""
+    say("widths", width)
+    cfg = around([(mlstm(2, 16, 16, 15.0), None), (grouped(2, 1, 16, 16, 9), dense(40))], width=width)
+    m = Model(cfg, tmp_path)
+    toks = m.tokens(6, seed=3)
+    want = so.run(cfg, m.W, toks)
+    with state(m, "f16") as inf:
+        assert logit_error(np.stack([inf.forward_token(t) for t in toks]), want) < TOL["f16"]
 
 
 @pytest.mark.parametrize("window", [1, 2, 15, 16, 17, 63, 64, 65, 100])
