@@ -392,6 +392,52 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
     }
 }
 
+// Few long rows: the four waves of a workgroup share one, each with every fourth 512-column step, U of them requested at once, so a
+// row is one or two trips to memory instead of one per 2048 columns (and the last trip asks for nothing behind the row).
+// With a wave per row such a matrix has some five waves on a CU and a chain of several trips in each.  Cold weights: 1152 x 6912 Q8_0
+// 7.4 -> 5.0 us, F16 6.7 -> 5.8; 1536 x 4096 Q8_0 5.0 -> 3.9, 1024 x 4096 F16 4.3 -> 3.7.  Bound by the launch and one trip.
+template <int FMT, int U>
+__global__ __launch_bounds__(TB) void k_matvec_split(const void *__restrict__ Wp, const half_t *__restrict__ scales,
+                                                     const float *__restrict__ x, float *__restrict__ y, int cols)
+{
+    __shared__ float red[4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const size_t row = (size_t)blockIdx.x * cols;
+    float acc = 0.f;
+    for (int c0 = 512 * wave; c0 < cols; c0 += 2048 * U) {
+        half8 w16[U];
+        uint2v w8[U];
+        float d[U];
+        float4v x0[U], x1[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int c = min(c0 + 2048 * u + lane * 8, cols - 8);          // clamped: loads stay unconditional
+            if (FMT == 0) w16[u] = __builtin_nontemporal_load(reinterpret_cast<const half8 *>((const half_t *)Wp + row + c));
+            else {
+                w8[u] = __builtin_nontemporal_load(reinterpret_cast<const uint2v *>((const int8_t *)Wp + row + c));
+                d[u] = (float)scales[(row + c) >> 5];
+            }
+            x0[u] = *reinterpret_cast<const float4v *>(&x[c]);
+            x1[u] = *reinterpret_cast<const float4v *>(&x[c + 4]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool live = c0 + 2048 * u + lane * 8 < cols;
+            float p = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float xv = live ? (e < 4 ? x0[u][e & 3] : x1[u][e & 3]) : 0.f;
+                p = fmaf(FMT == 0 ? (float)w16[u][e] : (float)(int8_t)(w8[u][e >> 2] >> (8 * (e & 3))), xv, FMT == 0 && e == 0 ? acc : p);
+            }
+            acc = FMT == 0 ? p : fmaf(d[u], p, acc);
+        }
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) red[wave] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) y[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
 // Any cols / alignment: one wave per row, lanes stride single elements.
 __global__ __launch_bounds__(TB) void k_matvec_any(const half_t *__restrict__ W, const float *__restrict__ X,
                                                    float *__restrict__ Y, int rows, int cols, int B)
@@ -408,6 +454,11 @@ __global__ __launch_bounds__(TB) void k_matvec_any(const half_t *__restrict__ W,
     }
 }
 
+// A workgroup per row (k_matvec_split) up to this many rows and bytes: beyond them the waves of k_matvec keep memory busy by
+// themselves and its longer runs per row are faster (F16, wave / workgroup per row: 1536 x 8192 7.35 / 7.7 us, 2048 x 8192 7.0 / 9.3,
+// 2560 x 9728 11.5 / 13.9).
+constexpr int SPLIT_ROWS = 1536;
+constexpr size_t SPLIT_BYTES = (size_t)20 << 20;
 // Rows per wave grow with the matrix so that mid-sized weights (a few thousand rows) still put 16 waves on every CU.
 template <int FMT>
 void launch_matvec(const void *W, const half_t *scales, const float *x, float *y, int rows, int cols)
@@ -422,10 +473,18 @@ void launch_matvec(const void *W, const half_t *scales, const float *x, float *y
     if (prof) hipExtLaunchKernelGGL((k_matvec<FMT, R_, U_, XL_>), grid, dim3(TB), L_, stream(), ev_a, ev_b, 0, W, scales, x, y, rows, cols, NormIn{}); \
     else hipLaunchKernelGGL((k_matvec<FMT, R_, U_, XL_>), grid, dim3(TB), L_, stream(), W, scales, x, y, rows, cols, NormIn{}); \
     HIP_CHECK(hipGetLastError()); } while (0)
+#define SPLIT_LAUNCH(U_) do { \
+    if (prof) hipExtLaunchKernelGGL((k_matvec_split<FMT, U_>), dim3(rows), dim3(TB), 0, stream(), ev_a, ev_b, 0, W, scales, x, y, cols); \
+    else hipLaunchKernelGGL((k_matvec_split<FMT, U_>), dim3(rows), dim3(TB), 0, stream(), W, scales, x, y, cols); \
+    HIP_CHECK(hipGetLastError()); } while (0)
     if (rows >= 32768 && lds <= 40 * 1024) MATVEC_LAUNCH(4, 2, 1, 16, lds);
     else if (rows >= 32768) MATVEC_LAUNCH(4, 2, 0, 16, 0);
     else if (rows >= 8192) MATVEC_LAUNCH(2, 2, 0, 8, 0);
+    else if (rows <= SPLIT_ROWS && cols >= 4096 && (size_t)rows * cols * (FMT == 0 ? 2 : 1) <= SPLIT_BYTES) {
+        if (cols > 4096) SPLIT_LAUNCH(4); else SPLIT_LAUNCH(2);
+    }
     else MATVEC_LAUNCH(1, 4, 0, 4, 0);
+#undef SPLIT_LAUNCH
 #undef MATVEC_LAUNCH
 }
 

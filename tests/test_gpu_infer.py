@@ -49,6 +49,25 @@ def test_f16_matvec(dev, rows, cols):
     assert maxrel(yb.read(F), ref) < 2e-5
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 4096), (37, 4104), (1536, 4608), (1537, 4128), (130, 6912), (9, 8192), (1300, 8192), (3, 8200), (50, 16896)])
+def test_matvec_with_a_row_per_workgroup(dev, rows, cols):
+    """Few long rows: the last step of 512 columns full and not, waves with unequal numbers of steps, more than one trip; Q8_0
+    where the columns are whole blocks."""
+    say("matvec, a row per workgroup", rows, cols)
+    rng = np.random.default_rng(rows + cols)
+    W, x, ref = rnd(rng, rows, cols, scale=0.05).astype(np.float16), rnd(rng, cols), np.zeros(rows, F)
+    op("f32", "or_f16_batch_matvec", W.view(np.uint16), x, ref, rows, cols, 1)
+    wb, xb, yb = dev.up(W), dev.up(x), dev.empty(rows * 4)
+    dev.L.metal_enqueue_f16_matvec(wb.h, xb.h, yb.h, rows, cols)
+    assert maxrel(yb.read(F), ref) < 2e-5
+    if cols % 32 == 0:
+        blocks = oracle.q8_quantize(W.astype(F))
+        op("f32", "or_q8_matvec", blocks, x, ref, rows, cols // 32)
+        qb = dev.up(blocks)
+        dev.L.metal_enqueue_q8_matvec(qb.h, xb.h, yb.h, rows, cols // 32)
+        assert maxrel(yb.read(F), ref) < 2e-5
+
+
 @pytest.mark.parametrize("rows,cols,B", [(4112, 1024, 2), (300, 2560, 3), (4096, 512, 4), (515, 1152, 5), (4096, 256, 8),
                                          (1000, 512, 9), (2048, 640, 32), (64, 50, 3)])
 def test_f16_batch_matvec(dev, rows, cols, B):
