@@ -646,7 +646,7 @@ int gemm_ring_enabled() { return g_ring; }
 
 // Which kernel multiplies an [M, K] activation block with an [N, K] weight.  Measured on MI355X (Qwen3-4B shapes):
 // the 128 x 256 LDS-tiled kernel wins for F16 weights once there is about one block per CU (2048 rows: 490-650
-// against 300 TFLOP/s for the weight-streaming kernel).  With Q8_0 weights the streaming kernel, whose waves overlap
+// against 300 TFLOP/s for the weight-streaming kernel); between 65 and 1023 rows mid_takes_big compares what each would take.  With Q8_0 weights the streaming kernel, whose waves overlap
 // each other's unpacking and MFMAs, is ahead of the large-M kernel unpacking tiles into LDS itself (400-470 against
 // 340-460 TFLOP/s), but from 1024 rows on it pays to dequantise the operand once into an F16 image (3 bytes of extra
 // HBM traffic per weight) and run the large-M kernel on that instead of unpacking every tile again for each 64 rows

@@ -2,7 +2,7 @@
 // (batch * seq = 2048 in the Q8_0 configuration), where a weight tile is reused by enough activation rows
 // that the matrix cores, not HBM, bound the product.  Same operands as the weight-streaming kernel
 // (gemm.h: tiled fp16 activations with per-row power-of-two factors; F16 or Q8_0 weight tiles), same
-// arithmetic (v_mfma_f32_32x32x16_f16, fp32 accumulation), one launch, no K split.
+// arithmetic (v_mfma_f32_32x32x16_f16, fp32 accumulation), one launch; K chunks (planes) where the blocks leave CUs idle.
 //
 // A workgroup of four waves owns a 128 x 256 block of C and walks K in steps of 64.  Per step every wave
 // fetches one 32-row block of the activation tile and two of the weight tile from L2/HBM in the MFMA

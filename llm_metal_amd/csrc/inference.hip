@@ -3,10 +3,10 @@
 // Every step is enqueued on the library's one stream; the host waits once per token, for the logits or for
 // the argmax computed on the GPU.
 //
-// One decode step computes what src/nn/fast_inference.c:376-467 computes, in 9 launches per layer instead of 17
-// (10 instead of 23 with adapters): Q|K|V and gate|up are one matrix each (row concatenation, built when the state is
-// created), the residual add travels with the RMSNorm that follows it, and one kernel does LoRA up-projection,
-// per-head RMSNorm, RoPE and the KV-cache store for all heads.
+// One decode step computes what src/nn/fast_inference.c:376-467 computes, in 5 launches per layer instead of 17: Q|K|V and
+// gate|up are one matrix each (row concatenation, built when the state is created), the products that follow a norm form it
+// themselves (matvec_norm, matvec_norms_around), and the attention launch does LoRA up-projection, per-head RMSNorm, RoPE and
+// the KV-cache store for the new token.  Prompts of five tokens and more run many tokens per step (PromptRun).
 #include "backend.h"
 #include "devutil.h"
 #include "fused.h"
