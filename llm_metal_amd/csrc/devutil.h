@@ -14,14 +14,14 @@ typedef float    float4v __attribute__((ext_vector_type(4)));
 #define WAVE 64
 
 // v + (or max with) the value of lane ^ O, without the trip through LDS that __shfl_xor takes: DPP inside rows of sixteen lanes,
-// gfx950's row and half swaps across them.  Every lane of the wave active.  The same operands meet as with __shfl_xor, so the
-// results are the same bit for bit; six dependent steps take some 50 cycles instead of 700 (Q8_0 head of
+// gfx950's row and half swaps across them.  Every lane of the wave active.  The same operands meet in the same order as with
+// __shfl_xor (a sum of products needs wave_sum_products for that); six dependent steps take some 50 cycles instead of 700 (Q8_0 head of
 // 262 144 rows, one reduction per row: 86 -> 77 us; k_qkv_bwd_rows at 64 rows 9.6 -> 8.0; gated product with its norms 12.9 -> 11.7).
 template <int CTRL, int BANKS = 0xF> __device__ __forceinline__ float dpp_move(float old, float v)
 {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v), CTRL, 0xF, BANKS, false));
 }
-struct LanePair { float a, b; };                           // v of this lane and of lane ^ O, in either order
+struct LanePair { float a, b; };                           // v of this lane and of lane ^ O; in either order, the lower lane's first where O is 16 or 32
 template <int O> __device__ __forceinline__ LanePair lane_pair(float v)
 {
     static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "a power of two below 64");
@@ -45,6 +45,16 @@ __device__ __forceinline__ float wave_sum(float v)
     return xor_add<1>(xor_add<2>(xor_add<4>(xor_add<8>(xor_add<16>(xor_add<32>(v))))));
 }
 
+// The sum of a b over the wave.  Its first step adds the lane's own product, not yet rounded, to the rounded one of lane ^ 32:
+// one fused operation, which `v += __shfl_xor(v, 32)` becomes when v is a product, and wave_sum(a * b), whose swap takes rounded
+// products from both, does not.  (The last bit of a row's log-sum-exp turns roundings of its loss gradient to fp16: adapters after a
+// step 1e-4 .. 2e-3 apart.)
+__device__ __forceinline__ float wave_sum_products(float a, float b)
+{
+    const LanePair p = lane_pair<32>(__fmul_rn(a, b));     // a: of the lower half's lane, b: of the upper half's
+    return xor_add<1>(xor_add<2>(xor_add<4>(xor_add<8>(xor_add<16>(fmaf(a, b, threadIdx.x & 32 ? p.a : p.b))))));
+}
+
 __device__ __forceinline__ float wave_max(float v)
 {
     return xor_max<1>(xor_max<2>(xor_max<4>(xor_max<8>(xor_max<16>(xor_max<32>(v))))));
@@ -53,9 +63,8 @@ __device__ __forceinline__ float wave_max(float v)
 // Workgroup reductions for blocks of up to 1024 threads (16 waves).  `smem`
 // must hold 16 floats; every thread gets the result.  Two barriers per call,
 // so the same `smem` may be reused by the next call.
-__device__ __forceinline__ float block_sum(float v, float *smem)
+__device__ __forceinline__ float block_sum_waves(float v, float *smem)       // v: the sum of the thread's wave
 {
-    v = wave_sum(v);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     if (lane == 0) smem[w] = v;
     __syncthreads();
@@ -65,10 +74,12 @@ __device__ __forceinline__ float block_sum(float v, float *smem)
     return r;
 }
 
+__device__ __forceinline__ float block_sum(float v, float *smem) { return block_sum_waves(wave_sum(v), smem); }
+__device__ __forceinline__ float block_sum_products(float a, float b, float *smem) { return block_sum_waves(wave_sum_products(a, b), smem); }
+
 // Two sums for one pair of barriers; `smem` must hold 32 floats.  Each sum is formed in the order block_sum forms it.
-__device__ __forceinline__ void block_sum2(float &a, float &b, float *smem)
+__device__ __forceinline__ void block_sum2_waves(float &a, float &b, float *smem)
 {
-    a = wave_sum(a); b = wave_sum(b);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     if (lane == 0) { smem[w] = a; smem[16 + w] = b; }
     __syncthreads();
@@ -77,6 +88,7 @@ __device__ __forceinline__ void block_sum2(float &a, float &b, float *smem)
     __syncthreads();
     a = ra; b = rb;
 }
+__device__ __forceinline__ void block_sum2(float &a, float &b, float *smem) { a = wave_sum(a); b = wave_sum(b); block_sum2_waves(a, b, smem); }
 
 // A sum and a maximum for one pair of barriers; `smem` must hold 32 floats.  The sum is formed in the order block_sum forms it.
 __device__ __forceinline__ void block_sum_max(float &a, float &m, float *smem)

@@ -820,7 +820,7 @@ __global__ __launch_bounds__(TB) void k_lora_grads(LoraGradArgs a)
         a.grad[idx] = s;
         gval = s;
     }
-    const float sq = block_sum(gval * gval, sm);
+    const float sq = block_sum_products(gval, gval, sm);
     if (threadIdx.x == 0) a.sq_slots[blockIdx.x] = sq;
 }
 
@@ -1254,7 +1254,7 @@ __global__ __launch_bounds__(256) void k_ce_partial(CeArgs a)
         ts += expf(x.x - tm) + expf(x.y - tm) + expf(x.z - tm) + expf(x.w - tm);
     }
     const float mx = block_max(tm, sm);
-    const float sum = block_sum(ts * expf(tm - mx), sm);   // a thread without elements: 0 * exp(-1e30 - mx) = 0
+    const float sum = block_sum_products(ts, expf(tm - mx), sm);   // a thread without elements: 0 * exp(-1e30 - mx) = 0
     if (threadIdx.x == 0) a.partials[r * CE_CHUNKS + chunk] = make_float2(mx, sum);
 }
 

@@ -121,9 +121,9 @@ __global__ __launch_bounds__(256) void k_delta_decode(DecodeDelta s, DecodeMoe e
     } else gate = silu(a.cin[s.o_g + vch]);
     const float beta = sigmoid(a.cin[a.o_b + h]);
     const float gh = PC ? 1.f : expf(-a.a_exp[h] * softplus(a.cin[a.o_a + h] + a.dt_bias[h]));
-    float sq = qv * qv, sk = kv * kv;
-    block_sum2(sq, sk, red);
-    const float dot = block_sum(qv * kv, red);
+    float sq = wave_sum_products(qv, qv), sk = wave_sum_products(kv, kv);
+    block_sum2_waves(sq, sk, red);
+    const float dot = block_sum_products(qv, kv, red);
     const float iq = 1.f / (sqrtf(sq + 1e-6f) * sqrtf((float)a.dim)), ik = 1.f / sqrtf(sk + 1e-6f), kq = dot * iq * ik;
     if (tid < DP) { qs[tid] = qv * iq; ks[tid] = kv * ik; if (PC) gs[tid] = gv; }   // zeros beyond dim
     __syncthreads();

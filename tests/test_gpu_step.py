@@ -495,3 +495,23 @@ def test_the_step_is_deterministic(fmt):
     assert runs[0][0] == runs[1][0], (runs[0][0], runs[1][0])
     for a, b in zip(runs[0][1:], runs[1][1:]):
         assert np.array_equal(a, b)
+
+
+def test_gradient_norm_in_its_order_of_sums():
+    """The squares of a workgroup's 256 gradients (a rank without a kernel of its own): per wave, lane i adds its unrounded product
+    to the rounded one of lane i + 32, then rounded sums over 16, 8, 4, 2, 1 lanes; the waves in order; workgroups in 64 bits."""
+    F = np.float32
+    cfg = C1.with_(name="norm_order", NL=1, D=64, Hq=2, Hkv=1, hd=32, IS=64, V=256, R=2, alpha=4.0, seq=8)
+    model = make_model(cfg, seed=1)
+    with SFTState(cfg, model) as st:
+        for seed in range(96):                                     # (the last bits meet in the norm in one of fourteen)
+            st.train_step(*make_batch(cfg, seed=50 + seed), 0.0)
+            g, norm = st.lora_grads(), F(st.grad_norm())
+            assert 0 < norm < 1                                    # not clipped: the gradients are as they were summed
+            g = np.concatenate([g, np.zeros(-g.size % 256, F)]).reshape(-1, 4, 64)
+            v = (g[..., :32].astype(np.longdouble) ** 2 + (g[..., 32:] * g[..., 32:]).astype(np.longdouble)).astype(F)
+            for o in (16, 8, 4, 2, 1):
+                v = v[..., :o] + v[..., o:2 * o]
+            v = v[..., 0]
+            slots = ((F(0) + v[:, 0] + v[:, 1]) + v[:, 2]) + v[:, 3]
+            assert norm == F(np.sqrt(slots.astype(np.float64).sum())), seed
