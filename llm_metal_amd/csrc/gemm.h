@@ -91,7 +91,7 @@ int gemm_ring_enabled();            // 1 (default): products of up to 64 rows ta
 // half_scale != 0 (ring plans only, a_inv_scale null): the planes are written as halves, each chunk sum times half_scale
 // (see gemm_ring); plane_stride and ldp then count halves, and only planes_at4_multi reads such planes.
 void launch_gemm(const half_t *A_tiled, const float *a_inv_scale, const WeightOp &W,
-                 float *P, int ldp, size_t plane_stride, int M, int N, int K, const GemmPlan &p, float half_scale = 0.f);
+                 float *P, int ldp, size_t plane_stride, int M, int N, int K, const GemmPlan &p, float half_scale = 0.f, bool short_sums = false);
 // Largest sum of |w| over a row of a tiled F16 matrix [N, K]: with operand rows scaled below 8192 (row_scale_for), no
 // chunk sum of a product with this matrix exceeds 8192 times it.  Synchronises the stream.
 // the same over the values a weight operand of any format multiplies with (0 when the operand mixes Q8_0 and F16 tiles)
@@ -129,6 +129,17 @@ void set_big_gemm_block(int mode);     // F16 tiles: 0 block shape by the measur
 // Returns the number of planes written (fewer than `chunks` when K has too few steps for that many).
 int launch_gemm_big(const half_t *A_tiled, const float *a_inv_scale, const WeightOp &W, float *C, int ldc, int M, int N, int K,
                     int chunks = 1, size_t plane_stride = 0);
+// A product whose operand rows hold more than fp16 does (value and residual rows): planes [M, N] whose sums are formed from parts
+// of at most sixteen MFMAs each, so that rounding the accumulators costs no more than the fp32 matrix-vector kernels lose.
+struct ShortPlan {
+    int big, chunks;                   // the large-M kernel with that many K chunks, else t
+    GemmPlan t;
+    int planes() const { return big ? chunks : t.S; }
+};
+ShortPlan plan_short_sums(int M, int N, int K, int nbq, int fmt);
+// P: planes() planes; returns how many of them were written.  W: F16 tiles (f16_image_of) where the plan says big.
+int launch_short_sums(const half_t *A_tiled, const WeightOp &W, float *P, size_t plane_stride, int M, int N, int K, const ShortPlan &p);
+int big_gemm_policy();                 // hip_gemm_force_large_m's choice
 // The same with F16 tiles for rows that belong to different weights [N, K] of one shape (the experts of a mixture), their
 // tiled images group_stride halves apart: row block i of 128 rows is multiplied with weight group_of[i] (device), and only the
 // first group_of[M / 128] blocks have rows (the rest of C is not written).  M is a multiple of 128; `groups`: how many weights.

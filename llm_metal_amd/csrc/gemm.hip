@@ -385,8 +385,9 @@ GemmPlan plan_gemm(int M, int N, int K, int nbq, int fmt)
 }
 
 void launch_gemm(const half_t *A, const float *a_inv_scale, const WeightOp &W,
-                 float *P, int ldp, size_t plane_stride, int M, int N, int K, const GemmPlan &p, float half_scale)
+                 float *P, int ldp, size_t plane_stride, int M, int N, int K, const GemmPlan &p, float half_scale, bool short_sums)
 {
+    short_sums = short_sums && W.fmt == 0 && !a_inv_scale && half_scale == 0.f;      // (the ring kernels that leave fp32 planes of F16 tiles)
     if (half_scale != 0.f && (!p.ring || a_inv_scale)) { fprintf(stderr, "[fast_hip] gemm: half planes need a ring plan without row factors\n"); abort(); }
     if (M <= 0 || N <= 0 || K <= 0) return;
     const int Kb = tiled_kb(K), Nb = tiled_rb(N), Mb = tiled_rb(M);
@@ -423,7 +424,9 @@ void launch_gemm(const half_t *A, const float *a_inv_scale, const WeightOp &W,
         if (p.wide) {
 #define WIDE_LAUNCH(SC, HP, WFV) launch_kargs<24>(gemm_ring_wide<SC, HP, WFV>, rgrid, rblock, 0, stream(), g, g_prof_on ? ra : nullptr, g_prof_on ? rb : nullptr)
 #define WIDE_PICK(WFV) do { if (a_inv_scale) WIDE_LAUNCH(1, 0, WFV); else if (half_scale != 0.f) WIDE_LAUNCH(0, 1, WFV); else WIDE_LAUNCH(0, 0, WFV); } while (0)
-            if (W.fmt == 1) WIDE_PICK(1); else if (W.fmt == 2) WIDE_PICK(2); else WIDE_PICK(0);
+            if (W.fmt == 1) WIDE_PICK(1); else if (W.fmt == 2) WIDE_PICK(2);
+            else if (short_sums) launch_kargs<24>(gemm_ring_wide<0, 0, 0, 1>, rgrid, rblock, 0, stream(), g, g_prof_on ? ra : nullptr, g_prof_on ? rb : nullptr);
+            else WIDE_PICK(0);
 #undef WIDE_PICK
 #undef WIDE_LAUNCH
             HIP_CHECK(hipGetLastError());
@@ -435,6 +438,7 @@ void launch_gemm(const half_t *A, const float *a_inv_scale, const WeightOp &W,
 #define RING_LAUNCH_Q8(SC, HP, WFV) launch_kargs<24>(gemm_ring<2, SC, HP, WFV>, rgrid, rblock, 0, stream(), g, g_prof_on ? ra : nullptr, g_prof_on ? rb : nullptr)
         if (W.fmt == 1) { if (a_inv_scale) RING_LAUNCH_Q8(1, 0, 1); else if (half_scale != 0.f) RING_LAUNCH_Q8(0, 1, 1); else RING_LAUNCH_Q8(0, 0, 1); }
         else if (W.fmt == 2) { if (a_inv_scale) RING_LAUNCH_Q8(1, 0, 2); else if (half_scale != 0.f) RING_LAUNCH_Q8(0, 1, 2); else RING_LAUNCH_Q8(0, 0, 2); }
+        else if (short_sums && p.kg == 2) launch_kargs<24>(gemm_ring<2, 0, 0, 0, 1>, rgrid, rblock, 0, stream(), g, g_prof_on ? ra : nullptr, g_prof_on ? rb : nullptr);
         else if (p.kg == 1) RING_PICK(1); else if (p.kg == 2) RING_PICK(2); else RING_PICK(4);
 #undef RING_LAUNCH_Q8
 #undef RING_PICK
@@ -652,6 +656,7 @@ int gemm_ring_enabled() { return g_ring; }
 // HBM traffic per weight) and run the large-M kernel on that instead of unpacking every tile again for each 64 rows
 // of activations: 4 x 512 rows, 112.9 ms per step against 123 ms (streaming) and 125 ms (Q8_0 inside the large-M kernel).
 int g_big_policy = 0;                                     // 0 measured rule, 1 always, -1 never, 2 always and Q8_0 tiles stay quantised
+int big_gemm_policy() { return g_big_policy; }
 bool use_big_gemm(int M, int N, int K, int fmt, bool one_plane)
 {
     if (g_big_policy) return g_big_policy > 0;

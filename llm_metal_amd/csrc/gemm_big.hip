@@ -263,8 +263,13 @@ __global__ __launch_bounds__(256) void gemm_big(GemmKArgs g)
 //
 // GROUPED: the 128-row blocks of A belong to different weights of one shape, laid group.stride halves apart: block mt is
 // multiplied with number group.of[mt]; only the first group.of[M / 128] blocks have rows.
+//
+// SHORT: no sum of more than twelve MFMAs in one accumulator.  The matrix cores round an accumulator at every instruction, so a
+// sum over K = 2560 in one is 2.5 times as far from the exact one as a matrix-vector product's (units of 2^-24 of the result's
+// norm, 64 rows: 5.5 against 2.2; K = 9728: 10.5 against 3.9).  Two of the eight accumulators of a wave are added to sums of their own
+// in each of four half steps out of six, under the MFMAs of the others, and start again from zero.
 struct GroupArgs { const int *of; size_t stride; };
-template <bool GROUPED>
+template <bool GROUPED, bool SHORT = false>
 __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group)
 {
     constexpr int HB = 12 * 2 * 64;                       // half8 per buffer: [4 A + 8 W row blocks][2 slices][64 lanes]
@@ -310,13 +315,13 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
     const int dst[3] = {wave, 4 + 2 * wave, 5 + 2 * wave};
     float *const Cp = g.P + (size_t)chunk * g.plane_stride;
 
-    float16v acc[2][4];
+    float16v acc[2][4], sum[2][4];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+            for (int v = 0; v < 16; v++) acc[i][j][v] = sum[i][j][v] = 0.f;
 
     typedef __attribute__((address_space(3))) void lds_void;
     uint32_t loff[3][2];
@@ -343,19 +348,25 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
 #pragma unroll
         for (int k = 0; k < 4; k++) w[k] = cur[((4 + 4 * wn + k) * 2 + j) * 64 + lane];
     };
-    auto multiply = [&](const half8 (&a)[2], const half8 (&w)[4]) __attribute__((always_inline)) {
+    auto multiply = [&](const half8 (&a)[2], const half8 (&w)[4], int out) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], acc[i][k], 0, 0, 0);
+            for (int k = 0; k < 4; k++) {
+                if (SHORT && k == out) {
+                    sum[i][k] += acc[i][k];
+                    acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], float16v{}, 0, 0, 0);
+                } else acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], acc[i][k], 0, 0, 0);
+            }
     };
-    auto step = [&](int hs, const half8 (&cur)[HB], const half8 (&nxt)[HB], half8 (&free_buf)[HB]) __attribute__((always_inline)) {
+    // (out: SHORT's column of accumulators to add to the sums)
+    auto step = [&](int hs, int out, const half8 (&cur)[HB], const half8 (&nxt)[HB], half8 (&free_buf)[HB]) __attribute__((always_inline)) {
         request(free_buf, min(hs + 5, last));
         half8 a1[2], w1[4];
         read(a1, w1, cur, 1);
-        multiply(a0, w0);
+        multiply(a0, w0, out);
         read(a0, w0, nxt, 0);
-        multiply(a1, w1);
+        multiply(a1, w1, -1);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
 #pragma unroll
         for (int i = 0; i < 16; i++) {
@@ -371,19 +382,25 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
     read(a0, w0, lb0, 0);
     const int full = nhalf / 6 * 6;
     for (int h0 = 0; h0 < full; h0 += 6) {
-        step(h0, lb0, lb1, lb5);
-        step(h0 + 1, lb1, lb2, lb0);
-        step(h0 + 2, lb2, lb3, lb1);
-        step(h0 + 3, lb3, lb4, lb2);
-        step(h0 + 4, lb4, lb5, lb3);
-        step(h0 + 5, lb5, lb0, lb4);
+        step(h0, 0, lb0, lb1, lb5);
+        step(h0 + 1, 1, lb1, lb2, lb0);
+        step(h0 + 2, 2, lb2, lb3, lb1);
+        step(h0 + 3, 3, lb3, lb4, lb2);
+        step(h0 + 4, 4, lb4, lb5, lb3);
+        step(h0 + 5, 5, lb5, lb0, lb4);
     }
-    if (full < nhalf) step(full, lb0, lb1, lb5);
-    if (full + 1 < nhalf) step(full + 1, lb1, lb2, lb0);
-    if (full + 2 < nhalf) step(full + 2, lb2, lb3, lb1);
-    if (full + 3 < nhalf) step(full + 3, lb3, lb4, lb2);
-    if (full + 4 < nhalf) step(full + 4, lb4, lb5, lb3);
+    if (full < nhalf) step(full, 0, lb0, lb1, lb5);
+    if (full + 1 < nhalf) step(full + 1, 1, lb1, lb2, lb0);
+    if (full + 2 < nhalf) step(full + 2, 2, lb2, lb3, lb1);
+    if (full + 3 < nhalf) step(full + 3, 3, lb3, lb4, lb2);
+    if (full + 4 < nhalf) step(full + 4, 4, lb4, lb5, lb3);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (SHORT) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) acc[i][k] += sum[i][k];
+    }
 
     if (mb0 * 32 + 128 <= g.M && (nb0 + 8) * 32 <= g.N) {
         float sc[2][16];
@@ -977,6 +994,47 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
     }
     HIP_CHECK(hipGetLastError());
     return 1;
+}
+
+// The plan: the streaming kernel (its waves and planes in any case form short sums; at most four K steps per wave, sixteen MFMAs) or
+// the 128 x 256 block, by the times of mid_plan at any number of rows -- the 256 x 256 block has no registers for a second set of
+// sums.  Operands that are not F16 tiles: use_big_gemm's rule.
+ShortPlan plan_short_sums(int M, int N, int K, int nbq, int fmt)
+{
+    ShortPlan p{0, 1, plan_gemm(M, N, K, nbq, fmt)};
+    const int cus = num_cus() > 0 ? num_cus() : 256, Kb = tiled_kb(K);
+    if (!p.t.ring && p.t.steps > 4 * p.t.nw) { p.t.steps = 4 * p.t.nw; p.t.S = (Kb + p.t.steps - 1) / p.t.steps; }
+    const int policy = big_gemm_policy();
+    if (policy < 0 || (policy == 0 && (M <= 64 || (fmt != 0 && !use_big_gemm(M, N, K, fmt))))) return p;
+    double best = policy || fmt ? 1e30 : 5.1 + 0.152 * (2e-6 * N * K) + 1.65 * (2e-9 * M * N * K) + (0.115 + 0.2) * (4e-6 * p.t.S * M * N);
+    for (int S = 1; S <= 20 && (S == 1 || S * 4 <= Kb); S++) {
+        const double us = mid_big_us(0, M, N, K, S, cus);
+        if (us < best) { best = us; p.big = 1; p.chunks = S; }
+    }
+    if (p.big && g_big_split != 1) p.chunks = std::min(std::max(1, g_big_split), Kb);
+    return p;
+}
+
+int launch_short_sums(const half_t *A, const WeightOp &W, float *P, size_t plane_stride, int M, int N, int K, const ShortPlan &p)
+{
+    if (!p.big) { launch_gemm(A, nullptr, W, P, N, plane_stride, M, N, K, p.t, 0.f, true); return p.t.S; }
+    if (W.fmt != 0) return launch_gemm_big(A, nullptr, W, P, N, M, N, K, 1, plane_stride);      // (Q8_0 tiles in the large-M kernel are asked for)
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (!W.w16 || p.chunks < 1) { fprintf(stderr, "[fast_hip] gemm_short: bad launch M=%d N=%d K=%d chunks=%d\n", M, N, K, p.chunks); abort(); }
+    GemmKArgs g{};
+    g.A = reinterpret_cast<const half8 *>(A); g.W = W;
+    g.P = P; g.ldp = N; g.plane_stride = plane_stride;
+    g.M = M; g.N = N; g.Mb = tiled_rb(M); g.Nb = tiled_rb(N); g.Kb = tiled_kb(K);
+    g.steps_per_chunk = (g.Kb + p.chunks - 1) / p.chunks;
+    g.S = (g.Kb + g.steps_per_chunk - 1) / g.steps_per_chunk;
+    g.m_tiles = 1;
+    const dim3 grid(8 * ((M + 127) / 128) * (((N + 255) / 256 * g.S + 7) / 8));
+    hipEvent_t ev_a = nullptr, ev_b = nullptr;
+    if (gemm_prof_begin(weight_stream_bytes(W, N, K), 2.0 * M * N * K, &ev_a, &ev_b))
+        hipExtLaunchKernelGGL((gemm_big_f16<false, true>), grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g, GroupArgs{});
+    else hipLaunchKernelGGL((gemm_big_f16<false, true>), grid, dim3(256), 0, stream(), g, GroupArgs{});
+    HIP_CHECK(hipGetLastError());
+    return g.S;
 }
 
 void launch_gemm_groups(const half_t *A, const float *a_inv_scale, const half_t *W, size_t group_stride, const int *group_of, float *C, int ldc,

@@ -313,7 +313,9 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // matrix (fmt 1: row blocks from nbq on), the K steps from kbq on of its transposed image (fmt 2) -- take the F16 way
 // through the same slot; which way is uniform per wave and stage.  Every wave issues four loads per round either way (a
 // quantised tile's fourth asks for its scales once more), so that one count serves the waits.
-template <int KG, int SCALE, int HALFP = 0, int WF = 0>
+//
+// SHORT: every fourth round's accumulator is added to a sum of its own (gemm_big_f16, gemm_big.hip): at most sixteen MFMAs in one.
+template <int KG, int SCALE, int HALFP = 0, int WF = 0, int SHORT = 0>
 __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
 {
     static_assert(!(SCALE && HALFP), "final outputs stay fp32");
@@ -379,9 +381,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
             else asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(src + (size_t)step * 256 + j * 64), "s"(sb + (uint32_t)(j * 1024)) : "m0", "memory");
         }
     };
-    float16v acc;
+    float16v acc, sum;
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    for (int v = 0; v < 16; v++) acc[v] = sum[v] = 0.f;
     request(0);
     if (rounds > 1) request(1);
     for (int rd = 0; rd < rounds; rd++) {
@@ -419,7 +421,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
 #pragma unroll
             for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], w[j], acc, 0, 0, 0);
         }
+        if (SHORT && (rd & 3) == 3) { sum += acc; acc = float16v{}; }
     }
+    if (SHORT) acc += sum;
     // Exchange: wave (q, kg) ends up with registers [kg Q, kg Q + Q) of quadrant q, Q = 16 / KG, summed over the groups.
     constexpr int Q = 16 / KG;
     float res[Q];
@@ -486,7 +490,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
 // waves 0 .. 3 request one weight tile each (four loads: a quantised tile's 2 KB and its scales, twice; or the four
 // pieces of an F16 tile that the operand carries), waves 4 .. 7 two pieces each of the activation blocks; the waits count
 // per wave.
-template <int SCALE, int HALFP, int WF = 0>
+template <int SCALE, int HALFP, int WF = 0, int SHORT = 0>
 __global__ __launch_bounds__(512) void gemm_ring_wide(KARGS24)
 {
     static_assert(!(SCALE && HALFP), "final outputs stay fp32");
@@ -565,9 +569,9 @@ __global__ __launch_bounds__(512) void gemm_ring_wide(KARGS24)
                 asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(qsrc + (size_t)step * 256 + j * 64), "s"(sb + qoff + (uint32_t)(j * 1024)) : "m0", "memory");
         }
     };
-    float16v acc;
+    float16v acc, sum;
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    for (int v = 0; v < 16; v++) acc[v] = sum[v] = 0.f;
     request(0);
     if (nsteps > 1) request(1);
     for (int rd = 0; rd < nsteps; rd++) {
@@ -604,7 +608,9 @@ __global__ __launch_bounds__(512) void gemm_ring_wide(KARGS24)
         if (rd + 2 < nsteps) request(rd + 2);
 #pragma unroll
         for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], w[j], acc, 0, 0, 0);
+        if (SHORT && (rd & 3) == 3) { sum += acc; acc = float16v{}; }
     }
+    if (SHORT) acc += sum;
     // D layout of v_mfma_f32_32x32x16: column = lane & 31, row = 8 (v / 4) + 4 (lane / 32) + v % 4
     const int n = (tile * WB + qn) * 32 + r;
     const bool inside = 64 <= g.M && (tile + 1) * 32 * WB <= g.N;

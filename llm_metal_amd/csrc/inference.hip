@@ -1190,15 +1190,9 @@ SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const
     const half_t *a16 = dptr_as<half_t>(r.a16);
     auto planes = [&](const WeightOp &op, int m, MetalBuf *&buf, size_t &stride) {
         stride = (size_t)m * rows;
-        if (use_big_gemm(m, rows, cols, op.fmt)) {
-            const WeightOp f = f16_image_of(op, rows, cols);
-            const int chunks = big_gemm_chunks_for(m, rows, cols, f);
-            float *P = at_least(buf, stride * chunks);
-            return launch_gemm_big(a16, nullptr, f, P, rows, m, rows, cols, chunks, stride);
-        }
-        const GemmPlan p = plan_gemm(m, rows, cols, (op.fmt == 1 && op.nbq < tiled_rb(rows)) ? op.nbq : 0, op.fmt);
-        launch_gemm(a16, nullptr, op, at_least(buf, stride * p.S), rows, stride, m, rows, cols, p);
-        return p.S;
+        const ShortPlan p = plan_short_sums(m, rows, cols, (op.fmt == 1 && op.nbq < tiled_rb(rows)) ? op.nbq : 0, op.fmt);
+        float *P = at_least(buf, stride * p.planes());
+        return launch_short_sums(a16, p.big ? f16_image_of(op, rows, cols) : op, P, stride, m, rows, cols, p);
     };
     SplitPlanes out{};
     out.inv = inv; out.N = rows;

@@ -1,6 +1,7 @@
 // Many tokens of one sequence in one step, for the models whose decoding runs a token at a time (prompt.hip; the host side is
 // in inference.hip).  Every product reads its weight once for all of them on the matrix cores, with 22 bits of every fp32
-// activation kept (rows_to_f16_split); everything else is fp32.
+// activation kept (rows_to_f16_split), in sums of short parts (plan_short_sums); everything else is fp32.  No further from 64 bits
+// than the tokens one by one (tests/test_gpu_prompt.py).
 #pragma once
 #include "gemm.h"
 

@@ -104,15 +104,20 @@ __device__ __attribute__((noinline)) void attend_plain(const float *Q, const flo
     for (int u = 0; u < U; u++) if (lane + 64 * u < HD) out[((size_t)m * Hq + head) * HD + lane + 64 * u] = o[u] / l;
 }
 
-// Attention in fp32 on the matrix cores (v_mfma_f32_32x32x2_f32: products and sums as exact as the decoding kernel's).
+// Attention in fp32 on the matrix cores (v_mfma_f32_32x32x2_f32).
 // A workgroup serves 32 (token, query head) pairs of one key head -- row r of the key head is token r / G, head r % G of its
 // group, so a tile spans few positions whatever G is -- and its four waves take the key tiles in turn, 32 keys each, with a
 // running softmax of their own that the workgroup merges at the end: the chain of a wave is a quarter of the keys.  Scores are
 // formed transposed (keys x rows): a row is a lane, and the accumulator that holds a row's probabilities is, register by
 // register, the operand of the product with the values (the keys of a step are those the two lane halves hold), so nothing
-// passes through LDS until the merge.  Per tile 2 HD matrix instructions of 64 cycles: bound by them for long prompts
-// (a 2048-token one reads 17 MB of keys per 128 rows from L2), by the chain of one wave for short ones: 500 tokens, 504
-// workgroups, 55-59 us.
+// passes through LDS until the merge.
+// An accumulator is rounded at every instruction, so no sum stays in one for long: a score is added up from parts of eight
+// instructions (sixteen columns), a value sum from parts of four (eight keys), each part added while the next is multiplied.
+// Error against 64 bits at 33 / 500 keys, units of 2^-24 of the result's norm: 1.8 / 2.4 for heads of 128, 1.8 / 2.6 for 256,
+// single-token kernel 2.3 / 3.0 and 1.9 / 3.2 (last row); whole sums in one accumulator 3.5 / 5.1 and 4.4 / 6.7.
+// Per tile HD matrix instructions of 64 cycles, half for the scores: bound by them for long prompts, by the chain of one wave for
+// short ones.  32 heads of 128 over 8: 13.3 us at 120 tokens, 52.6 at 500 (12.5 and 49.6 with whole sums); 4 heads of 256 over
+// one: 23.7 and 61.0 (21.4 and 50.6).
 template <int HD>
 __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const float *__restrict__ Q, const float *__restrict__ Kc, const float *__restrict__ Vc,
                                                                        float *__restrict__ out, int M, int pos, int Hq, int G, int max_seq, float scale)
@@ -123,7 +128,7 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
     const int kvh = blockIdx.y, rows = M * G, row0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 32;      // the longest first
     const int r = min(row0 + col, rows - 1), m = r / G, head = kvh * G + r % G, qpos = pos + m;
-    const int first = pos + row0 / G, last = pos + min(row0 + 31, rows - 1) / G, tiles = last / 32 + 1;
+    const int last = pos + min(row0 + 31, rows - 1) / G, tiles = last / 32 + 1;
     const float *Kh = Kc + (size_t)kvh * max_seq * HD, *Vh = Vc + (size_t)kvh * max_seq * HD;
 
     float4v q[HH / 4];                                     // columns half * HH .. of the lane's row
@@ -134,12 +139,14 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
     float16v O[CB] = {};
     float mx = -3.0e38f, l = 0.f, bad = 0.f;
     for (int t = wave; t < tiles; t += 4) {
-        const float *kp = Kh + (size_t)min(t * 32 + col, last) * HD + half * HH;
-        float16v S = {};
+        // (a tile's part of every address is scalar, a lane's 32 bits)
+        const float *Kt = Kh + (size_t)t * 32 * HD, *Vt = Vh + (size_t)t * 32 * HD;
+        const uint32_t left = (uint32_t)(last - t * 32), k0 = min((uint32_t)col, left) * HD + half * HH;
+        float16v S = {}, T[2];
         float4v k[2][4];                                   // sixteen columns while the sixteen before are multiplied
         auto keys = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) k[i & 1][e] = *reinterpret_cast<const float4v *>(kp + 16 * i + 4 * e);
+            for (int e = 0; e < 4; e++) k[i & 1][e] = *reinterpret_cast<const float4v *>(Kt + (k0 + 16 * i + 4 * e));
         };
         keys(0);
 #pragma unroll
@@ -147,17 +154,25 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
             if (i + 1 < HH / 16) keys(i + 1);
             __builtin_amdgcn_sched_barrier(0);             // (all of a tile's loads together spill)
 #pragma unroll
-            for (int e = 0; e < 16; e++) S = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i & 1][e >> 2][e & 3], q[4 * i + (e >> 2)][e & 3], S, 0, 0, 0);
+            for (int u = 0; u < 2; u++) {
+                float16v &t8 = T[u];
+                t8 = float16v{};
+#pragma unroll
+                for (int e = 0; e < 8; e++) t8 = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i & 1][2 * u + (e >> 2)][e & 3], q[4 * i + 2 * u + (e >> 2)][e & 3], t8, 0, 0, 0);
+                if (i + u > 0) S += T[u ^ 1];
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+        S += T[1];
         // value rows of four of the sixteen keys that the lane's half holds, keys 8 b + 4 half .. + 3 of the tile; the next
         // four are requested while these are multiplied
         float v[2][4][CB];
         auto values = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const float *vp = Vh + (size_t)min(t * 32 + 8 * b + 4 * half + e, last) * HD + col;
+                const uint32_t v0 = min((uint32_t)(8 * b + 4 * half + e), left) * HD + col;
 #pragma unroll
-                for (int c = 0; c < CB; c++) v[b & 1][e][c] = vp[32 * c];
+                for (int c = 0; c < CB; c++) v[b & 1][e][c] = Vt[v0 + 32 * c];
             }
         };
         values(0);
@@ -175,27 +190,29 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
 #pragma unroll
         for (int j = 0; j < 16; j++) { S[j] = expf(S[j] - now); sum += S[j]; }       // (a key that is not seen: 0)
         l = fmaf(l, keep, sum);
-        if (__any(keep != 1.f)) {
+        auto flush = [&](int n) __attribute__((always_inline)) {
+            const int c = n % CB;
 #pragma unroll
-            for (int c = 0; c < CB; c++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) O[c][j] *= keep;
-        }
-        const bool partly = t * 32 + 31 > first;           // some rows do not see some keys of this tile
+            for (int j = 0; j < 16; j++) O[c][j] = n < CB ? fmaf(O[c][j], keep, T[n & 1][j]) : O[c][j] + T[n & 1][j];
+        };
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             if (b < 3) values(b + 1);
-            if (partly) {
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int c = 0; c < CB; c++) bad += v[b & 1][e][c] * 0.f;
-            }
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int c = 0; c < CB; c++) O[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[b & 1][e][c], S[4 * b + e], O[c], 0, 0, 0);
+                for (int c = 0; c < CB; c++) bad = fmaf(v[b & 1][e][c], 0.f, bad);     // (a branch for tiles that all rows see whole lets the sums below pile up behind it)
+#pragma unroll
+            for (int c = 0; c < CB; c++) {
+                float16v &t4 = T[(b * CB + c) & 1];
+                t4 = float16v{};
+#pragma unroll
+                for (int e = 0; e < 4; e++) t4 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[b & 1][e][c], S[4 * b + e], t4, 0, 0, 0);
+                if (b + c > 0) flush(b * CB + c - 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+        flush(4 * CB - 1);
     }
     if (__syncthreads_or(bad != 0.f)) {                    // a probability of zero has met an infinity or NaN
         for (int i = wave; i < 32 && row0 + i < rows; i += 4) attend_plain<HD>(Q, Kh, Vh, out, (row0 + i) / G, kvh * G + (row0 + i) % G, pos + (row0 + i) / G, Hq, scale);
