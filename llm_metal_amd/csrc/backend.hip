@@ -3,7 +3,6 @@
 // (:69-249): one device, one in-order stream, explicit HBM allocations.
 #include "backend.h"
 #include <string.h>
-#include <unistd.h>
 #include <vector>
 
 namespace {
@@ -134,18 +133,10 @@ size_t metal_buf_size(MetalBuf *b) { return b ? b->size : 0; }
 
 void *hip_buf_device_ptr(MetalBuf *b) { return b ? lmhip::dptr(b) : nullptr; }
 
-// The driver clears freed memory before it counts as free again, some milliseconds after hipFree has returned: the figure is
-// read until it has stood still for 20 ms (half a second at most).
 void hip_mem_info(size_t *free_bytes, size_t *total_bytes)
 {
-    size_t f = 0, t = 0, before = 0;
+    size_t f = 0, t = 0;
     HIP_CHECK(hipMemGetInfo(&f, &t));
-    for (int same = 0, i = 0; same < 4 && i < 100; i++) {
-        before = f;
-        usleep(5000);
-        HIP_CHECK(hipMemGetInfo(&f, &t));
-        same = f == before ? same + 1 : 0;
-    }
     if (free_bytes) *free_bytes = f;
     if (total_bytes) *total_bytes = t;
 }

@@ -12,18 +12,11 @@ from llm_metal_amd import lib as _lib
 from llm_metal_amd.sft import InferenceState, SFTState
 from llm_metal_amd.synth import make_batch, make_model
 from tests.decode_chain import oracle_decode
-from tests.gpu_util import maxrel
+from tests.gpu_util import maxrel, settled_free_bytes
 
 pytestmark = pytest.mark.gpu
 F = np.float32
 TINY_GEMMA = SFTConfig("tiny_gemma3", GEMMA3, NL=7, D=128, Hq=4, Hkv=1, hd=32, IS=256, V=512, seq=6, tied=True)
-
-
-def _free_bytes(L):
-    import ctypes
-    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
-    L.hip_mem_info(ctypes.byref(free), ctypes.byref(total))
-    return free.value
 
 
 def say(*a):
@@ -225,10 +218,10 @@ def test_decode_at_the_benchmarked_widths(fmt, with_lora, from_sft):
         L = _lib.load()
         weight_count = c.NL * (c.D * (c.Hq + 2 * c.Hkv) * c.hd + c.D * c.Hq * c.hd + 3 * c.D * c.IS) + c.V * c.D
         with SFTState(c, model) as sft:
-            free0 = _free_bytes(L)
+            free0 = settled_free_bytes(L)
             with InferenceState(sft=sft, max_seq=64) as inf:
                 check(inf)
-                assert free0 - _free_bytes(L) < weight_count // 2, (free0 - _free_bytes(L), weight_count)
+                assert free0 - settled_free_bytes(L) < weight_count // 2, (free0 - settled_free_bytes(L), weight_count)
     elif with_lora:
         with SFTState(c, model) as sft:
             with InferenceState(c, model, max_seq=64, use_fp16=True) as inf:

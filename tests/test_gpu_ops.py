@@ -331,3 +331,15 @@ def test_metal_buf_ptr_is_coherent_at_flush(dev):
     dev.be.flush()
     assert np.array_equal(host[1024:1040], np.arange(1024, 1040, dtype=F)) and host[1040] == 2080
     dev.L.metal_buf_free(view)
+
+
+def test_memory_figures_come_at_once(dev):
+    import ctypes as C
+    import time
+    free, total = C.c_size_t(0), C.c_size_t(0)
+
+    def seconds():
+        t = time.perf_counter()
+        dev.L.hip_mem_info(C.byref(free), C.byref(total))
+        return time.perf_counter() - t
+    assert min(seconds() for _ in range(5)) < 5e-3 and 0 < free.value <= total.value

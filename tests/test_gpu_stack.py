@@ -13,6 +13,7 @@ from llm_metal_amd.configs import C1
 from llm_metal_amd.sft import InferenceState
 from llm_metal_amd.synth import make_model, write_stack_checkpoint
 from oracle import stack_oracle as so
+from tests.gpu_util import settled_free_bytes
 from tests.stack_models import MODELS, Model, around, channel, config, delta, dense, grouped, latent, logit_error, mlstm, moe
 
 pytestmark = pytest.mark.gpu
@@ -346,7 +347,6 @@ def test_what_is_refused(tmp_path):
 
 
 def test_states_give_their_memory_back(tmp_path):
-    import ctypes
     from llm_metal_amd import lib
     cfg, ra, rg = MODELS["mixed"]
     m = Model(cfg, tmp_path, ra, rg)
@@ -358,9 +358,7 @@ def test_states_give_their_memory_back(tmp_path):
             with state(m, "f16") as inf:
                 inf.generate(prompt, 5)
                 inf.generate_batch(prompt, 5, 3)
-            f, t = ctypes.c_size_t(0), ctypes.c_size_t(0)
-            lib.load().hip_mem_info(ctypes.byref(f), ctypes.byref(t))
-            free.append(f.value)
+            free.append(settled_free_bytes(lib.load()))
     assert free[1] == free[2] == free[3]
 
 

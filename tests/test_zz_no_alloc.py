@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle.oracle import op
-from tests.gpu_util import Dev, rel
+from tests.gpu_util import Dev, rel, settled_free_bytes
 
 pytestmark = pytest.mark.gpu
 F = np.float32
@@ -49,7 +49,6 @@ def test_no_alloc_attention_leaves_device_memory_as_it_was():
     without slice partials) allocate nothing.  fast_metal_init has resolved the fixed array's address on this device
     before, so the calls themselves resolve nothing either (a caller under graph capture must have initialised the
     library on its device first)."""
-    import ctypes as C
     dev = Dev()
     try:
         L = dev.L
@@ -61,13 +60,12 @@ def test_no_alloc_attention_leaves_device_memory_as_it_was():
         out = dev.empty(Hq * hd * 4)
         ptrs = [L.hip_buf_device_ptr(b.h) for b in (Q, Kc, Vc, out)]
         L.metal_flush()
-        free0, free1, total = C.c_size_t(), C.c_size_t(), C.c_size_t()
-        L.hip_mem_info(C.byref(free0), C.byref(total))
+        free0 = settled_free_bytes(L)
         for n_attend in (4096, 100, 2500, 257):
             assert L.hip_attention_noalloc(*ptrs, n_attend, hd, max_seq, Hq, G) == 0
         L.metal_flush()
-        L.hip_mem_info(C.byref(free1), C.byref(total))
-        assert free1.value == free0.value, (free0.value, free1.value)
+        free1 = settled_free_bytes(L)
+        assert free1 == free0, (free0, free1)
         assert np.isfinite(out.read(F)).all()
     finally:
         dev.close()
