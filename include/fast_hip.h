@@ -186,7 +186,8 @@ void hip_gemm_large_m_split(int mode);
 void hip_gemm_large_m_block(int mode);
 /* A training state with frozen Q8_0 weights whose products run on the large-M kernel keeps the F16 image of every
  * weight it has used (made once instead of once per product) while they fit this many MB per state (default 65536;
- * the 4B model needs 16 GB); weights beyond that, or all with 0, get an image per product. */
+ * the 4B model needs 16 GB); weights beyond that, or all with 0, get an image per product.  With 0 the prompts of a
+ * generation state form the tiles of its F16 weights per product too, instead of keeping them: the same results. */
 void hip_gemm_image_budget_mb(int mb);
 /* Training attention without the [seq, seq] probability matrices in memory (running softmax in the forward, the
  * probabilities formed again in the backward): -1 = for head_dim 64 / 128 when ceil(seq / 128) * query heads * batch

@@ -118,6 +118,7 @@ double weight_stream_bytes(const WeightOp &W, int N, int K);
 // `keep`: the image goes there (tiled_elems(N, K) halves, the caller's) instead of the scratch arena; with
 // f16_part_only only the tiles that are F16 in W are written (the Q8_0 part of `keep` holds its image from before).
 WeightOp f16_image_of(const WeightOp &W, int N, int K, void *keep = nullptr, bool f16_part_only = false);
+size_t image_budget();                                    // bytes (hip_gemm_image_budget_mb, sft.hip)
 bool large_m_unpacks_q8();                                // the large-M policy that reads Q8_0 tiles itself is in force
 // chunks > 1 (F16 tiles only): the K steps are cut into that many chunks, chunk c writing the plane at C + c * plane_stride;
 // big_gemm_chunks: what the measured rule picks for a product
@@ -166,7 +167,7 @@ void gemm_f32a_exact(const float *A, struct ::MetalBuf *W, float *C, int M, int 
 // plan_gemm(2M, N, K) into planes of [2M, N]; C [M, N] from the planes.
 const half_t *tiled_weight_of(struct ::MetalBuf *W, int N, int K);
 void launch_rows_to_f16_split(const float *A, half_t *a16, float *inv, int M, int K);
-void launch_reduce_planes_split(const float *P, int S, size_t plane_stride, int ldp, const float *inv, float *C, int M, int N);
+void launch_reduce_planes_split(const float *P, int S, size_t plane_stride, int ldp, const float *inv, float *C, int M, int N, int ldc = 0);   // (ldc 0: N)
 // element (m, n) of such a product: the planes of row m and of row M + m summed, each sum times its row's factor
 __device__ __forceinline__ float split_planes_value(const float *__restrict__ P, int S, size_t plane_stride, int ldp,
                                                     const float *__restrict__ inv, int M, int m, int n)

@@ -139,12 +139,12 @@ __global__ void fill_random_f16(half_t *p, size_t n, uint32_t seed)
 
 // C[m, n] = sum over planes of row m and of row M + m, each times its row factor
 __global__ void reduce_planes_split(const float *__restrict__ P, int S, size_t plane_stride, int ldp,
-                                    const float *__restrict__ row_scale, float *__restrict__ C, int M, int N)
+                                    const float *__restrict__ row_scale, float *__restrict__ C, int M, int N, int ldc)
 {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)M * N) return;
     const int m = (int)(idx / N), n = (int)(idx % N);
-    C[idx] = lmhip::split_planes_value(P, S, plane_stride, ldp, row_scale, M, m, n);
+    C[(size_t)m * ldc + n] = lmhip::split_planes_value(P, S, plane_stride, ldp, row_scale, M, m, n);
 }
 
 __global__ void reduce_planes(const float *__restrict__ P, int S, size_t plane_stride, int ldp,
@@ -765,10 +765,10 @@ void launch_rows_to_f16_split(const float *A, half_t *a16, float *inv, int M, in
     else hipLaunchKernelGGL(rows_to_f16_split, dim3(M), dim3(256), 0, stream(), A, K, a16, inv, M, K, tiled_kb(K));
 }
 
-void launch_reduce_planes_split(const float *P, int S, size_t plane_stride, int ldp, const float *inv, float *C, int M, int N)
+void launch_reduce_planes_split(const float *P, int S, size_t plane_stride, int ldp, const float *inv, float *C, int M, int N, int ldc)
 {
     const size_t n = (size_t)M * N;
-    hipLaunchKernelGGL(reduce_planes_split, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream(), P, S, plane_stride, ldp, inv, C, M, N);
+    hipLaunchKernelGGL(reduce_planes_split, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream(), P, S, plane_stride, ldp, inv, C, M, N, ldc ? ldc : N);
 }
 
 // C[M, N] fp32 = A[M, K] fp32 * W^T, W an F16 [N, K] weight buffer, with A split into value and residual rows

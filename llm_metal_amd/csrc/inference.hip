@@ -22,6 +22,7 @@
 #include <string.h>
 #include <string>
 #include <sys/stat.h>
+#include <unistd.h>
 #include <vector>
 
 using namespace lmhip;
@@ -82,6 +83,9 @@ struct InferenceState {
     float scaling;
     MetalBuf *lora_t;                    // [2R]: A_q ln | A_v ln
     PromptRun *prompt;                   // scratch of prompts taken many tokens at a time (NULL until used)
+    bool prompt_refused;                 // no room for it
+    uint64_t q8_fit_version;             // versions of the weights that q8_fit was found for (0: none)
+    bool q8_fit;
     BatchRun *batch;                     // scratch and caches of the lock-step batch path, kept from call to call (NULL until used)
 };
 
@@ -1099,6 +1103,7 @@ void step_on_run(InferenceState *s, int token, int pos)
 
 constexpr int PROMPT_ROWS = 1024;        // tokens of one step
 constexpr int PROMPT_WANT = 32;          // rows of logits formed together
+constexpr int PROMPT_HEAD_ROWS = 65536;  // rows of the head multiplied at a time
 
 struct PromptRun {
     int cap;                             // rows the buffers are sized for
@@ -1121,50 +1126,83 @@ size_t free_memory()
     return f;
 }
 
-// Whether n tokens go many to a step: from five on.  A step of 2 to 32 rows takes 1.0 ms on F16 weights (nine layers of the 4B
-// shape; 1.8 tokens one by one) and 2.5 ms on Q8_0 ones (4.5 tokens: their tiled images are formed anew for every product), and
-// 500 tokens take 4.3 instead of 458 ms; portions of up to four stay bit for bit what single tokens give.
-// The first time: room for the tiled images of F16 weights (kept, as the batch path keeps them) besides 2 GB, and no Q8_0
-// weight beyond what a half holds; a state that does not qualify takes its tokens one by one.
-bool prompt_takes(InferenceState *s, int n)
+// Whether `bytes` are free besides 2 GB for everything allocated later.  The driver clears freed memory before it counts as free
+// again, some milliseconds after the call that freed it; settled: a figure that is too low is read until it stands still for 20 ms.
+bool memory_for(size_t bytes, bool settled)
+{
+    bytes += (size_t)2 << 30;
+    size_t before = free_memory();
+    for (int same = 0, i = 0; settled && before < bytes && same < 4 && i < 100; i++) {
+        usleep(5000);
+        const size_t now = free_memory();
+        same = now == before ? same + 1 : 0;
+        before = now;
+    }
+    return before >= bytes;
+}
+
+// What the products of a step of up to `cap` tokens need: planes, and the F16 images of the largest matrix where none is kept
+size_t prompt_product_bytes(const InferenceState *s, int cap)
 {
     const bool q8 = !s->use_fp16 && !s->borrows_tiles;
-    if (s->stack || n < 5 || !prompt_attention_supported(s->hd) || s->D > 8192 || s->R > 64) return false;
-    if (s->prompt) return true;
-    if (!s->borrows_tiles) {
-        size_t need = (size_t)2 << 30;
-        MetalBuf *top = nullptr;
-        if (q8) {
-            top = metal_buf_create(sizeof(unsigned));
-            HIP_CHECK(hipMemsetAsync(dptr(top), 0, sizeof(unsigned), stream()));
+    const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
+    const int shapes[4][2] = {{qd + 2 * kd + (s->borrows_tiles ? 2 * s->R : 0), s->D}, {s->D, qd}, {2 * s->IS, s->D}, {s->D, s->IS}};
+    const int head = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V), want = 2 * std::min(PROMPT_WANT, cap);
+    size_t planes = (size_t)plan_short_sums(want, head, s->D, 0, 0).planes() * want * head * sizeof(float), planes2 = 0, image = tiled_elems(head, s->D) * sizeof(half_t);
+    for (const auto &sh : shapes) {
+        image = std::max(image, tiled_elems(sh[0], sh[1]) * sizeof(half_t));
+        for (int m = 64; m - 64 < 2 * cap; m += 64) {
+            const int M = std::min(m, 2 * cap);
+            const size_t n = (size_t)plan_short_sums(M, sh[0], sh[1], 0, 0).planes() * M * sh[0] * sizeof(float);
+            planes = std::max(planes, n);
+            if (M <= cap) planes2 = std::max(planes2, n);
         }
-        const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
-        for (int L = 0; L < s->NL; L++) {
-            const InferenceState::Layer &lw = s->layers[L];
-            for (const WMat *w : {&lw.qkv, (const WMat *)lw.o, &lw.gu, (const WMat *)lw.down}) {
-                if (q8) q8_max_scale(w->mbuf, w->rows, w->cols, dptr_as<unsigned>(top));
-                else if (!w->mbuf->tiled[0].dev) need += tiled_elems(w->rows, w->cols) * sizeof(half_t);
-            }
-        }
-        bool fits = true;
-        if (q8) {
-            unsigned bits = 0;
-            HIP_CHECK(hipMemcpyAsync(&bits, dptr(top), sizeof bits, hipMemcpyDeviceToHost, stream()));
-            HIP_CHECK(hipStreamSynchronize(stream()));
-            metal_buf_free(top);
-            float d;
-            memcpy(&d, &bits, sizeof d);
-            fits = d * 128.f < 65504.f;                                   // (false for a NaN)
-            need += 2 * sizeof(half_t) * std::max({tiled_elems(qd + 2 * kd, s->D), tiled_elems(2 * s->IS, s->D), tiled_elems(s->D, s->IS), tiled_elems(s->D, qd)});
-        }
-        if (!fits || free_memory() < need) return false;
     }
-    s->prompt = new PromptRun{};
-    PromptRun &r = *s->prompt;
+    return planes + (q8 ? planes2 + 2 * image : image);
+}
+
+// The weights' Q8_0 scales are small enough that two F16 images hold d q.  Asked once for what the weights hold (their versions).
+bool q8_scales_fit(InferenceState *s)
+{
+    uint64_t version = 1;                                             // (0: not asked yet)
+    for (int L = 0; L < s->NL; L++) {
+        const InferenceState::Layer &lw = s->layers[L];
+        for (const WMat *w : {&lw.qkv, (const WMat *)lw.o, &lw.gu, (const WMat *)lw.down}) version += w->mbuf->version;
+    }
+    if (s->q8_fit_version == version) return s->q8_fit;
+    MetalBuf *top = metal_buf_create(sizeof(unsigned));
+    unsigned bits = 0;
+    metal_buf_write(top, 0, &bits, sizeof bits);
+    for (int L = 0; L < s->NL; L++) {
+        const InferenceState::Layer &lw = s->layers[L];
+        for (const WMat *w : {&lw.qkv, (const WMat *)lw.o, &lw.gu, (const WMat *)lw.down}) q8_max_scale(w->mbuf, w->rows, w->cols, dptr_as<unsigned>(top));
+    }
+    metal_buf_read(top, 0, &bits, sizeof bits);
+    metal_buf_free(top);
+    float d;
+    memcpy(&d, &bits, sizeof d);
+    s->q8_fit_version = version;
+    return s->q8_fit = d * 128.f < 65504.f;                           // (false for a NaN)
+}
+
+// Whether n tokens go many to a step: from five on.  A step of 2 to 32 rows takes 1.0 ms on F16 weights (nine layers of the 4B
+// shape; 1.8 tokens one by one) and 2.4 ms on Q8_0 ones (4.5 tokens: their tiled images are formed anew for every product), and
+// 500 tokens take 3.6 instead of 458 ms; portions of up to four stay bit for bit what single tokens give.
+// A state takes its tokens one by one where a Q8_0 weight is beyond what a half holds and, decided once with its first prompt,
+// where there is no room for a step's buffers.
+bool prompt_takes(InferenceState *s, int n)
+{
+    if (s->stack || n < 5 || !prompt_attention_supported(s->hd) || s->D > 8192 || s->R > 64 || s->prompt_refused) return false;
+    if (!s->use_fp16 && !s->borrows_tiles && !q8_scales_fit(s)) return false;
+    if (s->prompt) return true;
     const int qd = s->Hq * s->hd, cap = std::min(PROMPT_ROWS, s->max_seq);
-    r.cap = cap;
     size_t a16 = 0;
     for (int K : {s->D, qd, s->IS}) a16 = std::max(a16, tiled_elems(2 * cap, K));
+    const size_t rows = (size_t)cap * (2 * (size_t)s->D + 2 * (size_t)qd + (prompt_glu_supported(s->IS) ? 0 : s->IS) + 4 + 2 * s->R) + s->max_seq + (size_t)PROMPT_WANT * s->D;
+    if (!memory_for(rows * sizeof(float) + a16 * sizeof(half_t) + prompt_product_bytes(s, cap), true)) { s->prompt_refused = true; return false; }
+    s->prompt = new PromptRun{};
+    PromptRun &r = *s->prompt;
+    r.cap = cap;
     r.x = fbuf((size_t)cap * s->D); r.ln = fbuf((size_t)cap * s->D);
     r.q = fbuf((size_t)cap * qd); r.att = fbuf((size_t)cap * qd);
     if (!prompt_glu_supported(s->IS)) r.act = fbuf((size_t)cap * s->IS);
@@ -1176,6 +1214,20 @@ bool prompt_takes(InferenceState *s, int n)
     return true;
 }
 
+// Rows row0 .. row0 + rows of a row-major F16 matrix as GEMM tiles (row0 a multiple of 32): a part of its image, which is kept with
+// the matrix when there is room for it, or else formed in scratch for this product -- the same tiles, so the same results.
+const half_t *prompt_tiles(const WMat *w, int row0, int rows)
+{
+    const size_t Kb = tiled_kb(w->cols);
+    if (w->mbuf->tiled[0].dev || (image_budget() && memory_for(tiled_elems(w->rows, w->cols) * sizeof(half_t), false)))
+        return tiled_weight_of(w->mbuf, w->rows, w->cols) + (size_t)(row0 / 32) * Kb * 2048;
+    const size_t n = tiled_elems(rows, w->cols);
+    half_t *img = (half_t *)scratch(SCR_WF16, n * sizeof(half_t));
+    if (rows % 32 || w->cols % 64) launch_fill_f32((float *)img, 0.f, n / 2);         // (the tiling writes no padding)
+    launch_tile_f16(dptr_as<half_t>(w->mbuf) + (size_t)row0 * w->cols, rows, w->cols, img, (int)Kb, 0, 0, 0);
+    return img;
+}
+
 // a buffer of at least n floats (what it held is gone when it grows)
 float *at_least(MetalBuf *&b, size_t n)
 {
@@ -1185,7 +1237,7 @@ float *at_least(MetalBuf *&b, size_t n)
 
 // planes of (the operand in r.a16, rows split by `inv`) x w^T: w the state's own matrix (its tiled F16 image, or for Q8_0 the
 // two images of d q and of what rounding that to F16 lost) or a training state's tiles
-SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv, int M)
+SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv, int M, int row0 = 0)
 {
     const half_t *a16 = dptr_as<half_t>(r.a16);
     auto planes = [&](const WeightOp &op, int m, MetalBuf *&buf, size_t &stride) {
@@ -1197,7 +1249,7 @@ SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const
     SplitPlanes out{};
     out.inv = inv; out.N = rows;
     if (tiles) out.S = planes(*tiles, 2 * M, r.planes, out.plane);
-    else if (s->use_fp16) out.S = planes(weight_f16(tiled_weight_of(w->mbuf, rows, cols)), 2 * M, r.planes, out.plane);
+    else if (s->use_fp16) out.S = planes(weight_f16(prompt_tiles(w, row0, rows)), 2 * M, r.planes, out.plane);
     else {
         const size_t n = tiled_elems(rows, cols);
         half_t *hi = (half_t *)scratch(SCR_WF16, 2 * n * sizeof(half_t)), *lo = hi + n;
@@ -1275,9 +1327,7 @@ void prompt_logits(InferenceState *s, PromptRun &r, const int *m, int count, flo
     auto row = [&](int i, float *dst) {
         HIP_CHECK(hipMemcpyAsync(dst, dptr_as<float>(r.ln) + (size_t)m[i] * D, (size_t)D * 4, hipMemcpyDeviceToDevice, stream()));
     };
-    bool one_by_one = !s->borrows_tiles && (!s->use_fp16 || count < 4);
-    if (!s->borrows_tiles && !one_by_one && !s->lm_head->mbuf->tiled[0].dev)            // room for the head's tiled image
-        one_by_one = free_memory() < tiled_elems(s->V, D) * sizeof(half_t) + ((size_t)2 << 30);
+    const bool one_by_one = !s->borrows_tiles && (!s->use_fp16 || count < 4);
     if (one_by_one) {
         for (int i = 0; i < count; i++) {
             row(i, dptr_as<float>(s->ln));
@@ -1290,8 +1340,11 @@ void prompt_logits(InferenceState *s, PromptRun &r, const int *m, int count, flo
     }
     for (int i = 0; i < count; i++) row(i, dptr_as<float>(r.sel) + (size_t)i * D);
     launch_rows_to_f16_split(dptr_as<float>(r.sel), dptr_as<half_t>(r.a16), dptr_as<float>(r.inv_br), count, D);
-    const SplitPlanes lg = prompt_product(s, r, s->lm_head, s->borrows_tiles ? &s->borrowed_lm : nullptr, s->V, D, dptr_as<float>(r.inv_br), count);
-    launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, out, count, lg.N);
+    for (int n0 = 0, n; n0 < s->V; n0 += n) {              // (own weights: in parts, for which there is room in scratch if not for the whole head's image)
+        n = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V - n0);
+        const SplitPlanes lg = prompt_product(s, r, s->lm_head, s->borrows_tiles ? &s->borrowed_lm : nullptr, n, D, dptr_as<float>(r.inv_br), count, n0);
+        launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, out + n0, count, n, s->V);
+    }
 }
 
 // n tokens from position pos on, in portions of equal size; after each, f(first token of the portion, its length)

@@ -714,6 +714,8 @@ MetalBuf *host_buf(size_t bytes, void **cpu)
 
 }  // namespace
 
+namespace lmhip { size_t image_budget() { return g_image_budget; } }
+
 extern "C" {
 
 SFTState *sft_state_create_from_ref(const SFTModelRef *m, int batch, int seq_len, int lora_rank, float lora_alpha,

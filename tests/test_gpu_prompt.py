@@ -4,6 +4,7 @@ they agree to about sqrt(layers) ulps of the largest logit: 2e-5 leaves a factor
 import numpy as np
 import pytest
 
+from llm_metal_amd import lib
 from llm_metal_amd.configs import C1, GEMMA3, QWEN3, SFTConfig
 from llm_metal_amd.sft import InferenceState, SFTState
 from llm_metal_amd.synth import make_batch, make_model
@@ -144,3 +145,23 @@ def test_prompt_is_as_exact_as_single_tokens(c, n):
         got = inf.forward_tokens(toks, range(n))
     print(rel(got, want), rel(single, want))
     assert rel(got, want) < 1.1 * rel(single, want)
+
+
+def test_prompt_tiles_kept_or_formed_per_product():
+    """Without room for the tiles of its weights a state forms them in scratch for every product: the same logits, bit for bit, the
+    head's included (70000 rows go in two parts; 1312 columns and 2084 rows leave padding)."""
+    c = C1.with_(name="tiles", D=1312, IS=2084, NL=2, Hq=12, Hkv=4, V=70000)
+    model, toks, got = make_model(c, seed=41, gamma_jitter=0.1), tokens(c, 90, 42), []
+    L = lib.load()
+    for mb in (0, 65536):
+        L.hip_gemm_image_budget_mb(mb)
+        try:
+            with InferenceState(c, model, max_seq=90) as inf:
+                want = one_by_one(inf, toks[:40]) if not got else None
+                inf.reset()
+                got.append(inf.forward_tokens(toks, range(3, 40)))
+                if want is not None:
+                    assert maxrel(got[0], want[3:]) < TOL
+        finally:
+            L.hip_gemm_image_budget_mb(65536)
+    assert np.array_equal(got[0], got[1])
