@@ -351,7 +351,8 @@ __global__ __launch_bounds__(256) void k_apply_retile(half8 *__restrict__ W, hal
 __global__ __launch_bounds__(256) void k_untile_tiles(const half8 *__restrict__ src, int Kb, int rb0, int rows, int cols, half_t *__restrict__ dst)
 {
     __shared__ half8 t[4][32][9];                          // (a row's eight pieces and one of padding)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = blockIdx.x * 4 + wave, rb = blockIdx.y;
+    const int across = ((cols + 63) / 64 + 3) / 4;         // workgroups along a row block (1-D grid: the row blocks may be more than 65535)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = blockIdx.x % across * 4 + wave, rb = blockIdx.x / across;
     if (kb * 64 < cols) {
         const half8 *p = src + ((size_t)(rb0 + rb) * Kb + kb) * 256 + lane;
 #pragma unroll
@@ -459,7 +460,7 @@ void launch_untile_f16(const half_t *src_tiled, int Kb, int row_off, int k_off, 
     const size_t n = (size_t)rows * cols;
     if (!n) return;
     if (!transpose && k_off == 0 && row_off % 32 == 0 && cols % 8 == 0 && !((uintptr_t)dst & 15)) {
-        LAUNCH(k_untile_tiles, dim3((tiled_kb(cols) + 3) / 4, tiled_rb(rows)), dim3(256), 0, reinterpret_cast<const half8 *>(src_tiled), Kb, row_off / 32, rows, cols, dst);
+        LAUNCH(k_untile_tiles, dim3((unsigned)((tiled_kb(cols) + 3) / 4) * tiled_rb(rows)), dim3(256), 0, reinterpret_cast<const half8 *>(src_tiled), Kb, row_off / 32, rows, cols, dst);
         return;
     }
     LAUNCH(k_untile_f16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, src_tiled, Kb, row_off, k_off, transpose, rows, cols, dst);

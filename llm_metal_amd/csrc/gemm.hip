@@ -196,7 +196,8 @@ __global__ __launch_bounds__(256) void q8_operand_to_f16(lmhip::WeightOp W, int 
 __global__ __launch_bounds__(256) void tile_f16_rows(const half_t *__restrict__ src, int rows, int cols, half8 *__restrict__ dst, int Kb, int rb0)
 {
     __shared__ half8 t[4][32][9];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = blockIdx.x * 4 + wave, rb = blockIdx.y;
+    const int across = ((cols + 63) / 64 + 3) / 4;         // workgroups along a row block (1-D grid: the row blocks may be more than 65535)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = blockIdx.x % across * 4 + wave, rb = blockIdx.x / across;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int r = rb * 32 + 8 * i + (lane >> 3), c = kb * 64 + 8 * (lane & 7);
@@ -518,7 +519,7 @@ void launch_tile_f16(const half_t *src, int rows, int cols, half_t *dst_tiled, i
 {
     if (rows <= 0 || cols <= 0) return;
     if (!transpose && k_off == 0 && row_off % 32 == 0 && cols % 8 == 0 && !((uintptr_t)src & 15)) {
-        hipLaunchKernelGGL(tile_f16_rows, dim3((tiled_kb(cols) + 3) / 4, tiled_rb(rows)), dim3(256), 0, stream(), src, rows, cols,
+        hipLaunchKernelGGL(tile_f16_rows, dim3((unsigned)((tiled_kb(cols) + 3) / 4) * tiled_rb(rows)), dim3(256), 0, stream(), src, rows, cols,
                            reinterpret_cast<half8 *>(dst_tiled), Kb_dst, row_off / 32);
         HIP_CHECK(hipGetLastError());
         return;

@@ -69,7 +69,7 @@ def test_matvec_with_a_row_per_workgroup(dev, rows, cols):
 
 
 @pytest.mark.parametrize("rows,cols,B", [(4112, 1024, 2), (300, 2560, 3), (4096, 512, 4), (515, 1152, 5), (4096, 256, 8),
-                                         (1000, 512, 9), (2048, 640, 32), (64, 50, 3)])
+                                         (1000, 512, 9), (2048, 640, 32), (64, 50, 3), (65536 * 32 + 7, 8, 2)])   # (more row blocks than a grid's second dimension holds)
 def test_f16_batch_matvec(dev, rows, cols, B):
     say("f16_batch_matvec", rows, cols, B)
     rng = np.random.default_rng(rows + cols + B)
