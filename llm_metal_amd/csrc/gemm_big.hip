@@ -233,7 +233,6 @@ __global__ __launch_bounds__(256) void gemm_big(GemmKArgs g)
         return;
     }
     // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
-    const EdgeStore edge(g.P + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
     uint32_t col[NW];
 #pragma unroll
     for (int k = 0; k < NW; k++) { const int n = (nb0 + NW * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
@@ -244,9 +243,11 @@ __global__ __launch_bounds__(256) void gemm_big(GemmKArgs g)
         for (int v = 0; v < 16; v++)
             sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
 #pragma unroll
-        for (int v = 0; v < 16; v++)
+        for (int v = 0; v < 16; v++) {
+            const EdgeStore edge(g.P, (mb0 + 2 * wm + i) * 32 + 8 * (v >> 2), g.M, g.ldp);
 #pragma unroll
-            for (int k = 0; k < NW; k++) edge.f32((2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+            for (int k = 0; k < NW; k++) edge.f32(4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+        }
     }
 }
 
@@ -421,7 +422,6 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
         return;
     }
     // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
-    const EdgeStore edge(Cp + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
     uint32_t col[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
@@ -432,9 +432,11 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
         for (int v = 0; v < 16; v++)
             sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
 #pragma unroll
-        for (int v = 0; v < 16; v++)
+        for (int v = 0; v < 16; v++) {
+            const EdgeStore edge(Cp, (mb0 + 2 * wm + i) * 32 + 8 * (v >> 2), g.M, g.ldp);
 #pragma unroll
-            for (int k = 0; k < 4; k++) edge.f32((2 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+            for (int k = 0; k < 4; k++) edge.f32(4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+        }
     }
 }
 
@@ -581,7 +583,6 @@ __global__ __launch_bounds__(256) void gemm_big_f16_256(GemmKArgs g)
         return;
     }
     // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
-    const EdgeStore edge(Cp + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
     uint32_t col[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
@@ -592,9 +593,11 @@ __global__ __launch_bounds__(256) void gemm_big_f16_256(GemmKArgs g)
         for (int v = 0; v < 16; v++)
             sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
 #pragma unroll
-        for (int v = 0; v < 16; v++)
+        for (int v = 0; v < 16; v++) {
+            const EdgeStore edge(Cp, (mb0 + 4 * wm + i) * 32 + 8 * (v >> 2), g.M, g.ldp);
 #pragma unroll
-            for (int k = 0; k < 4; k++) edge.f32((4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+            for (int k = 0; k < 4; k++) edge.f32(4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+        }
     }
 }
 
@@ -800,7 +803,6 @@ __global__ __launch_bounds__(256) void gemm_big_q8(GemmKArgs g)
         return;
     }
     // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
-    const EdgeStore edge(Cp + (size_t)mb0 * 32 * g.ldp, g.M - mb0 * 32, g.ldp);
     uint32_t col[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
@@ -811,9 +813,11 @@ __global__ __launch_bounds__(256) void gemm_big_q8(GemmKArgs g)
         for (int v = 0; v < 16; v++)
             sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + MI * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
 #pragma unroll
-        for (int v = 0; v < 16; v++)
+        for (int v = 0; v < 16; v++) {
+            const EdgeStore edge(Cp, (mb0 + MI * wm + i) * 32 + 8 * (v >> 2), g.M, g.ldp);
 #pragma unroll
-            for (int k = 0; k < 4; k++) edge.f32((MI * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+            for (int k = 0; k < 4; k++) edge.f32(4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
+        }
     }
 }
 

@@ -91,17 +91,19 @@ __device__ __forceinline__ void load_w_q8_cols(half8 (&w)[4], const WeightOp &W,
 
 // Stores of a tile that reaches past the matrix.  Under a test per element the compiler branches around every store and drains
 // the queue before it -- 12 to 15 us per launch of the large-M kernels (250 rows: 33 us on 6176 x 2560 against 18 at 256,
-// whose tiles lie inside).  Here nothing branches: the stores go through a buffer descriptor that ends with the matrix's last
-// row, and an element in a column past the end gets an offset past that end; the hardware drops what lies outside.
+// whose tiles lie inside).  Here nothing branches: the stores go through buffer descriptors that end with the matrix's last
+// row, and an element in a column past the end gets an offset past that end; the hardware drops what lies outside.  A descriptor
+// covers eight rows: offsets have 31 bits, which 256 rows of 2^21 floats would pass (eight: of 2^26).
 struct EdgeStore {
     __amdgpu_buffer_rsrc_t window;
     int row_bytes;
-    // base: the tile's first row; rows: of the matrix from there on (a tile has at most 256); ld: row stride
-    template <typename T> __device__ __forceinline__ EdgeStore(T *base, int rows, int ld)
+    // base: the matrix's first row; row: the first of the eight (uniform); rows: of the matrix; ld: row stride
+    template <typename T> __device__ __forceinline__ EdgeStore(T *base, int row, int rows, int ld)
     {
+        row = __builtin_amdgcn_readfirstlane(row);
         row_bytes = ld * (int)sizeof(T);
-        const size_t n = (size_t)min(rows, 256) * (size_t)row_bytes;
-        window = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(n < 0x7fffffff ? n : 0x7fffffff), 0x00020000);
+        const int n = __builtin_amdgcn_readfirstlane(min(max(rows - row, 0), 8));      // (a descriptor the compiler takes for divergent costs a loop per store)
+        window = __builtin_amdgcn_make_buffer_rsrc((void *)(base + (size_t)row * ld), 0, n * row_bytes, 0x00020000);
     }
     static __device__ __forceinline__ uint32_t column(bool in, int bytes) { return in ? (uint32_t)bytes : 0x80000000u; }
     __device__ __forceinline__ void f32(int row, uint32_t col, float v) const
@@ -268,10 +270,10 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_tiled(GemmKArgs g)
                 Pp[(size_t)m * g.ldp + n] = sres[k]; \
             } \
         } else { \
-            const EdgeStore edge(Pp + (size_t)mb0 * 32 * g.ldp, M - mb0 * 32, g.ldp); \
             _Pragma("unroll") for (int k = 0; k < Q; k++) { \
                 const int i = i0 + k, mb = i / (NB * 16), b = (i / 16) % NB, v = i % 16, n = (nb0 + b) * 32 + r; \
-                edge.f32(mb * 32 + 8 * (v >> 2) + 4 * h + (v & 3), EdgeStore::column(n < N, n * 4), sres[k]); \
+                const EdgeStore edge(Pp, (mb0 + mb) * 32 + 8 * (v >> 2), M, g.ldp); \
+                edge.f32(4 * h + (v & 3), EdgeStore::column(n < N, n * 4), sres[k]); \
             } \
         } } }
     ALL_WAVES(PART_STORE, 0)
@@ -454,10 +456,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
 #pragma unroll
             for (int k = 0; k < Q; k++) { const int v = kg * Q + k; Ph[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = f2h(res[k] * g.half_scale); }
         } else {
-            const EdgeStore edge(Ph, g.M, g.ldp);
             const uint32_t col = EdgeStore::column(n < g.N, n * 2);
 #pragma unroll
-            for (int k = 0; k < Q; k++) { const int v = kg * Q + k; edge.f16(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, f2h(res[k] * g.half_scale)); }
+            for (int k = 0; k < Q; k++) { const int v = kg * Q + k; EdgeStore(Ph, qm * 32 + 8 * (v >> 2), g.M, g.ldp).f16(4 * h + (v & 3), col, f2h(res[k] * g.half_scale)); }
         }
         return;
     }
@@ -473,10 +474,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_ring(KARGS24)
 #pragma unroll
         for (int k = 0; k < Q; k++) { const int v = kg * Q + k; Pp[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = res[k]; }
     } else {
-        const EdgeStore edge(Pp, g.M, g.ldp);
         const uint32_t col = EdgeStore::column(n < g.N, n * 4);
 #pragma unroll
-        for (int k = 0; k < Q; k++) { const int v = kg * Q + k; edge.f32(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, res[k]); }
+        for (int k = 0; k < Q; k++) { const int v = kg * Q + k; EdgeStore(Pp, qm * 32 + 8 * (v >> 2), g.M, g.ldp).f32(4 * h + (v & 3), col, res[k]); }
     }
 }
 
@@ -620,10 +620,9 @@ __global__ __launch_bounds__(512) void gemm_ring_wide(KARGS24)
 #pragma unroll
             for (int v = 0; v < 16; v++) Ph[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = f2h(acc[v] * g.half_scale);
         } else {
-            const EdgeStore edge(Ph, g.M, g.ldp);
             const uint32_t col = EdgeStore::column(n < g.N, n * 2);
 #pragma unroll
-            for (int v = 0; v < 16; v++) edge.f16(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, f2h(acc[v] * g.half_scale));
+            for (int v = 0; v < 16; v++) { EdgeStore(Ph, qm * 32 + 8 * (v >> 2), g.M, g.ldp).f16(4 * h + (v & 3), col, f2h(acc[v] * g.half_scale)); }
         }
         return;
     }
@@ -636,10 +635,9 @@ __global__ __launch_bounds__(512) void gemm_ring_wide(KARGS24)
 #pragma unroll
         for (int v = 0; v < 16; v++) Pp[(size_t)(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * g.ldp + n] = acc[v];
     } else {
-        const EdgeStore edge(Pp, g.M, g.ldp);
         const uint32_t col = EdgeStore::column(n < g.N, n * 4);
 #pragma unroll
-        for (int v = 0; v < 16; v++) edge.f32(qm * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col, acc[v]);
+        for (int v = 0; v < 16; v++) { EdgeStore(Pp, qm * 32 + 8 * (v >> 2), g.M, g.ldp).f32(4 * h + (v & 3), col, acc[v]); }
     }
 }
 

@@ -8,7 +8,7 @@ from llm_metal_amd import lib
 from llm_metal_amd.configs import C1, GEMMA3, QWEN3, SFTConfig
 from llm_metal_amd.sft import InferenceState, SFTState
 from llm_metal_amd.synth import make_batch, make_model
-from tests.gpu_util import rel
+from tests.gpu_util import maxrel, rel
 
 pytestmark = pytest.mark.gpu
 # widths that no tile divides: 2084 = 65 blocks of 32 + 4, 1312 = 20.5 K steps, 8212 columns in the head
@@ -72,3 +72,24 @@ def test_prompt_equals_streaming_kernel(n):
             finally:
                 L.hip_gemm_force_large_m(0)
     assert rel(got[1], got[0]) < 5e-6 and rel(got[2], got[0]) < 5e-6          # operands of 22 bits
+
+
+def test_rows_of_many_columns():
+    """Blocks that reach past a matrix of 2.6 million columns: 256 of its rows are more bytes than one descriptor's offsets have
+    bits.  Targets in the last, ragged block of columns, in the last rows of the only block of rows."""
+    c = C1.with_(name="wide_head", NL=1, D=64, Hq=2, Hkv=1, hd=32, IS=64, V=2_600_004, seq=256, R=2, tied=True)
+    model = make_model(c, seed=27)
+    tok, _ = make_batch(c, seed=28)
+    tgt = (c.V - 1 - np.arange(c.BN) % 100).astype(np.uint32)
+    L, got = lib.load(), []
+    for policy, block in ((-1, 0), (1, 2), (1, 1)):
+        L.hip_gemm_force_large_m(policy)
+        L.hip_gemm_large_m_block(block)
+        try:
+            with SFTState(c, model) as st:
+                st.train_step(tok, tgt, 0.0)
+                got.append(st.losses())
+        finally:
+            L.hip_gemm_force_large_m(0)
+            L.hip_gemm_large_m_block(0)
+    assert np.ptp(got[0]) > 0 and maxrel(got[1], got[0]) < 1e-5 and maxrel(got[2], got[0]) < 1e-5
