@@ -410,13 +410,14 @@ void forward_token(InferenceState *s, int token, int pos)
     // (matvec_norm) and the sum goes to the other of two residual buffers; the Q|K|V product only without adapters,
     // whose down-projection reads the normed vector too.
     MetalBuf *x = s->x, *x_other = s->x2;
-    // (Gemma3's branch is normed on its way into the sum: matvec_norms_around does that too)
+    // (Gemma3's branch is normed on its way into the sum: matvec_norms_around does that too; a model may come without the norm of
+    // its feed-forward branch)
     const bool fuse_ffn = D <= 12288, fuse_qkv = fuse_ffn && s->lora.empty();
     const int q8 = s->use_fp16 ? 0 : 1;
     auto normed_product = [&](MetalBuf *W, MetalBuf *branch, MetalBuf *g_branch, MetalBuf *g, MetalBuf *y, int rows, int glu) {
         NormIn n{dptr_as<float>(x), branch ? dptr_as<float>(branch) : nullptr, dptr_as<float>(g), branch ? dptr_as<float>(x_other) : nullptr,
                  s->eps, D, g_branch ? dptr_as<float>(g_branch) : nullptr, nullptr};
-        if (gemma) { matvec_norms_around(W, n, dptr_as<float>(y), rows, D, q8, glu); mark_written(y); }
+        if (gemma && (g_branch || !branch)) { matvec_norms_around(W, n, dptr_as<float>(y), rows, D, q8, glu); mark_written(y); }
         else matvec_norm(W, n, y, rows, D, q8, glu);
         if (branch) std::swap(x, x_other);
     };

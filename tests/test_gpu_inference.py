@@ -446,3 +446,17 @@ def test_sft_state_from_a_loaded_model_description(tmp_path):
     L.sft_state_free(h)
     L.model_ref_free(ref)
     assert la == lb                                                            # the same weights, the same arithmetic
+
+
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+def test_gemma_without_the_norm_behind_its_feed_forward(fmt):
+    """post_ff_norm_g of a model may be absent: the branch enters the sum as it is, token by token, in a prompt and in a batch."""
+    model = make_model(TINY_GEMMA, seed=61, gamma_jitter=0.1)
+    model["g_post_ff"] = [None] * TINY_GEMMA.NL
+    toks = [3, 70, 11, 500, 42, 7, 9, 300]
+    with InferenceState(TINY_GEMMA, model, max_seq=16, use_fp16=fmt == "f16") as inf:
+        got = np.stack([inf.forward_token(t) for t in toks])
+        inf.reset()
+        assert maxrel(inf.forward_tokens(toks, range(8)), got) < 2e-5
+        if fmt == "f16":
+            assert maxrel(np.stack([inf.step_batch([t, t], i)[1] for i, t in enumerate(toks)]), got) < 2e-5
