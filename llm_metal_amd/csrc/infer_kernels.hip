@@ -802,7 +802,8 @@ __global__ __launch_bounds__(TB) void k_attn_decode(const float *__restrict__ Q,
 // (columns d and d + HD / 2 of a rotary pair are in the same lane from HD = 128 on); the newest key and value do not take the
 // way through the cache, which the first head of a key head's group writes for the launches to come.
 // Against k_attn_decode<4, true> at up to 129 keys: 16.4 -> 5.8 us (four heads of 256), 9.6 -> 4.2 (8 x 32 heads of 128),
-// 11.1 -> 7.0 where 128 more workgroups request the next weights.
+// 11.1 -> 7.3 where 128 more workgroups request the next weights.  Sums are kept as short as that kernel's (lane_dot, the merge):
+// error against 64 bits 0.96 to 1.00 of its at 60 keys, 0.99 to 1.00 at 250 (heads of 64, 128, 256).
 constexpr int SHORT_KEYS = 256;
 template <int HD>
 __global__ __launch_bounds__(TB) void k_attn_short(float *__restrict__ out, int hd, int max_seq, int G, float scale, HeadPost hp)
@@ -826,6 +827,16 @@ __global__ __launch_bounds__(TB) void k_attn_short(float *__restrict__ out, int 
         v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));    // 7 - lane of eight
         v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, false));    // 15 - lane of sixteen
         return v;
+    };
+    // a lane's part of a sum over a head, in four sums of C: one over all 4 C columns rounds at each, and a score was up to 1.5 times
+    // as far from 64 bits as k_attn_decode's
+    auto lane_dot = [](const float4v (&x)[C], const float4v (&y)[C]) __attribute__((always_inline)) {
+        float4v s = x[0] * y[0];
+#pragma unroll
+        for (int c = 1; c < C; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[e] = fmaf(x[c][e], y[c][e], s[e]);
+        return (s[0] + s[1]) + (s[2] + s[3]);
     };
     float4v q[C], kn[C], vn[C], gq[C], gk[C], k[U][C], v[U][C];
     float2 rot[C][4];
@@ -856,12 +867,7 @@ __global__ __launch_bounds__(TB) void k_attn_short(float *__restrict__ out, int 
     // RMSNorm and RoPE of a head in the group's lanes
     auto finish = [&](float4v (&x)[C], const float4v (&g)[C], bool normed) __attribute__((always_inline)) {
         if (normed) {
-            float ss = 0.f;
-#pragma unroll
-            for (int c = 0; c < C; c++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) ss += x[c][e] * x[c][e];
-            const float inv = rsqrtf(sum16(ss) / (float)HD + hp.eps);
+            const float inv = rsqrtf(sum16(lane_dot(x, x)) / (float)HD + hp.eps);
 #pragma unroll
             for (int c = 0; c < C; c++)
 #pragma unroll
@@ -893,12 +899,7 @@ __global__ __launch_bounds__(TB) void k_attn_short(float *__restrict__ out, int 
         }
     }
     auto dot = [&](const float4v (&x)[C]) __attribute__((always_inline)) {
-        float s = 0.f;
-#pragma unroll
-        for (int c = 0; c < C; c++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) s = fmaf(q[c][e], x[c][e], s);
-        return sum16(s) * scale;
+        return sum16(lane_dot(q, x)) * scale;
     };
     // the newest key belongs to group 0
     const float s0 = dot(kn);
@@ -941,14 +942,14 @@ __global__ __launch_bounds__(TB) void k_attn_short(float *__restrict__ out, int 
     float all = pm[0];
 #pragma unroll
     for (int g = 1; g < 16; g++) all = fmaxf(all, pm[g]);
-    float den = 0.f, num = 0.f;
+    float den[4] = {}, num[4] = {};                        // (sums of four groups)
 #pragma unroll
     for (int g = 0; g < 16; g++) {
         const float w = __expf(pm[g] - all);
-        den = fmaf(pl[g], w, den);
-        num = fmaf(po[g][tid], w, num);
+        den[g >> 2] = fmaf(pl[g], w, den[g >> 2]);
+        num[g >> 2] = fmaf(po[g][tid], w, num[g >> 2]);
     }
-    out[((size_t)z * hp.Hq + hq) * HD + tid] = num / den;
+    out[((size_t)z * hp.Hq + hq) * HD + tid] = ((num[0] + num[1]) + (num[2] + num[3])) / ((den[0] + den[1]) + (den[2] + den[3]));
 }
 
 // merge of the slices of one query head: grid = Hq (times the sequences of a batch), block = hd threads (<= 256)
