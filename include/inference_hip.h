@@ -81,9 +81,10 @@ int inference_step_batch(InferenceState *state, const int *tokens, int batch_siz
 
 /* The next n tokens at the current position, which advances by n, and the logits [n_want][vocab] (host) at the places
  * want[0 .. n_want) among them, ascending; n_want may be 0.  A prompt may be cut into calls anywhere.  They run as
- * one step (long prompts: a few); the models that are not described layer by layer take portions of up to four tokens, and
- * all tokens where head_dim is not 32, 64, 128 or 256 or memory for the products' operands is short, one by one.  No counterpart in the reference.  Returns 0,
- * -1 when the arguments do not fit. */
+ * one step (long prompts: a few).  The models that are not described layer by layer take portions of up to four tokens one by
+ * one, and all tokens where head_dim is not 32, 64, 128 or 256, d_model is above 8192, the adapters' rank above 64, a Q8_0 scale
+ * beyond what fp16 products hold, or, found once by a state's first prompt, memory for a step's buffers short.  No counterpart
+ * in the reference.  Returns 0, -1 when the arguments do not fit. */
 int  inference_forward_tokens(InferenceState *state, const int *tokens, int n, const int *want, int n_want, float *logits);
 
 ModelType inference_state_model_type(InferenceState *state);         /* src/nn/fast_inference.h:31 */

@@ -393,7 +393,7 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
 }
 
 // Few long rows: the four waves of a workgroup share one, each with every fourth 512-column step, U of them requested at once, so a
-// row is one or two trips to memory instead of one per 2048 columns (and the last trip asks for nothing behind the row).
+// row is one or two trips to memory instead of one per 2048 columns.  (Steps behind the row ask for its last eight columns again.)
 // With a wave per row such a matrix has some five waves on a CU and a chain of several trips in each.  Cold weights: 1152 x 6912 Q8_0
 // 7.4 -> 5.0 us, F16 6.7 -> 5.8; 1536 x 4096 Q8_0 5.0 -> 3.9, 1024 x 4096 F16 4.3 -> 3.7.  Bound by the launch and one trip.
 template <int FMT, int U>
@@ -1329,7 +1329,7 @@ void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, floa
 #undef LN_LAUNCH
 }
 
-// glu 0: y = W . v; 1, 2: the gated pairs of matvec_glu (W has 2 * rows rows; 1 SiLU, 2 GELU); 3: tanh-GELU of it
+// act 0: y = W . v; 1, 2: the gated pairs of matvec_glu (W has 2 * rows rows; 1 SiLU, 2 GELU); 3: tanh-GELU of it
 void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int cols, int q8, int act)
 {
     bool ok = rows > 0 && nin.dim > 0 && nin.dim <= cols && !(cols & (q8 ? 31 : 7)) && cols <= 15360 && aligned16(dptr(W)) && nin.xr && nin.g && nin.x_out != nin.xr;

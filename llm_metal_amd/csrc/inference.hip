@@ -1188,7 +1188,8 @@ bool q8_scales_fit(InferenceState *s)
 
 // Whether n tokens go many to a step: from five on.  A step of 2 to 32 rows takes 1.0 ms on F16 weights (nine layers of the 4B
 // shape; 1.8 tokens one by one) and 2.4 ms on Q8_0 ones (4.5 tokens: their tiled images are formed anew for every product), and
-// 500 tokens take 3.6 instead of 458 ms; portions of up to four stay bit for bit what single tokens give.
+// 500 tokens take 3.7 instead of 460 ms; portions of up to four stay bit for bit what single tokens give.  A state's first prompt
+// pays for the buffers and the tiles that are kept besides: at five tokens up to 2 ms more than one by one, once, at sixteen none.
 // A state takes its tokens one by one where a Q8_0 weight is beyond what a half holds and, decided once with its first prompt,
 // where there is no room for a step's buffers.
 bool prompt_takes(InferenceState *s, int n)
