@@ -508,3 +508,19 @@ def test_gradient_norm_in_its_order_of_sums():
             v = v[..., 0]
             slots = ((F(0) + v[:, 0] + v[:, 1]) + v[:, 2]) + v[:, 3]
             assert norm == F(np.sqrt(slots.astype(np.float64).sum())), seed
+
+
+@pytest.mark.parametrize("batch,seq", [(1, 3), (1, 64), (1, 65), (3, 47), (2, 300)])
+def test_adapter_gradients_over_rows_and_columns_that_fill_no_tile(batch, seq):
+    """Rank 16: rows in groups of four over four or sixteen waves, columns of dY (108 and 36) and of the input (100) in blocks
+    of 64.  The bar is that of the steps above: fp16 operands of the products in front of these sums."""
+    cfg = C1.with_(name="adapter_grads", NL=2, D=100, Hq=3, Hkv=1, hd=36, IS=128, V=260, batch=batch, seq=seq)
+    model = make_model(cfg, seed=21, gamma_jitter=0.1)
+    tok, tgt = make_batch(cfg, seed=30)
+    r = run_oracle(cfg, model, [(tok, tgt)], 1e-4)[0]
+    with SFTState(cfg, model) as st:
+        st.train_step(tok, tgt, 1e-4)
+        assert abs(st.grad_norm() - r["grad_norm"]) <= 1e-2 * r["grad_norm"]
+        for L, (gv, rv) in enumerate(zip(lora_views(cfg, st.lora_grads()), lora_views(cfg, r["grad"]))):
+            for k in ("A_q", "B_q", "A_v", "B_v"):
+                assert rel(gv[k], rv[k]) < 1e-2, (L, k, rel(gv[k], rv[k]))
