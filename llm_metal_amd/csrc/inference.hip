@@ -11,6 +11,7 @@
 #include "devutil.h"
 #include "fused.h"
 #include "prompt.h"
+#include "few_rows.h"
 #include "stack.h"
 #include "../../include/inference_hip.h"
 #include "../../include/loader_hip.h"
@@ -932,6 +933,7 @@ __global__ __launch_bounds__(AM_WGS) void k_argmax_final_batch(const float *__re
 struct BatchRun {
     StackRun *stk;                                                       // a layer-by-layer model's caches, states and scratch (then only logits and best besides)
     int B, R, len;                                                       // sequences; adapter rank the scratch was sized for; positions held by the caches
+    bool few;                                                            // its products take the kernels for a few rows (few_rows_fit)
     MetalBuf *x, *ln, *qkv, *att, *act, *logits, *best, *lora_t;
     MetalBuf *a16, *inv_ln, *inv_br, *planes;                            // a product's operand, its factors (of ln | of att and act), its planes
     std::vector<MetalBuf *> kc, vc;                                      // per layer: [B][Hkv, max_seq, hd]
@@ -949,11 +951,33 @@ void batch_release(BatchRun *r)
     delete r;
 }
 
+// A state whose batches take the kernels of few_rows.h: F16 weights, widths that fill their loads.  GPU time per step of 8 sequences,
+// nine layers of the 4B shape: 662 us against 788 for the ring kernel's products with their planes summed, gated and split
+// between them, which Q8_0 tiles and other widths keep.  It holds for any batch: four layers and logits, 2 / 8 / 32 sequences, ms
+// per step 0.32 / 0.36 / 0.45 (before 0.36 / 0.38 / 0.51), of the Gemma3-1B shape 0.22 / 0.24 / 0.28 (0.27 / 0.28 / 0.36).
+bool few_rows_fit(const InferenceState *s)
+{
+    const int qd = s->Hq * s->hd;
+    if (s->D % 4 || s->D > 8192 || qd % 4 || s->IS % 32) return false;
+    auto aligned = [](const MetalBuf *g) { return !g || ((uintptr_t)dptr(g) & 15) == 0; };
+    if (!aligned(s->g_final) || (s->borrows_tiles && s->borrowed_lm.fmt)) return false;
+    for (int L = 0; L < s->NL; L++) {
+        const InferenceState::Layer &w = s->layers[L];
+        if (!aligned(w.g_in) || !aligned(w.g_post_attn) || !aligned(w.g_pre_ff) || !aligned(w.g_post_ff)) return false;
+        if (s->borrows_tiles) {
+            const BorrowedLayer &b = s->borrowed[L];
+            if (b.qkv.fmt || b.o.fmt || b.gu.fmt || b.down.fmt) return false;
+        }
+    }
+    return true;
+}
+
 // One step for B tokens at the same position: forward_token_batch, src/nn/fast_inference.c:808-893.  Every product
-// reads its weight once for all B vectors (matrix cores over the tiled image, the arithmetic of gemm_f32a_exact); what
+// reads its weight once for all B vectors (matrix cores over the tiled image, 22 bits of every activation); what
 // is per sequence -- adapter terms, per-head RMSNorm, RoPE, cache store, attention -- has the sequence as a grid
-// dimension, so a layer is the same 11 launches (12 with adapters) for any B.  A product's planes are summed by the kernel
-// that consumes them and the norm kernel writes the next product's operand itself, where a row is one workgroup's.
+// dimension, so a layer is the same 7 launches (one more with adapters) for any B, or 11 where few_rows_fit does not hold.  A
+// product's planes are summed by the kernel that consumes them and the norm kernel writes the next product's operand itself,
+// where a row is one workgroup's.
 void forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int pos)
 {
     if (s->stack) {
@@ -972,15 +996,17 @@ void forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
     float *inv_ln = dptr_as<float>(r.inv_ln), *inv_br = dptr_as<float>(r.inv_br), *P = dptr_as<float>(r.planes);
     // x += branch (the planes `br` of the product before, none at the start); ln = RMSNorm(x) as fp32 (only the adapters
     // read it) and as the operand of the next product
-    auto add_norm_b = [&](const SplitPlanes &br, MetalBuf *g_branch, MetalBuf *g) {
+    auto add_norm_b = [&](const auto &br, MetalBuf *g_branch, MetalBuf *g) {
         float *ln = (s->lora.empty() || s->borrows_tiles) ? nullptr : dptr_as<float>(r.ln);      // fp32 copy: only k_lora_down reads it
         const float *gb = g_branch ? dptr_as<float>(g_branch) : nullptr;
-        launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, B, D, s->eps);
+        if constexpr (std::is_same_v<std::decay_t<decltype(br)>, FewPlanes>) launch_few_norm(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, B, D, s->eps);
+        else launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, B, D, s->eps);
     };
     // planes of (the operand in a16) x w^T; `inv`: the factors that operand's rows were split with.  The weight: the
     // tiled image of the state's own row-major matrix (made on first use), or the training state's tiles
+    auto weight = [&](const WMat *w, const WeightOp *tiles, int rows, int cols) { return tiles ? *tiles : weight_f16(tiled_weight_of(w->mbuf, rows, cols)); };
     auto product = [&](const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv) {
-        const WeightOp op = tiles ? *tiles : weight_f16(tiled_weight_of(w->mbuf, rows, cols));
+        const WeightOp op = weight(w, tiles, rows, cols);
         const GemmPlan p = plan_gemm(2 * B, rows, cols, op.fmt ? op.nbq : 0, op.fmt);
         const size_t plane = (size_t)2 * B * rows;
         launch_gemm(a16, nullptr, op, P, rows, plane, 2 * B, rows, cols, p);
@@ -989,17 +1015,22 @@ void forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
     const bool bt = s->borrows_tiles;
     auto split = [&](MetalBuf *in, int K) { launch_rows_to_f16_split(dptr_as<float>(in), a16, inv_br, B, K); };
     SplitPlanes pending{};                                               // FFN branch of the layer before, added by the next norm kernel
+    FewPlanes pending_few{};
     MetalBuf *pending_g = nullptr;
     for (int L = 0; L < s->NL; L++) {
         const InferenceState::Layer &lw = s->layers[L];
         const BorrowedLayer *bl = bt ? &s->borrowed[L] : nullptr;
-        add_norm_b(pending, pending_g, lw.g_in);
+        if (r.few) add_norm_b(pending_few, pending_g, lw.g_in);
+        else add_norm_b(pending, pending_g, lw.g_in);
         // a training state's fused matrix continues with the rows of A_q and A_v (their fp16 images, as its own forward
         // reads them): the product then yields the adapters' down-projections as well, and no launch forms them
         const bool t_in_product = bt && !s->lora.empty();
         const int nq_rows = nqkv + (t_in_product ? 2 * s->R : 0);
-        const SplitPlanes qkv = product(&lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D, inv_ln);
-        launch_reduce_planes_split(qkv.P, qkv.S, qkv.plane, qkv.N, qkv.inv, dptr_as<float>(r.qkv), B, qkv.N);
+        if (r.few) launch_few_full(a16, inv_ln, weight(&lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D).w16, dptr_as<float>(r.qkv), nq_rows, B, nq_rows, D);
+        else {
+            const SplitPlanes qkv = product(&lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D, inv_ln);
+            launch_reduce_planes_split(qkv.P, qkv.S, qkv.plane, qkv.N, qkv.inv, dptr_as<float>(r.qkv), B, qkv.N);
+        }
         HeadPost a{};
         a.qkv = dptr_as<float>(r.qkv); a.qkv_step = (size_t)nq_rows;
         a.g_q = lw.g_q ? dptr_as<float>(lw.g_q) : nullptr; a.g_k = lw.g_k ? dptr_as<float>(lw.g_k) : nullptr;
@@ -1017,18 +1048,32 @@ void forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
             a.Bq = dptr_as<float>(lr.Bq); a.Bv = dptr_as<float>(lr.Bv); a.R = s->R; a.sc = s->scaling;
         }
         attention_decode_fused(a, r.kc[L], r.vc[L], dptr_as<float>(r.att), hd, s->max_seq, B);
-        split(r.att, qd);
-        const SplitPlanes o = product(lw.o, bt ? &bl->o : nullptr, D, qd, inv_br);
-        add_norm_b(o, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn);
-        const SplitPlanes gu = product(&lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln);
-        hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, B), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), B, IS, gemma ? 1 : 0);
-        split(r.act, IS);
-        pending = product(lw.down, bt ? &bl->down : nullptr, D, IS, inv_br);
+        MetalBuf *g_post = gemma ? lw.g_post_attn : nullptr, *g_ff = gemma ? lw.g_pre_ff : lw.g_post_attn;
+        if (r.few) {
+            add_norm_b(launch_few_split(dptr_as<float>(r.att), weight(lw.o, bt ? &bl->o : nullptr, D, qd).w16, P, B, D, qd), g_post, g_ff);
+            launch_few_glu(a16, inv_ln, weight(&lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D).w16, dptr_as<float>(r.act), B, IS, D, gemma ? 1 : 0);
+            pending_few = launch_few_split(dptr_as<float>(r.act), weight(lw.down, bt ? &bl->down : nullptr, D, IS).w16, P, B, D, IS);
+        }
+        else {
+            split(r.att, qd);
+            const SplitPlanes o = product(lw.o, bt ? &bl->o : nullptr, D, qd, inv_br);
+            add_norm_b(o, g_post, g_ff);
+            const SplitPlanes gu = product(&lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln);
+            hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, B), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), B, IS, gemma ? 1 : 0);
+            split(r.act, IS);
+            pending = product(lw.down, bt ? &bl->down : nullptr, D, IS, inv_br);
+        }
         pending_g = gemma ? lw.g_post_ff : nullptr;
     }
-    add_norm_b(pending, pending_g, s->g_final);
-    const SplitPlanes lg = product(s->lm_head, bt ? &s->borrowed_lm : nullptr, s->V, D, inv_ln);
-    launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, dptr_as<float>(r.logits), B, lg.N);
+    if (r.few) {
+        add_norm_b(pending_few, pending_g, s->g_final);
+        launch_few_full(a16, inv_ln, weight(s->lm_head, bt ? &s->borrowed_lm : nullptr, s->V, D).w16, dptr_as<float>(r.logits), s->V, B, s->V, D);
+    }
+    else {
+        add_norm_b(pending, pending_g, s->g_final);
+        const SplitPlanes lg = product(s->lm_head, bt ? &s->borrowed_lm : nullptr, s->V, D, inv_ln);
+        launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, dptr_as<float>(r.logits), B, lg.N);
+    }
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1084,6 +1129,8 @@ BatchRun &batch_acquire(InferenceState *s, BatchRun *&slot, int B)
                 set_gemm_ring_wide(wide_was);
             }
     }
+    r.few = few_rows_fit(s);
+    if (r.few) plane_floats = std::max(plane_floats, (size_t)std::max(few_planes(D, qd), few_planes(D, IS)) * B * D);
     r.a16 = metal_buf_create(a16_elems * sizeof(half_t)); r.planes = fbuf(plane_floats);
     r.inv_ln = fbuf((size_t)2 * B); r.inv_br = fbuf((size_t)2 * B);
     r.best = metal_buf_create(((size_t)B + (size_t)B * 2 * AM_WGS) * sizeof(int));

@@ -167,6 +167,32 @@ def test_batch_steps_with_a_token_of_their_own_per_sequence(with_lora):
             check(inf)
 
 
+# widths that fill no K tile (160, 96), one K tile per wave and some beyond (D 4416: 69 tiles over eight and four waves; two columns
+# groups of the norm kernel), K chunks of one, two and four tiles per wave (IS 96, 9728, and 2 560 rows of 4 096), a vocabulary that
+# fills no block of 32 rows, an FFN whose gate blocks would be split (80: the products' planes as before)
+@pytest.mark.parametrize("kw,batches", [(dict(D=160, Hq=3, Hkv=1, hd=32, IS=96, V=260), (1, 2, 15, 16, 17, 32)),
+                                        (dict(D=160, Hq=3, Hkv=1, hd=32, IS=80, V=260), (3, 20)),
+                                        (dict(D=4416, Hq=2, Hkv=1, hd=64, IS=160, V=516), (5, 18)),
+                                        (dict(D=2560, Hq=32, Hkv=8, hd=128, IS=9728, V=512), (8, 31))],
+                         ids=["ragged", "ffn_80", "wide", "c3_widths"])
+@pytest.mark.parametrize("model_type", [0, 1], ids=["qwen3", "gemma3"])
+def test_batch_steps_over_shapes_that_fill_no_tile(kw, batches, model_type):
+    """Every sequence's logits against the single-sequence path, which sums whole fp32 rows: 22 bits of every activation
+    are left in a batch's products (2^-22 = 2.4e-7 each, a few hundred of them in a row of products and norms)."""
+    say("batch steps", kw, model_type)
+    c = C1.with_(name="few", model_type=model_type, NL=2, seq=8, tied=True, **kw)
+    model = make_model(c, seed=41, gamma_jitter=0.1)
+    n = 3
+    with InferenceState(c, model, max_seq=8, use_fp16=True) as inf:
+        for B in batches:
+            seqs = np.random.default_rng(B).integers(1, c.V, (B, n))
+            got = np.stack([inf.step_batch(seqs[:, i], i) for i in range(n)], axis=1)
+            for b in sorted({0, 1 % B, B // 2, B - 1}):
+                inf.reset()
+                single = np.stack([inf.forward_token(int(t)) for t in seqs[b]])
+                assert maxrel(got[b], single) < 1e-4, (B, b, maxrel(got[b], single))
+
+
 # Qwen3-4B's widths (hidden 2560, 32 / 8 heads of 128, FFN 9728): the instantiations that `bench.py --decode` launches --
 # two weight rows per wave with the SiLU gate and the norm inside the launch at 19456 x 2560, the norm-fused Q|K|V
 # product at 6144 x 2560, the attention kernel with four-key steps, the fused per-head prologue and the O weights asked
