@@ -392,6 +392,164 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
     }
 }
 
+// The same products over a normed vector of up to 512 S columns, without LDS and without barriers: the eight columns per step that a
+// lane multiplies are all it needs of the vector, so every wave forms the norm for itself -- its loads ahead of the first weights,
+// sums through DPP -- and keeps v g in registers for the `reps` units it takes one after the other, a unit's weights requested
+// before those of the unit before are used.  A unit is two rows, or with act 1 (SiLU) and 2 (GELU) a row of the gate and one of
+// the up matrix; act 3: GELU of every sum.  NORM as above.
+// Bound by the launch, the trip for the vector and the weights' stream.  With the vector in LDS behind two block reductions (k_matvec):
+// 6912 Q8_0 pairs of 1152 with both norms 11.5 us, 8.8 so; 9728 F16 pairs of 2560 20.4 -> 18.1 (5.5 TB/s), 6144 rows 8.9 -> 7.9; 8192 rows of
+// 2048 with both norms 12.3 -> 10.3; 16 384 rows of 1024 with a layer norm 14.3 -> 12.3.  Four rows in a unit are no faster (registers).
+template <int FMT, int NORM, int S>
+__global__ __launch_bounds__(TB, 2) void k_matvec_normed(const void *__restrict__ Wp, const half_t *__restrict__ scales, float *__restrict__ y, int rows, int cols,
+                                                         int act, int reps, NormIn nin)
+{
+    struct Stage {
+        half8  w16[FMT == 0 ? 2 : 1][S];
+        uint2v w8[FMT == 1 ? 2 : 1][S];
+        half_t d[FMT == 1 ? 2 : 1][S];
+    };
+    const int lane = threadIdx.x & 63, wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const bool pair = act == 1 || act == 2;
+    const int units = pair ? rows : (rows + 1) >> 1, last = min(wid * reps + reps, units) - 1;
+    int unit = wid * reps;
+    if (unit > last) return;
+    uint32_t at[S];                                        // (clamped: loads stay unconditional)
+#pragma unroll
+    for (int s = 0; s < S; s++) at[s] = min(lane * 8 + 512 * s, cols - 8);
+    float4v v[S][2], g[S][2], b[S][2], gb[S][2];
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            v[s][h] = *reinterpret_cast<const float4v *>(nin.xr + at[s] + 4 * h);
+            if (NORM != 2 && nin.br) {
+                b[s][h] = *reinterpret_cast<const float4v *>(nin.br + at[s] + 4 * h);
+                if (NORM == 3) gb[s][h] = *reinterpret_cast<const float4v *>(nin.g_br + at[s] + 4 * h);
+                if (NORM == 3 && nin.b_br) b[s][h] += *reinterpret_cast<const float4v *>(nin.b_br + at[s] + 4 * h);
+            }
+            g[s][h] = *reinterpret_cast<const float4v *>(nin.g + at[s] + 4 * h);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    auto load = [&](Stage &w, int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const size_t row = pair ? (size_t)u + (r ? rows : 0) : min(2 * u + r, rows - 1);
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                if (FMT == 0) w.w16[r][s] = __builtin_nontemporal_load(reinterpret_cast<const half8 *>((const half_t *)Wp + row * cols + at[s]));
+                else {
+                    w.w8[r][s] = __builtin_nontemporal_load(reinterpret_cast<const uint2v *>((const int8_t *)Wp + row * cols + at[s]));
+                    w.d[r][s] = (scales + row * (cols >> 5))[at[s] >> 5];
+                }
+            }
+        }
+    };
+    Stage A, B;
+    load(A, unit);
+    __builtin_amdgcn_sched_barrier(0);
+    // the norm; a column past the last (a lane that repeats another's) or past dim counts for nothing
+    auto live = [&](int s, int e) __attribute__((always_inline)) { return lane * 8 + 512 * s < cols && (NORM == 1 || (int)at[s] + e < nin.dim); };
+    float norm_inv;
+    if (NORM == 2) {
+        float sum = 0.f, ss = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) sum += live(s, e) ? v[s][e >> 2][e & 3] : 0.f;
+        const float mean = wave_sum(sum) / (float)nin.dim;
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float x = live(s, e) ? v[s][e >> 2][e & 3] - mean : 0.f;
+                v[s][e >> 2][e & 3] = x;
+                ss = fmaf(x, x, ss);
+            }
+        norm_inv = 1.f / sqrtf(wave_sum(ss) / (float)nin.dim + nin.eps);
+    } else {
+        if (nin.br) {
+            if (NORM == 3) {
+                float ss = 0.f;
+#pragma unroll
+                for (int s = 0; s < S; s++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const float x = live(s, e) ? b[s][e >> 2][e & 3] : 0.f;
+                        b[s][e >> 2][e & 3] = x;
+                        ss = fmaf(x, x, ss);
+                    }
+                const float post = 1.f / sqrtf(wave_sum(ss) / (float)nin.dim + nin.eps);
+#pragma unroll
+                for (int s = 0; s < S; s++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[s][e >> 2][e & 3] = fmaf(b[s][e >> 2][e & 3] * post, gb[s][e >> 2][e & 3], v[s][e >> 2][e & 3]);
+            } else
+#pragma unroll
+                for (int s = 0; s < S; s++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) v[s][h] += b[s][h];
+            if (wid == 0 && nin.x_out)
+#pragma unroll
+                for (int s = 0; s < S; s++)
+                    if (lane * 8 + 512 * s < cols)
+#pragma unroll
+                        for (int h = 0; h < 2; h++) *reinterpret_cast<float4v *>(nin.x_out + at[s] + 4 * h) = v[s][h];
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float x = lane * 8 + 512 * s < cols ? v[s][e >> 2][e & 3] : 0.f;
+                v[s][e >> 2][e & 3] = x;
+                ss = fmaf(x, x, ss);
+            }
+        ss = wave_sum(ss);
+        norm_inv = NORM == 1 ? rsqrtf(ss / (float)cols + nin.eps) : 1.f / sqrtf(ss / (float)nin.dim + nin.eps);
+    }
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) v[s][h] *= g[s][h];
+    auto use = [&](const Stage &w, int u) __attribute__((always_inline)) {
+        float acc[2];
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            acc[r] = 0.f;
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                if (FMT == 0) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) acc[r] = fmaf((float)w.w16[r][s][e], v[s][e >> 2][e & 3], acc[r]);
+                } else {
+                    float p = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) p = fmaf((float)(int8_t)(w.w8[r][s][e >> 2] >> (8 * (e & 3))), v[s][e >> 2][e & 3], p);
+                    acc[r] = fmaf((float)w.d[r][s], p, acc[r]);
+                }
+            }
+        }
+        const float s0 = wave_sum(acc[0]) * norm_inv, s1 = wave_sum(acc[1]) * norm_inv;
+        auto gelu = [](float x) { return 0.5f * x * (1.0f + tanhf(gelu_inner(x))); };
+        if (lane) return;
+        if (pair) y[u] = (act == 1 ? s0 / (1.0f + expf(-s0)) : gelu(s0)) * s1;
+        else {
+            y[2 * u] = act == 3 ? gelu(s0) : s0;
+            if (2 * u + 1 < rows) y[2 * u + 1] = act == 3 ? gelu(s1) : s1;
+        }
+    };
+    for (;;) {
+        if (unit == last) { use(A, unit); break; }
+        load(B, unit + 1);
+        use(A, unit);
+        if (++unit == last) { use(B, unit); break; }
+        load(A, unit + 1);
+        use(B, unit);
+        unit++;
+    }
+}
+
 // Few long rows: the four waves of a workgroup share one, each with every fourth 512-column step, U of them requested at once, so a
 // row is one or two trips to memory instead of one per 2048 columns.  (Steps behind the row ask for its last eight columns again.)
 // With a wave per row such a matrix has some five waves on a CU and a chain of several trips in each.  Cold weights: 1152 x 6912 Q8_0
@@ -503,6 +661,25 @@ void launch_matvec_glu(const void *W, const half_t *scales, const float *x, floa
 #undef GLU_LAUNCH
 }
 
+// k_matvec_normed takes vectors of up to 2560 columns (the vector and two stages of weights in registers; k_matvec those beyond).  Every
+// wave is resident: two workgroups per CU, or one where a unit's two rows have more than 1536 columns -- fewer waves then keep
+// memory busy, and 256 workgroups fill the CUs evenly (one / two per CU: 6144 x 2560 F16 7.9 / 9.0 us, Q8_0 6.2 / 7.8, 9728 pairs F16 18.1 / 18.5;
+// 6912 pairs of 1152 F16 10.0 / 9.6, Q8_0 9.3 / 8.8).
+constexpr int NORMED_COLS = 2560;
+template <int FMT, int NORM>
+void launch_matvec_normed(const void *W, const half_t *scales, const NormIn &nin, float *y, int rows, int cols, int act, hipEvent_t ev_a, hipEvent_t ev_b)
+{
+    const int units = act == 1 || act == 2 ? rows : (rows + 1) / 2, waves = cols > 1536 ? 1024 : 2048, reps = (units + waves - 1) / waves;
+    const dim3 grid((units + 4 * reps - 1) / (4 * reps));
+#define NORMED_LAUNCH(S_) do { \
+    if (ev_a) hipExtLaunchKernelGGL((k_matvec_normed<FMT, NORM, S_>), grid, dim3(TB), 0, stream(), ev_a, ev_b, 0, W, scales, y, rows, cols, act, reps, nin); \
+    else hipLaunchKernelGGL((k_matvec_normed<FMT, NORM, S_>), grid, dim3(TB), 0, stream(), W, scales, y, rows, cols, act, reps, nin); \
+    HIP_CHECK(hipGetLastError()); } while (0)
+    if (cols <= 512) NORMED_LAUNCH(1); else if (cols <= 1024) NORMED_LAUNCH(2); else if (cols <= 1536) NORMED_LAUNCH(3);
+    else if (cols <= 2048) NORMED_LAUNCH(4); else NORMED_LAUNCH(5);
+#undef NORMED_LAUNCH
+}
+
 // Either product over RMSNorm(xr + br; g), formed by the kernel itself (NORM): glu 0 plain rows, 1 SiLU, 2 GELU pairs.
 template <int FMT>
 void launch_matvec_norm(const void *W, const half_t *scales, const NormIn &nin, float *y, int rows, int cols, int glu)
@@ -510,6 +687,7 @@ void launch_matvec_norm(const void *W, const half_t *scales, const NormIn &nin, 
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     const double mats = glu ? 2.0 : 1.0;
     const bool prof = gemm_prof_begin(mats * rows * cols * (FMT == 0 ? 2.0 : 34.0 / 32.0), 2.0 * mats * rows * cols, &ev_a, &ev_b);
+    if (cols <= NORMED_COLS) { launch_matvec_normed<FMT, 1>(W, scales, nin, y, rows, cols, glu, ev_a, ev_b); return; }
     const size_t lds = (size_t)cols * 4;
 #define NORM_LAUNCH(G_, RPW_, REPS_) do { \
     const dim3 grid((rows + RPW_ * REPS_ - 1) / (RPW_ * REPS_)); \
@@ -1318,8 +1496,9 @@ void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, floa
     const NormIn nin{x, nullptr, g, nullptr, eps, dim};
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     const bool prof = gemm_prof_begin(2.0 * rows * cols, 2.0 * rows * cols, &ev_a, &ev_b);
-    const size_t lds = (size_t)cols * 4;
     const half_t *scales = nullptr;
+    if (cols <= NORMED_COLS) { launch_matvec_normed<0, 2>(dptr(W), scales, nin, y, rows, cols, 0, ev_a, ev_b); return; }
+    const size_t lds = (size_t)cols * 4;
 #define LN_LAUNCH(REPS_) do { \
     const dim3 grid((rows + 8 * REPS_ - 1) / (8 * REPS_)); \
     if (prof) hipExtLaunchKernelGGL((k_matvec<0, 2, 2, 1, 0, 2, REPS_>), grid, dim3(TB), lds, stream(), ev_a, ev_b, 0, dptr(W), scales, nullptr, y, rows, cols, nin); \
@@ -1345,16 +1524,17 @@ void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int
     } else REQUIRE_BYTES(W, (size_t)wrows * cols * 2, "matvec_norms_around");
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     const bool prof = gemm_prof_begin((q8 ? 34.0 / 32.0 : 2.0) * wrows * cols, 2.0 * wrows * cols, &ev_a, &ev_b);
+    if (cols <= NORMED_COLS) {
+        if (q8) launch_matvec_normed<1, 3>(w, scales, nin, y, rows, cols, act, ev_a, ev_b);
+        else launch_matvec_normed<0, 3>(w, scales, nin, y, rows, cols, act, ev_a, ev_b);
+        return;
+    }
     const size_t lds = (size_t)cols * 4;
-    // columns of up to three steps of 512: a wave asks for whole rows at once (1152 columns, gated Q8_0 pairs: 14.3 us with two
-    // steps, the second stage of which is all but empty, 13.7 with three)
-#define AROUND_LAUNCH_U(FMT_, U_, GLU_, RPW_, REPS_, ACT_) do { \
-    const dim3 grid((rows + RPW_ * REPS_ - 1) / (RPW_ * REPS_)); \
-    if (prof) hipExtLaunchKernelGGL((k_matvec<FMT_, 2, U_, 1, GLU_, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), ev_a, ev_b, 0, w, scales, nullptr, y, rows, cols, nin); \
-    else hipLaunchKernelGGL((k_matvec<FMT_, 2, U_, 1, GLU_, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), w, scales, nullptr, y, rows, cols, nin); \
-    HIP_CHECK(hipGetLastError()); } while (0)
 #define AROUND_LAUNCH(FMT_, GLU_, RPW_, REPS_, ACT_) do { \
-    if (cols > 1024 && cols <= 1536) AROUND_LAUNCH_U(FMT_, 3, GLU_, RPW_, REPS_, ACT_); else AROUND_LAUNCH_U(FMT_, 2, GLU_, RPW_, REPS_, ACT_); } while (0)
+    const dim3 grid((rows + RPW_ * REPS_ - 1) / (RPW_ * REPS_)); \
+    if (prof) hipExtLaunchKernelGGL((k_matvec<FMT_, 2, 2, 1, GLU_, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), ev_a, ev_b, 0, w, scales, nullptr, y, rows, cols, nin); \
+    else hipLaunchKernelGGL((k_matvec<FMT_, 2, 2, 1, GLU_, 3, REPS_, ACT_>), grid, dim3(TB), lds, stream(), w, scales, nullptr, y, rows, cols, nin); \
+    HIP_CHECK(hipGetLastError()); } while (0)
     if (act == 3) { if (rows >= 16384) AROUND_LAUNCH(0, 0, 8, 4, 1); else AROUND_LAUNCH(0, 0, 8, 1, 1); }
     else if (act == 0) {
         if (q8) AROUND_LAUNCH(1, 0, 8, 1, 0);
@@ -1363,7 +1543,6 @@ void matvec_norms_around(MetalBuf *W, const NormIn &nin, float *y, int rows, int
     }
     else if (q8) { if (act == 1) AROUND_LAUNCH(1, 1, 4, 2, 0); else AROUND_LAUNCH(1, 2, 4, 2, 0); }
     else { if (act == 1) AROUND_LAUNCH(0, 1, 4, 2, 0); else AROUND_LAUNCH(0, 2, 4, 2, 0); }
-#undef AROUND_LAUNCH_U
 #undef AROUND_LAUNCH
 }
 
