@@ -161,12 +161,18 @@ __global__ __launch_bounds__(256) void k_transpose_scaled_jobs(TransposeJobs js,
 // eight XCDs in turn; an XCD takes a contiguous share of the list of (matrix, row pair, column group) items, so the
 // workgroups that read the same two row blocks of Y^T run on one XCD, one after the other, and fetch them into one L2
 // instead of one each.
-struct WgradJob { const half8 *XT; const float *x_inv; const half8 *YT; const float *y_inv; half_t *target; int M_out, N_in; };
+struct WgradJob { const half8 *XT; const float *x_inv; const half8 *YT; const float *y_inv; half_t *target, *WT; int M_out, N_in; };
 struct WgradJobs { WgradJob j[4]; int first[5]; int n; };
 
-template <int SGD>
+// MODE 0: target = the accumulator G, + dW.  1: target = W, - lr dW (sft_backward_sgd).  2: what mode 0 on a cleared accumulator and
+// k_apply_retile behind it leave, bit for bit -- W = half(W - lr half(dW)) and its transposed image WT -- without G: 6 instead of
+// 14 bytes of traffic per weight, and the 64 x 64 block that WT takes is the wave's own, turned through LDS.
+// Gemma3-1B, 640 tokens: head (302 M weights) 769 + 513 us in two launches, 897 so; a layer's four matrices 71 + 28, 80.
+template <int MODE>
 __global__ __launch_bounds__(256) void k_wgrad(WgradJobs js, int Kt, float lr)
 {
+    constexpr int LDT = 72;                               // halves per row of the turned block: 16-byte reads, rows four banks apart
+    __shared__ half_t turned[MODE == 2 ? 4 * 64 * LDT : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l31 = lane & 31, h = lane >> 5;
     const int total = js.first[js.n], per_xcd = (total + 7) >> 3;
     int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -225,6 +231,9 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradJobs js, int Kt, float lr)
                         acc[mt][nh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[nh][j], y[mt][j], acc[mt][nh], 0, 0, 0);
         }
     };
+    auto update = [&](half_t old, float a) __attribute__((always_inline)) {             // contraction is off in this file
+        return MODE == 0 ? f2h(h2f(old) + a) : MODE == 1 ? f2h(h2f(old) - lr * a) : f2h(h2f(old) - lr * h2f(f2h(0.f + a)));
+    };
     if (active && (mb0 + 2) * 32 <= M_out && nk * 64 + 64 <= N_in) {
         // Block inside the matrix: everything the read-modify-write needs is requested at once, before the contraction
         // (whose loads it then travels with), then computed, then stored.  With the bounds tests of the general path
@@ -259,12 +268,33 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradJobs js, int Kt, float lr)
                     const float xs[4] = {xi[nh][j4].x, xi[nh][j4].y, xi[nh][j4].z, xi[nh][j4].w};
                     half4 o = g[mt][nh][j4];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float a = acc[mt][nh][4 * j4 + i] * sy[mt] * xs[i];
-                        o[i] = SGD ? f2h(h2f(o[i]) - lr * a) : f2h(h2f(o[i]) + a);
-                    }
+                    for (int i = 0; i < 4; i++) o[i] = update(o[i], acc[mt][nh][4 * j4 + i] * sy[mt] * xs[i]);
                     __builtin_nontemporal_store(o, gp[mt][nh][j4]);
+                    if (MODE == 2) {
+                        // rows m and m + 1 (neighbouring lanes) of two columns each: the even lane takes columns 0 and 1, the odd one 2 and 3
+                        typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+                        const u2 mine = __builtin_bit_cast(u2, o);
+                        const uint32_t keep = l31 & 1 ? mine[1] : mine[0], give = l31 & 1 ? mine[0] : mine[1];
+                        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xF, 0xF, false);   // quad_perm [1, 0, 3, 2]
+                        const uint32_t lo = l31 & 1 ? got : keep, hi = l31 & 1 ? keep : got;                               // row m's pair, row m + 1's
+                        const int n = nh * 32 + 8 * j4 + 4 * h + 2 * (l31 & 1), m = mt * 32 + (l31 & ~1);
+                        uint32_t *to = reinterpret_cast<uint32_t *>(turned + (wave * 64 + n) * LDT + m);
+                        to[0] = (lo & 0xFFFFu) | hi << 16;
+                        to[LDT / 2] = lo >> 16 | (hi & 0xFFFF0000u);
+                    }
                 }
+        if (MODE == 2) {                                  // (a wave's own block: no barrier)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            half8 *to = reinterpret_cast<half8 *>(js.j[k].WT);
+            const int KbT = tiled_kb(M_out);
+#pragma unroll
+            for (int th = 0; th < 2; th++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    __builtin_nontemporal_store(*reinterpret_cast<const half8 *>(turned + (wave * 64 + th * 32 + l31) * LDT + 32 * h + 8 * j),
+                                                &to[(((size_t)nk * 2 + th) * KbT + (mb0 >> 1)) * 256 + j * 64 + lane]);
+        }
         return;
     }
     contract_tokens();
@@ -285,8 +315,8 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradJobs js, int Kt, float lr)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     if (n0 + i >= N_in) continue;
-                    const float a = acc[mt][nh][4 * j4 + i] * sy * x_inv[n0 + i];
-                    g[i] = SGD ? f2h(h2f(g[i]) - lr * a) : f2h(h2f(g[i]) + a);        // contraction is off in this file
+                    g[i] = update(g[i], acc[mt][nh][4 * j4 + i] * sy * x_inv[n0 + i]);
+                    if (MODE == 2) js.j[k].WT[tiled_index(n0 + i, m, tiled_kb(M_out))] = g[i];
                 }
                 *reinterpret_cast<half4 *>(target + addr) = g;
             }
@@ -414,7 +444,7 @@ void launch_transpose_scaled_jobs(const TransposeOperand *ops, int n, int T)
     LAUNCH_TIMED(0.0, 0.0, k_transpose_scaled_jobs, dim3(total), dim3(256), 0, js, T);
 }
 
-void launch_wgrads(const WgradOperands *w, int n, int T, int sgd, float lr)
+void launch_wgrads(const WgradOperands *w, int n, int T, int mode, float lr)
 {
     if (n <= 0 || n > 4 || T <= 0) { fprintf(stderr, "[fast_hip] wgrads: %d matrices\n", n); abort(); }
     WgradJobs js{};
@@ -423,7 +453,7 @@ void launch_wgrads(const WgradOperands *w, int n, int T, int sgd, float lr)
     for (int i = 0; i < n; i++) {
         if (w[i].M_out <= 0 || w[i].N_in <= 0) { fprintf(stderr, "[fast_hip] wgrads: empty matrix\n"); abort(); }
         js.j[i] = WgradJob{reinterpret_cast<const half8 *>(w[i].XT), w[i].x_inv, reinterpret_cast<const half8 *>(w[i].YT), w[i].y_inv,
-                           w[i].target_tiled, w[i].M_out, w[i].N_in};
+                           w[i].target_tiled, w[i].transposed, w[i].M_out, w[i].N_in};
         js.first[i] = total;
         total += ((tiled_kb(w[i].N_in) + 3) / 4) * ((tiled_rb(w[i].M_out) + 1) / 2);
     }
@@ -431,17 +461,18 @@ void launch_wgrads(const WgradOperands *w, int n, int T, int sgd, float lr)
     const dim3 grid((total + 7) / 8 * 8);                 // whole rounds of the eight XCDs; k_wgrad maps ids to tiles
     double weights = 0.0;
     for (int i = 0; i < n; i++) weights += (double)w[i].M_out * w[i].N_in;
-    // the F16 target is read and written once: 4 bytes per weight
-    if (sgd) LAUNCH_TIMED(4.0 * weights, 2.0 * T * weights, k_wgrad<1>, grid, dim3(256), 0, js, tiled_kb(T), lr);
-    else     LAUNCH_TIMED(4.0 * weights, 2.0 * T * weights, k_wgrad<0>, grid, dim3(256), 0, js, tiled_kb(T), lr);
+    // the F16 target is read and written once: 4 bytes per weight, and with its transposed image 6
+    if (mode == 2) LAUNCH_TIMED(6.0 * weights, 2.0 * T * weights, k_wgrad<2>, grid, dim3(256), 0, js, tiled_kb(T), lr);
+    else if (mode == 1) LAUNCH_TIMED(4.0 * weights, 2.0 * T * weights, k_wgrad<1>, grid, dim3(256), 0, js, tiled_kb(T), lr);
+    else LAUNCH_TIMED(4.0 * weights, 2.0 * T * weights, k_wgrad<0>, grid, dim3(256), 0, js, tiled_kb(T), lr);
 }
 
 void launch_wgrad(const half_t *XT, const float *x_inv, const half_t *YT, const float *y_inv, half_t *target_tiled,
-                  int M_out, int N_in, int T, int sgd, float lr)
+                  int M_out, int N_in, int T, int mode, float lr, half_t *transposed)
 {
     if (M_out <= 0 || N_in <= 0 || T <= 0) return;
-    const WgradOperands w{XT, x_inv, YT, y_inv, target_tiled, M_out, N_in};
-    launch_wgrads(&w, 1, T, sgd, lr);
+    const WgradOperands w{XT, x_inv, YT, y_inv, target_tiled, M_out, N_in, transposed};
+    launch_wgrads(&w, 1, T, mode, lr);
 }
 
 void launch_apply_retile(half_t *W_tiled, half_t *G_tiled, half_t *WT_tiled, int M_out, int N_in, float lr,

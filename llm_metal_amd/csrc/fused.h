@@ -265,12 +265,13 @@ void launch_transpose_scaled_pair(const half_t *in0, const float *in0_inv, int F
 struct TransposeOperand { const half_t *in; const float *in_inv; int F; half_t *out; float *out_inv; };
 void launch_transpose_scaled_jobs(const TransposeOperand *ops, int n, int T);
 // target (tiled [M_out, N_in] F16) <- half(target + alpha * Y^T X), XT/YT = transposed operands over T tokens;
-// sgd: alpha = -lr (f16_sgd_fused), else alpha = 1 (f16_grad_accum)
+// mode 0: alpha = 1 (f16_grad_accum); 1: alpha = -lr (f16_sgd_fused); 2: f16_grad_accum into a cleared accumulator and f16_sgd_apply in
+// one, target = W and `transposed` (tiled [N_in, M_out]) its transposed image
 void launch_wgrad(const half_t *XT, const float *x_inv, const half_t *YT, const float *y_inv, half_t *target_tiled,
-                  int M_out, int N_in, int T, int sgd, float lr);
+                  int M_out, int N_in, int T, int mode, float lr, half_t *transposed = nullptr);
 // the same for up to four matrices in one launch
-struct WgradOperands { const half_t *XT; const float *x_inv; const half_t *YT; const float *y_inv; half_t *target_tiled; int M_out, N_in; };
-void launch_wgrads(const WgradOperands *w, int n, int T, int sgd, float lr);
+struct WgradOperands { const half_t *XT; const float *x_inv; const half_t *YT; const float *y_inv; half_t *target_tiled; int M_out, N_in; half_t *transposed; };
+void launch_wgrads(const WgradOperands *w, int n, int T, int mode, float lr);
 // G != null: W = half(W - lr G), G = 0 (f16_sgd_apply); always: WT (tiled [N_in, M_out]) <- W^T.  `matrices` of the same
 // shape in one launch, `stride` halves apart in W and G and `strideT` in WT (the layers of an arena).
 void launch_apply_retile(half_t *W_tiled, half_t *G_tiled, half_t *WT_tiled, int M_out, int N_in, float lr,

@@ -93,6 +93,7 @@ struct SFTState {
     // backward has run, and all eight operands of its weight gradients are transposed in one launch
     MetalBuf *dy16[4], *dy_inv[4], *lyT[4], *lyT_inv[4], *lxT[4], *lxT_inv[4];
     MetalBuf *gqkv, *go, *ggu, *gd, *glm;   // F16 gradient accumulators, tiled like the weights (sft_alloc_grad_accum)
+    bool accum_clear;                    // nothing has been added to them since they were zeroed
     MetalBuf *grpo_old_lp, *grpo_advs, *grpo_new_lp;   // host-visible [BN] inputs/outputs of the policy gradient
     float *grpo_old_lp_cpu, *grpo_advs_cpu, *grpo_new_lp_cpu;
     MetalBuf *lora_acc;                  // LoRA gradients summed over the completions of a GRPO group
@@ -112,7 +113,8 @@ struct SFTState {
     WMat lm_head_out;
 };
 
-enum { BWD_LORA = 0, BWD_ACCUM = 1, BWD_SGD = 2 };
+// BWD_APPLY: BWD_ACCUM on cleared accumulators with sft_apply_grad_sgd behind it, without the accumulators; same results
+enum { BWD_LORA = 0, BWD_ACCUM = 1, BWD_SGD = 2, BWD_APPLY = 3 };
 
 namespace {
 
@@ -487,7 +489,7 @@ void forward_impl(SFTState *s, bool gather, bool zero_rows = false)
 }
 
 // dW = dY^T X for one (fused) matrix [M_out, N_in] at element offsets w_off / wt_off of its arenas:
-// added into the accumulator (BWD_ACCUM) or applied at once to both weight images (BWD_SGD).
+// added into the accumulator (BWD_ACCUM) or applied at once to both weight images (BWD_SGD, BWD_APPLY).
 void weight_grad(SFTState *s, int mode, float lr, const half_t *dY16, const float *dy_inv, int M_out,
                  const half_t *X16, const float *x_inv, int N_in,
                  MetalBuf *W, MetalBuf *WT, MetalBuf *G, size_t w_off, size_t wt_off)
@@ -498,6 +500,9 @@ void weight_grad(SFTState *s, int mode, float lr, const half_t *dY16, const floa
     if (mode == BWD_ACCUM) {
         launch_wgrad(at<half_t>(s->xT), at<float>(s->xT_inv), at<half_t>(s->yT), at<float>(s->yT_inv),
                      at<half_t>(G, w_off), M_out, N_in, s->BN, 0, 0.f);
+    } else if (mode == BWD_APPLY) {
+        launch_wgrad(at<half_t>(s->xT), at<float>(s->xT_inv), at<half_t>(s->yT), at<float>(s->yT_inv),
+                     at<half_t>(W, w_off), M_out, N_in, s->BN, 2, lr, at<half_t>(WT, wt_off));
     } else {
         launch_wgrad(at<half_t>(s->xT), at<float>(s->xT_inv), at<half_t>(s->yT), at<float>(s->yT_inv),
                      at<half_t>(W, w_off), M_out, N_in, s->BN, 1, lr);
@@ -506,7 +511,7 @@ void weight_grad(SFTState *s, int mode, float lr, const half_t *dY16, const floa
 }
 
 // Backward from the fp16 loss gradient in dl16 / dl_inv.  mode: BWD_LORA (adapter gradients),
-// BWD_ACCUM / BWD_SGD (full-parameter: sft_backward_accum / sft_backward_sgd, src/nn/fast_sft.c:984-986).
+// BWD_ACCUM / BWD_SGD (full-parameter: sft_backward_accum / sft_backward_sgd, src/nn/fast_sft.c:984-986), BWD_APPLY.
 void backward_impl(SFTState *s, int mode = BWD_LORA, float lr = 0.f)
 {
     const int BN = s->BN, D = s->D, IS = s->IS, qd = s->qd, kd = s->kd, R = s->R, NL = s->NL;
@@ -519,7 +524,8 @@ void backward_impl(SFTState *s, int mode = BWD_LORA, float lr = 0.f)
     // so that all four weight gradients can be formed after the layer's last row kernel: one launch transposes their
     // eight operands instead of four launches of two (the weights do not change before the apply, so the order of the
     // reference's f16_grad_accum calls, src/nn/fast_sft.c:804-946, does not matter).  Otherwise one buffer serves all.
-    const bool defer = mode == BWD_ACCUM && s->dy16[0];
+    const bool defer = (mode == BWD_ACCUM || mode == BWD_APPLY) && s->dy16[0];
+    if (mode == BWD_ACCUM) s->accum_clear = false;
     half_t *d16[4];
     float *dinv[4];
     for (int i = 0; i < 4; i++) { d16[i] = defer ? at<half_t>(s->dy16[i]) : a16; dinv[i] = defer ? at<float>(s->dy_inv[i]) : ainv; }
@@ -613,27 +619,6 @@ void backward_impl(SFTState *s, int mode = BWD_LORA, float lr = 0.f)
         const bool input_grad = mode != BWD_LORA || L > 0;
         if (mode == BWD_LORA && input_grad) qb.pf = prefetch_for(s, wop(s, W_QKV, L, true), D, s->nq_ext, 1024);
         launch_qkv_bwd(qb, BN);
-        if (defer) {
-            // the layer's four weight gradients: eight transposes in one launch, then G += dY^T X for the four matrices in one
-            const int m_out[4] = {D, 2 * IS, D, s->nq_ext}, n_in[4] = {IS, D, qd, D};
-            const half_t *x16[4] = {at<half_t>(s->act16, L * s->st_act), at<half_t>(s->ln2_16, L * s->st_ln1),
-                                    at<half_t>(s->attn16, L * s->st_attn), at<half_t>(s->ln1_16, (size_t)L * s->st_ln1)};
-            const float *xinv[4] = {at<float>(s->act_inv, (size_t)L * BN), at<float>(s->ln2_inv, (size_t)L * BN), at<float>(s->ones),
-                                    at<float>(s->ln1_inv, (size_t)L * BN)};
-            MetalBuf *G[4] = {s->gd, s->ggu, s->go, s->gqkv};
-            const size_t goff[4] = {L * s->st_d, L * s->st_gu, L * s->st_o, L * s->st_qkv};
-            TransposeOperand ops[8];
-            for (int i = 0; i < 4; i++) {
-                ops[2 * i] = TransposeOperand{d16[i], dinv[i], m_out[i], at<half_t>(s->lyT[i]), at<float>(s->lyT_inv[i])};
-                ops[2 * i + 1] = TransposeOperand{x16[i], xinv[i], n_in[i], at<half_t>(s->lxT[i]), at<float>(s->lxT_inv[i])};
-            }
-            launch_transpose_scaled_jobs(ops, 8, BN);
-            WgradOperands wg[4];
-            for (int i = 0; i < 4; i++)
-                wg[i] = WgradOperands{at<half_t>(s->lxT[i]), at<float>(s->lxT_inv[i]), at<half_t>(s->lyT[i]), at<float>(s->lyT_inv[i]),
-                                      at<half_t>(G[i], goff[i]), m_out[i], n_in[i]};
-            launch_wgrads(wg, 4, BN, 0, 0.f);
-        }
         // full-parameter: W_q, W_k, W_v are updated BEFORE the dX product, which then multiplies with the
         // new weights in SGD mode, as the reference does                       [:922-946]
         if (mode != BWD_LORA && !defer)
@@ -643,6 +628,30 @@ void backward_impl(SFTState *s, int mode = BWD_LORA, float lr = 0.f)
         // dln1 = [dq|dk|dv|dh] [Wq;Wk;Wv;A_q;A_v]; dx += RNB(x_in, dln1; g_in); clamp     [:956-980]
         if (!input_grad) break;
         Planes pl = gemm(s, d16[3], dinv[3], wop(s, W_QKV, L, true), D, s->nq_ext);
+        if (defer) {
+            // the layer's four weight gradients: eight transposes in one launch, then G += dY^T X for the four matrices in one; behind
+            // the layer's last product, whose weights BWD_APPLY changes, and ahead of the norm that writes d16[0] again
+            const int m_out[4] = {D, 2 * IS, D, s->nq_ext}, n_in[4] = {IS, D, qd, D};
+            const half_t *x16[4] = {at<half_t>(s->act16, L * s->st_act), at<half_t>(s->ln2_16, L * s->st_ln1),
+                                    at<half_t>(s->attn16, L * s->st_attn), at<half_t>(s->ln1_16, (size_t)L * s->st_ln1)};
+            const float *xinv[4] = {at<float>(s->act_inv, (size_t)L * BN), at<float>(s->ln2_inv, (size_t)L * BN), at<float>(s->ones),
+                                    at<float>(s->ln1_inv, (size_t)L * BN)};
+            const bool apply = mode == BWD_APPLY;
+            MetalBuf *G[4] = {apply ? s->wd : s->gd, apply ? s->wgu : s->ggu, apply ? s->wo : s->go, apply ? s->wqkv : s->gqkv};
+            MetalBuf *WT[4] = {s->wdT, s->wguT, s->woT, s->wqkvT};
+            const size_t goff[4] = {L * s->st_d, L * s->st_gu, L * s->st_o, L * s->st_qkv}, toff[4] = {L * s->st_dT, L * s->st_guT, L * s->st_oT, L * s->st_qkvT};
+            TransposeOperand ops[8];
+            for (int i = 0; i < 4; i++) {
+                ops[2 * i] = TransposeOperand{d16[i], dinv[i], m_out[i], at<half_t>(s->lyT[i]), at<float>(s->lyT_inv[i])};
+                ops[2 * i + 1] = TransposeOperand{x16[i], xinv[i], n_in[i], at<half_t>(s->lxT[i]), at<float>(s->lxT_inv[i])};
+            }
+            launch_transpose_scaled_jobs(ops, 8, BN);
+            WgradOperands wg[4];
+            for (int i = 0; i < 4; i++)
+                wg[i] = WgradOperands{at<half_t>(s->lxT[i]), at<float>(s->lxT_inv[i]), at<half_t>(s->lyT[i]), at<float>(s->lyT_inv[i]),
+                                      at<half_t>(G[i], goff[i]), m_out[i], n_in[i], apply ? at<half_t>(WT[i], toff[i]) : nullptr};
+            launch_wgrads(wg, 4, BN, apply ? 2 : 0, lr);
+        }
         NormBwdArgs n1{};
         n1.dy = pl; n1.x_saved = at<float>(s->xs, (size_t)(2 * L) * xsz); n1.g = at<float>(s->g_in, (size_t)L * D);
         n1.eps = s->eps; n1.D = D; n1.dx_prev = at<float>(s->dx[cur]); n1.dx_out = at<float>(s->dx[cur ^ 1]); n1.clamp = 1e6f;
@@ -1095,6 +1104,7 @@ void sft_alloc_grad_accum(SFTState *s)
     s->ggu = hbuf(s->NL * s->st_gu);   s->gd = hbuf(s->NL * s->st_d);
     s->glm = hbuf(tiled_elems(s->V, s->D));
     for (MetalBuf *b : {s->gqkv, s->go, s->ggu, s->gd, s->glm}) HIP_CHECK(hipMemsetAsync(dptr(b), 0, b->size, stream()));
+    s->accum_clear = true;
     const int m_out[4] = {s->D, 2 * s->IS, s->D, s->nq_ext}, n_in[4] = {s->IS, s->D, s->qd, s->D};
     for (int i = 0; i < 4; i++) {
         s->dy16[i] = hbuf(tiled_elems(s->BN, m_out[i])); s->dy_inv[i] = fbuf(s->BN);
@@ -1117,6 +1127,7 @@ void sft_apply_grad_sgd(SFTState *s, float lr)
     launch_apply_retile(at<half_t>(s->wgu), at<half_t>(s->ggu), at<half_t>(s->wguT), 2 * s->IS, s->D, lr, s->NL, s->st_gu, s->st_guT);
     launch_apply_retile(at<half_t>(s->wd), at<half_t>(s->gd), at<half_t>(s->wdT), s->D, s->IS, lr, s->NL, s->st_d, s->st_dT);
     launch_apply_retile(at<half_t>(s->wlm), at<half_t>(s->glm), at<half_t>(s->wlmT), s->V, s->D, lr);
+    s->accum_clear = true;
     metal_flush();
 }
 
@@ -1360,6 +1371,9 @@ void grpo_apply_completions(SFTState *s, const GRPOCompletions *c, float lr, flo
         if (!s->lora_acc) s->lora_acc = fbuf(s->lora_n);
         HIP_CHECK(hipMemsetAsync(dptr(s->lora_acc), 0, s->lora_n * 4, stream()));
     }
+    // a whole group in one pass, with nothing accumulated before it: gradients are applied as they are formed
+    const bool at_once = accurate && s->accum_clear && G <= B;
+    bool applied = false;
     // A state built with batch B takes B completions per pass (one forward and backward for all of them: every weight
     // is streamed once per pass instead of once per completion); sequence slots beyond the group are all zero rows.
     for (int i0 = 0; i0 < G; i0 += B) {
@@ -1400,7 +1414,9 @@ void grpo_apply_completions(SFTState *s, const GRPOCompletions *c, float lr, flo
         ce.clip_eps = c->clip_eps; ce.dl_scale = 1.0f / (float)G;                 // [:445-452]
         launch_ce_rows(ce, s->BN);
         if (s->full_param) {
-            backward_impl(s, s->gqkv ? BWD_ACCUM : BWD_SGD, lr / (float)G);       // [:454-461]
+            if (at_once) backward_impl(s, BWD_APPLY, lr);
+            else backward_impl(s, s->gqkv ? BWD_ACCUM : BWD_SGD, lr / (float)G);  // [:454-461]
+            applied = at_once;
         } else {
             backward_impl(s);                                                     // [:462-473]
             metal_enqueue_add_scaled(s->lora_acc, s->lora_grad, 1.0f, (int)s->lora_n);
@@ -1410,7 +1426,8 @@ void grpo_apply_completions(SFTState *s, const GRPOCompletions *c, float lr, flo
             for (int b = 0; b < B && i0 + b < G; b++)
                 memcpy(new_logprobs + (size_t)(i0 + b) * seq_len, s->grpo_new_lp_cpu + (size_t)b * seq_len, (size_t)seq_len * 4);
     }
-    if (accurate) {                                                               // [:479-481]
+    if (applied) {
+    } else if (accurate) {                                                        // [:479-481]
         sft_apply_grad_sgd(s, lr);
     } else if (!s->full_param) {                                                  // [:482-491]
         metal_enqueue_copy(s->lora_acc, s->lora_grad, (int)s->lora_n);

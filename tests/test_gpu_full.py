@@ -186,6 +186,38 @@ def test_grpo_accumulate_and_apply(cfg):
             assert rel(d_gpu, d_ref) < 3e-2, (L, k, rel(d_gpu, d_ref))
 
 
+@pytest.mark.parametrize("cfg", [FULL_Q.with_(batch=3, seq=40), FULL_G.with_(batch=2), FULL_Q3, FULL_Q3.with_(name="wide", D=320, Hq=5, Hkv=1, IS=704, V=2080, seq=24)],
+                         ids=["c1", "gemma3", "odd_tiles", "inner_blocks"])
+def test_a_group_in_one_pass_is_applied_as_its_gradients_are_formed(cfg):
+    """grpo_apply_completions on a state that holds the whole group never fills the accumulators; a group twice as large, whose
+    second half is empty, takes a second pass and with it accumulate and apply.  With its advantages doubled (the loss is
+    divided by the group's size) both form the same numbers, and every weight comes out the same, bit for bit, in both images, as
+    it does when gradients were accumulated beforehand and applied with a rate of zero."""
+    model = make_model(cfg, seed=61, gamma_jitter=0.1)
+    rng = np.random.default_rng(62)
+    G, P = cfg.batch, 5
+    prompt, toks, adv = _completions(cfg, rng, G, P, [cfg.seq - P - 3 * i for i in range(G)])
+    old = [np.full(len(t), -np.log(cfg.V), np.float32) + 0.1 * rng.standard_normal(len(t)).astype(np.float32) for t in toks]
+    none = np.zeros(0)
+    out = []
+    for way in range(3):
+        with SFTState(cfg, model) as st:
+            if way == 2:
+                st.alloc_grad_accum()
+                st.apply_grad_sgd(0.0)
+            for _ in range(2):
+                if way == 1:
+                    lp = st.grpo_apply_completions(prompt, toks + [none] * G, old + [none] * G, np.concatenate([2 * adv, 0 * adv]), 0.2, 0.05)[:G]
+                else:
+                    lp = st.grpo_apply_completions(prompt, toks, old, adv, 0.2, 0.05)
+            out.append((lp, [st.matrix_f16(L, k, src) for L, k in all_matrices(cfg) for src in (0, 1, 2)]))
+    assert any(np.any(a != b) for a, b in zip(out[0][1][0::3], [oracle.f32_to_f16_bits(oracle_matrix(cfg, oracle.weights_as_used(model), L, k)) for L, k in all_matrices(cfg)]))
+    for other in out[1:]:
+        assert np.array_equal(out[0][0], other[0])
+        for i, (a, b) in enumerate(zip(out[0][1], other[1])):
+            assert np.array_equal(a, b), (i // 3, i % 3)
+
+
 @pytest.mark.parametrize("batch", [1, 2], ids=["one_per_pass", "two_per_pass"])
 def test_grpo_lora_mode_sums_adapter_gradients_then_adamw(batch):
     cfg = C1.with_(name="grpo_lora", seq=32)
