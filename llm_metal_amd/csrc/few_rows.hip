@@ -1,9 +1,10 @@
-// A batch's step reads every weight once for 2 .. 32 rows: bound by the weights' bytes and by what stands between the launches, so
+// A batch's step or a short prompt reads every weight once for up to 32 rows: bound by the weights' bytes and by what stands between the launches, so
 // its products take their operand as the kernels before leave it and leave what the kernels behind need (few_rows.h).
 #include "backend.h"
 #include "devutil.h"
 #include "few_rows.h"
 #include <stdio.h>
+#include <algorithm>
 #include <type_traits>
 
 using namespace lmhip;
@@ -15,6 +16,51 @@ constexpr float RESIDUAL = 2048.f;                         // a residual image i
 __device__ __forceinline__ float gated(float g, float u, int gelu)
 {
     return (gelu ? 0.5f * g * (1.0f + tanhf(gelu_inner(g))) : g / (1.0f + expf(-g))) * u;
+}
+
+// The sums of a workgroup's waves for 32 weight rows (WT 2: gate and up rows) times the images of up to 16 MT vectors, acc[row block][image tile],
+// meet in `part`, half of the waves at a time; value and residual images times their factors are added and the results stored.
+// TOKENS: an accumulator's rows are the images and its columns the weight rows, else the other way round.
+template <int MT, int WT, int WAVES, bool TOKENS>
+__device__ __forceinline__ void few_finish(float *part, const float16v (&acc)[WT][MT], const float *__restrict__ inv, float *__restrict__ out, int ldo, int B, int N, int gelu)
+{
+    constexpr int HALF = WAVES / 2;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float *p = part + (size_t)(wave & (HALF - 1)) * WT * MT * 1024;
+    if (wave >= HALF) {
+#pragma unroll
+        for (int q = 0; q < WT; q++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) p[((q * MT + m) * 16 + i) * 64 + lane] = acc[q][m][i];
+    }
+    __syncthreads();
+    if (wave < HALF) {
+#pragma unroll
+        for (int q = 0; q < WT; q++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) p[((q * MT + m) * 16 + i) * 64 + lane] += acc[q][m][i];
+    }
+    __syncthreads();
+    // row r of an accumulator is register 4 (r / 8) + r % 4 of the lanes of half (r / 4) % 2
+    const int m = threadIdx.x & 31, n = blockIdx.x * 32 + m;
+    if (n >= N) return;
+    auto image = [&](int q, int row) __attribute__((always_inline)) {
+        const int r = TOKENS ? row & 31 : m, c = TOKENS ? m : row & 31;
+        const float *s = part + (q * MT + (MT > 1 ? row >> 5 : 0)) * 1024 + (4 * (r >> 3) + (r & 3)) * 64 + 32 * ((r >> 2) & 1) + c;
+        float v = s[0];
+#pragma unroll
+        for (int h = 1; h < HALF; h++) v += s[h * WT * MT * 1024];
+        return v * inv[row];
+    };
+    for (int b = threadIdx.x >> 5; b < B; b += 64 * WAVES / 32) {
+        float v = image(0, b) + image(0, B + b);
+        if (WT == 2) v = gated(v, image(WT - 1, b) + image(WT - 1, B + b), gelu);
+        out[(size_t)b * ldo + n] = v;
+    }
 }
 
 // WT 1: 32 weight rows of [N, K] per workgroup, WT 2: the 32 gate rows and the 32 up rows of as many FFN columns.  All of K in one
@@ -78,41 +124,128 @@ __global__ __launch_bounds__(64 * WAVES, WT * MT == 4 || U > 3 ? 2 : 4) void k_f
     if (U > 3 && left == 3) tiles(std::integral_constant<int, U < 3 ? U : 3>{}, t0);
     if (U > 2 && left == 2) tiles(std::integral_constant<int, U < 2 ? U : 2>{}, t0);
     if (left == 1) tiles(std::integral_constant<int, 1>{}, t0);
-    float *p = part + (size_t)(wave & (HALF - 1)) * WT * MT * 1024;
-    if (wave >= HALF) {
+    few_finish<MT, WT, WAVES, false>(part, acc, inv, out, ldo, B, N, gelu);
+}
+
+// Eight codes of a Q8_0 row as fp16 integers, exactly: 1024 + (code + 128) is a half's bits, 1152 taken off
+__device__ __forceinline__ half8 codes8(uint32_t a, uint32_t b)
+{
+    half8 r;
+    const uint32_t w[2] = {a ^ 0x80808080u, b ^ 0x80808080u};
 #pragma unroll
-        for (int q = 0; q < WT; q++)
-#pragma unroll
-            for (int m = 0; m < MT; m++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) p[((q * MT + m) * 16 + i) * 64 + lane] = acc[q][m][i];
+    for (int i = 0; i < 4; i++) {
+        const uint32_t p = __builtin_amdgcn_perm(0x64646464u, w[i >> 1], i & 1 ? 0x04030402u : 0x04010400u);
+        const half2v h = __builtin_bit_cast(half2v, p) - half2v{(half_t)1152, (half_t)1152};
+        r[2 * i] = h[0];
+        r[2 * i + 1] = h[1];
     }
-    __syncthreads();
-    if (wave < HALF) {
+    return r;
+}
+
+// k_few_full over the rows of a Q8_0 matrix as they lie (codes [rows][K], a scale per 32 of them): 1.06 bytes per weight, and exact ones.
+// A wave takes four blocks of its 32 rows at a time, a whole 128-byte line of each, the next ones on their way: read eight lanes to a
+// line (a lane to a row made 32 lines of every load, which took the address unit 3.5 us a group) and turned through LDS of the
+// wave's own.  Both lane halves multiply one block -- the operand's two column blocks, a lane half each, change places -- so
+// that a block's two MFMAs multiply integers and its scale, one per lane with the weight rows as the accumulator's columns,
+// goes onto their sum in fp32.  blockIdx.y: chunks of K (few_chunks), a plane of the result each.
+// 4B shape, 8 / 32 vectors: Q|K|V 8.1 / 12.7 us, gate|up 21.8 / 29.4, O 7.4 / 10.5, down 12.4 / 20.6 (bound by the address unit and the
+// trips, not by 1.06 bytes per weight); the two F16 images formed for every such product took 97 us a layer and their products 105.
+// QUAD: a row's scales come in fours, in one load.
+template <int MT, int WT, int WAVES, bool QUAD>
+__global__ __launch_bounds__(64 * WAVES, MT * WT == 1 ? 4 : 2) void k_few_q8(const half8 *__restrict__ A, const float *__restrict__ inv, const int8_t *__restrict__ Wq,
+                                                                            const half_t *__restrict__ Wd, float *__restrict__ out, int ldo, int B, int N, int K, int up_row, int gelu)
+{
+    constexpr int G = 4, LDR = 144;                        // bytes of a row's line in LDS
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    __shared__ float part[WAVES / 2 * WT * MT * 16 * 64];
+    __shared__ u4 lines[WAVES][WT][32 * LDR / 16];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), h = lane >> 5;
+    const int nb = K >> 5, Kb = tiled_kb(K), all = (nb + G - 1) / G, each = (all + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int first = blockIdx.y * each, groups = min(first + each, all), row0 = blockIdx.x * 32;
+    struct Stage { u4 c[WT][G]; half4 d[WT]; };
+    auto load = [&](Stage &w, int g) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < WT; q++)
+        for (int q = 0; q < WT; q++) {
 #pragma unroll
-            for (int m = 0; m < MT; m++)
+            for (int u = 0; u < G; u++) {                  // rows 8 u + lane / 8, sixteen codes of the line
+                const size_t r = min(row0 + 8 * u + (lane >> 3), N - 1) + (q ? up_row : 0);
+                w.c[q][u] = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(Wq + r * K + min(g * 128 + 16 * (lane & 7), K - 16)));
+            }
+            const half_t *d = Wd + (size_t)(min(row0 + (lane & 31), N - 1) + (q ? up_row : 0)) * nb;
+            if (QUAD) w.d[q] = *reinterpret_cast<const half4 *>(d + min(g, all - 1) * G);
+            else
 #pragma unroll
-                for (int i = 0; i < 16; i++) p[((q * MT + m) * 16 + i) * 64 + lane] += acc[q][m][i];
-    }
-    __syncthreads();
-    // weight row m of the block is register 4 (m / 8) + m % 4 of the lanes of half (m / 4) % 2
-    const int m = threadIdx.x & 31, n = blockIdx.x * 32 + m;
-    if (n >= N) return;
-    const int at = (4 * (m >> 3) + (m & 3)) * 64 + 32 * ((m >> 2) & 1);
-    auto image = [&](int q, int row) __attribute__((always_inline)) {
-        const float *s = part + (q * MT + (MT > 1 ? row >> 5 : 0)) * 1024 + at + (row & 31);
-        float v = s[0];
-#pragma unroll
-        for (int h = 1; h < HALF; h++) v += s[h * WT * MT * 1024];
-        return v * inv[row];
+                for (int u = 0; u < G; u++) w.d[q][u] = d[min(g * G + u, nb - 1)];
+        }
     };
-    for (int b = threadIdx.x >> 5; b < B; b += 64 * WAVES / 32) {
-        float v = image(0, b) + image(0, B + b);
-        if (WT == 2) v = gated(v, image(WT - 1, b) + image(WT - 1, B + b), gelu);
-        out[(size_t)b * ldo + n] = v;
+    uint32_t slot[MT];                                     // (image rows past the last repeat it)
+#pragma unroll
+    for (int m = 0; m < MT; m++) slot[m] = a_lane((lane & 32) | (min(32 * m + (lane & 31), 2 * B - 1) & 31));
+    float16v sum[WT][MT] = {};
+    Stage w;
+    load(w, first + wave);                                 // (a wave behind the last group asks for the last columns; nothing of it is used)
+    for (int g = first + wave; g < groups; g += WAVES) {
+        half8 a[MT][2][4];                                 // the group's two tiles
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const half8 *at = A + (size_t)min(2 * g + t, Kb - 1) * 256;
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) a[m][t][j] = (m ? at + (size_t)Kb * 256 : at)[slot[m] + 64 * j];
+        }
+        float d[WT][G];
+#pragma unroll
+        for (int q = 0; q < WT; q++)
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                *reinterpret_cast<u4 *>(reinterpret_cast<char *>(lines[wave][q]) + (8 * u + (lane >> 3)) * LDR + 16 * (lane & 7)) = w.c[q][u];
+                d[q][u] = (float)w.d[q][u];
+            }
+        load(w, g + WAVES);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // (a wave's own lines: no barrier)
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        // column blocks 0 and 1 of a tile, a lane half each: slices 2 e and 2 e + 1 become block 0's and block 1's
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int e = 0; e < 4; e += 2) {
+                    u4 x = __builtin_bit_cast(u4, a[m][t][e]), y = __builtin_bit_cast(u4, a[m][t][e + 1]);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const auto r = __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false);
+                        x[i] = r[0];
+                        y[i] = r[1];
+                    }
+                    a[m][t][e] = __builtin_bit_cast(half8, x);
+                    a[m][t][e + 1] = __builtin_bit_cast(half8, y);
+                }
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            if (g * G + u >= nb) break;
+#pragma unroll
+            for (int q = 0; q < WT; q++) {
+                const char *line = reinterpret_cast<const char *>(lines[wave][q]) + (lane & 31) * LDR + 32 * u + 8 * h;
+                const u2 c0 = *reinterpret_cast<const u2 *>(line), c1 = *reinterpret_cast<const u2 *>(line + 16);
+                const half8 w0 = codes8(c0[0], c0[1]), w1 = codes8(c1[0], c1[1]);
+#pragma unroll
+                for (int m = 0; m < MT; m++) {
+                    float16v acc = {};
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[m][u >> 1][u & 1], w0, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[m][u >> 1][2 + (u & 1)], w1, acc, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) sum[q][m][i] = fmaf(acc[i], d[q][u], sum[q][m][i]);
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
+    few_finish<MT, WT, WAVES, true>(part, sum, inv, out + (size_t)blockIdx.y * B * ldo, ldo, B, N, gelu);
 }
 
 // 128 weight rows and 2 T K tiles per workgroup: each of its eight waves holds the T weight tiles of one row block and one half of
@@ -349,6 +482,35 @@ void launch_few_norm(float *x, const FewPlanes &br, const float *g_branch, const
     else { if (br.S && g_branch) FN(2, true); else FN(2, false); }
 #undef FN
 }
+
+// K chunks of a product of [N, K] Q8_0 rows whose planes its consumer adds: 256 workgroups, at least two groups of columns per wave
+int few_chunks(int N, int K)
+{
+    const int most = std::max(1, (K / 128) / 16);
+    return std::min(most, (256 + tiled_rb(N) - 1) / tiled_rb(N));
+}
+
+#define FEW_Q8(MT_, WT_, WAVES_, OUT_, LDO_, UP_, GELU_) do { \
+    if (K % 128 == 0 && ((uintptr_t)W.d & 7) == 0) hipLaunchKernelGGL((k_few_q8<MT_, WT_, WAVES_, true>), grid, dim3(64 * WAVES_), 0, stream(), A, inv, W.q, W.d, OUT_, LDO_, B, N, K, UP_, GELU_); \
+    else hipLaunchKernelGGL((k_few_q8<MT_, WT_, WAVES_, false>), grid, dim3(64 * WAVES_), 0, stream(), A, inv, W.q, W.d, OUT_, LDO_, B, N, K, UP_, GELU_); } while (0)
+FewPlanes launch_few_full_q8(const half_t *a16, const float *inv, const FewQ8 &W, float *out, int ldo, int B, int N, int K, int chunks)
+{
+    check(B >= 1 && B <= FEW_ROWS && N >= 1 && K >= 32 && K % 32 == 0 && ldo >= N && chunks >= 1 && chunks < 65536 && ((uintptr_t)W.q & 15) == 0, "few_full_q8");
+    const dim3 grid(tiled_rb(N), chunks);
+    const half8 *A = reinterpret_cast<const half8 *>(a16);
+    if (2 * B > 32) FEW_Q8(2, 1, 8, out, ldo, 0, 0); else FEW_Q8(1, 1, 8, out, ldo, 0, 0);
+    return FewPlanes{out, (size_t)B * ldo, chunks, ldo};
+}
+
+void launch_few_glu_q8(const half_t *a16, const float *inv, const FewQ8 &W, float *act, int B, int IS, int K, int gelu)
+{
+    check(B >= 1 && B <= FEW_ROWS && IS >= 32 && IS % 32 == 0 && K >= 32 && K % 32 == 0 && ((uintptr_t)W.q & 15) == 0, "few_glu_q8");
+    const dim3 grid(IS / 32);
+    const half8 *A = reinterpret_cast<const half8 *>(a16);
+    const int N = IS;
+    if (2 * B > 32) FEW_Q8(2, 2, 4, act, IS, IS, gelu); else FEW_Q8(1, 2, 4, act, IS, IS, gelu);
+}
+#undef FEW_Q8
 
 int few_planes(int N, int K)
 {

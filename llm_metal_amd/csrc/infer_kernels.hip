@@ -12,6 +12,7 @@
 #include "devutil.h"
 #include "gemm.h"
 #include "prompt.h"
+#include "few_rows.h"
 #include <hip/hip_ext.h>
 
 using namespace lmhip;
@@ -1574,6 +1575,14 @@ void matvec_norm(MetalBuf *W, const NormIn &nin, MetalBuf *y, int rows, int cols
         launch_matvec_norm<0>(dptr(W), nullptr, nin, dptr_as<float>(y), rows, cols, glu);
     }
     mark_written(y);
+}
+
+FewQ8 few_q8_of(MetalBuf *W, int rows, int cols)
+{
+    if (rows <= 0 || cols <= 0 || (cols & 31) || W->size < (size_t)rows * (cols / 32) * 34) { fprintf(stderr, "[fast_hip] few_q8_of: unsupported shape %d x %d\n", rows, cols); abort(); }
+    FewQ8 r{};
+    r.q = q8_split_of(W, rows, cols / 32, &r.d);
+    return r;
 }
 
 void q8_to_tiled_pair(MetalBuf *W, int rows, int cols, half_t *hi, half_t *lo)

@@ -1233,9 +1233,9 @@ bool q8_scales_fit(InferenceState *s)
     return s->q8_fit = d * 128.f < 65504.f;                           // (false for a NaN)
 }
 
-// Whether n tokens go many to a step: from five on.  A step of 2 to 32 rows takes 1.0 ms on F16 weights (nine layers of the 4B
-// shape; 1.8 tokens one by one) and 2.4 ms on Q8_0 ones (4.5 tokens: their tiled images are formed anew for every product), and
-// 500 tokens take 3.7 instead of 460 ms; portions of up to four stay bit for bit what single tokens give.  A state's first prompt
+// Whether n tokens go many to a step: from five on.  Nine layers of the 4B shape, ms at 5 / 8 / 16 / 32 / 64 tokens: F16 weights
+// 0.75 / 0.79 / 0.85 / 1.02 / 1.27, Q8_0 0.78 / 0.81 / 0.86 / 1.03 / 1.98 (1.8 and 2.4 four tokens one by one); 500 tokens take 3.7 instead of
+// 460 ms; portions of up to four stay bit for bit what single tokens give.  A state's first prompt
 // pays for the buffers and the tiles that are kept besides: at five tokens up to 2 ms more than one by one, once, at sixteen none.
 // A state takes its tokens one by one where a Q8_0 weight is beyond what a half holds and, decided once with its first prompt,
 // where there is no room for a step's buffers.
@@ -1311,8 +1311,12 @@ SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const
     return out;
 }
 
+// A step of up to FEW_ROWS tokens takes the batch's products (few_rows.h) where the state's widths fit them: at 8 / 32 tokens of nine 4B
+// layers 0.79 / 1.02 ms against 0.94 / 1.07 of the short sums (F16), 0.81 / 1.03 against 2.40 / 2.45 with F16 images formed for each product (Q8_0)
+bool prompt_few(const InferenceState *s, int M) { return M <= FEW_ROWS && few_rows_fit(s); }
+
 // One step: the M tokens at positions pos .. pos + M - 1, their keys and values into kc and vc (the first sequence's part),
-// the final norm's rows into r.ln.  Per layer the launches of forward_token_batch, with the tokens as rows: ten, whatever M.
+// the final norm's rows into r.ln.  Per layer the launches of forward_token_batch, with the tokens as rows: ten, for a few rows eight.
 void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, std::vector<MetalBuf *> &vc, int M, int pos)
 {
     const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd, IS = s->IS, qd = Hq * hd, nqkv = qd + 2 * Hkv * hd;
@@ -1327,15 +1331,38 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
         const float *gb = g_branch ? dptr_as<float>(g_branch) : nullptr;
         launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, M, D, s->eps);
     };
+    const bool few = prompt_few(s, M), q8 = !s->use_fp16 && !bt;
+    const int nq_rows = nqkv + (bt && adapters ? 2 * s->R : 0);               // (a training state's fused matrix continues with the rows of A_q and A_v)
+    float *P = nullptr, *act = nullptr;
+    if (few) {
+        P = at_least(r.planes, (size_t)M * std::max(nq_rows, D * (q8 ? std::max(few_chunks(D, qd), few_chunks(D, IS)) : std::max(few_planes(D, qd), few_planes(D, IS)))));
+        act = at_least(r.act, (size_t)std::min(FEW_ROWS, r.cap) * IS);
+    }
+    auto few_norm = [&](const FewPlanes &br, MetalBuf *g_branch, MetalBuf *g, bool keep) {
+        launch_few_norm(dptr_as<float>(r.x), br, g_branch ? dptr_as<float>(g_branch) : nullptr, dptr_as<float>(g), keep ? dptr_as<float>(r.ln) : nullptr, a16, inv_ln, M, D, s->eps);
+    };
+    auto tiles = [&](const WMat *w, const WeightOp *op, int rows) { return op ? op->w16 : prompt_tiles(w, 0, rows); };
+    auto few_branch = [&](const WMat *w, const WeightOp *op, const float *in, int K) {       // [M, D] of the rows `in`
+        if (!q8) return launch_few_split(in, tiles(w, op, D), P, M, D, K);
+        launch_rows_to_f16_split(in, a16, inv_br, M, K);
+        return launch_few_full_q8(a16, inv_br, few_q8_of(w->mbuf, D, K), P, D, M, D, K, few_chunks(D, K));
+    };
     SplitPlanes pending{};
+    FewPlanes pending_few{};
     MetalBuf *pending_g = nullptr;
     for (int L = 0; L < s->NL; L++) {
         const InferenceState::Layer &lw = s->layers[L];
         const BorrowedLayer *bl = bt ? &s->borrowed[L] : nullptr;
-        norm(pending, pending_g, lw.g_in, adapters && !bt);
         PromptHeads h{};
-        // (a training state's fused matrix continues with the rows of A_q and A_v)
-        h.qkv = prompt_product(s, r, &lw.qkv, bt ? &bl->qkv : nullptr, nqkv + (bt && adapters ? 2 * s->R : 0), D, inv_ln, M);
+        if (few) {
+            few_norm(pending_few, pending_g, lw.g_in, adapters && !bt);
+            if (q8) launch_few_full_q8(a16, inv_ln, few_q8_of(lw.qkv.mbuf, nq_rows, D), P, nq_rows, M, nq_rows, D);
+            else launch_few_full(a16, inv_ln, tiles(&lw.qkv, bt ? &bl->qkv : nullptr, nq_rows), P, nq_rows, M, nq_rows, D);
+            h.qkv.P = P; h.qkv.S = 1; h.qkv.N = nq_rows;
+        } else {
+            norm(pending, pending_g, lw.g_in, adapters && !bt);
+            h.qkv = prompt_product(s, r, &lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D, inv_ln, M);
+        }
         h.g_q = lw.g_q ? dptr_as<float>(lw.g_q) : nullptr; h.g_k = lw.g_k ? dptr_as<float>(lw.g_k) : nullptr;
         h.rope = dptr_as<float2>(s->rope_tabs) + ((size_t)s->theta_slot[L] * s->max_seq + pos) * (hd / 2);
         h.q = dptr_as<float>(r.q); h.kc = dptr_as<float>(kc[L]); h.vc = dptr_as<float>(vc[L]);
@@ -1352,6 +1379,14 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
         launch_prompt_heads(h);
         launch_prompt_attention(h.q, h.kc, h.vc, dptr_as<float>(r.att), M, pos, Hq, Hkv, hd, s->max_seq);
         mark_written(kc[L]); mark_written(vc[L]);
+        if (few) {
+            few_norm(few_branch(lw.o, bt ? &bl->o : nullptr, dptr_as<float>(r.att), qd), gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, false);
+            if (q8) launch_few_glu_q8(a16, inv_ln, few_q8_of(lw.gu.mbuf, 2 * IS, D), act, M, IS, D, gemma ? 1 : 0);
+            else launch_few_glu(a16, inv_ln, tiles(&lw.gu, bt ? &bl->gu : nullptr, 2 * IS), act, M, IS, D, gemma ? 1 : 0);
+            pending_few = few_branch(lw.down, bt ? &bl->down : nullptr, act, IS);
+            pending_g = gemma ? lw.g_post_ff : nullptr;
+            continue;
+        }
         launch_rows_to_f16_split(dptr_as<float>(r.att), a16, inv_br, M, qd);
         const SplitPlanes o = prompt_product(s, r, lw.o, bt ? &bl->o : nullptr, D, qd, inv_br, M);
         norm(o, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, false);
@@ -1364,7 +1399,8 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
         pending = prompt_product(s, r, lw.down, bt ? &bl->down : nullptr, D, IS, inv_br, M);
         pending_g = gemma ? lw.g_post_ff : nullptr;
     }
-    norm(pending, pending_g, s->g_final, true);
+    if (few) few_norm(pending_few, pending_g, s->g_final, true);
+    else norm(pending, pending_g, s->g_final, true);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1401,7 +1437,11 @@ void prompt_portions(InferenceState *s, const int *tokens, int n, int pos, std::
                      const std::function<void(int, int)> &f)
 {
     PromptRun &r = *s->prompt;
-    const int portions = (n + r.cap - 1) / r.cap, each = (n + portions - 1) / portions;
+    // (Q8_0: two short steps take less time than one whose products form F16 images of their weights -- 1.98 against 2.71 ms for 64 tokens
+    // of nine 4B layers -- three do not)
+    const bool q8 = !s->use_fp16 && !s->borrows_tiles;
+    const int cap = q8 && n <= 2 * FEW_ROWS && few_rows_fit(s) ? std::min(FEW_ROWS, r.cap) : r.cap;
+    const int portions = (n + cap - 1) / cap, each = (n + portions - 1) / portions;
     for (int i = 0; i < n; i++) r.ids_host[pos + i] = tokens[i];
     for (int at = 0; at < n; at += each) {
         const int M = std::min(each, n - at);

@@ -9,6 +9,7 @@ namespace lmhip {
 
 // A product as the GEMM leaves it: S planes of [2M, N], rows m and M + m the value and residual images of row m, inv their
 // factors.  P2 not null: S2 more planes of [M, N] of the value rows with what rounding the weights to fp16 lost, times 2^11.
+// inv null (planes_at only): P is the product itself, [M, N].
 struct SplitPlanes {
     const float *P, *inv;
     size_t plane;
@@ -20,6 +21,7 @@ struct SplitPlanes {
 constexpr float Q8_RESIDUAL_SCALE = 2048.f;
 __device__ __forceinline__ float planes_at(const SplitPlanes &p, int M, int m, int n)
 {
+    if (!p.inv) return p.P[(size_t)m * p.N + n];
     float v = split_planes_value(p.P, p.S, p.plane, p.N, p.inv, M, m, n);
     if (p.P2) {
         float r = 0.f;

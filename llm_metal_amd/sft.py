@@ -34,7 +34,7 @@ class _HostView:
 
 
 class _HostPool:
-    """Arrays that a state hands out, in pinned memory: the GPU writes them in place.  New pageable pages cost a fault each and a
+    """Arrays of a batch's logits, step after step, in pinned memory: the GPU writes them in place.  New pageable pages cost a fault each and a
     copy through the runtime's staging: 32 sequences of a vocabulary of 16 384, 2 MB a step, 700 us of which the kernels 278;
     eight of 32 768, 1 MB, 875 us of which 662.  At most `LIMIT` bytes at a time, idle ones among them; what goes beyond is ordinary
     memory, as is what is too small for its pages to count.  Blocks that no array looks at are kept for the next ones of their
@@ -341,7 +341,7 @@ class InferenceState:
         """The next tokens at the current position; logits [len(want), V] at the places `want` (ascending) among them."""
         t = np.ascontiguousarray(tokens, dtype=np.int32)
         w = np.ascontiguousarray(want, dtype=np.int32)
-        out = self._host.empty((len(w), self.V))
+        out = np.empty((len(w), self.V), dtype=np.float32)
         if self.L.inference_forward_tokens(self.h, _vp(t), len(t), _vp(w), len(w), _vp(out)) != 0:
             raise RuntimeError("inference_forward_tokens refused its arguments")
         return out

@@ -52,6 +52,22 @@ def test_prompt_equals_tokens_one_by_one(c, fmt, n):
         assert maxrel(inf.forward_tokens(toks[cut:n], [n - cut - 1]), want[n - 1:n]) < TOL
 
 
+@pytest.mark.parametrize("n", [5, 16, 17, 32, 64])
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+@pytest.mark.parametrize("kw", [dict(D=1184, Hq=2, Hkv=1, hd=128, IS=2080), dict(D=2560, Hq=4, Hkv=2, hd=128, IS=9728)], ids=["ragged", "many_chunks"])
+@pytest.mark.parametrize("model_type", [QWEN3, GEMMA3], ids=["qwen3", "gemma3"])
+def test_short_prompts_on_either_side_of_an_operand_tile(kw, fmt, n, model_type):
+    """16 tokens fill the 32 rows of one operand tile with their two images, 32 those of two, 64 are two steps of a Q8_0 state; columns
+    that fill no group of four Q8_0 blocks (1184), K in one chunk and in several."""
+    print(kw, fmt, n, flush=True)
+    c = SFTConfig("short", model_type, NL=2, V=260, tied=True, **kw)
+    model, toks = make_model(c, seed=6, gamma_jitter=0.1), tokens(c, n, n)
+    with InferenceState(c, model, max_seq=n, use_fp16=fmt == "f16") as inf:
+        want = one_by_one(inf, toks)
+        inf.reset()
+        assert maxrel(inf.forward_tokens(toks, range(n)), want) < TOL
+
+
 def test_prompt_of_several_steps():
     c = C1.with_(name="long", NL=1, V=256)
     model, toks = make_model(c, seed=4), tokens(c, 2500, 5)
