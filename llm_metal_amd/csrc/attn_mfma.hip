@@ -220,7 +220,7 @@ __device__ __forceinline__ void load_probs(float4 (&p)[M32], const AttnTileArgs 
 constexpr int DKV_TS = 40;                                 // halves per key: 80 bytes apart, so that eight lanes' 16-byte reads cover all banks
 template <int BWD, int M32, int DKV = 0>
 __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int ldx, int xlo, int nk, int N, int i0, int b, int h, int tid,
-                                         const float4 (&p_early)[BWD ? M32 : 1], uint16_t *Ts = nullptr)
+                                         const float4 (&p_early)[BWD ? M32 : 1], uint16_t *Ts = nullptr, bool keep = true)
 {
     const int rr = tid >> 3, part = tid & 7, i = i0 + rr;
     const bool row_ok = i < N;
@@ -286,7 +286,7 @@ __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int l
                 }
             }
         }
-        if (!DKV && row_ok && j < N) {
+        if (!DKV && keep && row_ok && j < N) {
             if ((N & 3) == 0) *reinterpret_cast<float4 *>(gdst + 32 * m) = o;
             else { const float *q = &o.x; for (int c = 0; c < 4; c++) if (j + c < N) gdst[32 * m + c] = q[c]; }
         }
@@ -296,19 +296,25 @@ __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int l
 // grid (query blocks of 32, Hq, batch), block 256; LDS: Ahi, Alo [32][HD+8] bf16, Xs[32][ldx] fp32 / bf16 pairs
 // M32: 32-key blocks a row can hold (2, 8, 16 or 32: sequences up to 64, 256, 512, 1024); a template parameter so
 // that the kernel's code is one straight run (the kernel runs once per workgroup, and what it skips it still fetches).
-template <int BWD, int HD, int M32, int DKV = 0>
+// CS 2 (heads of 256): two workgroups per block form the same scores and rows and half of the head's columns each (launch_tile_hd).
+template <int BWD, int HD, int M32, int DKV = 0, int CS = 1>
 __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
 {
+    static_assert(CS == 1 || HD == 256, "a wave has two column blocks to share");
     extern __shared__ float lds[];
-    constexpr int lda = HD + 8;                            // halves; rows 16-byte aligned and 4 banks apart: conflict-free 16-byte reads
+    // heads of 256 over more than 512 keys: the A rows are in LDS one half of their columns at a time, which leaves room for 1024 scores
+    // a row (the wave-per-query kernels, which sequences beyond 928 keys took before, need 380 + 641 + 344 us at 1000 positions of four heads)
+    constexpr bool HALVES = HD == 256 && M32 == 32;
+    constexpr int lda = (HALVES ? HD / 2 : HD) + 8;        // halves; rows 16-byte aligned and 4 banks apart: conflict-free 16-byte reads
     const int N = a.seq;
     if ((int)blockIdx.z >= a.batch) {
         const int per_z = gridDim.x * gridDim.y;
         prefetch_weight_tiles<256>(a.pf, (blockIdx.z - a.batch) * per_z + blockIdx.y * gridDim.x + blockIdx.x);
         return;
     }
-    const int qb = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int qb = blockIdx.x, h = blockIdx.y / CS, share = blockIdx.y % CS, b = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l31 = lane & 31, hh = lane >> 5;
+    const int dt0 = wave + 4 * share, dt_end = CS > 1 ? dt0 + 1 : HD / 32;      // the wave's column blocks: dt0, dt0 + 4 .. below dt_end
     const int qd = a.Hq * HD, kd = a.Hkv * HD, hk = h / (a.Hq / a.Hkv);
     const size_t r0 = (size_t)b * N;
     const int i0 = qb * 32;
@@ -327,8 +333,8 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
     const int nkb = nk >> 5;
     const int nitems = wave < nkb ? ((nkb - wave + 3) >> 2) * NCB : 0;
     auto b_item = [&](int q) {
-        const int qq = nitems ? min(q, nitems - 1) : 0;
-        const int jb = nitems ? wave + 4 * (qq / NCB) : 0, c = qq % NCB;
+        const int qq = nitems ? min(q, nitems - 1) : 0, nq = max(nitems / NCB, 1);
+        const int jb = nitems ? wave + 4 * (HALVES ? qq % nq : qq / NCB) : 0, c = HALVES ? qq / nq : qq % NCB;
         return a.BT + ((((size_t)b * a.Hkv + hk) * (HD / 4) + c * (CB / 4) + hh * (CB / 8)) * ldt + min(jb * 32 + l31, N - 1)) * 4;
     };
     BTile<CB> bt0, bt1;
@@ -337,7 +343,7 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
     if constexpr (BWD && M32 <= 8) load_probs<M32>(p_early, a, N, i0, b, h, tid);
     // DKV: this lane's q values for the shares formed at the end (query rows 16 u + 8 hh + e of the block, head column
     // dt * 32 + l31 for the wave's blocks dt = wave, wave + 4): requested now, used last
-    constexpr int NDT = DKV ? (HD + 127) / 128 : 1;
+    constexpr int NDT = DKV ? (HD + 127) / 128 / CS : 1;
     float q_early[NDT][2][8];
     if constexpr (BWD && DKV) {
 #pragma unroll
@@ -346,17 +352,17 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
             for (int u = 0; u < 2; u++)
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    const int i = i0 + 16 * u + 8 * hh + e, d = min((wave + 4 * t) * 32, HD - 32) + l31;
+                    const int i = i0 + 16 * u + 8 * hh + e, d = min((dt0 + 4 * t) * 32, HD - 32) + l31;
                     q_early[t][u][e] = a.q[(r0 + min(i, N - 1)) * qd + h * HD + d];
                 }
     }
     CRing cring;
     const float *c_lane0 = a.C + r0 * kd + hk * HD + l31;
-    c_ring_start<M32>(cring, c_lane0 + (wave * 32 < HD ? wave * 32 : 0), (size_t)kd, nk, hh, N);
+    c_ring_start<M32>(cring, c_lane0 + (dt0 * 32 < HD ? dt0 * 32 : 0), (size_t)kd, nk, hh, N);
 
     // ---- A rows into LDS (rows past the sequence as zeros); the loads of all HD / 32 rounds are issued together
+    float4 av[HD / 32];
     {
-        float4 av[HD / 32];
         if (BWD) {
             size_t rows[HD / 32]; int cols[HD / 32]; bool ok[HD / 32];
 #pragma unroll
@@ -375,18 +381,23 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
                 if (i0 + rr < N) av[u] = ld4(a.A + (r0 + i0 + rr) * qd + h * HD + 4 * c4);
             }
         }
+    }
+    auto stage = [&](int half) __attribute__((always_inline)) {       // HALVES: a thread's columns all lie in one of the two
 #pragma unroll
         for (int u = 0; u < HD / 32; u++) {
             const int idx = tid + 256 * u, rr = idx / (HD >> 2), c4 = idx % (HD >> 2);
-            if (BWD && !DKV && i0 + rr < N) st4(a.A_out + (r0 + i0 + rr) * qd + h * HD + 4 * c4, av[u]);
-            *reinterpret_cast<u32x2 *>(Ahi + rr * lda + 4 * c4) = u32x2{pack_hi(av[u].x, av[u].y), pack_hi(av[u].z, av[u].w)};
-            *reinterpret_cast<u32x2 *>(Alo + rr * lda + 4 * c4) = u32x2{pack_hi(rest(av[u].x), rest(av[u].y)), pack_hi(rest(av[u].z), rest(av[u].w))};
+            if (BWD && !DKV && half == 0 && share == 0 && i0 + rr < N) st4(a.A_out + (r0 + i0 + rr) * qd + h * HD + 4 * c4, av[u]);
+            if (HALVES && c4 / (HD >> 3) != half) continue;
+            const int at = rr * lda + 4 * (HALVES ? c4 % (HD >> 3) : c4);
+            *reinterpret_cast<u32x2 *>(Ahi + at) = u32x2{pack_hi(av[u].x, av[u].y), pack_hi(av[u].z, av[u].w)};
+            *reinterpret_cast<u32x2 *>(Alo + at) = u32x2{pack_hi(rest(av[u].x), rest(av[u].y)), pack_hi(rest(av[u].z), rest(av[u].w))};
         }
-    }
+    };
+    stage(0);
     __syncthreads();
     // a head of 256 columns at up to 64 keys: the C values of the wave's second column block are asked for now and
     // arrive during phase 1 and the row step (at the start of the kernel they would not fit among a wave's 63 loads in flight)
-    constexpr bool RING2 = HD > 128 && M32 == 2;
+    constexpr bool RING2 = HD > 128 && M32 == 2 && CS == 1;
     CRing cring2;
     if constexpr (RING2) c_ring_start<M32>(cring2, c_lane0 + (wave + 4) * 32, (size_t)kd, nk, hh, N);
 
@@ -395,7 +406,28 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
 #pragma unroll
         for (int v = 0; v < 16; v++) Xs[(8 * (v >> 2) + 4 * hh + (v & 3)) * ldx + jb * 32 + l31] = acc[v];
     };
-    {
+    if constexpr (HALVES) {
+        const int nq = nitems / NCB;
+        for (int c = 0; c < NCB; c++) {
+            if (c) { __syncthreads(); stage(c); __syncthreads(); }
+            auto run = [&](int q, const BTile<CB> &bt) __attribute__((always_inline)) {
+                Acc2 acc{zero16(), zero16()};
+                tile_abt<CB>(acc, Ahi, Alo, lda, 0, lane, bt);
+                float16v x = acc.a + acc.b;
+                const int jb = wave + 4 * q;
+                if (c)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) x[v] += Xs[(8 * (v >> 2) + 4 * hh + (v & 3)) * ldx + jb * 32 + l31];   // (the lane's own)
+                put_x(x, jb);
+            };
+            for (int q = 0; q < nq; q += 2) {              // (the tile behind a pass's last one is the next pass's first)
+                b_tile_load<CB>(bt1, b_item(c * nq + q + 1), ldt);
+                run(q, bt0);
+                b_tile_load<CB>(bt0, b_item(c * nq + min(q + 2, nq)), ldt);
+                if (q + 1 < nq) run(q + 1, bt1);
+            }
+        }
+    } else {
         Acc2 acc{zero16(), zero16()};
         auto run = [&](int q, const BTile<CB> &bt) __attribute__((always_inline)) {
             const int jb = wave + 4 * (q / NCB), c = q % NCB;
@@ -423,7 +455,7 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
     __syncthreads();
 
     // ---- row step
-    row_step<BWD, M32, DKV>(a, Xs, ldx, N32, nk, N, i0, b, h, tid, p_early, Ts);    // whole rows of N entries are written
+    row_step<BWD, M32, DKV>(a, Xs, ldx, N32, nk, N, i0, b, h, tid, p_early, Ts, share == 0);    // whole rows of N entries are written
     __syncthreads();
 
     // ---- phase 3: Y = X C, one 32-column block of the head per wave and round
@@ -442,8 +474,8 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
         put_y(tile_xc_2(reinterpret_cast<const __bf16 *>(Xs), 2 * ldx, N32, nk, lane, cring), wave);
         put_y(tile_xc_2(reinterpret_cast<const __bf16 *>(Xs), 2 * ldx, N32, nk, lane, cring2), wave + 4);
     } else {
-        for (int dt = wave; dt * 32 < HD; dt += 4) {
-            if (dt != wave) c_ring_start<M32>(cring, c_lane0 + dt * 32, (size_t)kd, nk, hh, N);
+        for (int dt = dt0; dt < dt_end; dt += 4) {
+            if (dt != dt0) c_ring_start<M32>(cring, c_lane0 + dt * 32, (size_t)kd, nk, hh, N);
             float16v acc;
             if constexpr (M32 == 2) acc = tile_xc_2(reinterpret_cast<const __bf16 *>(Xs), 2 * ldx, N32, nk, lane, cring);
             else acc = tile_xc(reinterpret_cast<const __bf16 *>(Xs), 2 * ldx, N32, nk, c_lane0 + dt * 32, (size_t)kd, N, lane, cring);
@@ -459,7 +491,7 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
         const int img = N32 * DKV_TS;
 #pragma unroll
         for (int t = 0; t < NDT; t++) {
-            const int dt = wave + 4 * t;
+            const int dt = dt0 + 4 * t;
             if (dt * 32 >= HD) break;
             const int d = dt * 32 + l31;
             HL qB[2], oB[2];
@@ -497,7 +529,7 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
             }
         }
     }
-    if (!BWD && h == a.Hq - 1)                             // zero the K padding of the operand rows once
+    if (!BWD && h == a.Hq - 1 && share == 0)               // zero the K padding of the operand rows once
         for (int idx = tid; idx < 32 * (Kb * 64 - qd); idx += 256) {
             const int rr = idx / (Kb * 64 - qd), c = qd + idx % (Kb * 64 - qd);
             if (i0 + rr < N) a.out16[tiled_a_index((int)(r0 + i0 + rr), c, Kb)] = (half_t)0;
@@ -572,18 +604,25 @@ __global__ __launch_bounds__(256) void k_attn_dkv_tile(AttnDkvArgs a)
 size_t tile_lds_bytes(int hd, int seq, int dkv = 0)
 {
     const size_t n32 = (seq + 31) & ~31;
+    if (hd == 256 && seq > 512) hd = 128;                  // (k_attn_tile: HALVES)
     return (size_t)32 * (hd + 8 + n32 + 4) * sizeof(float) + (dkv ? 4 * n32 * DKV_TS * sizeof(uint16_t) : 0);
 }
 
-template <int BWD, int HD, int M32, int DKV = 0>
+template <int BWD, int HD, int M32, int DKV = 0, int CS = 1>
 void launch_tile_m(const AttnTileArgs &a)
 {
+    if constexpr (HD == 256 && CS == 1) {
+        // few blocks leave most CUs idle: a second workgroup for each takes half of the columns behind the rows off it.  Four heads, forward
+        // / backward: 1 x 64 (8 blocks) 10.2 / 20.5 -> 8.0 / 16.5 us, 1 x 200 20.7 / 23.0 -> 17.2 / 18.9, 4 x 160 (80) 20.3 / 25.2 -> 16.4 / 22.1;
+        // beyond 128 blocks two workgroups would share a CU and form the scores twice for nothing
+        if ((long)((a.seq + 31) / 32) * a.Hq * a.batch <= 128) { launch_tile_m<BWD, HD, M32, DKV, 2>(a); return; }
+    }
     static bool attr_set = false;
-    if (!attr_set) { HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_attn_tile<BWD, HD, M32, DKV>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024)); attr_set = true; }
+    if (!attr_set) { HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_attn_tile<BWD, HD, M32, DKV, CS>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024)); attr_set = true; }
     const size_t lds = tile_lds_bytes(HD, a.seq, DKV);
-    const int per_z = ((a.seq + 31) / 32) * a.Hq;
+    const int per_z = ((a.seq + 31) / 32) * a.Hq * CS;
     const int extra = a.pf.base ? a.pf.wgs / per_z : 0;   // the planner made pf.wgs a multiple of per_z
-    LAUNCH((k_attn_tile<BWD, HD, M32, DKV>), dim3((a.seq + 31) / 32, a.Hq, a.batch + extra), dim3(256), lds, a);
+    LAUNCH((k_attn_tile<BWD, HD, M32, DKV, CS>), dim3((a.seq + 31) / 32, a.Hq * CS, a.batch + extra), dim3(256), lds, a);
 }
 
 template <int BWD, int HD>

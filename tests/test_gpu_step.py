@@ -524,3 +524,21 @@ def test_adapter_gradients_over_rows_and_columns_that_fill_no_tile(batch, seq):
         for L, (gv, rv) in enumerate(zip(lora_views(cfg, st.lora_grads()), lora_views(cfg, r["grad"]))):
             for k in ("A_q", "B_q", "A_v", "B_v"):
                 assert rel(gv[k], rv[k]) < 1e-2, (L, k, rel(gv[k], rv[k]))
+
+
+@pytest.mark.parametrize("batch,seq,heads,window", [(1, 70, 2, 0), (1, 300, 2, 0), (2, 420, 6, 0), (1, 513, 2, 0), (1, 650, 2, 200), (3, 530, 4, 0), (1, 1000, 2, 0),
+                                                    (1, 1024, 1, 0)])
+def test_heads_of_256_over_every_length_of_the_score_rows(batch, seq, heads, window):
+    """Two workgroups per block of 32 queries, each with half of the head's columns, up to 128 blocks and one beyond ((2, 420, 6) and
+    (3, 530, 4)); more than 512 keys with half of the operand's columns in LDS at a time.  The bar is that of the steps above."""
+    cfg = C1.with_(name="hd256", NL=1, D=64, Hq=heads, Hkv=1, hd=256, IS=96, V=256, batch=batch, seq=seq, window=window)
+    model = make_model(cfg, seed=21, gamma_jitter=0.1)
+    tok, tgt = make_batch(cfg, seed=30)
+    r = run_oracle(cfg, model, [(tok, tgt)], 1e-4)[0]
+    with SFTState(cfg, model) as st:
+        loss = st.train_step(tok, tgt, 1e-4)
+        assert abs(loss - r["loss"]) <= 1e-3 * abs(r["loss"]), (loss, r["loss"])
+        assert rel(st.logits(), r["logits"]) < 1e-2
+        for gv, rv in zip(lora_views(cfg, st.lora_grads()), lora_views(cfg, r["grad"])):
+            for k in ("A_q", "B_q", "A_v", "B_v"):
+                assert rel(gv[k], rv[k]) < 1e-2, (k, rel(gv[k], rv[k]))
