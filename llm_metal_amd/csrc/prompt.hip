@@ -265,6 +265,78 @@ __global__ __launch_bounds__(TB, HD <= 128 ? 2 : 1) void k_prompt_attn(const flo
         }
 }
 
+// The same for short contexts: one (token, query head) per wave, all in registers.  Sixteen lanes take a key, four columns each and 64
+// apart, so four keys are read side by side, four such groups requested together; a score is a sum over sixteen lanes, a row of up to
+// 64 scores sixteen registers, and the four lane groups' shares of the output meet at the end.  Up to 64 keys the tiles above are one
+// or two, each the whole chain of HD matrix instructions of 64 cycles in one wave while others idle.  32 heads of 128 over 8 at 8 / 32 / 64
+// tokens: 12.5 / 12.3 / 13.0 us, 4.0 / 4.9 / 7.6 so; 4 heads of 256 over one 21 / 21 / 22, 4.8 / 6.7 / 9.2.  The reads grow with the square
+// of the tokens: 32 heads break even at some 100, so the line is at the sixteen registers.
+constexpr int SHORT_KEYS = 64;
+template <int HD>
+__global__ __launch_bounds__(TB) void k_prompt_attn_short(const float *__restrict__ Q, const float *__restrict__ Kc, const float *__restrict__ Vc,
+                                                          float *__restrict__ out, int M, int pos, int Hq, int G, int max_seq, float scale)
+{
+    constexpr int C = HD / 64, NI = SHORT_KEYS / 4;
+    const int lane = threadIdx.x & 63, id = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (id >= M * Hq) return;
+    const int m = id / Hq, head = id % Hq, qpos = pos + m, g = lane >> 4, c = 4 * (lane & 15);
+    const float *Kh = Kc + (size_t)(head / G) * max_seq * HD, *Vh = Vc + (size_t)(head / G) * max_seq * HD, *q = Q + (size_t)id * HD;
+    float4v qv[C];
+#pragma unroll
+    for (int i = 0; i < C; i++) qv[i] = *reinterpret_cast<const float4v *>(q + c + 64 * i);
+    auto row = [&](const float *X, int it, float4v (&r)[C]) __attribute__((always_inline)) {       // (keys behind the query's repeat its own)
+        const float *at = X + (uint32_t)(min(4 * it + g, qpos) * HD + c);
+#pragma unroll
+        for (int i = 0; i < C; i++) r[i] = *reinterpret_cast<const float4v *>(at + 64 * i);
+    };
+    float s[NI], mx = -3.0e38f;
+#pragma unroll
+    for (int i0 = 0; i0 < NI; i0 += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[i0 + u] = -INFINITY;
+        if (4 * i0 > qpos) continue;                       // (uniform)
+        float4v k[4][C];
+#pragma unroll
+        for (int u = 0; u < 4; u++) row(Kh, i0 + u, k[u]);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            float d = 0.f;
+#pragma unroll
+            for (int i = 0; i < C; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) d = fmaf(qv[i][e], k[u][i][e], d);
+            d = xor_add<8>(xor_add<4>(xor_add<2>(xor_add<1>(d)))) * scale;
+            if (4 * (i0 + u) + g <= qpos) { s[i0 + u] = d; mx = fmaxf(mx, d); }
+        }
+    }
+    mx = xor_max<32>(xor_max<16>(mx));
+    float l = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; i++) { s[i] = expf(s[i] - mx); l += s[i]; }
+    l = xor_add<32>(xor_add<16>(l));
+    float4v o[C] = {};
+#pragma unroll
+    for (int i0 = 0; i0 < NI; i0 += 4) {
+        if (4 * i0 > qpos) continue;
+        float4v v[4][C];
+#pragma unroll
+        for (int u = 0; u < 4; u++) row(Vh, i0 + u, v[u]);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (4 * (i0 + u) + g <= qpos)
+#pragma unroll
+                for (int i = 0; i < C; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[i][e] = fmaf(s[i0 + u], v[u][i][e], o[i][e]);
+    }
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[i][e] = xor_add<32>(xor_add<16>(o[i][e])) / l;
+        if (g == i % 4) *reinterpret_cast<float4v *>(out + (size_t)id * HD + c + 64 * i) = o[i];
+    }
+}
+
 // One workgroup per token, the gated row in registers (C chunks of four columns per thread): the planes are read once and the
 // next product's operand leaves as two fp16 rows, where a gate kernel and a split kernel wrote and read the fp32 row between them.
 // 500 rows of 9728: 20.7 us.  (A few rows leave most CUs without one: at eight, 11.8 us against 9.2 for the two kernels, which a
@@ -351,6 +423,12 @@ void launch_prompt_attention(const float *q, const float *kc, const float *vc, f
     const int G = Hq / Hkv;
     const dim3 grid((M * G + 31) / 32, Hkv);
     const float scale = 1.0f / sqrtf((float)hd);
+    if (pos + M <= SHORT_KEYS && (hd == 128 || hd == 256) && ((uintptr_t)vc & 15) == 0) {
+        const dim3 waves((M * Hq + 3) / 4);
+        if (hd == 128) hipLaunchKernelGGL(k_prompt_attn_short<128>, waves, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale);
+        else hipLaunchKernelGGL(k_prompt_attn_short<256>, waves, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale);
+        return;
+    }
 #define PA(HD_) hipLaunchKernelGGL(k_prompt_attn<HD_>, grid, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale)
     if (hd == 32) PA(32); else if (hd == 64) PA(64); else if (hd == 128) PA(128); else if (hd == 256) PA(256);
     else { fprintf(stderr, "[fast_hip] prompt_attention: unsupported head size %d\n", hd); abort(); }
