@@ -71,6 +71,7 @@ struct NormIn {
     int dim;                             // layer norm and norms around: entries of xr that count
     const float *g_br, *b_br;            // norms around: RMS norm weight and bias (may be null) of br
 };
+constexpr int NORMED_COLS = 2560;        // widest vector that the products below norm in every wave (k_matvec_normed)
 // infer_kernels.hip: y = W . RMSNorm(xr + br; g) (glu 0), or the gated pair product of matvec_glu over it (1 SiLU, 2 GELU)
 void matvec_norm(MetalBuf *W, const NormIn &nin, MetalBuf *y, int rows, int cols, int q8, int glu);
 // infer_kernels.hip: y = W . LayerNorm(x; g) over the first dim of cols entries (F16 rows)

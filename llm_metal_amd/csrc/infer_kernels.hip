@@ -662,11 +662,11 @@ void launch_matvec_glu(const void *W, const half_t *scales, const float *x, floa
 #undef GLU_LAUNCH
 }
 
-// k_matvec_normed takes vectors of up to 2560 columns (the vector and two stages of weights in registers; k_matvec those beyond).  Every
+// k_matvec_normed takes vectors of up to NORMED_COLS = 2560 columns (the vector and two stages of weights in registers; k_matvec those beyond).  Every
 // wave is resident: two workgroups per CU, or one where a unit's two rows have more than 1536 columns -- fewer waves then keep
 // memory busy, and 256 workgroups fill the CUs evenly (one / two per CU: 6144 x 2560 F16 7.9 / 9.0 us, Q8_0 6.2 / 7.8, 9728 pairs F16 18.1 / 18.5;
-// 6912 pairs of 1152 F16 10.0 / 9.6, Q8_0 9.3 / 8.8).
-constexpr int NORMED_COLS = 2560;
+// 6912 pairs of 1152 F16 10.0 / 9.6, Q8_0 9.3 / 8.8).  The head, against k_matvec behind a launch for its norm:
+// 262 144 Q8_0 rows of 1152 3.4 + 77 -> 64 us (5.0 TB/s), 32 768 F16 rows of 2560 4.7 + 26 -> 27.
 template <int FMT, int NORM>
 void launch_matvec_normed(const void *W, const half_t *scales, const NormIn &nin, float *y, int rows, int cols, int act, hipEvent_t ev_a, hipEvent_t ev_b)
 {
@@ -695,8 +695,8 @@ void launch_matvec_norm(const void *W, const half_t *scales, const NormIn &nin, 
     if (prof) hipExtLaunchKernelGGL((k_matvec<FMT, 2, 2, 1, G_, 1, REPS_>), grid, dim3(TB), lds, stream(), ev_a, ev_b, 0, W, scales, nullptr, y, rows, cols, nin); \
     else hipLaunchKernelGGL((k_matvec<FMT, 2, 2, 1, G_, 1, REPS_>), grid, dim3(TB), lds, stream(), W, scales, nullptr, y, rows, cols, nin); \
     HIP_CHECK(hipGetLastError()); } while (0)
-    // measured at 9728 x 2560 pairs and 6144 x 2560 rows: two row groups per wave for the pairs (2432 workgroups forming
-    // the vector cost what the norm's own launch did), one for the rows (384 workgroups leave CUs idle)
+    // beyond NORMED_COLS: two row groups per wave for the pairs (thousands of workgroups each forming the vector cost what the
+    // norm's own launch did), one for the rows (a few hundred workgroups leave CUs idle)
     if (glu == 0) NORM_LAUNCH(0, 8, 1); else if (glu == 1) NORM_LAUNCH(1, 4, 2); else NORM_LAUNCH(2, 4, 2);
 #undef NORM_LAUNCH
 }

@@ -461,9 +461,12 @@ void forward_token(InferenceState *s, int token, int pos)
         pending = s->branch;
         pending_g = gemma ? lw.g_post_ff : nullptr;
     }
-    add_norm(s, x, pending, pending_g, s->g_final);
+    if (D <= NORMED_COLS) normed_product(s->lm_head->mbuf, pending, pending_g, s->g_final, s->logits, s->V, 0);
+    else {
+        add_norm(s, x, pending, pending_g, s->g_final);
+        matvec(s, s->lm_head, s->ln, s->logits);
+    }
     HIP_CHECK(hipGetLastError());
-    matvec(s, s->lm_head, s->ln, s->logits);
 }
 
 const float *logits_to_host(InferenceState *s)

@@ -488,6 +488,22 @@ def test_gemma_without_the_norm_behind_its_feed_forward(fmt):
             assert maxrel(np.stack([inf.step_batch([t, t], i)[1] for i, t in enumerate(toks)]), got) < 2e-5
 
 
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+@pytest.mark.parametrize("model_type", [0, 1], ids=["qwen3", "gemma3"])
+@pytest.mark.parametrize("D,V", [(128, 259), (160, 8195), (1536, 4097), (2560, 4099), (2592, 259)])
+def test_logits_of_an_odd_vocabulary_behind_the_last_norm(D, V, model_type, fmt):
+    """The head's rows in pairs: an odd one left over, one pair and several per wave; the last width takes the norm as a launch of
+    its own.  A few hundred fp32 roundings per row (2^-24 = 6e-8 each) over one layer, as the other comparisons here."""
+    say("odd vocabulary", D, V, model_type, fmt)
+    c = C1.with_(name="head", model_type=model_type, NL=1, seq=8, tied=True, D=D, Hq=2, Hkv=1, hd=32, IS=96, V=V, weight_format=fmt)
+    model = make_model(c, seed=43, gamma_jitter=0.1)
+    toks = [int(t) for t in np.random.default_rng(44).integers(1, V, 3)]
+    want = oracle_decode(c, model, fmt, toks, max_seq=8, precision="f64")
+    with InferenceState(c, model, max_seq=8, use_fp16=(fmt == "f16")) as inf:
+        got = np.stack([inf.forward_token(t) for t in toks])
+    assert maxrel(got, want) < 5e-4, maxrel(got, want)
+
+
 @pytest.mark.parametrize("c", [SFTConfig("q64", QWEN3, NL=1, D=128, Hq=8, Hkv=2, hd=64, IS=128, V=512),
                                SFTConfig("q128", QWEN3, NL=1, D=128, Hq=8, Hkv=2, hd=128, IS=128, V=512),
                                SFTConfig("g256", GEMMA3, NL=1, D=128, Hq=8, Hkv=2, hd=256, IS=128, V=512, tied=True)], ids=lambda c: c.name)
