@@ -597,6 +597,65 @@ __global__ __launch_bounds__(TB) void k_matvec_split(const void *__restrict__ Wp
     if (threadIdx.x == 0) y[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// Two rows per workgroup, their columns dealt to the four waves in 512-column steps, S of them each: all that a wave multiplies is requested
+// at once, and a part of the vector (twice a row's bytes of it, from L2) serves two rows.  With a wave per row the weights came in a chain
+// of up to five trips.  Cold weights, us, a wave per row -> so (with four and five rows): F16 2560 x 4096 4.9 -> 4.35 (4.6, 4.8),
+// 2560 x 9728 11.9 -> 11.1 = 4.5 TB/s (11.2, 10.9), 2048 x 8192 7.8 -> 7.8; Q8_0 2560 x 4096 and 2560 x 9728 16.9 -> 13.2 together,
+// 1152 x 1024 3.3 -> 2.9.  Eight steps in flight for the wave per row: 13.4 and 5.8.  Bound by the launch and one trip, then by memory.
+template <int FMT, int S>
+__global__ __launch_bounds__(TB) void k_matvec_rows(const void *__restrict__ Wp, const half_t *__restrict__ scales,
+                                                    const float *__restrict__ x, float *__restrict__ y, int rows, int cols)
+{
+    constexpr int R = 2;
+    __shared__ float red[4][R];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), row0 = blockIdx.x * R;
+    float4v xv[S][2];
+    half8 w16[R][S];
+    uint2v w8[R][S];
+    half_t d[R][S];
+    uint32_t at[S];                                          // (clamped: loads stay unconditional)
+#pragma unroll
+    for (int s = 0; s < S; s++) at[s] = min(512 * (4 * s + wave) + lane * 8, cols - 8);
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) xv[s][h] = *reinterpret_cast<const float4v *>(x + at[s] + 4 * h);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const size_t row = (size_t)min(row0 + r, rows - 1);
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            if (FMT == 0) w16[r][s] = __builtin_nontemporal_load(reinterpret_cast<const half8 *>((const half_t *)Wp + row * cols + at[s]));
+            else {
+                w8[r][s] = __builtin_nontemporal_load(reinterpret_cast<const uint2v *>((const int8_t *)Wp + row * cols + at[s]));
+                d[r][s] = (scales + row * (cols >> 5))[at[s] >> 5];
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        acc[r] = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            if (512 * (4 * s + wave) + lane * 8 >= cols) continue;
+            float p = FMT == 0 ? acc[r] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) p = fmaf(FMT == 0 ? (float)w16[r][s][e] : (float)(int8_t)(w8[r][s][e >> 2] >> (8 * (e & 3))), xv[s][e >> 2][e & 3], p);
+            acc[r] = FMT == 0 ? p : fmaf((float)d[r][s], p, acc[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float v = wave_sum(acc[r]);
+        if (lane == 0) red[wave][r] = v;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < R && row0 + t < rows) y[row0 + t] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+}
+
 // Any cols / alignment: one wave per row, lanes stride single elements.
 __global__ __launch_bounds__(TB) void k_matvec_any(const half_t *__restrict__ W, const float *__restrict__ X,
                                                    float *__restrict__ Y, int rows, int cols, int B)
@@ -618,7 +677,8 @@ __global__ __launch_bounds__(TB) void k_matvec_any(const half_t *__restrict__ W,
 // 2560 x 9728 11.5 / 13.9).
 constexpr int SPLIT_ROWS = 1536;
 constexpr size_t SPLIT_BYTES = (size_t)20 << 20;
-// Rows per wave grow with the matrix so that mid-sized weights (a few thousand rows) still put 16 waves on every CU.
+// Rows per wave grow with the matrix; below 8192 rows (and behind SPLIT_ROWS) a workgroup takes two, so that mid-sized weights still put
+// enough waves on every CU.
 template <int FMT>
 void launch_matvec(const void *W, const half_t *scales, const float *x, float *y, int rows, int cols)
 {
@@ -636,13 +696,24 @@ void launch_matvec(const void *W, const half_t *scales, const float *x, float *y
     if (prof) hipExtLaunchKernelGGL((k_matvec_split<FMT, U_>), dim3(rows), dim3(TB), 0, stream(), ev_a, ev_b, 0, W, scales, x, y, cols); \
     else hipLaunchKernelGGL((k_matvec_split<FMT, U_>), dim3(rows), dim3(TB), 0, stream(), W, scales, x, y, cols); \
     HIP_CHECK(hipGetLastError()); } while (0)
+#define ROWS_LAUNCH(S_) do { \
+    const dim3 grid((rows + 1) / 2); \
+    if (prof) hipExtLaunchKernelGGL((k_matvec_rows<FMT, S_>), grid, dim3(TB), 0, stream(), ev_a, ev_b, 0, W, scales, x, y, rows, cols); \
+    else hipLaunchKernelGGL((k_matvec_rows<FMT, S_>), grid, dim3(TB), 0, stream(), W, scales, x, y, rows, cols); \
+    HIP_CHECK(hipGetLastError()); } while (0)
     if (rows >= 32768 && lds <= 40 * 1024) MATVEC_LAUNCH(4, 2, 1, 16, lds);
     else if (rows >= 32768) MATVEC_LAUNCH(4, 2, 0, 16, 0);
     else if (rows >= 8192) MATVEC_LAUNCH(2, 2, 0, 8, 0);
     else if (rows <= SPLIT_ROWS && cols >= 4096 && (size_t)rows * cols * (FMT == 0 ? 2 : 1) <= SPLIT_BYTES) {
         if (cols > 4096) SPLIT_LAUNCH(4); else SPLIT_LAUNCH(2);
     }
+    else if (cols > 512 && cols <= 5 * 2048) {               // what ROWS_LAUNCH holds in registers; a single step leaves it one wave
+        const int steps = (cols + 2047) / 2048;
+        if (steps == 1) ROWS_LAUNCH(1); else if (steps == 2) ROWS_LAUNCH(2); else if (steps == 3) ROWS_LAUNCH(3);
+        else if (steps == 4) ROWS_LAUNCH(4); else ROWS_LAUNCH(5);
+    }
     else MATVEC_LAUNCH(1, 4, 0, 4, 0);
+#undef ROWS_LAUNCH
 #undef SPLIT_LAUNCH
 #undef MATVEC_LAUNCH
 }

@@ -68,6 +68,33 @@ def test_matvec_with_a_row_per_workgroup(dev, rows, cols):
         assert maxrel(yb.read(F), ref) < 2e-5
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 520), (129, 512), (3, 1024), (2049, 2048), (2051, 2080), (1537, 4096), (8191, 544), (1539, 6176), (1601, 8192),
+                                       (2561, 9728), (5, 2056), (1539, 10240), (1541, 10272)])
+def test_matvec_with_two_rows_per_workgroup(dev, rows, cols):
+    """An odd row left over, a last 512-column step full, begun and missing for some waves, every count of steps and the widths on
+    either side of the range; within it the lanes past the row do not multiply its last weights, here infinite in one row, by zero."""
+    say("matvec, two rows per workgroup", rows, cols)
+    rng = np.random.default_rng(rows + cols)
+    W, x, ref = rnd(rng, rows, cols, scale=0.05).astype(np.float16), rnd(rng, cols), np.zeros(rows, F)
+    op("f32", "or_f16_batch_matvec", W.view(np.uint16), x, ref, rows, cols, 1)
+    V = W.copy()
+    V[rows // 2, cols - 1] = np.inf
+    for w in (W, V) if 512 < cols <= 10240 else (W,):
+        wb, xb, yb = dev.up(w), dev.up(x), dev.empty(rows * 4)
+        dev.L.metal_enqueue_f16_matvec(wb.h, xb.h, yb.h, rows, cols)
+        got = yb.read(F)
+        if w is V:
+            assert np.isinf(got[rows // 2]) and (got[rows // 2] > 0) == (x[-1] > 0)
+            got[rows // 2] = ref[rows // 2]
+        assert maxrel(got, ref) < 2e-5
+    if cols % 32 == 0:
+        blocks = oracle.q8_quantize(W.astype(F))
+        op("f32", "or_q8_matvec", blocks, x, ref, rows, cols // 32)
+        qb = dev.up(blocks)
+        dev.L.metal_enqueue_q8_matvec(qb.h, xb.h, yb.h, rows, cols // 32)
+        assert maxrel(yb.read(F), ref) < 2e-5
+
+
 @pytest.mark.parametrize("rows,cols,B", [(4112, 1024, 2), (300, 2560, 3), (4096, 512, 4), (515, 1152, 5), (4096, 256, 8),
                                          (1000, 512, 9), (2048, 640, 32), (64, 50, 3), (65536 * 32 + 7, 8, 2)])   # (more row blocks than a grid's second dimension holds)
 def test_f16_batch_matvec(dev, rows, cols, B):
