@@ -188,11 +188,11 @@ struct LoraGradArgs {
     const half_t *ln16; const float *ln_inv_scale;  // tiled [rows, D]
     int rows, D, qd, kd, R; float sc;
     float *grad;                  // arena: dA_q | dB_q | dA_v | dB_v per layer
-    float *sq_slots;              // one partial sum of squares per workgroup
+    float *sq_slots;              // a sum of squares per 64 gradients or columns of them; four in a row are a slot
     int layers;
     size_t st_dq, st_dv, st_t, st_dh, st_ln16, st_lninv, st_grad, st_slots;   // layer strides in elements
 };
-int  lora_grad_blocks(int D, int qd, int kd, int R);
+int  lora_grad_slots(int D, int qd, int kd, int R);   // sums of squares of a layer, a multiple of four
 void launch_lora_grads(const LoraGradArgs &a);
 
 struct GluArgs {
@@ -235,7 +235,7 @@ void launch_ce_rows(const CeArgs &a, int rows);
 
 struct AdamArgs {
     float *p, *g, *m, *v; size_t n;
-    const float *sq_slots; int n_slots;
+    const float *sq_slots; int n_slots;             // (n_slots: sums of squares, four to a slot)
     const float *hyper;           // device-visible: [0] lr, [1] 1-b1^t, [2] 1-b2^t, written by the host per step
     float b1, b2, eps, wd, max_norm;
     // fp16 shadows of A_q / A_v: rows a_row0.. of the tiled image wqkv ([*, D]) and columns a_row0.. of the

@@ -12,6 +12,7 @@
 #include "fused.h"
 #include "planes.h"
 #include "kargs.h"
+#include <type_traits>
 
 namespace lmhip {
 namespace {
@@ -781,10 +782,9 @@ __global__ __launch_bounds__(NT) void k_qkv_bwd_rows(QkvBwdArgs a)
 // ------------------------------------------------------------------ LoRA gradients
 // dB = sc * dY^T t, dA = dh^T ln1 (float_matmul_tn + scale, src/nn/fast_sft.c:948-952,
 // 962-966): one thread per gradient element, looping over the rows.  Each
-// workgroup also leaves the sum of squares of what it wrote (for the global norm).
+// wave also leaves the sum of squares of what it wrote (for the global norm).
 __global__ __launch_bounds__(TB) void k_lora_grads(LoraGradArgs a)
 {
-    __shared__ float sm[16];
     {                                                     // blockIdx.y = layer
         const size_t L = blockIdx.y;
         a.dq_f += L * a.st_dq; a.dv_f += L * a.st_dv; a.tq += L * a.st_t; a.tv += L * a.st_t; a.dh += L * a.st_dh;
@@ -820,121 +820,140 @@ __global__ __launch_bounds__(TB) void k_lora_grads(LoraGradArgs a)
         a.grad[idx] = s;
         gval = s;
     }
-    const float sq = block_sum_products(gval, gval, sm);
-    if (threadIdx.x == 0) a.sq_slots[blockIdx.x] = sq;
+    const float sq = wave_sum_products(gval, gval);
+    if ((threadIdx.x & 63) == 0) a.sq_slots[4 * blockIdx.x + (threadIdx.x >> 6)] = sq;
 }
 
-// The same for rank 16 on the matrix cores (v_mfma_f32_16x16x4_f32, fp32 throughout): a workgroup owns 64 columns of dY (or of
-// the input) and its NW waves take the rows four at a time in turn, so that a wave sums rows / NW rows and has eight groups of them
-// in flight; the waves' sums meet in LDS.  A lane holds four neighbouring columns of one row per load, which are four operands.
-// Bound by the bytes of dY and of the input: 36 layers of 2048 rows of the 4B shape 442 us (1.9 GB at 4.3 TB/s), of 64 rows 31.1; four
-// layers of 2000 rows of the Gemma3-1B shape 31.4 us, 26 of 64 rows 12.3.  With a thread for each column and all rows of it, a
-// row's factors read from LDS one by one: 863, 33.6, 570 (40 workgroups) and 24.1 us.
-// grid.x = lora_grad_blocks(), block 64 NW; qd and kd multiples of four (heads are).
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_lora_grads_r16(LoraGradArgs a)
+// The same for rank 16 on the matrix cores: a workgroup owns 64 columns of dY (or of the input), a wave half of them (or all of dA_q, or
+// of dA_v) and all rows, a step of U groups of four on its way while the one before is multiplied.  v_mfma_f32_16x16x4_f32 is four
+// fmaf, one row after the other (bit for bit, subnormal values too), so every sum runs over the rows in the order above and the
+// gradients are the same numbers however the columns are dealt: AdamW's first steps make whole steps of the last bits of gradients near
+// zero.  For that no sum is shared between waves.
+// Bound by the bytes of dY and of the input, short models under many rows by a chain's trips to memory: 36 layers of 2048 rows of the 4B shape
+// 495 us (1.9 GB at 3.8 TB/s), of 64 rows 25.0; four layers of 2000 rows of the Gemma3-1B shape 60, 26 of 64 rows 12.5.  A thread for each
+// column, a row's factors read from LDS one by one (the same sums): 863, 33.6, 570 (40 workgroups) and 24.1; rows dealt to up to sixteen
+// waves whose sums met in LDS (other sums): 442, 31.1, 31.4 and 12.3.
+// grid.x = lora_grad_slots(), block 128; qd and kd multiples of four (heads are), columns past the last are not written.
+__global__ __launch_bounds__(128) void k_lora_grads_r16(LoraGradArgs a)
 {
-    constexpr int R = 16, U = 8, H = NW / 2, OPEN = 4;
-    __shared__ float part[H * 32 * 64];
-    __shared__ float sm[16];
+    typedef float float2v __attribute__((ext_vector_type(2)));
+    constexpr int R = 16, LB = 20, LA = 65;               // LB, LA: floats per column of dB and per row of dA in LDS
+    __shared__ float part[2 * R * LA > 64 * LB ? 2 * R * LA : 64 * LB];
     {                                                     // blockIdx.y = layer
         const size_t L = blockIdx.y;
         a.dq_f += L * a.st_dq; a.dv_f += L * a.st_dv; a.tq += L * a.st_t; a.tv += L * a.st_t; a.dh += L * a.st_dh;
         a.ln16 += L * a.st_ln16; a.ln_inv_scale += L * a.st_lninv; a.grad += L * a.st_grad; a.sq_slots += L * a.st_slots;
     }
-    const int nbq = (a.qd + 63) / 64, nbv = (a.kd + 63) / 64;
-    const int bx = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, k = lane >> 4, col = lane & 15;
-    const int groups = (a.rows + 3) / 4;
+    const int nbq = 4 * ((a.qd + 255) / 256), nbv = 4 * ((a.kd + 255) / 256);
+    const int bx = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), k = lane >> 4, col = lane & 15;
+    const bool isB = bx < nbq + nbv, isv = isB ? bx >= nbq : wave;
+    const int c0 = (bx < nbq ? bx : isB ? bx - nbq : bx - nbq - nbv) * 64, W = !isB ? a.D : isv ? a.kd : a.qd;
+    if (c0 >= W) {                                        // (part of a slot of 256 columns)
+        if (tid == 0) a.sq_slots[bx] = 0.f;
+        return;
+    }
     const size_t nA = (size_t)R * a.D, nBq = (size_t)a.qd * R;
-    float sq = 0.f;
-    // acc: n accumulators, each four values of a lane; n * 256 sums of all waves end up in part, accumulator by accumulator
-    auto meet = [&](float4v *acc, int n) __attribute__((always_inline)) {
-        float *p = part + (size_t)(wave % H) * 32 * 64;
-        if (wave >= H)
-            for (int i = 0; i < n; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) p[(4 * i + e) * 64 + lane] = acc[i][e];
-        __syncthreads();
-        if (wave < H)
-            for (int i = 0; i < n; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) p[(4 * i + e) * 64 + lane] += acc[i][e];
-        __syncthreads();
-    };
-    auto total = [&](int at) __attribute__((always_inline)) {
-        float v = part[at];
-#pragma unroll
-        for (int w = 1; w < H; w++) v += part[(size_t)w * 32 * 64 + at];
-        return v;
-    };
-    if (bx < nbq + nbv) {                                 // dB_q, dB_v
-        const bool isv = bx >= nbq;
-        const int c0 = (isv ? bx - nbq : bx) * 64, W = isv ? a.kd : a.qd;
-        const int c = min(c0 + 4 * col, W - 4);           // (columns past the last are not written)
-        const float *dy = (isv ? a.dv_f : a.dq_f) + c, *t = (isv ? a.tv : a.tq) + col;
-        float4v acc[4] = {};
-        for (int g0 = wave; g0 < groups; g0 += U * NW) {
-            float4v y[U];
-            float f[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int i = min(4 * (g0 + u * NW) + k, a.rows - 1);
-                y[u] = *reinterpret_cast<const float4v *>(dy + (size_t)i * W);
-                f[u] = t[(size_t)i * R];
+    float sq = 0.f;                                       // a column's squares, lane by lane of wave 0
+    // load(stage, first row, whole), use(stage, first row, whole); whole: all rows of the step are there, and an address is scalar but for
+    // the lane's offset.  (No branch around a load in the loop: the wait behind it would be for all of them.)
+    auto walk = [&](auto rows_of_step, auto &s0, auto &s1, auto load, auto use) __attribute__((always_inline)) {
+        constexpr int S = decltype(rows_of_step)::value;
+        constexpr std::true_type whole{};
+        constexpr std::false_type ragged{};
+        int at = 0;
+        if (3 * S <= a.rows) {
+            load(s0, 0, whole);
+            for (; at + 3 * S <= a.rows; at += 2 * S) {
+                load(s1, at + S, whole);
+                __builtin_amdgcn_sched_barrier(0);
+                use(s0, at, whole);
+                load(s0, at + 2 * S, whole);
+                __builtin_amdgcn_sched_barrier(0);
+                use(s1, at + S, whole);
             }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool in = 4 * (g0 + u * NW) + k < a.rows;
-                const float fu = in ? f[u] : 0.f;
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? y[u][j] : 0.f, fu, acc[j], 0, 0, 0);
-            }
+        } else load(s0, 0, ragged);
+        for (;; at += 2 * S) {                            // up to two steps more
+            if (at + S < a.rows) load(s1, at + S, ragged);
+            use(s0, at, ragged);
+            if (at + S >= a.rows) break;
+            if (at + 2 * S < a.rows) load(s0, at + 2 * S, ragged);
+            use(s1, at + S, ragged);
+            if (at + 2 * S >= a.rows) break;
         }
-        meet(acc, 4);
+    };
+    if (isB) {                                            // dB_q, dB_v: columns 2 col and 2 col + 1 of the wave's 32
+        constexpr int U = 16;
+        struct Stage { float2v y[U]; float f[U]; } s0, s1;
+        const float *dy = isv ? a.dv_f : a.dq_f, *t = isv ? a.tv : a.tq;
+        const int c = min(c0 + 32 * wave + 2 * col, W - 2);
+        float4v acc[2] = {};
+        walk(std::integral_constant<int, 4 * U>{}, s0, s1, [&](Stage &s, int at, auto whole) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = whole ? k : min(k, a.rows - 1 - at - 4 * u), i0 = at + 4 * u;     // (row i0 + i; i may be negative)
+                s.y[u] = *reinterpret_cast<const float2v *>(dy + (size_t)i0 * W + (i * W + c));
+                s.f[u] = (t + (size_t)i0 * R)[i * R + col];
+            }
+        }, [&](const Stage &s, int at, auto whole) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool in = whole || at + 4 * u + k < a.rows;
+                const float f = in ? s.f[u] : 0.f;
+#pragma unroll
+                for (int i = 0; i < 2; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? s.y[u][i] : 0.f, f, acc[i], 0, 0, 0);
+            }
+        });
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) part[(32 * wave + 2 * (4 * k + e) + i) * LB + col] = acc[i][e] * a.sc;
+        __syncthreads();
         float *out = a.grad + (isv ? 2 * nA + nBq : nA) + (size_t)c0 * R;
-        for (int e = tid; e < 64 * R; e += 64 * NW) {     // element (column e / 16, r = e % 16): accumulator column % 4
-            const int cc = e >> 4, r = e & 15;
-            if (c0 + cc >= W) break;
-            const float v = total((4 * (cc & 3) + ((cc >> 2) & 3)) * 64 + ((cc >> 4) << 4) + r) * a.sc;
-            out[e] = v;
-            sq += v * v;
+        for (int at = tid; at < 16 * R; at += 128)
+            if (c0 + (at >> 2) < W) st4(out + 4 * at, ld4(part + (at >> 2) * LB + 4 * (at & 3)));
+        if (wave == 0 && c0 + lane < W) {
+#pragma unroll
+            for (int r = 0; r < R; r += 4) sq += sumsq4(ld4(part + lane * LB + r));
         }
-    } else {                                              // dA_q, dA_v
-        const int kb = bx - nbq - nbv, Kb = tiled_kb(a.D), d0 = kb * 64;
-        float4v acc[8] = {};                              // dA_q of the four columns, then dA_v
-        for (int g0 = wave; g0 < groups; g0 += OPEN * NW) {
-            half4 x[OPEN];
-            float f[OPEN], hq[OPEN], hv[OPEN];
+    } else {                                              // dA_q, dA_v: columns 4 col .. 4 col + 3
+        constexpr int U = 8;
+        struct Stage { half4 x[U]; float f[U], h[U]; } s0, s1;
+        const int Kb = tiled_kb(a.D), hc = (isv ? R : 0) + col;
+        float4v acc[4] = {};
+        walk(std::integral_constant<int, 4 * U>{}, s0, s1, [&](Stage &s, int at, auto whole) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < OPEN; u++) {
-                const int i = min(4 * (g0 + u * NW) + k, a.rows - 1);
-                x[u] = *reinterpret_cast<const half4 *>(a.ln16 + tiled_a_index(i, d0 + 4 * col, Kb));
-                f[u] = a.ln_inv_scale[i];
-                hq[u] = a.dh[(size_t)i * 2 * R + col];
-                hv[u] = a.dh[(size_t)i * 2 * R + R + col];
+            for (int u = 0; u < U; u++) {
+                const int i = whole ? k : min(k, a.rows - 1 - at - 4 * u), i0 = at + 4 * u;
+                // (at is a multiple of 32: the step's rows are one row block, row i0 + i its row 4 u + i)
+                s.x[u] = *reinterpret_cast<const half4 *>(a.ln16 + tiled_a_index(at, c0, Kb) + (uint32_t)tiled_a_index(4 * u + i, 4 * col, 1));
+                s.f[u] = (a.ln_inv_scale + i0)[i];
+                s.h[u] = (a.dh + (size_t)i0 * 2 * R)[i * 2 * R + hc];
             }
+        }, [&](const Stage &s, int at, auto whole) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < OPEN; u++) {
-                const bool in = 4 * (g0 + u * NW) + k < a.rows;
-                const float q = in ? hq[u] : 0.f, v = in ? hv[u] : 0.f;
+            for (int u = 0; u < U; u++) {
+                const bool in = whole || at + 4 * u + k < a.rows;
+                const float h = in ? s.h[u] : 0.f;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float xv = in ? h2f(x[u][j]) * f[u] : 0.f;
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, xv, acc[j], 0, 0, 0);
-                    acc[4 + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, xv, acc[4 + j], 0, 0, 0);
-                }
+                for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(h, in ? h2f(s.x[u][i]) * s.f[u] : 0.f, acc[i], 0, 0, 0);
             }
-        }
-        meet(acc, 8);
-        for (int e = tid; e < 2 * 64 * R; e += 64 * NW) { // element (q or v, r, column d0 + d)
-            const int isv = e >> 10, r = (e >> 6) & 15, d = e & 63;
-            if (d0 + d >= a.D) continue;
-            const float v = total((16 * isv + 4 * (d & 3) + (r & 3)) * 64 + ((r >> 2) << 4) + (d >> 2));
-            a.grad[(isv ? nA + nBq : 0) + (size_t)r * a.D + d0 + d] = v;
-            sq += v * v;
+        });
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) part[((isv ? R : 0) + 4 * k + e) * LA + 4 * col + i] = acc[i][e];
+        __syncthreads();
+        if (c0 + lane < W) {
+            float *out = a.grad + (isv ? nA + nBq : 0) + c0 + lane;
+#pragma unroll 4
+            for (int r = 0; r < R; r++) out[(size_t)r * a.D] = part[((isv ? R : 0) + r) * LA + lane];
+            if (wave == 0) {
+#pragma unroll
+                for (int r = 0; r < R; r++) sq += part[r * LA + lane] * part[r * LA + lane] + part[(R + r) * LA + lane] * part[(R + r) * LA + lane];
+            }
         }
     }
-    sq = block_sum(sq, sm);
+    sq = wave_sum(sq);
     if (tid == 0) a.sq_slots[bx] = sq;
 }
 
@@ -1426,15 +1445,18 @@ __global__ __launch_bounds__(256) void k_ce_rows8(CeArgs a, int rows)
 
 // ------------------------------------------------------------------ optimiser
 // clip_grad_norm + adamw_update, src/nn/fast_sft.c:1045-1107, in one pass over the
-// flat LoRA arena: the global norm comes from the per-workgroup sums of squares
-// (double accumulator, as the reference), gradients are rescaled in place when
+// flat LoRA arena: the global norm comes from the waves' sums of squares, four in a
+// row to a slot (double accumulator over the slots, as the reference), gradients are rescaled in place when
 // the norm exceeds max_norm, and the fp16 images of A_q / A_v inside the fused
 // QKV weight (and its transpose) are refreshed for the next step's GEMMs.
 __global__ __launch_bounds__(1024) void k_grad_norm(const float *__restrict__ slots, int n, float *out)
 {
     __shared__ double sd[16];
     double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += (double)slots[i];
+    for (int i = threadIdx.x; i < n / 4; i += blockDim.x) {
+        const float4 p = ld4(slots + 4 * (size_t)i);
+        s += (double)(((p.x + p.y) + p.z) + p.w);
+    }
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, WAVE);
     if ((threadIdx.x & 63) == 0) sd[threadIdx.x >> 6] = s;
     __syncthreads();
@@ -1586,20 +1608,18 @@ void launch_qkv_bwd(const QkvBwdArgs &a, int rows)
     }
 }
 
-int lora_grad_blocks(int D, int qd, int kd, int R)
+int lora_grad_slots(int D, int qd, int kd, int R)
 {
-    if (R == 16) return (qd + 63) / 64 + (kd + 63) / 64 + (D + 63) / 64;
+    if (R == 16) return 4 * ((qd + 255) / 256 + (kd + 255) / 256 + (D + 255) / 256);
     const size_t n = (size_t)2 * R * D + (size_t)qd * R + (size_t)kd * R;
-    return (int)((n + TB - 1) / TB);
+    return 4 * (int)((n + TB - 1) / TB);
 }
 
 void launch_lora_grads(const LoraGradArgs &a)
 {
-    const dim3 grid(lora_grad_blocks(a.D, a.qd, a.kd, a.R), a.layers > 0 ? a.layers : 1);
-    // (up to 64 rows four waves hold all of them in one round of loads)
-    if (a.R != 16) LAUNCH(k_lora_grads, grid, dim3(TB), 0, a);
-    else if (a.rows <= 64) LAUNCH(k_lora_grads_r16<4>, grid, dim3(256), 0, a);
-    else LAUNCH(k_lora_grads_r16<16>, grid, dim3(1024), 0, a);
+    const int slots = lora_grad_slots(a.D, a.qd, a.kd, a.R), layers = a.layers > 0 ? a.layers : 1;
+    if (a.R != 16) LAUNCH(k_lora_grads, dim3(slots / 4, layers), dim3(TB), 0, a);
+    else LAUNCH(k_lora_grads_r16, dim3(slots, layers), dim3(128), 0, a);
 }
 
 void launch_glu_fwd(const GluArgs &a, int rows)

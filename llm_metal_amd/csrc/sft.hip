@@ -869,7 +869,7 @@ SFTState *sft_state_create_from_ref(const SFTModelRef *m, int batch, int seq_len
     // ---- LoRA arena, gradients, optimiser state ----
     s->lsz = (size_t)2 * R * D + (size_t)qd * R + (size_t)kd * R;
     s->lora_n = s->lsz * NL;
-    s->slots_per_layer = R ? lora_grad_blocks(D, qd, kd, R) : 1;
+    s->slots_per_layer = R ? lora_grad_slots(D, qd, kd, R) : 1;
     s->lora = fbuf(s->lora_n ? s->lora_n : 1); s->lora_grad = fbuf(s->lora_n ? s->lora_n : 1);
     s->lora16 = hbuf(s->lora_n ? s->lora_n : 1);
     s->adam_m = fbuf(s->lora_n ? s->lora_n : 1); s->adam_v = fbuf(s->lora_n ? s->lora_n : 1);

@@ -542,3 +542,34 @@ def test_heads_of_256_over_every_length_of_the_score_rows(batch, seq, heads, win
         for gv, rv in zip(lora_views(cfg, st.lora_grads()), lora_views(cfg, r["grad"])):
             for k in ("A_q", "B_q", "A_v", "B_v"):
                 assert rel(gv[k], rv[k]) < 1e-2, (k, rel(gv[k], rv[k]))
+
+
+@pytest.mark.parametrize("batch,seq", [(1, 3), (1, 64), (1, 65), (3, 47), (2, 300)])
+def test_adapter_gradients_of_rank_16_are_summed_row_by_row(batch, seq):
+    """The matrix-core kernel of rank 16 adds the rows one after the other in fp32, as the kernel of the other ranks does: with two rows
+    of A and two columns of B zero, fourteen of its ranks are those of rank 14, bit for bit.  (A sum in parts is as good to a few
+    2^-24 of its size, but AdamW's first steps turn the sign of a gradient near zero into a whole step.)  A column of B has one
+    entry, 2^-6: the factors dY B of dA, which the two ranks' kernels sum in another order, are single products then."""
+    cfg = C1.with_(name="rank16", NL=1, D=100, Hq=3, Hkv=1, hd=36, IS=128, V=260, batch=batch, seq=seq, alpha=4.0)
+    small = cfg.with_(R=14, alpha=3.5)                                     # the same scaling
+    model = make_model(cfg, seed=21, gamma_jitter=0.1)
+    wide = lora_views(cfg, model["lora"])[0]
+    for k in ("B_q", "B_v"):
+        wide[k][:] = 0
+        wide[k][5 * np.arange(16) % len(wide[k]), np.arange(16)] = 2.0 ** -6
+    cut = {"A_q": wide["A_q"][:14], "B_q": wide["B_q"][:, :14], "A_v": wide["A_v"][:14], "B_v": wide["B_v"][:, :14]}
+    narrow = dict(model, lora=np.concatenate([np.ascontiguousarray(cut[k]).ravel() for k in ("A_q", "B_q", "A_v", "B_v")]))
+    for k in ("A_q", "A_v"):
+        wide[k][14:] = 0
+    for k in ("B_q", "B_v"):
+        wide[k][:, 14:] = 0
+    grads = []
+    for c, m in ((cfg, model), (small, narrow)):
+        with SFTState(c, m) as st:
+            st.train_step(*make_batch(c, seed=30), 0.0)
+            assert 0 < st.grad_norm() < 1                                  # not clipped: the gradients are as they were summed
+            grads.append(lora_views(c, st.lora_grads())[0])
+    for k in ("A_q", "B_q", "A_v", "B_v"):
+        a = grads[0][k][:14] if k[0] == "A" else grads[0][k][:, :14]
+        assert np.array_equal(a, grads[1][k]), (k, np.abs(a - grads[1][k]).max())
+        assert np.any(a)
