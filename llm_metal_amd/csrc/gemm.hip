@@ -317,18 +317,6 @@ static int ring_chunks(int n_tiles, int Kb, int K, int cus)
         const double score = eff - 0.05 * S * (K > 2560 ? 2560.0 / K : 1.0);
         if (score > best_score + 1e-9) { best_score = score; best = S; }
     }
-    // A few row tiles under a long K: the score, made of shares of the CUs, leaves them in one chunk, a chain of half a microsecond for
-    // every two K steps.  Cut where that takes 4 us off (a launch that only adds planes takes 3.5), a plane costing its consumer
-    // some 0.15 us: 256 x 4096 at 64 rows 19.0 us -> 4.8 in eleven chunks, 256 x 1536 9.0 -> 4.5 in six.
-    auto chain = [&](int S) { const int steps = (Kb + S - 1) / S; return 0.5 * ((steps + 1) / 2) + 0.15 * S; };
-    if (8L * n_tiles * best <= cus) {
-        int cut = best;
-        for (int S = best + 1; S <= 32 && S <= Kb && (long)n_tiles * S <= cus; S++) {
-            const int steps = (Kb + S - 1) / S;
-            if ((Kb + steps - 1) / steps == S && chain(S) < chain(cut) - 1e-9) cut = S;
-        }
-        if (chain(best) - chain(cut) >= 4.0) best = cut;
-    }
     return best;
 }
 

@@ -573,3 +573,26 @@ def test_adapter_gradients_of_rank_16_are_summed_row_by_row(batch, seq):
         a = grads[0][k][:14] if k[0] == "A" else grads[0][k][:, :14]
         assert np.array_equal(a, grads[1][k]), (k, np.abs(a - grads[1][k]).max())
         assert np.any(a)
+
+
+def test_products_that_leave_halves_round_their_sum_once():
+    """gate|up forward over K = 1536 with two row tiles: columns d and d + 768 of the operand are the same and those of the weights cancel
+    but for 2^-8, so the sum over any part of K is some 150 times the whole.  As one half it is off by 2^-12 (and the down
+    product's by as much, through the gate's slope and the norm: 2^-9 in all); as halves of parts it would be off by 150 times that."""
+    cfg = C1.with_(name="halves", NL=1, D=1536, Hq=2, Hkv=1, hd=32, IS=64, V=512, seq=64)
+    model = make_model(cfg, seed=71, gamma_jitter=0.1)
+    rng, h = np.random.default_rng(72), cfg.D // 2
+    model["token_emb"][:, h:] = model["token_emb"][:, :h]
+    model["wo"][0][:] = 0                                                  # the FFN's row is the embedding's
+    model["g_post_attn"][0][h:] = model["g_post_attn"][0][:h]
+    for k in ("wg", "wu"):
+        w = rng.standard_normal((cfg.IS, h)) * 9
+        model[k][0][:] = np.concatenate([w, rng.standard_normal(w.shape) * 9 / 256 - w], axis=1)
+    got = []
+    for on in (0, 1):
+        with SFTState(cfg, model) as st:
+            st.L.hip_gemm_half_planes(on)
+            st.train_step(*make_batch(cfg, seed=73), 0.0)
+            got.append(st.logits())
+            st.L.hip_gemm_half_planes(1)
+    assert 0 < rel(got[1], got[0]) < 2.0 ** -9, rel(got[1], got[0])
