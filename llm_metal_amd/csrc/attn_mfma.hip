@@ -296,16 +296,13 @@ __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int l
 // grid (query blocks of 32, Hq, batch), block 256; LDS: Ahi, Alo [32][HD+8] bf16, Xs[32][ldx] fp32 / bf16 pairs
 // M32: 32-key blocks a row can hold (2, 8, 16 or 32: sequences up to 64, 256, 512, 1024); a template parameter so
 // that the kernel's code is one straight run (the kernel runs once per workgroup, and what it skips it still fetches).
-// CS 2 (heads of 256): two workgroups per block form the same scores and rows and half of the head's columns each (launch_tile_hd).
+// CS 2 (heads of 256): two workgroups per block form the same scores and rows and half of the head's columns each (launch_tile_m).
 template <int BWD, int HD, int M32, int DKV = 0, int CS = 1>
 __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
 {
     static_assert(CS == 1 || HD == 256, "a wave has two column blocks to share");
     extern __shared__ float lds[];
-    // heads of 256 over more than 512 keys: the A rows are in LDS one half of their columns at a time, which leaves room for 1024 scores
-    // a row (the wave-per-query kernels, which sequences beyond 928 keys took before, need 380 + 641 + 344 us at 1000 positions of four heads)
-    constexpr bool HALVES = HD == 256 && M32 == 32;
-    constexpr int lda = (HALVES ? HD / 2 : HD) + 8;        // halves; rows 16-byte aligned and 4 banks apart: conflict-free 16-byte reads
+    constexpr int lda = HD + 8;                            // halves; rows 16-byte aligned and 4 banks apart: conflict-free 16-byte reads
     const int N = a.seq;
     if ((int)blockIdx.z >= a.batch) {
         const int per_z = gridDim.x * gridDim.y;
@@ -333,8 +330,8 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
     const int nkb = nk >> 5;
     const int nitems = wave < nkb ? ((nkb - wave + 3) >> 2) * NCB : 0;
     auto b_item = [&](int q) {
-        const int qq = nitems ? min(q, nitems - 1) : 0, nq = max(nitems / NCB, 1);
-        const int jb = nitems ? wave + 4 * (HALVES ? qq % nq : qq / NCB) : 0, c = HALVES ? qq / nq : qq % NCB;
+        const int qq = nitems ? min(q, nitems - 1) : 0;
+        const int jb = nitems ? wave + 4 * (qq / NCB) : 0, c = qq % NCB;
         return a.BT + ((((size_t)b * a.Hkv + hk) * (HD / 4) + c * (CB / 4) + hh * (CB / 8)) * ldt + min(jb * 32 + l31, N - 1)) * 4;
     };
     BTile<CB> bt0, bt1;
@@ -361,8 +358,8 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
     c_ring_start<M32>(cring, c_lane0 + (dt0 * 32 < HD ? dt0 * 32 : 0), (size_t)kd, nk, hh, N);
 
     // ---- A rows into LDS (rows past the sequence as zeros); the loads of all HD / 32 rounds are issued together
-    float4 av[HD / 32];
     {
+        float4 av[HD / 32];
         if (BWD) {
             size_t rows[HD / 32]; int cols[HD / 32]; bool ok[HD / 32];
 #pragma unroll
@@ -381,19 +378,14 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
                 if (i0 + rr < N) av[u] = ld4(a.A + (r0 + i0 + rr) * qd + h * HD + 4 * c4);
             }
         }
-    }
-    auto stage = [&](int half) __attribute__((always_inline)) {       // HALVES: a thread's columns all lie in one of the two
 #pragma unroll
         for (int u = 0; u < HD / 32; u++) {
             const int idx = tid + 256 * u, rr = idx / (HD >> 2), c4 = idx % (HD >> 2);
-            if (BWD && !DKV && half == 0 && share == 0 && i0 + rr < N) st4(a.A_out + (r0 + i0 + rr) * qd + h * HD + 4 * c4, av[u]);
-            if (HALVES && c4 / (HD >> 3) != half) continue;
-            const int at = rr * lda + 4 * (HALVES ? c4 % (HD >> 3) : c4);
-            *reinterpret_cast<u32x2 *>(Ahi + at) = u32x2{pack_hi(av[u].x, av[u].y), pack_hi(av[u].z, av[u].w)};
-            *reinterpret_cast<u32x2 *>(Alo + at) = u32x2{pack_hi(rest(av[u].x), rest(av[u].y)), pack_hi(rest(av[u].z), rest(av[u].w))};
+            if (BWD && !DKV && share == 0 && i0 + rr < N) st4(a.A_out + (r0 + i0 + rr) * qd + h * HD + 4 * c4, av[u]);
+            *reinterpret_cast<u32x2 *>(Ahi + rr * lda + 4 * c4) = u32x2{pack_hi(av[u].x, av[u].y), pack_hi(av[u].z, av[u].w)};
+            *reinterpret_cast<u32x2 *>(Alo + rr * lda + 4 * c4) = u32x2{pack_hi(rest(av[u].x), rest(av[u].y)), pack_hi(rest(av[u].z), rest(av[u].w))};
         }
-    };
-    stage(0);
+    }
     __syncthreads();
     // a head of 256 columns at up to 64 keys: the C values of the wave's second column block are asked for now and
     // arrive during phase 1 and the row step (at the start of the kernel they would not fit among a wave's 63 loads in flight)
@@ -406,28 +398,7 @@ __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
 #pragma unroll
         for (int v = 0; v < 16; v++) Xs[(8 * (v >> 2) + 4 * hh + (v & 3)) * ldx + jb * 32 + l31] = acc[v];
     };
-    if constexpr (HALVES) {
-        const int nq = nitems / NCB;
-        for (int c = 0; c < NCB; c++) {
-            if (c) { __syncthreads(); stage(c); __syncthreads(); }
-            auto run = [&](int q, const BTile<CB> &bt) __attribute__((always_inline)) {
-                Acc2 acc{zero16(), zero16()};
-                tile_abt<CB>(acc, Ahi, Alo, lda, 0, lane, bt);
-                float16v x = acc.a + acc.b;
-                const int jb = wave + 4 * q;
-                if (c)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) x[v] += Xs[(8 * (v >> 2) + 4 * hh + (v & 3)) * ldx + jb * 32 + l31];   // (the lane's own)
-                put_x(x, jb);
-            };
-            for (int q = 0; q < nq; q += 2) {              // (the tile behind a pass's last one is the next pass's first)
-                b_tile_load<CB>(bt1, b_item(c * nq + q + 1), ldt);
-                run(q, bt0);
-                b_tile_load<CB>(bt0, b_item(c * nq + min(q + 2, nq)), ldt);
-                if (q + 1 < nq) run(q + 1, bt1);
-            }
-        }
-    } else {
+    {
         Acc2 acc{zero16(), zero16()};
         auto run = [&](int q, const BTile<CB> &bt) __attribute__((always_inline)) {
             const int jb = wave + 4 * (q / NCB), c = q % NCB;
@@ -604,7 +575,6 @@ __global__ __launch_bounds__(256) void k_attn_dkv_tile(AttnDkvArgs a)
 size_t tile_lds_bytes(int hd, int seq, int dkv = 0)
 {
     const size_t n32 = (seq + 31) & ~31;
-    if (hd == 256 && seq > 512) hd = 128;                  // (k_attn_tile: HALVES)
     return (size_t)32 * (hd + 8 + n32 + 4) * sizeof(float) + (dkv ? 4 * n32 * DKV_TS * sizeof(uint16_t) : 0);
 }
 
@@ -657,6 +627,8 @@ bool attn_bwd_one_launch(int hd, int seq)
     return g_bwd_one_launch && attn_mfma_supported(hd, seq) && seq <= 64 && tile_lds_bytes(hd, seq, 1) <= 150 * 1024;
 }
 
+// (heads of 256 beyond 928 keys have no room for their rows of scores; with half of the operand's columns in LDS at a time they would, and
+// take a third of the time at 1000, but the kernels that they have are fp32 throughout, these work on bf16 pairs)
 bool attn_mfma_supported(int hd, int seq)
 {
     return (hd == 32 || hd == 64 || hd == 128 || hd == 256) && seq >= 1 && seq <= 1024 && tile_lds_bytes(hd, seq) <= 150 * 1024;

@@ -530,7 +530,7 @@ def test_adapter_gradients_over_rows_and_columns_that_fill_no_tile(batch, seq):
                                                     (1, 1024, 1, 0)])
 def test_heads_of_256_over_every_length_of_the_score_rows(batch, seq, heads, window):
     """Two workgroups per block of 32 queries, each with half of the head's columns, up to 128 blocks and one beyond ((2, 420, 6) and
-    (3, 530, 4)); more than 512 keys with half of the operand's columns in LDS at a time.  The bar is that of the steps above."""
+    (3, 530, 4)); beyond 928 keys the kernels without matrix cores.  The bar is that of the steps above."""
     cfg = C1.with_(name="hd256", NL=1, D=64, Hq=heads, Hkv=1, hd=256, IS=96, V=256, batch=batch, seq=seq, window=window)
     model = make_model(cfg, seed=21, gamma_jitter=0.1)
     tok, tgt = make_batch(cfg, seed=30)
@@ -596,3 +596,22 @@ def test_products_that_leave_halves_round_their_sum_once():
             got.append(st.logits())
             st.L.hip_gemm_half_planes(1)
     assert 0 < rel(got[1], got[0]) < 2.0 ** -9, rel(got[1], got[0])
+
+
+@pytest.mark.parametrize("batch,seq", [(1, 929), (2, 1000)])
+def test_long_rows_of_heads_of_256_are_summed_in_32_bits(batch, seq):
+    """Beyond 928 keys such heads take the wave-per-query kernels, fp32 throughout.  Three times q's norm weights and a third of k's are the
+    same scores but for a rounding of 2^-24 of every operand, 2^-19 of a probability where scores reach 32, and the four fp16
+    roundings behind the attention turn where that crosses one: sqrt(4 x 2^-19 x 2^-11) = 6e-5 of the result.  Operands in two bf16
+    parts are off by 2^-17, 2^-12 = 2.4e-4 of a probability, which the result shows as it is."""
+    cfg = C1.with_(name="hd256_long", NL=1, D=64, Hq=2, Hkv=1, hd=256, IS=96, V=256, batch=batch, seq=seq)
+    model = make_model(cfg, seed=21, gamma_jitter=0.1)
+    tok, tgt = make_batch(cfg, seed=30)
+    got = []
+    for f in (1, 3):
+        m = dict(model, g_q=[g * np.float32(4 * f) for g in model["g_q"]], g_k=[g * np.float32(4 / f) for g in model["g_k"]])
+        with SFTState(cfg, m) as st:
+            st.train_step(tok, tgt, 0.0)
+            got.append((st.logits(), st.lora_grads()))
+    assert rel(got[1][0], got[0][0]) < 1.2e-4, rel(got[1][0], got[0][0])
+    assert rel(got[1][1], got[0][1]) < 1.2e-4, rel(got[1][1], got[0][1])
