@@ -461,7 +461,8 @@ void forward_token(InferenceState *s, int token, int pos)
         pending = s->branch;
         pending_g = gemma ? lw.g_post_ff : nullptr;
     }
-    if (D <= NORMED_COLS) normed_product(s->lm_head->mbuf, pending, pending_g, s->g_final, s->logits, s->V, 0);
+    // (matvec_norm, which a branch without a norm of its own takes, wants whole blocks of 32 columns)
+    if (D <= NORMED_COLS && (D % 32 == 0 || pending_g)) normed_product(s->lm_head->mbuf, pending, pending_g, s->g_final, s->logits, s->V, 0);
     else {
         add_norm(s, x, pending, pending_g, s->g_final);
         matvec(s, s->lm_head, s->ln, s->logits);

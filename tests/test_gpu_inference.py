@@ -488,6 +488,23 @@ def test_gemma_without_the_norm_behind_its_feed_forward(fmt):
             assert maxrel(np.stack([inf.step_batch([t, t], i)[1] for i, t in enumerate(toks)]), got) < 2e-5
 
 
+@pytest.mark.parametrize("layers", [1, 2], ids=["one_layer", "adapters"])
+def test_widths_that_are_no_whole_blocks_without_the_norm_behind_the_feed_forward(layers):
+    """104 columns: a single layer, or several with adapters, whose first product takes its norm as a launch of its own; so does the
+    head there, its fused kernel behind a plain branch taking whole blocks of 32.  Against the batch's step (22 bits of an activation)."""
+    say("104 columns", layers)
+    c = TINY_GEMMA.with_(name="narrow", NL=layers, D=104, seq=8)
+    model = make_model(c, seed=62, gamma_jitter=0.1)
+    plain = dict(model, g_post_ff=[None] * c.NL)
+    toks = [3, 70, 11, 42, 7]
+    with SFTState(c, model) as st, InferenceState(c, plain, max_seq=8, use_fp16=True) as inf:
+        if layers > 1:
+            inf.attach_lora(st)
+        got = np.stack([inf.forward_token(t) for t in toks])
+        assert np.all(np.isfinite(got)) and np.any(got)
+        assert maxrel(np.stack([inf.step_batch([t, t], i)[1] for i, t in enumerate(toks)]), got) < 2e-5
+
+
 @pytest.mark.parametrize("fmt", ["f16", "q8_0"])
 @pytest.mark.parametrize("model_type", [0, 1], ids=["qwen3", "gemma3"])
 @pytest.mark.parametrize("D,V", [(128, 259), (160, 8195), (1536, 4097), (2560, 4099), (2592, 259)])
