@@ -59,9 +59,6 @@ size_t metal_buf_size(MetalBuf *b);
 void *hip_buf_device_ptr(MetalBuf *b);
 /* free and total bytes of the current device's memory (hipMemGetInfo): lets a caller see that a call allocated nothing */
 void hip_mem_info(size_t *free_bytes, size_t *total_bytes);
-// Pinned host memory, which the GPU writes and reads in place; NULL where there is none left.
-void *hip_host_alloc(size_t bytes);
-void hip_host_free(void *p);
 /* Non-owning window [offset, offset+size) of another buffer. */
 MetalBuf *metal_buf_view(MetalBuf *parent, size_t offset, size_t size);
 

@@ -133,15 +133,6 @@ size_t metal_buf_size(MetalBuf *b) { return b ? b->size : 0; }
 
 void *hip_buf_device_ptr(MetalBuf *b) { return b ? lmhip::dptr(b) : nullptr; }
 
-void *hip_host_alloc(size_t bytes)
-{
-    void *p = nullptr;
-    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    return p;
-}
-
-void hip_host_free(void *p) { if (p) (void)hipHostFree(p); }
-
 void hip_mem_info(size_t *free_bytes, size_t *total_bytes)
 {
     size_t f = 0, t = 0;

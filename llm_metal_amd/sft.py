@@ -2,7 +2,6 @@
 tests and bench.py: device buffers as thin handles, the SFT state as a class.
 Every method is one call into libllm_metal_hip.so."""
 import ctypes as C
-import threading
 
 import numpy as np
 
@@ -12,69 +11,6 @@ from .configs import SFTConfig
 
 def _vp(a):
     return a.ctypes.data_as(C.c_void_p)
-
-
-class _HostBlock:
-    """Pinned memory of a pool; back to it with the last array that looks at it."""
-
-    def __init__(self, pool, ptr, size):
-        self.pool, self.ptr, self.size = pool, ptr, size
-
-    def view(self, shape):
-        return np.asarray(_HostView(self, shape))
-
-    def __del__(self):
-        self.pool.give(self.ptr, self.size)
-
-
-class _HostView:
-    def __init__(self, block, shape):
-        self.block = block
-        self.__array_interface__ = {"shape": tuple(shape), "typestr": "<f4", "data": (block.ptr, False), "version": 3}
-
-
-class _HostPool:
-    """Arrays of a batch's logits, step after step, in pinned memory: the GPU writes them in place.  New pageable pages cost a fault each and a
-    copy through the runtime's staging: 32 sequences of a vocabulary of 16 384, 2 MB a step, 700 us of which the kernels 278;
-    eight of 32 768, 1 MB, 875 us of which 662.  At most `LIMIT` bytes at a time, idle ones among them; what goes beyond is ordinary
-    memory, as is what is too small for its pages to count.  Blocks that no array looks at are kept for the next ones of their
-    size and freed with the state; an array may outlive it."""
-    LIMIT, LEAST = 256 << 20, 64 << 10
-
-    def __init__(self, L):
-        self.L, self.lock, self.idle, self.held, self.open = L, threading.RLock(), {}, 0, True
-
-    def empty(self, shape):
-        size = 4 * int(np.prod(shape))
-        if size < self.LEAST:
-            return np.empty(shape, dtype=np.float32)
-        with self.lock:
-            ptr = self.idle[size].pop() if self.idle.get(size) else None
-            if ptr is None:
-                if self.held + size > self.LIMIT:
-                    self._drop_idle()
-                if self.open and self.held + size <= self.LIMIT:
-                    ptr = self.L.hip_host_alloc(size)
-                    self.held += size if ptr else 0
-        return _HostBlock(self, ptr, size).view(shape) if ptr else np.empty(shape, dtype=np.float32)
-
-    def give(self, ptr, size):
-        with self.lock:
-            self.idle.setdefault(size, []).append(ptr)
-            if not self.open:
-                self._drop_idle()
-
-    def _drop_idle(self):
-        idle, self.idle = self.idle, {}                    # (a collection in here may give more)
-        for size, ptrs in idle.items():
-            for p in ptrs:
-                self.L.hip_host_free(p)
-                self.held -= size
-
-    def close(self):
-        with self.lock:
-            self.open = False
-            self._drop_idle()
 
 
 class Backend:
@@ -326,7 +262,6 @@ class InferenceState:
         if not self.h:
             raise RuntimeError("inference state creation failed (no gfx950 device or unsupported dims)")
         self.V = self.L.inference_state_vocab_size(self.h)
-        self._host = _HostPool(self.L)
 
     def reset(self):
         self.L.inference_state_reset(self.h)
@@ -365,7 +300,7 @@ class InferenceState:
     def step_batch(self, tokens, pos, want_logits=True):
         """One lock-step step with a token per sequence at position `pos`; [batch, V] logits (None if not asked for)."""
         t = np.ascontiguousarray(tokens, dtype=np.int32)
-        out = self._host.empty((len(t), self.V)) if want_logits else None
+        out = np.empty((len(t), self.V), dtype=np.float32) if want_logits else None
         if self.L.inference_step_batch(self.h, _vp(t), len(t), int(pos), _vp(out) if want_logits else None) != 0:
             raise RuntimeError("inference_step_batch refused its arguments")
         return out
@@ -392,7 +327,6 @@ class InferenceState:
         if self.h:
             self.L.inference_state_free(self.h)
             self.h = None
-            self._host.close()
 
     def __enter__(self):
         return self

@@ -193,6 +193,27 @@ def test_batch_steps_over_shapes_that_fill_no_tile(kw, batches, model_type):
                 assert maxrel(got[b], single) < 1e-4, (B, b, maxrel(got[b], single))
 
 
+@pytest.mark.parametrize("V", [260, 40004], ids=["4_pages", "160_pages"])
+def test_logits_of_batch_steps_are_the_callers_own(V):
+    """Ordinary arrays, as numpy's own are: each owns its memory, may be resized, and keeps what it holds when further steps and the end
+    of the state pass; memory that ends in the middle of a page is written to its end and no further."""
+    say("logits of batch steps", V)
+    c = C1.with_(name="own", NL=1, seq=8, V=V, tied=True)
+    model = make_model(c, seed=45)
+    toks = np.random.default_rng(46).integers(1, V, (4, 3)).astype(np.int32)
+    with InferenceState(c, model, max_seq=8, use_fp16=True) as inf:
+        rows = [inf.step_batch(t, i) for i, t in enumerate(toks)]
+        was = [r.copy() for r in rows]
+        room = np.full(3 * V + 7, 5, np.float32)
+        assert inf.L.inference_step_batch(inf.h, toks[0].ctypes.data, 3, 0, room[3:].ctypes.data) == 0
+        assert np.array_equal(room[3:-4].reshape(3, V), was[0]) and np.all(room[:3] == 5) and np.all(room[-4:] == 5)
+        inf.step_batch(toks[1][:2], 0)                                     # another run, with staging of its own
+    for r, w in zip(rows, was):
+        assert r.flags.owndata and np.array_equal(r, w)
+        r.resize((4, V), refcheck=False)
+        assert np.array_equal(r[:3], w) and not r[3].any()
+
+
 # Qwen3-4B's widths (hidden 2560, 32 / 8 heads of 128, FFN 9728): the instantiations that `bench.py --decode` launches --
 # two weight rows per wave with the SiLU gate and the norm inside the launch at 19456 x 2560, the norm-fused Q|K|V
 # product at 6144 x 2560, the attention kernel with four-key steps, the fused per-head prologue and the O weights asked
