@@ -296,7 +296,7 @@ __device__ __forceinline__ void row_step(const AttnTileArgs &a, float *Xs, int l
 // grid (query blocks of 32, Hq, batch), block 256; LDS: Ahi, Alo [32][HD+8] bf16, Xs[32][ldx] fp32 / bf16 pairs
 // M32: 32-key blocks a row can hold (2, 8, 16 or 32: sequences up to 64, 256, 512, 1024); a template parameter so
 // that the kernel's code is one straight run (the kernel runs once per workgroup, and what it skips it still fetches).
-// CS 2 (heads of 256): two workgroups per block form the same scores and rows and half of the head's columns each (launch_tile_m).
+// CS 2 (heads of 256): two workgroups per block form the same scores and rows and half of the head's columns each (attn_column_shares).
 template <int BWD, int HD, int M32, int DKV = 0, int CS = 1>
 __global__ __launch_bounds__(256) void k_attn_tile(AttnTileArgs a)
 {
@@ -581,17 +581,13 @@ size_t tile_lds_bytes(int hd, int seq, int dkv = 0)
 template <int BWD, int HD, int M32, int DKV = 0, int CS = 1>
 void launch_tile_m(const AttnTileArgs &a)
 {
-    if constexpr (HD == 256 && CS == 1) {
-        // few blocks leave most CUs idle: a second workgroup for each takes half of the columns behind the rows off it.  Four heads, forward
-        // / backward: 1 x 64 (8 blocks) 10.2 / 20.5 -> 8.0 / 16.5 us, 1 x 200 20.7 / 23.0 -> 17.2 / 18.9, 4 x 160 (80) 20.3 / 25.2 -> 16.4 / 22.1;
-        // beyond 128 blocks two workgroups would share a CU and form the scores twice for nothing
-        if ((long)((a.seq + 31) / 32) * a.Hq * a.batch <= 128) { launch_tile_m<BWD, HD, M32, DKV, 2>(a); return; }
-    }
+    if constexpr (HD == 256 && CS == 1)
+        if (attn_column_shares(HD, a.seq, a.Hq, a.batch) == 2) { launch_tile_m<BWD, HD, M32, DKV, 2>(a); return; }
     static bool attr_set = false;
     if (!attr_set) { HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_attn_tile<BWD, HD, M32, DKV, CS>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024)); attr_set = true; }
     const size_t lds = tile_lds_bytes(HD, a.seq, DKV);
     const int per_z = ((a.seq + 31) / 32) * a.Hq * CS;
-    const int extra = a.pf.base ? a.pf.wgs / per_z : 0;   // the planner made pf.wgs a multiple of per_z
+    const int extra = a.pf.base ? a.pf.wgs / per_z : 0;   // the planner made pf.wgs a multiple of per_z (attn_column_shares)
     LAUNCH((k_attn_tile<BWD, HD, M32, DKV, CS>), dim3((a.seq + 31) / 32, a.Hq * CS, a.batch + extra), dim3(256), lds, a);
 }
 

@@ -128,6 +128,11 @@ void launch_attn_bwd(const AttnBwdArgs &a);
 // The same two operations on the fp32 matrix cores (attn_mfma.hip): head_dim a multiple of 32 and a
 // 32-row block of scores within the LDS budget; the wave-per-query kernels above remain the general path.
 bool attn_mfma_supported(int hd, int seq);
+// workgroups per (block of 32 queries, head, sequence) of the matrix-core kernels, each with its share of the head's columns.  Few blocks of
+// heads of 256 leave most CUs idle: a second workgroup for each takes half of the columns behind the rows off it.  Four heads, forward /
+// backward: 1 x 64 (8 blocks) 10.2 / 20.5 -> 8.0 / 16.5 us, 1 x 200 20.7 / 23.0 -> 17.2 / 18.9, 4 x 160 (80) 20.3 / 25.2 -> 16.4 / 22.1;
+// beyond 128 blocks two workgroups would share a CU and form the scores twice for nothing.
+inline int attn_column_shares(int hd, int seq, int Hq, int batch) { return hd == 256 && (long)((seq + 31) / 32) * Hq * batch <= 128 ? 2 : 1; }
 void launch_attn_fwd_mfma(const AttnFwdArgs &a);
 void launch_attn_bwd_mfma(const AttnBwdArgs &a);
 // dQ and the dK / dV shares in one launch (AttnBwdArgs::dkp): on by default wherever the matrix-core path runs on at

@@ -427,7 +427,7 @@ void forward_impl(SFTState *s, bool gather, bool zero_rows = false)
         aa.window = (s->window > 0 && s->layer_local[L]) ? s->window : 0;
         if (s->use_flash) {
         } else if (attn_mfma_supported(s->hd, s->N)) {
-            aa.pf = prefetch_for(s, wop(s, W_O, L, false), D, qd, 256, ((s->N + 31) / 32) * s->Hq);
+            aa.pf = prefetch_for(s, wop(s, W_O, L, false), D, qd, 256, ((s->N + 31) / 32) * s->Hq * attn_column_shares(s->hd, s->N, s->Hq, s->B));
             launch_attn_fwd_mfma(aa);
         } else launch_attn_fwd(aa);
         // full-parameter mode keeps the FFN GEMM operands of every layer as well

@@ -526,7 +526,7 @@ def test_adapter_gradients_over_rows_and_columns_that_fill_no_tile(batch, seq):
                 assert rel(gv[k], rv[k]) < 1e-2, (L, k, rel(gv[k], rv[k]))
 
 
-@pytest.mark.parametrize("batch,seq,heads,window", [(1, 70, 2, 0), (1, 300, 2, 0), (2, 420, 6, 0), (1, 513, 2, 0), (1, 650, 2, 200), (3, 530, 4, 0), (1, 1000, 2, 0),
+@pytest.mark.parametrize("batch,seq,heads,window", [(1, 64, 3, 0), (1, 70, 2, 0), (1, 300, 2, 0), (2, 420, 6, 0), (1, 513, 2, 0), (1, 650, 2, 200), (3, 530, 4, 0), (1, 1000, 2, 0),
                                                     (1, 1024, 1, 0)])
 def test_heads_of_256_over_every_length_of_the_score_rows(batch, seq, heads, window):
     """Two workgroups per block of 32 queries, each with half of the head's columns, up to 128 blocks and one beyond ((2, 420, 6) and
