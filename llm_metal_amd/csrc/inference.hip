@@ -1341,7 +1341,8 @@ SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const
 bool prompt_few(const InferenceState *s, int M) { return M <= FEW_ROWS && few_rows_fit(s); }
 
 // One step: the M tokens at positions pos .. pos + M - 1, their keys and values into kc and vc (the first sequence's part),
-// the final norm's rows into r.ln.  Per layer the launches of forward_token_batch, with the tokens as rows: ten, for a few rows eight.
+// the final norm's rows into r.ln.  Per layer the launches of forward_token_batch, with the tokens as rows: ten, for a few rows of
+// F16 weights eight (of Q8_0 ten: the rows ahead of O and of down are split by launches of their own).
 void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, std::vector<MetalBuf *> &vc, int M, int pos)
 {
     const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd, IS = s->IS, qd = Hq * hd, nqkv = qd + 2 * Hkv * hd;

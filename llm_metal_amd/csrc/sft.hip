@@ -522,8 +522,9 @@ void backward_impl(SFTState *s, int mode = BWD_LORA, float lr = 0.f)
     int cur = 0;                                          // dx ping-pong
     // Accumulate mode: each of a layer's four loss-gradient operands (of down, gate|up, o, qkv) has a buffer of its own,
     // so that all four weight gradients can be formed after the layer's last row kernel: one launch transposes their
-    // eight operands instead of four launches of two (the weights do not change before the apply, so the order of the
-    // reference's f16_grad_accum calls, src/nn/fast_sft.c:804-946, does not matter).  Otherwise one buffer serves all.
+    // eight operands instead of four launches of two (no product reads a layer's weights after its last one, so the order of
+    // the reference's f16_grad_accum calls, src/nn/fast_sft.c:804-946, does not matter; BWD_APPLY changes the weights behind it).
+    // Otherwise one buffer serves all.
     const bool defer = (mode == BWD_ACCUM || mode == BWD_APPLY) && s->dy16[0];
     if (mode == BWD_ACCUM) s->accum_clear = false;
     half_t *d16[4];
