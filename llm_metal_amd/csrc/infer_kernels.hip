@@ -733,10 +733,12 @@ void launch_matvec_glu(const void *W, const half_t *scales, const float *x, floa
 #undef GLU_LAUNCH
 }
 
-// k_matvec_normed takes vectors of up to NORMED_COLS = 2560 columns (the vector and two stages of weights in registers; k_matvec those beyond).  Every
-// wave is resident: two workgroups per CU, or one where a unit's two rows have more than 1536 columns -- fewer waves then keep
-// memory busy, and 256 workgroups fill the CUs evenly (one / two per CU: 6144 x 2560 F16 7.9 / 9.0 us, Q8_0 6.2 / 7.8, 9728 pairs F16 18.1 / 18.5;
-// 6912 pairs of 1152 F16 10.0 / 9.6, Q8_0 9.3 / 8.8).  The head, against k_matvec behind a launch for its norm:
+// k_matvec_normed takes vectors of up to NORMED_COLS = 2560 columns (k_matvec those beyond): five steps hold the vector and two stages of weights
+// in 171 to 224 registers of the 256 that a wave has, a sixth spills where norms stand on both sides of a branch.  Every wave is
+// resident: two workgroups per CU, or one where a unit's two rows have more than 1536 columns -- fewer waves then keep memory
+// busy, and 256 workgroups fill the CUs evenly (one / two per CU: 6144 x 2560 F16 7.9 / 9.0 us, Q8_0 6.2 / 7.8, 9728 pairs F16 18.1 / 18.5;
+// 6912 pairs of 1152 F16 10.0 / 9.6, Q8_0 9.3 / 8.8; a token of six layers, 1568 columns F16 185 / 188 us, 2048 Q8_0 182 / 184, with norms around
+// 1568 190 / 197, 2048 216 / 222, 2560 269 / 281; 1536 179 / 182 and 1152 161 / 161 is no difference).  The head, against k_matvec behind a launch for its norm:
 // 262 144 Q8_0 rows of 1152 3.4 + 77 -> 64 us (5.0 TB/s), 32 768 F16 rows of 2560 4.7 + 26 -> 27.
 template <int FMT, int NORM>
 void launch_matvec_normed(const void *W, const half_t *scales, const NormIn &nin, float *y, int rows, int cols, int act, hipEvent_t ev_a, hipEvent_t ev_b)

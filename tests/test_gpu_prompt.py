@@ -68,6 +68,23 @@ def test_short_prompts_on_either_side_of_an_operand_tile(kw, fmt, n, model_type)
         assert maxrel(inf.forward_tokens(toks, range(n)), want) < TOL
 
 
+@pytest.mark.parametrize("n", [63, 64, 65])
+@pytest.mark.parametrize("hd,group", [(128, 4), (256, 2), (256, 1)])
+def test_attention_on_either_side_of_64_keys(hd, group, n):
+    """Up to 64 keys a wave takes a token's head, beyond them the tiles do: whole prompts, and portions that end there and begin behind
+    others (positions 20 and 40), seven tokens of them so that the last wave of a workgroup has nothing to do."""
+    print(hd, group, n, flush=True)
+    c = SFTConfig("short_keys", QWEN3, NL=1, D=128, Hq=group, Hkv=1, hd=hd, IS=96, V=260, tied=True)
+    model, toks = make_model(c, seed=8, gamma_jitter=0.1), tokens(c, n, n)
+    with InferenceState(c, model, max_seq=n, use_fp16=True) as inf:
+        want = one_by_one(inf, toks)
+        for cuts in ((), (20,), (20, 40, n - 7)):
+            inf.reset()
+            at = (0,) + cuts + (n,)
+            got = np.concatenate([inf.forward_tokens(toks[a:b], range(b - a)) for a, b in zip(at, at[1:])])
+            assert maxrel(got, want) < TOL, cuts
+
+
 def test_prompt_of_several_steps():
     c = C1.with_(name="long", NL=1, V=256)
     model, toks = make_model(c, seed=4), tokens(c, 2500, 5)
