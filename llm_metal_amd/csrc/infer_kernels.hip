@@ -600,7 +600,7 @@ __global__ __launch_bounds__(TB) void k_matvec_split(const void *__restrict__ Wp
 // Two rows per workgroup, their columns dealt to the four waves in 512-column steps, S of them each: all that a wave multiplies is requested
 // at once, and a part of the vector (twice a row's bytes of it, from L2) serves two rows.  With a wave per row the weights came in a chain
 // of up to five trips.  Cold weights, us, a wave per row -> so (with four and five rows): F16 2560 x 4096 4.9 -> 4.35 (4.6, 4.8),
-// 2560 x 9728 11.9 -> 11.1 = 4.5 TB/s (11.2, 10.9), 2048 x 8192 7.8 -> 7.8; Q8_0 2560 x 4096 and 2560 x 9728 16.9 -> 13.2 together,
+// 2560 x 9728 11.9 -> 11.1 = 4.5 TB/s (11.2, 10.9); Q8_0 2560 x 4096 and 2560 x 9728 16.9 -> 13.2 together,
 // 1152 x 1024 3.3 -> 2.9.  Eight steps in flight for the wave per row: 13.4 and 5.8.  Bound by the launch and one trip, then by memory.
 template <int FMT, int S>
 __global__ __launch_bounds__(TB) void k_matvec_rows(const void *__restrict__ Wp, const half_t *__restrict__ scales,
@@ -707,6 +707,10 @@ void launch_matvec(const void *W, const half_t *scales, const float *x, float *y
     else if (rows <= SPLIT_ROWS && cols >= 4096 && (size_t)rows * cols * (FMT == 0 ? 2 : 1) <= SPLIT_BYTES) {
         if (cols > 4096) SPLIT_LAUNCH(4); else SPLIT_LAUNCH(2);
     }
+    // F16, up to two workgroups of the wave per row on each CU, its trips of 2048 columns whole: it is the faster one (wave per row / two
+    // rows: 2048 x 6144 5.4 / 5.7 us, x 8192 6.6 / 7.3, x 10240 7.9 / 8.6, 1600 x 8192 6.3 / 6.8; 2176 x 8192 9.1 / 8.3, Q8_0 2048 x 8192 7.3 / 6.7;
+    // 2048 x 9728 7.8 / 8.4 too, but its lanes past a row's end multiply the last weights by zero, which an infinite one does not survive)
+    else if (FMT == 0 && rows <= 2048 && cols >= 6144 && cols % 2048 == 0) MATVEC_LAUNCH(1, 4, 0, 4, 0);
     else if (cols > 512 && cols <= 5 * 2048) {               // what ROWS_LAUNCH holds in registers; a single step leaves it one wave
         const int steps = (cols + 2047) / 2048;
         if (steps == 1) ROWS_LAUNCH(1); else if (steps == 2) ROWS_LAUNCH(2); else if (steps == 3) ROWS_LAUNCH(3);
