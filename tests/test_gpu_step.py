@@ -512,7 +512,7 @@ def test_gradient_norm_in_its_order_of_sums():
 
 @pytest.mark.parametrize("batch,seq", [(1, 3), (1, 64), (1, 65), (3, 47), (2, 300)])
 def test_adapter_gradients_over_rows_and_columns_that_fill_no_tile(batch, seq):
-    """Rank 16: rows in groups of four over four or sixteen waves, columns of dY (108 and 36) and of the input (100) in blocks
+    """Rank 16: rows in groups of four, steps of 32 and of 64 of them, columns of dY (108 and 36) and of the input (100) in blocks
     of 64.  The bar is that of the steps above: fp16 operands of the products in front of these sums."""
     cfg = C1.with_(name="adapter_grads", NL=2, D=100, Hq=3, Hkv=1, hd=36, IS=128, V=260, batch=batch, seq=seq)
     model = make_model(cfg, seed=21, gamma_jitter=0.1)
