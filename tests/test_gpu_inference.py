@@ -193,7 +193,7 @@ def test_batch_steps_over_shapes_that_fill_no_tile(kw, batches, model_type):
                 assert maxrel(got[b], single) < 1e-4, (B, b, maxrel(got[b], single))
 
 
-@pytest.mark.parametrize("V", [260, 40004], ids=["4_pages", "160_pages"])
+@pytest.mark.parametrize("V", [260, 50004, 400004], ids=["one_part", "two_parts", "four_parts"])
 def test_logits_of_batch_steps_are_the_callers_own(V):
     """Ordinary arrays, as numpy's own are: each owns its memory, may be resized, and keeps what it holds when further steps and the end
     of the state pass; memory that ends in the middle of a page is written to its end and no further."""
