@@ -1654,6 +1654,15 @@ void matvec_norm(MetalBuf *W, const NormIn &nin, MetalBuf *y, int rows, int cols
     mark_written(y);
 }
 
+bool q8_rows_of(MetalBuf *W, int rows, int cols, const void **codes, const void **scales)
+{
+    if (rows <= 0 || cols <= 0 || (cols & 31) || W->size < (size_t)rows * (cols / 32) * 34 || !W->owns || W->host || W->parent) return false;
+    const half_t *d = nullptr;
+    *codes = q8_split_of(W, rows, cols / 32, &d);
+    *scales = d;
+    return true;
+}
+
 FewQ8 few_q8_of(MetalBuf *W, int rows, int cols)
 {
     if (rows <= 0 || cols <= 0 || (cols & 31) || W->size < (size_t)rows * (cols / 32) * 34) { fprintf(stderr, "[fast_hip] few_q8_of: unsupported shape %d x %d\n", rows, cols); abort(); }

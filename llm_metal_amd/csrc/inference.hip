@@ -3,7 +3,8 @@
 // Every step is enqueued on the library's one stream; the host waits once per token, for the logits or for
 // the argmax computed on the GPU.
 //
-// One decode step computes what src/nn/fast_inference.c:376-467 computes, in 5 launches per layer instead of 17: Q|K|V and
+// One decode step computes what src/nn/fast_inference.c:376-467 computes: where the host waits for the step, in one launch (token.hip),
+// otherwise, and for shapes, adapters and contexts that it does not take, in 5 launches per layer instead of 17: Q|K|V and
 // gate|up are one matrix each (row concatenation, built when the state is created), the products that follow a norm form it
 // themselves (matvec_norm, matvec_norms_around), and the attention launch does LoRA up-projection, per-head RMSNorm, RoPE and
 // the KV-cache store for the new token.  Prompts of five tokens and more run many tokens per step (PromptRun).
@@ -12,6 +13,7 @@
 #include "fused.h"
 #include "prompt.h"
 #include "few_rows.h"
+#include "token.h"
 #include "stack.h"
 #include "../../include/inference_hip.h"
 #include "../../include/loader_hip.h"
@@ -33,8 +35,10 @@ extern "C" MetalBuf *sft_get_token_emb_buf(SFTState *s);
 namespace {
 struct BatchRun;
 struct PromptRun;
+struct TokenRun;
 void batch_release(BatchRun *r);
 void prompt_release(PromptRun *r);
+void token_release(TokenRun *r);
 // a state on a training state's tiles, or of a layer-by-layer model: one token through the lock-step path with a run of
 // one sequence
 void step_on_run(InferenceState *s, int token, int pos);
@@ -87,12 +91,16 @@ struct InferenceState {
     bool prompt_refused;                 // no room for it
     uint64_t q8_fit_version;             // versions of the weights that q8_fit was found for (0: none)
     bool q8_fit;
+    TokenRun *one_launch;                // what a step in one launch needs (NULL until used)
+    bool steps_in_launches;              // it cannot be had, or a wait in it ran out
+    uint64_t step_ticks;                 // of the 100 MHz clock that a wait in it may last
     BatchRun *batch;                     // scratch and caches of the lock-step batch path, kept from call to call (NULL until used)
 };
 
 namespace {
 
 constexpr int TB = 256;
+constexpr uint64_t STEP_TICKS = 100000000;                   // a second: only a device that is not ours alone takes longer than some milliseconds
 
 // x = emb[token] * scale: the embedding row, scaled by sqrt(D) for Gemma3 (src/nn/fast_inference.c:385-391)
 __global__ __launch_bounds__(TB) void k_embed_row(const float *__restrict__ emb, int token, float scale, float *__restrict__ x, int D)
@@ -491,6 +499,127 @@ int argmax_to_host(InferenceState *s)
 // every step of the state is one of a run (BatchRun), also with a single sequence
 bool steps_on_run(const InferenceState *s) { return s->borrows_tiles || s->stack; }
 
+// ---- a step in one launch (token.hip)
+
+struct TokenRun {
+    TokenShape shape;
+    TokenArgs args;                      // what stays from step to step
+    MetalBuf *words, *table;             // hand-overs; the layers' addresses
+    std::vector<TokenLayer> layers;      // as the table holds them
+    int *fail;                           // pinned: a wait ran out
+    uint32_t tag;
+    long steps;
+};
+
+void token_release(TokenRun *r)
+{
+    if (!r) return;
+    metal_buf_free(r->words);
+    metal_buf_free(r->table);
+    if (r->fail) hipHostFree(r->fail);
+    delete r;
+}
+
+__global__ __launch_bounds__(TB) void k_clear_words(unsigned long long *w, size_t n)
+{
+    const size_t i = (size_t)blockIdx.x * TB + threadIdx.x;
+    if (i < n) w[i] = 0;
+}
+
+// addresses of a weight's rows; false where they do not stay with the buffer or are not aligned
+bool token_rows(InferenceState *s, const WMat *w, int rows, int cols, uint64_t *data, uint64_t *scales)
+{
+    const void *p = nullptr, *d = nullptr;
+    if (s->use_fp16) {
+        if (w->mbuf->size < (size_t)rows * cols * 2) return false;
+        p = dptr(w->mbuf);
+    } else if (!q8_rows_of(w->mbuf, rows, cols, &p, &d)) return false;
+    *data = (uint64_t)p; *scales = (uint64_t)d;
+    return !((uintptr_t)p & 15);
+}
+
+// The run, with the layers' addresses as they are now; NULL: the step goes in launches.  Those it is for: the matrix-vector pipeline's own
+// weights without adapters, contexts of up to TOKEN_KEYS keys (what its attention is made for; k_attn_short's line too), shapes that the kernel holds
+// (token_fits).  A profile of the products wants launches to count.
+TokenRun *token_acquire(InferenceState *s, int pos)
+{
+    if (s->steps_in_launches || steps_on_run(s) || !s->lora.empty() || pos >= TOKEN_KEYS || gemm_profiling()) return nullptr;
+    const bool gemma = s->model_type == MODEL_GEMMA3;
+    const TokenShape shape{s->D, s->IS, s->Hq, s->Hkv, s->hd, s->NL, s->V};
+    const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
+    bool ok = s->one_launch || token_fits(shape);
+    std::vector<TokenLayer> now(ok ? s->NL : 0);
+    for (int L = 0; ok && L < s->NL; L++) {
+        const InferenceState::Layer &lw = s->layers[L];
+        TokenLayer &t = now[L];
+        ok = token_rows(s, &lw.qkv, qd + 2 * kd, s->D, &t.qkv, &t.qkv_d) && token_rows(s, lw.o, s->D, qd, &t.o, &t.o_d) &&
+             token_rows(s, &lw.gu, 2 * s->IS, s->D, &t.gu, &t.gu_d) && token_rows(s, lw.down, s->D, s->IS, &t.down, &t.down_d);
+        auto norm = [](MetalBuf *b) { return b ? (uint64_t)dptr(b) : 0; };
+        t.g_in = norm(lw.g_in); t.g_post_attn = gemma ? norm(lw.g_post_attn) : 0; t.g_ff = norm(gemma ? lw.g_pre_ff : lw.g_post_attn);
+        t.g_post_ff = gemma ? norm(lw.g_post_ff) : 0; t.g_q = norm(lw.g_q); t.g_k = norm(lw.g_k);
+        t.kc = (uint64_t)dptr(s->kc[L]); t.vc = (uint64_t)dptr(s->vc[L]);
+        t.rope = (uint64_t)(dptr_as<float2>(s->rope_tabs) + (size_t)s->theta_slot[L] * s->max_seq * (s->hd / 2));
+        ok = ok && t.g_in && t.g_ff && (!gemma || (t.g_post_attn && t.g_post_ff));
+        for (uint64_t p : {t.g_in, t.g_post_attn, t.g_ff, t.g_post_ff, t.g_q, t.g_k, t.kc, t.vc, t.rope}) ok = ok && !(p & 15);
+    }
+    uint64_t head = 0, head_d = 0;
+    ok = ok && token_rows(s, s->lm_head, s->V, s->D, &head, &head_d) && s->emb && s->g_final && !(((uintptr_t)dptr(s->emb) | (uintptr_t)dptr(s->g_final)) & 15);
+    if (!ok) { s->steps_in_launches = true; return nullptr; }
+    if (!s->one_launch) {
+        TokenRun *r = new TokenRun();
+        if (hipHostMalloc((void **)&r->fail, sizeof(int), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            delete r;
+            s->steps_in_launches = true;
+            return nullptr;
+        }
+        *r->fail = 0;
+        r->shape = shape; r->tag = 1;
+        const size_t n = token_words(shape, nullptr, nullptr);
+        r->words = metal_buf_create(n * 8);
+        hipLaunchKernelGGL(k_clear_words, dim3((unsigned)((n + TB - 1) / TB)), dim3(TB), 0, stream(), dptr_as<unsigned long long>(r->words), n);
+        r->table = metal_buf_create(s->NL * sizeof(TokenLayer));
+        TokenArgs &a = r->args;
+        token_words(shape, &a, dptr_as<unsigned long long>(r->words));
+        a.layers = dptr_as<uint64_t>(r->table);
+        a.fail = r->fail;
+        a.NL = s->NL; a.D = s->D; a.IS = s->IS; a.Hq = s->Hq; a.Hkv = s->Hkv; a.hd = s->hd; a.max_seq = s->max_seq; a.V = s->V;
+        a.gemma = gemma; a.emb_scale = s->emb_scale; a.eps = s->eps; a.scale = 1.0f / sqrtf((float)s->hd);
+        s->one_launch = r;
+    }
+    TokenRun &r = *s->one_launch;
+    if (r.layers.size() != now.size() || memcmp(r.layers.data(), now.data(), now.size() * sizeof(TokenLayer)) != 0) {
+        r.layers = now;
+        HIP_CHECK(hipMemcpyAsync(dptr(r.table), r.layers.data(), now.size() * sizeof(TokenLayer), hipMemcpyHostToDevice, stream()));
+        HIP_CHECK(hipStreamSynchronize(stream()));
+    }
+    r.args.head = (const void *)head; r.args.head_d = (const void *)head_d;
+    r.args.g_final = dptr_as<float>(s->g_final);
+    r.args.logits = dptr_as<float>(s->logits);
+    return &r;
+}
+
+// One step and the wait for it: the logits in logits_host, or the argmax in best_host.  false: not taken, or a wait ran out (the step is
+// to be taken again, and this state's steps go in launches from here on).
+bool token_in_one_launch(InferenceState *s, int token, int pos, bool logits)
+{
+    TokenRun *r = token_acquire(s, pos);
+    if (!r) return false;
+    TokenArgs &a = r->args;
+    a.emb_row = dptr_as<float>(s->emb) + (size_t)token * s->D;
+    a.logits_host = logits ? s->logits_host : nullptr;
+    a.best_host = logits ? nullptr : s->best_host;
+    a.ticks = s->step_ticks; a.tag = r->tag; a.pos = pos;
+    r->tag += s->NL + 1;
+    launch_token(a, r->shape, s->use_fp16 ? 0 : 1);
+    for (int L = 0; L < s->NL; L++) { mark_written(s->kc[L]); mark_written(s->vc[L]); }
+    mark_written(s->logits);
+    HIP_CHECK(hipStreamSynchronize(stream()));
+    if (*(volatile int *)r->fail) { s->steps_in_launches = true; return false; }
+    r->steps++;
+    return true;
+}
+
 void default_eos(InferenceState *s)
 {
     if (s->stack) { s->n_eos = 0; return; }                           // a design without end tokens of its own
@@ -506,6 +635,7 @@ InferenceState *base_state(ModelType mt, int D, int V, int NL, int max_seq, Laye
     s->D = D; s->V = V; s->NL = NL;
     s->max_seq = max_seq; s->cur_len = 0; s->model_type = mt;
     s->stack = stack;
+    s->step_ticks = STEP_TICKS;
     default_eos(s);
     HIP_CHECK(hipHostMalloc((void **)&s->logits_host, (size_t)V * 4, hipHostMallocDefault));
     HIP_CHECK(hipHostMalloc((void **)&s->best_host, sizeof(int), hipHostMallocDefault));
@@ -790,6 +920,7 @@ void inference_state_free(InferenceState *s)
     batch_release(s->batch);
     batch_release(s->single);
     prompt_release(s->prompt);
+    token_release(s->one_launch);
     stack_free(s->stack);
     for (MetalBuf *b : {s->gate_v, s->up_v, s->x, s->x2, s->branch, s->ln, s->qkv, s->att, s->gu, s->logits, s->best, s->lora_t, s->rope_tabs})
         metal_buf_free(b);
@@ -817,6 +948,8 @@ void inference_state_free(InferenceState *s)
 ModelType inference_state_model_type(InferenceState *s) { return s->model_type; }
 int inference_state_vocab_size(InferenceState *s) { return s->V; }
 void inference_state_reset(InferenceState *s) { s->cur_len = 0; }
+long hip_inference_steps_in_one_launch(InferenceState *s) { return s && s->one_launch ? s->one_launch->steps : 0; }
+void hip_inference_step_wait(InferenceState *s, long long ticks) { if (s && ticks >= 0) s->step_ticks = (uint64_t)ticks; }
 int inference_state_position(InferenceState *s) { return s->cur_len; }
 
 static bool token_ok(InferenceState *s, int token)
@@ -833,21 +966,30 @@ static void step_token(InferenceState *s, int token, int pos)
 }
 static int argmax_host(InferenceState *s) { return steps_on_run(s) ? argmax_on_run(s) : argmax_to_host(s); }
 static const float *logits_host(InferenceState *s) { return steps_on_run(s) ? logits_on_run(s) : logits_to_host(s); }
+// a step whose result the host waits for
+static const float *step_logits(InferenceState *s, int token, int pos)
+{
+    if (token_in_one_launch(s, token, pos, true)) return s->logits_host;
+    step_token(s, token, pos);
+    return logits_host(s);
+}
+static int step_argmax(InferenceState *s, int token, int pos)
+{
+    if (token_in_one_launch(s, token, pos, false)) return *s->best_host;
+    step_token(s, token, pos);
+    return argmax_host(s);
+}
 
 const float *inference_forward_token(InferenceState *s, int token)
 {
     if (!token_ok(s, token)) return nullptr;
-    step_token(s, token, s->cur_len);
-    s->cur_len++;
-    return logits_host(s);
+    return step_logits(s, token, s->cur_len++);
 }
 
 int inference_forward_token_argmax(InferenceState *s, int token)
 {
     if (!token_ok(s, token)) return -1;
-    step_token(s, token, s->cur_len);
-    s->cur_len++;
-    return argmax_host(s);
+    return step_argmax(s, token, s->cur_len++);
 }
 
 // The next n tokens of the sequence from the current position on, and the logits at the places want[0 .. n_want)
@@ -862,9 +1004,9 @@ int inference_forward_tokens(InferenceState *s, const int *tokens, int n, const 
     if (s->stack) return forward_rows(s, tokens, n, want, n_want, logits);
     if (prompt_takes(s, n)) return prompt_forward(s, tokens, n, want, n_want, logits);
     for (int i = 0, w = 0; i < n; i++) {                                  // the other models take one token per step
-        step_token(s, tokens[i], s->cur_len);
+        if (w < n_want && want[w] == i) memcpy(logits + (size_t)w++ * s->V, step_logits(s, tokens[i], s->cur_len), (size_t)s->V * sizeof(float));
+        else step_token(s, tokens[i], s->cur_len);
         s->cur_len++;
-        if (w < n_want && want[w] == i) memcpy(logits + (size_t)w++ * s->V, logits_host(s), (size_t)s->V * sizeof(float));
     }
     metal_flush();
     return 0;
@@ -892,9 +1034,7 @@ int inference_generate(InferenceState *s, const uint32_t *prompt_tokens, int pro
         bool is_eos = false;
         for (int e = 0; e < s->n_eos; e++) is_eos |= next == s->eos[e];
         if (is_eos) break;
-        step_token(s, next, s->cur_len);
-        s->cur_len++;
-        next = argmax_host(s);
+        next = step_argmax(s, next, s->cur_len++);
         output_tokens[n_gen++] = (uint32_t)next;
     }
     return n_gen;

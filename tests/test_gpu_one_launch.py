@@ -1,0 +1,104 @@
+"""Steps of one sequence as one launch (token.hip) against the same steps in launches, which the oracle's decode chain is compared with
+elsewhere (test_gpu_inference.py): the largest and smallest widths that the one launch takes, shares of rows that do not come out even, columns
+behind whole steps of 512, contexts up to and over its last key, and what it leaves to the launches."""
+import sys
+
+import numpy as np
+import pytest
+
+from llm_metal_amd.configs import GEMMA3, QWEN3, SFTConfig
+from llm_metal_amd.sft import InferenceState, SFTState
+from llm_metal_amd.synth import make_model
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    # few workgroups (a share of D / 4), columns behind the last whole step
+    "gemma_320": SFTConfig("t", GEMMA3, NL=3, D=320, Hq=4, Hkv=1, hd=256, IS=448, V=516, tied=True),
+    # the widest that threads hold five and seven entries of
+    "gemma_1280_7168": SFTConfig("t", GEMMA3, NL=2, D=1280, Hq=4, Hkv=2, hd=256, IS=7168, V=1000, tied=True),
+    # a step of 64 columns behind two whole ones, heads of 128
+    "gemma_1088_hd128": SFTConfig("t", GEMMA3, NL=2, D=1088, Hq=6, Hkv=3, hd=128, IS=2880, V=2052, tied=True),
+    "qwen_1152": SFTConfig("t", QWEN3, NL=2, D=1152, Hq=4, Hkv=1, hd=256, IS=6912, V=4100),
+    # the widest of all, vocabulary in several parts per workgroup
+    "qwen_2560_10240": SFTConfig("t", QWEN3, NL=2, D=2560, Hq=32, Hkv=8, hd=128, IS=10240, V=45004),
+    "qwen_1344": SFTConfig("t", QWEN3, NL=4, D=1344, Hq=10, Hkv=2, hd=128, IS=4160, V=772),
+}
+
+
+def say(*a):
+    print(*a, flush=True, file=sys.stderr)
+
+
+def one_launch(inf):
+    return inf.L.hip_inference_steps_in_one_launch(inf.h)
+
+
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+@pytest.mark.parametrize("shape", list(SHAPES))
+def test_a_step_as_one_launch_is_the_step_in_launches(shape, fmt):
+    say("one launch", shape, fmt)
+    c = SHAPES[shape].with_(weight_format=fmt)
+    model = make_model(c, seed=41, gamma_jitter=0.1)
+    toks = [int(t) for t in np.random.default_rng(42).integers(0, c.V, 262)]
+    with InferenceState(c, model, max_seq=262, use_fp16=fmt == "f16") as inf:
+        inf.L.hip_gemm_profile_enable(1)                   # a profile counts launches
+        want = np.stack([inf.forward_token(t) for t in toks])
+        inf.L.hip_gemm_profile_enable(0)
+        assert one_launch(inf) == 0
+        inf.reset()
+        got = np.stack([inf.forward_token(t) for t in toks])
+        assert one_launch(inf) == 256                      # the last contexts are longer than it takes
+        # both sum the same fp32 products in another order: 2^-24 per operation, some 200 roundings in a row between embedding and logits
+        err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert err.max() < 200 * 2.0 ** -24, err.max()
+        inf.reset()
+        best = [inf.forward_token_argmax(t) for t in toks]
+        assert one_launch(inf) == 512
+        srt = np.sort(want, axis=1)
+        clear = srt[:, -1] - srt[:, -2] > 1e-4 * np.abs(srt[:, -1])
+        assert clear.mean() > 0.9 and (np.asarray(best)[clear] == want.argmax(1)[clear]).all()
+        # the first of equal maxima is the argmax of what the call beside it hands out
+        inf.reset()
+        assert best[0] == int(got[0].argmax()) == inf.forward_token_argmax(toks[0])
+
+
+def test_a_wait_that_runs_out_takes_the_step_again_in_launches():
+    c = SHAPES["gemma_320"].with_(weight_format="f16")
+    model = make_model(c, seed=43, gamma_jitter=0.1)
+    toks = [int(t) for t in np.random.default_rng(44).integers(0, c.V, 12)]
+    with InferenceState(c, model, max_seq=16, use_fp16=True) as inf:
+        inf.L.hip_gemm_profile_enable(1)
+        want = np.stack([inf.forward_token(t) for t in toks])
+        inf.L.hip_gemm_profile_enable(0)
+        inf.reset()
+        got = [np.array(inf.forward_token(t)) for t in toks[:5]]
+        inf.L.hip_inference_step_wait(inf.h, 0)            # every wait is over when it begins; the kernel runs to its end
+        got += [np.array(inf.forward_token(t)) for t in toks[5:]]
+        assert one_launch(inf) == 5
+        err = np.linalg.norm(np.stack(got) - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert err.max() < 200 * 2.0 ** -24, err.max()
+        best = inf.generate(toks[:3], 6)
+        assert one_launch(inf) == 5 and len(best) >= 1
+
+
+@pytest.mark.parametrize("kw", [dict(D=1120), dict(IS=6880), dict(V=1002), dict(hd=64, Hq=16), dict(D=2624), dict(IS=10304)], ids=str)
+def test_shapes_that_stay_with_the_launches(kw):
+    base = dict(NL=1, D=1152, Hq=4, Hkv=1, hd=256, IS=2048, V=1000)
+    c = SFTConfig("t", QWEN3, **{**base, **kw}).with_(weight_format="f16")
+    model = make_model(c, seed=45, gamma_jitter=0.1)
+    with InferenceState(c, model, max_seq=8, use_fp16=True) as inf:
+        for t in (1, 2, 3):
+            assert np.isfinite(inf.forward_token(t)).all()
+        assert one_launch(inf) == 0
+
+
+def test_adapters_stay_with_the_launches():
+    c = SHAPES["gemma_320"].with_(weight_format="f16", batch=1, seq=8)
+    model = make_model(c, seed=46, gamma_jitter=0.1)
+    with SFTState(c, model) as sft, InferenceState(c, model, max_seq=8, use_fp16=True) as inf:
+        inf.forward_token(1)
+        assert one_launch(inf) == 1
+        inf.attach_lora(sft)
+        inf.forward_token(2)
+        assert one_launch(inf) == 1
