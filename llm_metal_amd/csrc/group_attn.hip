@@ -1,6 +1,7 @@
 // Grouped attention inside chunks of positions, fp32: position i sees the positions of its chunk up to itself, a head reads
 // the keys and values of its group.  Rotated keys and values lie in rings per sequence and key head; a layer may read the
-// rings of an earlier one.  Slices of the visible keys are read once for several heads and merged behind.
+// rings of an earlier one.  A step of one token on few keys is one launch, a workgroup per head; else slices of the visible
+// keys are read once for several heads and merged behind.
 #include "group_rows.h"
 #include "rows.h"
 #include <algorithm>
@@ -188,6 +189,156 @@ __global__ __launch_bounds__(256) void k_group_merge(GroupRows a, int m0, int ns
     }
 }
 
+// A step of one token with heads of 128 that turn whole.  grid (H, rows): a workgroup finishes a head, so nothing is merged by a second launch.  A key
+// belongs to 16 lanes, the 64 groups take keys in turn, four of each asked for together with the head's part of the product, and
+// keep a running softmax of their own; its gate, newest key and value come straight from the product, and one workgroup per key
+// head puts them into the rings.  Consecutive workgroups are of different key heads (up to eight of those: a cache is read into
+// few of the eight L2s).  Bound by latency up to about 256 keys, then by what a compute unit draws (1 KB a key).
+constexpr int ONE_PASS_KEYS = 640;
+__global__ __launch_bounds__(1024) void k_group_token(GroupRows a)
+{
+    constexpr int D = 128, U = 4, GROUPS = 64;
+    __shared__ float po[16][D], pm[16], pl[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = tid >> 4, sub = tid & 15;
+    const int per = a.H / a.G, g = blockIdx.x % a.G, part = blockIdx.x / a.G, h = g * per + part, m = blockIdx.y, p = a.r.pos;
+    const int first = p / a.chunk * a.chunk, old = p - first + (a.own ? 0 : 1), slot0 = first % a.ring_rows;       // old: keys that lie in the ring
+    const float *row = a.cin + (size_t)m * a.ldc;
+    float *kr = key_ring(a, m, g), *vr = value_ring(a, m, g);
+    float4v k[U][2], v[U][2];
+    auto keys = [&](int j0) __attribute__((always_inline)) {               // (past the last cached key: that one again)
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int r = slot0 + max(min(j0 + GROUPS * u, old - 1), 0);
+            const size_t at = (size_t)(r >= a.ring_rows ? r - a.ring_rows : r) * D + 4 * sub;
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                k[u][c] = *reinterpret_cast<const float4v *>(kr + at + 64 * c);
+                v[u][c] = *reinterpret_cast<const float4v *>(vr + at + 64 * c);
+            }
+        }
+    };
+    // a head's part of the product, and with the turn of the position (entries d and d + 64 are in the same lane)
+    float4v cs[2];
+    auto fetch = [&](float4v (&x)[2], int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+            x[c] = *reinterpret_cast<const float4v *>(row + at + 4 * sub + 64 * c) + *reinterpret_cast<const float4v *>(a.bias + at + 4 * sub + 64 * c);
+    };
+    auto turn = [&](float4v (&x)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float u = x[0][e], w = x[1][e], co = cs[e >> 1][2 * (e & 1)], si = cs[e >> 1][2 * (e & 1) + 1];
+            x[0][e] = u * co - w * si;
+            x[1][e] = w * co + u * si;
+        }
+    };
+    const bool works = 4 * wave < old || (a.own && wave == 0);             // (uniform)
+    float gate = 1.f;
+    if (a.gated && tid < D) gate = sigmoid(row[a.o_g + h * D + tid]);
+    float4v o[2] = {};
+    float mx = -3.0e38f, l = 0.f;
+    if (works) {
+        float4v q[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) cs[i] = *reinterpret_cast<const float4v *>(group_angles(a, p) + 4 * sub + 2 * i);
+        fetch(q, a.o_q + h * D);
+        if (old) keys(grp);
+        turn(q);
+#pragma unroll
+        for (int c = 0; c < 2; c++) q[c] *= a.scale;
+        // (two sums of four: as short as the general kernel's)
+        auto score = [&](const float4v (&x)[2]) __attribute__((always_inline)) {
+            float4v s = q[0] * x[0];
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[e] = fmaf(q[1][e], x[1][e], s[e]);
+            return group_sum<16>((s[0] + s[1]) + (s[2] + s[3]));
+        };
+        if (a.own && wave == 0) {                          // the newest key belongs to the first group
+            float4v kn[2], vn[2];
+            fetch(kn, a.o_k + g * D);
+            fetch(vn, a.o_v + g * D);
+            turn(kn);
+            const float s0 = score(kn);
+            if (grp == 0) {
+                if (part == 0) {
+                    const size_t at = (size_t)(p % a.ring_rows) * D + 4 * sub;
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        *reinterpret_cast<float4v *>(kr + at + 64 * c) = kn[c];
+                        *reinterpret_cast<float4v *>(vr + at + 64 * c) = vn[c];
+                    }
+                }
+                mx = s0; l = 1.f;
+                if (!(s0 > -3.0e38f)) { mx = -3.0e38f; l = expf(s0 - mx); }    // (not a number, or minus infinity)
+#pragma unroll
+                for (int c = 0; c < 2; c++) o[c] = l * vn[c];
+            }
+        }
+        for (int j0 = grp; j0 < old; j0 += GROUPS * U) {
+            float s[U], top = mx;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                s[u] = score(k[u]);
+                if (j0 + GROUPS * u < old) top = fmaxf(top, s[u]);
+            }
+            const float keep = expf(mx - top);
+            mx = top;
+            l *= keep;
+#pragma unroll
+            for (int c = 0; c < 2; c++) o[c] *= keep;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool in = j0 + GROUPS * u < old;
+                const float e = in ? expf(s[u] - mx) : 0.f;
+                l += e;
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) o[c][i] = fmaf(e, in ? v[u][c][i] : 0.f, o[c][i]);
+            }
+            if (j0 + GROUPS * U < old) keys(j0 + GROUPS * U);
+        }
+        // the four groups of the wave together
+        const float all = xor_max<16>(xor_max<32>(mx)), e = expf(mx - all);
+        mx = all;
+        l = xor_add<16>(xor_add<32>(l * e));
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[c][i] = xor_add<16>(xor_add<32>(o[c][i] * e));
+    }
+    if (lane < 16) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) *reinterpret_cast<float4v *>(&po[wave][4 * sub + 64 * c]) = o[c];
+        if (sub == 0) { pm[wave] = mx; pl[wave] = l; }
+    }
+    __syncthreads();
+    if (tid >= D) return;
+    float all = pm[0];
+#pragma unroll
+    for (int i = 1; i < 16; i++) all = fmaxf(all, pm[i]);
+    float den[4] = {}, num[4] = {};                        // (sums of four waves)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float e = expf(pm[i] - all);
+        den[i & 3] = fmaf(pl[i], e, den[i & 3]);
+        num[i & 3] = fmaf(po[i][tid], e, num[i & 3]);
+    }
+    a.o[((size_t)m * a.H + h) * D + tid] = ((num[0] + num[1]) + (num[2] + num[3])) / ((den[0] + den[1]) + (den[2] + den[3])) * gate;
+}
+
+// The line for keys: microseconds of a token of models with three such layers, slices and merge -> this.  Widths 1024 / 2048 / 4096
+// (8 / 16 / 32 heads) alone: 64 keys 121.6 -> 110.4 / 163.8 -> 149.5 / 340.6 -> 324.2, 512 keys 123.9 -> 116.6 / 165.7 -> 157.8 /
+// 342.7 -> 332.2, 1000 keys 127.8 -> 127.2 / 166.9 -> 169.8 / 345.2 -> 345.1, 2000 keys 135.2 -> 156.8 / 179.8 -> 199.2 / 358.2 ->
+// 371.6; four sequences, 512 keys 263.8 -> 260.1 / 292.5 -> 285.6 / 442.3 -> 429.0, 1000 keys 266.6 -> 276.8 / 296.1 -> 299.0 /
+// 451.9 -> 449.2; eight (up to 256 workgroups, one per compute unit), 512 keys 274.2 -> 268.7 / 303.5 -> 291.5 / 455.6 -> 435.1.
+bool group_token_fits(const GroupRows &a)
+{
+    const int seen = a.r.pos % a.chunk + 1;
+    const bool even = !((a.ldc | a.o_q | a.o_k | a.o_v) & 3) && !(((uintptr_t)a.cin | (uintptr_t)a.bias | (uintptr_t)a.kring | (uintptr_t)a.vring | (uintptr_t)a.rope) & 15);
+    return a.r.T == 1 && a.dim == 128 && a.vdim == 128 && a.rot_dims == 128 && even && seen <= ONE_PASS_KEYS && a.H * a.r.n() <= 256;
+}
+
 }  // namespace
 
 void launch_group_cache(const GroupRows &a)
@@ -199,6 +350,7 @@ void launch_group_cache(const GroupRows &a)
 void launch_group_attend(const GroupRows &in)
 {
     GroupRows a = in;
+    if (group_token_fits(a)) { LAUNCH(k_group_token, dim3(a.H, a.r.n()), dim3(1024), 0, a); return; }
     const int keys = a.r.T == 1 ? 32 : 64, dp = pad4(a.dim), vp = pad4(a.vdim);      // decoding: more workgroups on fewer keys each
     // slices of the longest visible span among the step's rows: the whole chunk once a row starts a new one
     const int in_chunk = a.r.pos % a.chunk + a.r.T, most = in_chunk > a.chunk ? a.chunk : in_chunk, n = (most + keys - 1) / keys;

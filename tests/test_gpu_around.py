@@ -68,6 +68,33 @@ def test_chunk_edges(chunk, n, fmt, tmp_path):
             assert logit_error(g[None], o_in[None]) < TOL[fmt]
 
 
+@pytest.mark.parametrize("heads,kv_heads,dims,batch", [(4, 1, 128, 3), (6, 3, 128, 0), (2, 2, 128, 0), (5, 1, 64, 0)])
+def test_steps_of_one_token_on_few_and_many_keys(heads, kv_heads, dims, batch, tmp_path):
+    """Heads of 128: up to 640 keys a workgroup takes a head's keys in turn, 64 by 64 and four of those asked for at once, beyond
+    that (and where a head turns in part) slices are merged.  Steps around those lines and into the next chunk, as a ring begins
+    anew and for a reader of the same keys, against the oracle."""
+    chunk = 690
+    cfg = around([(grouped(heads, kv_heads, 128, 128, chunk=chunk, dims=dims), None), (grouped(heads, kv_heads, 128, 128, chunk=chunk, dims=dims, kv_from=0), None)], width=64)
+    m = Model(cfg, tmp_path)
+    n = chunk + 10
+    toks = m.tokens(n, seed=7)
+    want = so.run(cfg, m.W, toks)
+    for fmt in ("f32", "f16"):
+        with state(m, fmt, max_seq=n) as inf:
+            for start, steps in ((0, 6), (62, 5), (254, 6), (318, 4), (636, 8), (chunk - 2, 8)):
+                say(heads, kv_heads, dims, fmt, start)
+                inf.reset()
+                if start:
+                    inf.forward_tokens(toks[:start])
+                got = np.stack([inf.forward_token(t) for t in toks[start:start + steps]])
+                assert logit_error(got, want[start:start + steps]) < TOL[fmt], (fmt, start)
+            if batch:
+                seqs = np.array([toks[:70]] + [m.tokens(70, seed=60 + b) for b in range(1, batch)])
+                got = np.stack([inf.step_batch(seqs[:, t], t) for t in range(70)], axis=1)
+                for b in range(batch):
+                    assert logit_error(got[b], so.run(cfg, m.W, seqs[b])) < TOL[fmt], (fmt, b)
+
+
 @FMT
 def test_a_reader_with_longer_chunks_than_the_keys_owner(fmt, tmp_path):
     """Keys that the layer which wrote them no longer sees are there for the layer that borrows them, in prompts longer than a
