@@ -70,12 +70,13 @@ struct NormIn {
     float eps;
     int dim;                             // layer norm and norms around: entries of xr that count
     const float *g_br, *b_br;            // norms around: RMS norm weight and bias (may be null) of br
+    float *y_host;                       // a second place for y, in pinned memory, or null (rows without gates, up to NORMED_COLS columns)
 };
 constexpr int NORMED_COLS = 2560;        // widest vector that the products below norm in every wave (k_matvec_normed)
 // infer_kernels.hip: y = W . RMSNorm(xr + br; g) (glu 0), or the gated pair product of matvec_glu over it (1 SiLU, 2 GELU)
 void matvec_norm(MetalBuf *W, const NormIn &nin, MetalBuf *y, int rows, int cols, int q8, int glu);
 // infer_kernels.hip: y = W . LayerNorm(x; g) over the first dim of cols entries (F16 rows)
-void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, float eps, float *y, int rows, int cols);
+void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, float eps, float *y, int rows, int cols, float *y_host = nullptr);
 
 // infer_kernels.hip: y = W . RMSNorm(v; g) with v = xr + RMSNorm(br + b_br; g_br) (br may be null) over the first dim of cols
 // entries, v also to x_out; F16 rows or Q8_0 blocks.  act 0: as it is; 1, 2: the gated pairs of matvec_glu (SiLU, GELU); 3: its

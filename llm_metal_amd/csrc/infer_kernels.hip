@@ -401,6 +401,8 @@ __global__ __launch_bounds__(TB) void k_matvec(const void *__restrict__ Wp, cons
 // Bound by the launch, the trip for the vector and the weights' stream.  With the vector in LDS behind two block reductions (k_matvec):
 // 6912 Q8_0 pairs of 1152 with both norms 11.5 us, 8.8 so; 9728 F16 pairs of 2560 20.4 -> 18.1 (5.5 TB/s), 6144 rows 8.9 -> 7.9; 8192 rows of
 // 2048 with both norms 12.3 -> 10.3; 16 384 rows of 1024 with a layer norm 14.3 -> 12.3.  Four rows in a unit are no faster (registers).
+// nin.y_host: a step's logits arrive in pinned memory while the rest is summed, 64 rows of a wave at a time, where a copy behind the kernel
+// costs a launch, its bytes and the runtime's way there (128 KB: 20 us and more of the 234 that a token of the 2048 wide model took).
 template <int FMT, int NORM, int S>
 __global__ __launch_bounds__(TB, 2) void k_matvec_normed(const void *__restrict__ Wp, const half_t *__restrict__ scales, float *__restrict__ y, int rows, int cols,
                                                          int act, int reps, NormIn nin)
@@ -413,7 +415,9 @@ __global__ __launch_bounds__(TB, 2) void k_matvec_normed(const void *__restrict_
     const int lane = threadIdx.x & 63, wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const bool pair = act == 1 || act == 2;
     const int units = pair ? rows : (rows + 1) >> 1, last = min(wid * reps + reps, units) - 1;
-    int unit = wid * reps;
+    const int first = wid * reps;
+    int unit = first;
+    float held = 0.f;
     if (unit > last) return;
     uint32_t at[S];                                        // (clamped: loads stay unconditional)
 #pragma unroll
@@ -533,12 +537,19 @@ __global__ __launch_bounds__(TB, 2) void k_matvec_normed(const void *__restrict_
         }
         const float s0 = wave_sum(acc[0]) * norm_inv, s1 = wave_sum(acc[1]) * norm_inv;
         auto gelu = [](float x) { return 0.5f * x * (1.0f + tanhf(gelu_inner(x))); };
-        if (lane) return;
-        if (pair) y[u] = (act == 1 ? s0 / (1.0f + expf(-s0)) : gelu(s0)) * s1;
-        else {
-            y[2 * u] = act == 3 ? gelu(s0) : s0;
-            if (2 * u + 1 < rows) y[2 * u + 1] = act == 3 ? gelu(s1) : s1;
+        if (pair) {
+            if (lane == 0) y[u] = (act == 1 ? s0 / (1.0f + expf(-s0)) : gelu(s0)) * s1;
+            return;
         }
+        // the rows of up to 32 units in the lanes, then out together: to host memory a store of one row costs what one of sixteen does
+        const int at = 2 * (u - first) & 63;
+        if (lane >> 1 == at >> 1) held = lane & 1 ? s1 : s0;
+        if (at != 62 && u != last) return;
+        const int row = 2 * u - at + lane;
+        if (lane > at + 1 || row >= rows) return;
+        const float out = act == 3 ? gelu(held) : held;
+        y[row] = out;
+        if (nin.y_host) nin.y_host[row] = out;
     };
     for (;;) {
         if (unit == last) { use(A, unit); break; }
@@ -1565,13 +1576,13 @@ void matvec_glu(MetalBuf *W, MetalBuf *x, MetalBuf *y, int rows, int cols, int q
 }
 
 // y = W . LayerNorm(x; g), the norm of the first `dim` entries formed inside the launch (F16 rows of `cols` columns)
-void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, float eps, float *y, int rows, int cols)
+void matvec_layernorm(MetalBuf *W, const float *x, const float *g, int dim, float eps, float *y, int rows, int cols, float *y_host)
 {
     if (rows <= 0 || dim <= 0 || dim > cols || (cols & 7) || cols > 15360 || !aligned16(dptr(W)) || !x || !g || !aligned16(x) || !aligned16(g)) {
         fprintf(stderr, "[fast_hip] matvec_layernorm: unsupported shape %d x %d or operands\n", rows, cols); abort();
     }
     REQUIRE_BYTES(W, (size_t)rows * cols * 2, "matvec_layernorm");
-    const NormIn nin{x, nullptr, g, nullptr, eps, dim};
+    const NormIn nin{x, nullptr, g, nullptr, eps, dim, nullptr, nullptr, y_host};
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     const bool prof = gemm_prof_begin(2.0 * rows * cols, 2.0 * rows * cols, &ev_a, &ev_b);
     const half_t *scales = nullptr;

@@ -42,6 +42,7 @@ void token_release(TokenRun *r);
 // a state on a training state's tiles, or of a layer-by-layer model: one token through the lock-step path with a run of
 // one sequence
 void step_on_run(InferenceState *s, int token, int pos);
+const float *step_logits_on_run(InferenceState *s, int token, int pos);
 const float *logits_on_run(InferenceState *s);
 int argmax_on_run(InferenceState *s);
 void prefill_on_run(InferenceState *s, const uint32_t *tokens, int n, int pos);
@@ -408,7 +409,8 @@ void add_norm(InferenceState *s, MetalBuf *x, MetalBuf *branch, MetalBuf *g_bran
 }
 
 // src/nn/fast_inference.c:376-467
-void forward_token(InferenceState *s, int token, int pos)
+// host: pinned memory for the logits besides, or null; true: they go there as they are formed
+bool forward_token(InferenceState *s, int token, int pos, float *host = nullptr)
 {
     const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd;
     const bool gemma = s->model_type == MODEL_GEMMA3;
@@ -423,9 +425,9 @@ void forward_token(InferenceState *s, int token, int pos)
     // its feed-forward branch)
     const bool fuse_ffn = D <= 12288, fuse_qkv = fuse_ffn && s->lora.empty();
     const int q8 = s->use_fp16 ? 0 : 1;
-    auto normed_product = [&](MetalBuf *W, MetalBuf *branch, MetalBuf *g_branch, MetalBuf *g, MetalBuf *y, int rows, int glu) {
+    auto normed_product = [&](MetalBuf *W, MetalBuf *branch, MetalBuf *g_branch, MetalBuf *g, MetalBuf *y, int rows, int glu, float *y_host = nullptr) {
         NormIn n{dptr_as<float>(x), branch ? dptr_as<float>(branch) : nullptr, dptr_as<float>(g), branch ? dptr_as<float>(x_other) : nullptr,
-                 s->eps, D, g_branch ? dptr_as<float>(g_branch) : nullptr, nullptr};
+                 s->eps, D, g_branch ? dptr_as<float>(g_branch) : nullptr, nullptr, y_host};
         if (gemma && (g_branch || !branch)) { matvec_norms_around(W, n, dptr_as<float>(y), rows, D, q8, glu); mark_written(y); }
         else matvec_norm(W, n, y, rows, D, q8, glu);
         if (branch) std::swap(x, x_other);
@@ -470,12 +472,14 @@ void forward_token(InferenceState *s, int token, int pos)
         pending_g = gemma ? lw.g_post_ff : nullptr;
     }
     // (matvec_norm, which a branch without a norm of its own takes, wants whole blocks of 32 columns)
-    if (D <= NORMED_COLS && (D % 32 == 0 || pending_g)) normed_product(s->lm_head->mbuf, pending, pending_g, s->g_final, s->logits, s->V, 0);
+    const bool normed = D <= NORMED_COLS && (D % 32 == 0 || pending_g);
+    if (normed) normed_product(s->lm_head->mbuf, pending, pending_g, s->g_final, s->logits, s->V, 0, host);
     else {
         add_norm(s, x, pending, pending_g, s->g_final);
         matvec(s, s->lm_head, s->ln, s->logits);
     }
     HIP_CHECK(hipGetLastError());
+    return normed && host;
 }
 
 const float *logits_to_host(InferenceState *s)
@@ -965,13 +969,14 @@ static void step_token(InferenceState *s, int token, int pos)
     else forward_token(s, token, pos);
 }
 static int argmax_host(InferenceState *s) { return steps_on_run(s) ? argmax_on_run(s) : argmax_to_host(s); }
-static const float *logits_host(InferenceState *s) { return steps_on_run(s) ? logits_on_run(s) : logits_to_host(s); }
 // a step whose result the host waits for
 static const float *step_logits(InferenceState *s, int token, int pos)
 {
     if (token_in_one_launch(s, token, pos, true)) return s->logits_host;
-    step_token(s, token, pos);
-    return logits_host(s);
+    if (steps_on_run(s)) return step_logits_on_run(s, token, pos);
+    if (!forward_token(s, token, pos, s->logits_host)) return logits_to_host(s);
+    HIP_CHECK(hipStreamSynchronize(stream()));
+    return s->logits_host;
 }
 static int step_argmax(InferenceState *s, int token, int pos)
 {
@@ -1126,12 +1131,12 @@ bool few_rows_fit(const InferenceState *s)
 // dimension, so a layer is the same 7 launches (one more with adapters) for any B, or 11 where few_rows_fit does not hold.  A
 // product's planes are summed by the kernel that consumes them and the norm kernel writes the next product's operand itself,
 // where a row is one workgroup's.
-void forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int pos)
+// host: pinned memory for the logits of a single sequence besides, or null; true: they go there as they are formed.
+bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int pos, float *host = nullptr)
 {
     if (s->stack) {
         stack_forward(s->stack, r.stk, tokens, 1, pos);
-        stack_logits(s->stack, r.stk, nullptr, r.B, dptr_as<float>(r.logits));
-        return;
+        return stack_logits(s->stack, r.stk, nullptr, r.B, dptr_as<float>(r.logits), host);
     }
     const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd, IS = s->IS, B = r.B;
     const int qd = Hq * hd, kd = Hkv * hd, nqkv = qd + 2 * kd;
@@ -1223,6 +1228,7 @@ void forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
         launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, dptr_as<float>(r.logits), B, lg.N);
     }
     HIP_CHECK(hipGetLastError());
+    return false;
 }
 
 // argmax of every sequence's logits, computed on the GPU; one wait for all of them
@@ -1321,6 +1327,15 @@ void step_on_run(InferenceState *s, int token, int pos)
     BatchRun &r = batch_acquire(s, s->single, 1);
     forward_token_batch(s, r, &token, pos);
     r.len = pos + 1;
+}
+const float *step_logits_on_run(InferenceState *s, int token, int pos)
+{
+    BatchRun &r = batch_acquire(s, s->single, 1);
+    const bool there = forward_token_batch(s, r, &token, pos, s->logits_host);
+    r.len = pos + 1;
+    if (!there) return logits_on_run(s);
+    HIP_CHECK(hipStreamSynchronize(stream()));
+    return s->logits_host;
 }
 // ---- prompts of the models that decode a token at a time, many tokens per step
 

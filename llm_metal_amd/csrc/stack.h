@@ -131,7 +131,7 @@ struct StackRun {
     struct Layer { MetalBuf *S = nullptr, *conv = nullptr, *ring = nullptr, *vring = nullptr, *n = nullptr, *m = nullptr; int ring_rows = 0; };
     std::vector<Layer> layers;
     MetalBuf *x2 = nullptr;                              // the residual's other place (fused steps of NORMS_AROUND)
-    float *xr = nullptr;                                 // where the fused steps left it
+    const float *xr = nullptr;                                 // where the fused steps left it
     const float *post_g = nullptr, *post_b = nullptr;    // NORMS_AROUND: norm weight and bias of the sum that waits in cout
     MetalBuf *tok = nullptr, *want = nullptr;
     int *tok_host = nullptr, *want_host = nullptr;       // pinned; tok_host [B * max_seq], each portion in its own place
@@ -161,7 +161,8 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
 // most STACK_WANT of them; the stream must be synchronised before the next call), or with NULL the last token of each
 // sequence.
 constexpr int STACK_WANT = 64;
-void stack_logits(LayerStack *st, StackRun *r, const int *want, int n, float *logits);
+// host: pinned memory for a single row besides, or null; true: the kernel that forms it writes it there too
+bool stack_logits(LayerStack *st, StackRun *r, const int *want, int n, float *logits, float *host = nullptr);
 
 // ---------------------------------------------------------------- launches (rows: B * T tokens, row m = b * T + t)
 

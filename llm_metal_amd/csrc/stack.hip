@@ -621,18 +621,20 @@ void feed_forward(LayerStack *st, StackRun *r, StackLayer &L, int n)
 }
 
 // decoding one sequence with F16 weights and norms around the sublayers: the vector of every product is the residual with
-// the sum before it, both normed inside the product's launch; the residual goes back and forth between two places
-void decode_layers_around(LayerStack *st, StackRun *r, int pos)
+// the sum before it, both normed inside the product's launch; the residual goes back and forth between two places.
+// emb: the token's row where it is the residual as it lies in the table, or null (r->x holds it)
+void decode_layers_around(LayerStack *st, StackRun *r, int pos, const float *emb)
 {
     const Rows rows{1, 1, pos};
     float *cin = ptr<float>(r->cin), *cout = ptr<float>(r->cout), *act = ptr<float>(r->act);
-    float *at = ptr<float>(r->x), *next = ptr<float>(r->x2);
+    const float *at = emb ? emb : ptr<float>(r->x);
+    float *next = ptr<float>(r->x2), *other = ptr<float>(r->x);
     NormIn in{};
     in.eps = st->cfg.eps; in.dim = st->D;
     auto product_of = [&](const StackMat &w, MetalBuf *g, float *y, int gelu) {
         in.xr = at; in.g = ptr<float>(g); in.x_out = in.br ? next : nullptr;
         matvec_norms_around(w.buf, in, y, w.rows, w.cols, 0, gelu ? 3 : 0);
-        if (in.br) std::swap(at, next);
+        if (in.br) { at = next; std::swap(next, other); }
     };
     auto leave = [&](MetalBuf *g, MetalBuf *b) { in.br = cout; in.g_br = ptr<float>(g); in.b_br = ptr<float>(b); };
     for (size_t i = 0; i < st->layers.size(); i++) {
@@ -708,6 +710,12 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
 {
     const Rows rows{r->B, T, pos};
     const int n = rows.n();
+    r->T = T; r->pending = 0;
+    r->one = n == 1 && r->fused;
+    if (r->one && st->cfg.norms == NORMS_AROUND && st->cfg.emb_scale == 1.f && st->D == st->Dp) {
+        decode_layers_around(st, r, pos, ptr<float>(st->emb) + (size_t)tokens[0] * st->D);
+        return;
+    }
     if (n <= STACK_FEW) launch_embed_few(ptr<float>(st->emb), tokens, st->cfg.emb_scale, ptr<float>(r->x), st->D, st->Dp, n);
     else {
         // many tokens travel through pinned memory, every position in a place of its own: only a sequence that has gone back
@@ -719,9 +727,7 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
         HIP_CHECK(hipMemcpyAsync(dptr(r->tok), th, (size_t)n * sizeof(int), hipMemcpyHostToDevice, stream()));
         launch_embed_rows(ptr<float>(st->emb), ptr<int>(r->tok), st->cfg.emb_scale, ptr<float>(r->x), st->D, st->Dp, n);
     }
-    r->T = T; r->pending = 0;
-    r->one = n == 1 && r->fused;
-    if (r->one) { if (st->cfg.norms == NORMS_AROUND) decode_layers_around(st, r, pos); else decode_layers(st, r, pos); return; }
+    if (r->one) { if (st->cfg.norms == NORMS_AROUND) decode_layers_around(st, r, pos, nullptr); else decode_layers(st, r, pos); return; }
     for (size_t i = 0; i < st->layers.size(); i++) {
         StackLayer &L = st->layers[i];
         const LayerConfig &c = L.c;
@@ -763,15 +769,16 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
     }
 }
 
-void stack_logits(LayerStack *st, StackRun *r, const int *want, int n, float *logits)
+bool stack_logits(LayerStack *st, StackRun *r, const int *want, int n, float *logits, float *host)
 {
-    if (n <= 0) return;
+    if (n <= 0) return false;
     if (r->one) {                                         // whatever `want` says, it is the one row
+        if (st->head.cols > NORMED_COLS) host = nullptr;
         if (st->cfg.norms == NORMS_AROUND)
-            matvec_norms_around(st->head.buf, NormIn{r->xr, ptr<float>(r->cout), ptr<float>(st->g_final), nullptr, st->cfg.eps, st->D, r->post_g, r->post_b},
+            matvec_norms_around(st->head.buf, NormIn{r->xr, ptr<float>(r->cout), ptr<float>(st->g_final), nullptr, st->cfg.eps, st->D, r->post_g, r->post_b, host},
                                 logits, st->head.rows, st->head.cols, 0, 0);
-        else matvec_layernorm(st->head.buf, ptr<float>(r->x), ptr<float>(st->g_final), st->D, st->cfg.eps, logits, st->head.rows, st->head.cols);
-        return;
+        else matvec_layernorm(st->head.buf, ptr<float>(r->x), ptr<float>(st->g_final), st->D, st->cfg.eps, logits, st->head.rows, st->head.cols, host);
+        return host;
     }
     const int *list = nullptr;
     if (want) {
@@ -781,6 +788,7 @@ void stack_logits(LayerStack *st, StackRun *r, const int *want, int n, float *lo
     }
     norm(st, r, st->g_final, n, 0, false, list, r->T, r->T - 1);
     product(st, st->head, ptr<half_t>(r->a16), ptr<float>(r->inv), ptr<float>(r->h), st->Dp, logits, n);
+    return false;
 }
 
 }  // namespace lmhip

@@ -141,6 +141,23 @@ def test_widths_of_decoded_rows(width, tmp_path):
         assert logit_error(np.stack([inf.forward_token(t) for t in toks]), want) < TOL["f16"]
 
 
+@pytest.mark.parametrize("vocab", [3, 161, 4098, 140003])
+@pytest.mark.parametrize("around_layers", [False, True])
+def test_logits_that_go_to_the_host_as_they_are_formed(around_layers, vocab, tmp_path):
+    """A wave of the head writes its rows 64 at a time: fewer rows than waves, odd ones, and 70 per wave.  What a step hands out is
+    what the same step leaves on the device, from where a portion's wanted rows are copied."""
+    say("host logits", around_layers, vocab)
+    cfg = around([(grouped(2, 1, 16, 16, 9), dense(40))], width=64, vocab=vocab) if around_layers else config([(delta(2, 1, 16, 16, 2), None)], width=64, vocab=vocab)
+    m = Model(cfg, tmp_path)
+    toks = [0, 2, vocab - 1, 1]
+    want = so.run(cfg, m.W, toks)
+    with state(m, "f16") as inf:
+        got = np.stack([inf.forward_token(t) for t in toks])
+        assert logit_error(got, want) < TOL["f16"]
+        inf.reset()
+        assert np.array_equal(got, np.concatenate([inf.forward_tokens([t], [0]) for t in toks]))
+
+
 @pytest.mark.parametrize("window", [1, 2, 15, 16, 17, 63, 64, 65, 100])
 def test_window_edges(window, tmp_path):
     """One attention layer: a token just outside the window must not matter at all, one just inside must, in a prompt and in
