@@ -72,6 +72,8 @@ __device__ __forceinline__ void few_finish(float *part, const float16v (&acc)[WT
 // Eight vectors, 4B shape: Q|K|V 8.9 us (31 MB; the ring kernel 8.4 and 3.7 for its planes), gate|up 23.2 (100 MB; 20.0 and 4.8 for
 // the gate), head of 32 768 rows 32.0 (27.3 and 4.2).  304 gate blocks fill 256 CUs unevenly: with four waves of up to four tiles in
 // flight each 23.2, eight of two 24.2 (the operand tile of the next one then waits for registers).
+// An accumulator is rounded at every instruction, so a K tile's four make a sum of their own: 20 tokens of one layer of width 2560 are 4.2e-7
+// from 64 bits so, 5.0e-7 with up to forty instructions on one sum; the times differ by less than their noise.
 template <int MT, int WT, int U, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WT * MT == 4 || U > 3 ? 2 : 4) void k_few_full(const half8 *__restrict__ A, const float *__restrict__ inv, const half8 *__restrict__ W,
                                                                                 float *__restrict__ out, int ldo, int B, int N, int Kb, int up_block, int gelu)
@@ -108,12 +110,28 @@ __global__ __launch_bounds__(64 * WAVES, WT * MT == 4 || U > 3 ? 2 : 4) void k_f
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < C; u++) {
+            if (WAVES == 8) {                              // (128 registers: one tile's sum at a time)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+                for (int m = 0; m < MT; m++) {
+                    float16v sum = {};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u][0][j], a[u % CA][m][j], sum, 0, 0, 0);
+                    acc[0][m] += sum;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                float16v sum[WT][MT] = {};
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int q = 0; q < WT; q++)
+#pragma unroll
+                        for (int m = 0; m < MT; m++) sum[q][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u][q][j], a[u % CA][m][j], sum[q][m], 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < WT; q++)
 #pragma unroll
-                    for (int m = 0; m < MT; m++) acc[q][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u][q][j], a[u % CA][m][j], acc[q][m], 0, 0, 0);
+                    for (int m = 0; m < MT; m++) acc[q][m] += sum[q][m];
+            }
             if (u + CA < C) operand(u + CA);
             __builtin_amdgcn_sched_barrier(0);
         }
