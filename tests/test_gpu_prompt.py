@@ -85,6 +85,36 @@ def test_attention_on_either_side_of_64_keys(hd, group, n):
             assert maxrel(got, want) < TOL, cuts
 
 
+@pytest.mark.parametrize("n", [265, 300, 545])
+def test_attention_with_workgroups_in_either_order(n):
+    """Heads of 128 over eight key heads: up to 512 workgroups the second half comes shortest first, from 516 tokens on all of them longest
+    first; last tiles of rows and keys full and not, a portion that begins inside a tile."""
+    print(n, flush=True)
+    c = SFTConfig("orders", QWEN3, NL=1, D=128, Hq=32, Hkv=8, hd=128, IS=96, V=260, tied=True)
+    model, toks = make_model(c, seed=12, gamma_jitter=0.1), tokens(c, n, n)
+    with InferenceState(c, model, max_seq=n, use_fp16=True) as inf:
+        want = one_by_one(inf, toks)
+        for cuts in ((), (77,)):
+            inf.reset()
+            at = (0,) + cuts + (n,)
+            got = np.concatenate([inf.forward_tokens(toks[a:b], range(b - a)) for a, b in zip(at, at[1:])])
+            assert maxrel(got, want) < TOL, cuts
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+def test_infinite_values_inside_a_tile_stay_with_later_tokens(hd):
+    """Tokens before one whose keys and values are not finite, in the same 32 keys and in earlier ones, do not see it."""
+    c = SFTConfig("inf", QWEN3, NL=1, D=128, Hq=4, Hkv=2, hd=hd, IS=96, V=260)
+    model, toks = make_model(c, seed=13), list(range(150))
+    with InferenceState(c, model, max_seq=150) as inf:
+        want = inf.forward_tokens(toks, range(150))
+    model["token_emb"][110] = np.inf
+    with InferenceState(c, model, max_seq=150) as inf:
+        got = inf.forward_tokens(toks, range(150))
+    assert maxrel(got[:110], want[:110]) < TOL and np.isfinite(got[:110]).all()
+    assert not np.isfinite(got[110:]).any()
+
+
 def test_prompt_of_several_steps():
     c = C1.with_(name="long", NL=1, V=256)
     model, toks = make_model(c, seed=4), tokens(c, 2500, 5)
