@@ -156,6 +156,12 @@ def test_logits_that_go_to_the_host_as_they_are_formed(around_layers, vocab, tmp
         assert logit_error(got, want) < TOL["f16"]
         inf.reset()
         assert np.array_equal(got, np.concatenate([inf.forward_tokens([t], [0]) for t in toks]))
+        # a portion's single row travels through pinned memory, several do not
+        inf.reset()
+        several = inf.forward_tokens(toks, [1, 3])
+        inf.reset()
+        one = [inf.forward_tokens(toks[:2], [1])[0], inf.forward_tokens(toks[2:], [1])[0]]
+        assert logit_error(np.stack(one), several) < TOL["f16"] and logit_error(np.stack(one), want[1::2]) < TOL["f16"]
 
 
 @pytest.mark.parametrize("window", [1, 2, 15, 16, 17, 63, 64, 65, 100])
