@@ -72,8 +72,9 @@ __device__ __forceinline__ void few_finish(float *part, const float16v (&acc)[WT
 // Eight vectors, 4B shape: Q|K|V 8.9 us (31 MB; the ring kernel 8.4 and 3.7 for its planes), gate|up 23.2 (100 MB; 20.0 and 4.8 for
 // the gate), head of 32 768 rows 32.0 (27.3 and 4.2).  304 gate blocks fill 256 CUs unevenly: with four waves of up to four tiles in
 // flight each 23.2, eight of two 24.2 (the operand tile of the next one then waits for registers).
-// An accumulator is rounded at every instruction, so a K tile's four make a sum of their own: 20 tokens of one layer of width 2560 are 4.2e-7
-// from 64 bits so, 5.0e-7 with up to forty instructions on one sum; the times differ by less than their noise.
+// An accumulator is rounded at every instruction, so beyond sixteen vectors a K tile's four make a sum of their own: 20 tokens of one layer of width 2560
+// are 4.2e-7 from 64 bits so, 5.0e-7 with up to forty instructions on one sum; steps of 17 sequences take 0.5 to 0.9 % more, of 32 no more.  Up to sixteen, where the matrix cores have half the work beside
+// the same vector additions, that took 0.7 % of three sequences' steps and is left out.
 template <int MT, int WT, int U, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WT * MT == 4 || U > 3 ? 2 : 4) void k_few_full(const half8 *__restrict__ A, const float *__restrict__ inv, const half8 *__restrict__ W,
                                                                                 float *__restrict__ out, int ldo, int B, int N, int Kb, int up_block, int gelu)
@@ -110,7 +111,12 @@ __global__ __launch_bounds__(64 * WAVES, WT * MT == 4 || U > 3 ? 2 : 4) void k_f
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < C; u++) {
-            if (WAVES == 8) {                              // (128 registers: one tile's sum at a time)
+            if (MT == 1) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int q = 0; q < WT; q++) acc[q][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u][q][j], a[u % CA][0][j], acc[q][0], 0, 0, 0);
+            } else if (WAVES == 8) {                       // (128 registers: one tile's sum at a time)
 #pragma unroll
                 for (int m = 0; m < MT; m++) {
                     float16v sum = {};

@@ -309,7 +309,7 @@ __device__ __forceinline__ float exp_below(float x)
 // ahead.  The rows' operands are split once for the workgroup and lie in LDS (24 KB for heads of 128; two workgroups on a CU).  Scores are
 // summed 32 columns at a time, values by the sixteen keys of an instruction.  Key heads are the fast grid dimension: of eight, each is
 // read into one XCD's L2.
-// Bound by the splits: some 1450 vector instructions per tile, 800 of them splits, beside 96 matrix ones; a wave that has a SIMD for itself
+// Bound by the splits: some 1400 vector instructions per tile, 800 of them splits, beside 96 matrix ones; a wave that has a SIMD for itself
 // takes 5.6 us for a tile, 7.4 in 32 bits.  32 heads of 128 over 8, 70 / 500 tokens 12.5 / 55 -> 10.5 / 28.2 us (ring and order of workgroups alone,
 // still in 32 bits: 41); 4 heads of 256 over one 22.0 / 61 -> 18.0 / 43.7, 250 behind 777 121 -> 84.
 // Error against 64 bits, units of 2^-24 of the result's norm, 70 / 500 tokens of normal keys: 128 1.99 / 2.04 -> 1.78 / 1.82, 256 2.06 / 2.05 -> 1.81 / 1.74;
