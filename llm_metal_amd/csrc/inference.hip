@@ -544,14 +544,14 @@ bool token_rows(InferenceState *s, const WMat *w, int rows, int cols, uint64_t *
 
 // The run, with the layers' addresses as they are now; NULL: the step goes in launches.  Those it is for: the matrix-vector pipeline's own
 // weights without adapters, contexts of up to TOKEN_KEYS keys (what its attention is made for; k_attn_short's line too), shapes that the kernel holds
-// (token_fits).  A profile of the products wants launches to count.
+// (token_fits) and for which it is the faster way (token_pays).  A profile of the products wants launches to count.
 TokenRun *token_acquire(InferenceState *s, int pos)
 {
     if (s->steps_in_launches || steps_on_run(s) || !s->lora.empty() || pos >= TOKEN_KEYS || gemm_profiling()) return nullptr;
     const bool gemma = s->model_type == MODEL_GEMMA3;
     const TokenShape shape{s->D, s->IS, s->Hq, s->Hkv, s->hd, s->NL, s->V};
     const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
-    bool ok = s->one_launch || token_fits(shape);
+    bool ok = s->one_launch || (token_fits(shape) && token_pays(shape, s->use_fp16 ? 0 : 1));
     std::vector<TokenLayer> now(ok ? s->NL : 0);
     for (int L = 0; ok && L < s->NL; L++) {
         const InferenceState::Layer &lw = s->layers[L];

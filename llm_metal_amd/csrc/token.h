@@ -32,6 +32,7 @@ struct TokenArgs {
 };
 
 bool token_fits(const TokenShape &s);
+bool token_pays(const TokenShape &s, int q8);            // among those that fit
 // 64-bit words that a state needs for its hand-overs, zero before the first step; with a and base: their places
 size_t token_words(const TokenShape &s, TokenArgs *a, unsigned long long *base);
 void launch_token(const TokenArgs &a, const TokenShape &s, int q8);

@@ -695,6 +695,23 @@ bool token_fits(const TokenShape &s)
     return rows(s.D, wgs - heads) <= ROWS && rows(2 * s.IS, wgs) <= ROWS && rows((s.Hq + 2 * s.Hkv) * s.hd, wgs) <= ROWS;
 }
 
+// Whether the one launch is the faster way: an estimate in microseconds, behind which the launches' own time does not matter.  Measured, launches ->
+// one launch, greedy, contexts of 10 and 230, models of 1 to 28 layers and 4096 to 262 144 rows of the head:
+// - a step without its layers 38 -> 22 (chain of the head's norm, the argmax and the wait), of which a head of 64k rows takes eight back;
+// - a layer, heads of 256, widths 384 / 640 / 1152 / 1536 F16 17.5 -> 17.4 / 20.1 -> 18.2 / 27.8 -> 23.0 / 31.0 -> 29.5, Q8_0 18.3 -> 18.7 / 20.4 -> 19.2 /
+//   26.2 -> 20.7 / 28.5 -> 24.4; heads of 128, 640 / 1024 / 1536 F16 17.4 -> 16.1 / 18.9 -> 17.3 / 25.0 -> 23.5, Q8_0 17.5 -> 18.3 / 17.8 -> 19.4 /
+//   22.7 -> 20.7; 2048 F16 with 16 / 32 of them 30.8 -> 31.6 / 40.0 -> 37.8, Q8_0 26.0 -> 24.6 / 32.6 -> 29.1, 2560 with 32 F16 51.6 -> 48.0, Q8_0 38.5 -> 36.5;
+// - 64k rows of the head of widths 128 / 384 / 768 / 1152 / 2560, F16 2 -> 95 / 5 -> 33 / 14 -> 20 / 22 -> 28 / 51 -> 51, Q8_0 3 -> 105 / 4 -> 35 / 9 -> 20 /
+//   12 -> 17 / 30 -> 41: here a workgroup takes 47 ns for a row and draws 22 GB/s (Q8_0: 18) and a narrow model has few of them (token_workgroups), a head's own
+//   launch streams 6.5 TB/s with all CUs.
+bool token_pays(const TokenShape &s, int q8)
+{
+    const float wgs = (float)token_workgroups(s), rows = (float)s.V, mb = rows * (float)s.D * (q8 ? 1.0625e-6f : 2e-6f);
+    const float head = std::max(rows * 0.0465f / wgs, mb / (wgs * (q8 ? 0.018f : 0.0225f))) - mb / 6.5f;
+    const float layer = s.hd == 256 ? (s.D >= 1024 ? 3.f : 1.5f) : q8 ? (s.D < 1280 ? -1.f : 1.5f) : s.Hq * s.hd > s.D ? 2.5f : s.D < 2048 ? 1.f : 0.f;
+    return 15.f - 8.f * std::min(1.f, rows / 65536.f) + (float)s.NL * layer > head;
+}
+
 size_t token_words(const TokenShape &s, TokenArgs *a, u64 *base)
 {
     auto padded = [](int n) { return (size_t)(n + 511) / 512 * 512; };

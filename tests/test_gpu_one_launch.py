@@ -93,6 +93,20 @@ def test_shapes_that_stay_with_the_launches(kw):
         assert one_launch(inf) == 0
 
 
+# either side of the line: vocabularies that few workgroups read too slowly, layers of narrow Q8_0 models with heads of 128, which cost more than
+# the step saves
+@pytest.mark.parametrize("kw,fmt,taken", [(dict(V=516), "f16", True), (dict(V=65536), "f16", False), (dict(V=65536), "q8_0", False),
+                                          (dict(model_type=QWEN3, D=512, hd=128, Hq=8, Hkv=4, V=516, NL=4), "q8_0", True),
+                                          (dict(model_type=QWEN3, D=512, hd=128, Hq=8, Hkv=4, V=516, NL=20), "q8_0", False),
+                                          (dict(model_type=QWEN3, D=512, hd=128, Hq=8, Hkv=4, V=516, NL=20), "f16", True)], ids=str)
+def test_shapes_that_are_faster_in_launches_stay_there(kw, fmt, taken):
+    c = SHAPES["gemma_320"].with_(weight_format=fmt, **kw)
+    model = make_model(c, seed=47, gamma_jitter=0.1)
+    with InferenceState(c, model, max_seq=8, use_fp16=fmt == "f16") as inf:
+        assert np.isfinite(inf.forward_token(1)).all()
+        assert one_launch(inf) == int(taken)
+
+
 def test_adapters_stay_with_the_launches():
     c = SHAPES["gemma_320"].with_(weight_format="f16", batch=1, seq=8)
     model = make_model(c, seed=46, gamma_jitter=0.1)
