@@ -99,8 +99,8 @@ int  inference_forward_token_argmax(InferenceState *state, int token);
 /* A step that the host waits for (the two calls above, inference_generate, places of inference_forward_tokens taken one by one) is one launch in
  * which all CUs take part, where the state has its own weights without adapters, up to 256 keys, heads of 128 or 256, and widths of whole 64 columns (d_model
  * <= 2560, FFN <= 10240, vocabulary a multiple of 4); otherwise five launches per layer.  Its workgroups wait for each other; should some be kept off
- * the device for longer than `ticks` of 10 ns (a second unless set), the step is taken again in launches, and so are the state's further ones.  No
- * counterpart in the reference. */
+ * the device for longer than `ticks` of 10 ns (20 ms unless set), the step is taken again in launches, and the state's next 64 steps go so too (twice
+ * as many each further time, up to 4096).  No counterpart in the reference. */
 void hip_inference_step_wait(InferenceState *state, long long ticks);
 /* how many steps of the state have been one launch */
 long hip_inference_steps_in_one_launch(InferenceState *state);

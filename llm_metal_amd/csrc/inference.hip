@@ -93,7 +93,7 @@ struct InferenceState {
     uint64_t q8_fit_version;             // versions of the weights that q8_fit was found for (0: none)
     bool q8_fit;
     TokenRun *one_launch;                // what a step in one launch needs (NULL until used)
-    bool steps_in_launches;              // it cannot be had, or a wait in it ran out
+    bool steps_in_launches;              // it cannot be had
     uint64_t step_ticks;                 // of the 100 MHz clock that a wait in it may last
     BatchRun *batch;                     // scratch and caches of the lock-step batch path, kept from call to call (NULL until used)
 };
@@ -101,7 +101,10 @@ struct InferenceState {
 namespace {
 
 constexpr int TB = 256;
-constexpr uint64_t STEP_TICKS = 100000000;                   // a second: only a device that is not ours alone takes longer than some milliseconds
+constexpr uint64_t STEP_TICKS = 2000000;                     // 20 ms: a step takes up to six, longer only on a device that is not ours alone
+// Steps in launches after a wait that ran out, twice as many after each further one up to PAUSE_MOST, half as many once as many have gone well: two
+// processes that decode on one device may hold a part of its CUs each whenever their steps meet, and lose a hundredth of their time so
+constexpr int PAUSE = 64, PAUSE_MOST = 4096;
 
 // x = emb[token] * scale: the embedding row, scaled by sqrt(D) for Gemma3 (src/nn/fast_inference.c:385-391)
 __global__ __launch_bounds__(TB) void k_embed_row(const float *__restrict__ emb, int token, float scale, float *__restrict__ x, int D)
@@ -513,6 +516,7 @@ struct TokenRun {
     int *fail;                           // pinned: a wait ran out
     uint32_t tag;
     long steps;
+    int rest, pause, good;               // steps that go in launches yet; as many after the next wait that runs out; taken since the last one
 };
 
 void token_release(TokenRun *r)
@@ -578,7 +582,7 @@ TokenRun *token_acquire(InferenceState *s, int pos)
             return nullptr;
         }
         *r->fail = 0;
-        r->shape = shape; r->tag = 1;
+        r->shape = shape; r->tag = 1; r->pause = PAUSE;
         const size_t n = token_words(shape, nullptr, nullptr);
         r->words = metal_buf_create(n * 8);
         hipLaunchKernelGGL(k_clear_words, dim3((unsigned)((n + TB - 1) / TB)), dim3(TB), 0, stream(), dptr_as<unsigned long long>(r->words), n);
@@ -604,11 +608,12 @@ TokenRun *token_acquire(InferenceState *s, int pos)
 }
 
 // One step and the wait for it: the logits in logits_host, or the argmax in best_host.  false: not taken, or a wait ran out (the step is
-// to be taken again, and this state's steps go in launches from here on).
+// to be taken again, and the state's next ones go in launches).
 bool token_in_one_launch(InferenceState *s, int token, int pos, bool logits)
 {
     TokenRun *r = token_acquire(s, pos);
     if (!r) return false;
+    if (r->rest > 0) { r->rest--; return false; }
     TokenArgs &a = r->args;
     a.emb_row = dptr_as<float>(s->emb) + (size_t)token * s->D;
     a.logits_host = logits ? s->logits_host : nullptr;
@@ -619,8 +624,13 @@ bool token_in_one_launch(InferenceState *s, int token, int pos, bool logits)
     for (int L = 0; L < s->NL; L++) { mark_written(s->kc[L]); mark_written(s->vc[L]); }
     mark_written(s->logits);
     HIP_CHECK(hipStreamSynchronize(stream()));
-    if (*(volatile int *)r->fail) { s->steps_in_launches = true; return false; }
+    if (*(volatile int *)r->fail) {
+        *r->fail = 0;
+        r->rest = r->pause; r->pause = std::min(2 * r->pause, PAUSE_MOST); r->good = 0;
+        return false;
+    }
     r->steps++;
+    if (++r->good >= r->pause) { r->pause = std::max(r->pause / 2, PAUSE); r->good = 0; }
     return true;
 }
 

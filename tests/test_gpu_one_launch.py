@@ -82,6 +82,35 @@ def test_a_wait_that_runs_out_takes_the_step_again_in_launches():
         assert one_launch(inf) == 5 and len(best) >= 1
 
 
+def test_steps_are_one_launch_again_some_steps_after_a_wait_that_ran_out():
+    c = SHAPES["gemma_320"].with_(weight_format="f16")
+    model = make_model(c, seed=48, gamma_jitter=0.1)
+    with InferenceState(c, model, max_seq=256, use_fp16=True) as inf:
+        L, h, tok = inf.L, inf.h, lambda n: [inf.forward_token(t % c.V) for t in range(n)]
+        tok(3)
+        for rest in (64, 128):                             # twice as many after the second one
+            n = one_launch(inf)
+            L.hip_inference_step_wait(h, 0)
+            tok(1)
+            L.hip_inference_step_wait(h, 100000000)
+            tok(rest)
+            assert one_launch(inf) == n
+            tok(2)
+            assert one_launch(inf) == n + 2
+        # what the steps hand out behind a failed one, and behind the pause, is what they hand out without
+        got = inf.forward_token(5)
+        at = inf.position() - 1
+        inf.reset()
+        L.hip_gemm_profile_enable(1)
+        history = [t for n in (3, 1, 64, 2, 1, 128, 2) for t in range(n)]
+        assert len(history) == at
+        for t in history:
+            inf.forward_token(t % c.V)
+        want = inf.forward_token(5)
+        L.hip_gemm_profile_enable(0)
+        assert np.linalg.norm(got - want) < 200 * 2.0 ** -24 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("kw", [dict(D=1120), dict(IS=6880), dict(V=1002), dict(hd=64, Hq=16), dict(D=2624), dict(IS=10304)], ids=str)
 def test_shapes_that_stay_with_the_launches(kw):
     base = dict(NL=1, D=1152, Hq=4, Hkv=1, hd=256, IS=2048, V=1000)
