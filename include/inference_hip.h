@@ -102,6 +102,9 @@ int  inference_forward_token_argmax(InferenceState *state, int token);
  * the device for longer than `ticks` of 10 ns (20 ms unless set), the step is taken again in launches, and the state's next 64 steps go so too (twice
  * as many each further time, up to 4096).  No counterpart in the reference. */
 void hip_inference_step_wait(InferenceState *state, long long ticks);
+/* Such steps take some 200 KB of device memory per state, asked for by the first one; where the device has them no more, or a limit of `bytes` set
+ * before it forbids them, the state's steps go in launches. */
+void hip_inference_step_memory(InferenceState *state, size_t bytes);
 /* how many steps of the state have been one launch */
 long hip_inference_steps_in_one_launch(InferenceState *state);
 

@@ -95,6 +95,7 @@ struct InferenceState {
     TokenRun *one_launch;                // what a step in one launch needs (NULL until used)
     bool steps_in_launches;              // it cannot be had
     uint64_t step_ticks;                 // of the 100 MHz clock that a wait in it may last
+    size_t step_bytes;                   // of device memory that it may take
     BatchRun *batch;                     // scratch and caches of the lock-step batch path, kept from call to call (NULL until used)
 };
 
@@ -511,7 +512,8 @@ bool steps_on_run(const InferenceState *s) { return s->borrows_tiles || s->stack
 struct TokenRun {
     TokenShape shape;
     TokenArgs args;                      // what stays from step to step
-    MetalBuf *words, *table;             // hand-overs; the layers' addresses
+    unsigned long long *words;           // hand-overs, and behind them
+    uint64_t *table;                     // the layers' addresses
     std::vector<TokenLayer> layers;      // as the table holds them
     int *fail;                           // pinned: a wait ran out
     uint32_t tag;
@@ -522,8 +524,8 @@ struct TokenRun {
 void token_release(TokenRun *r)
 {
     if (!r) return;
-    metal_buf_free(r->words);
-    metal_buf_free(r->table);
+    hipStreamSynchronize(stream());
+    if (r->words) hipFree(r->words);
     if (r->fail) hipHostFree(r->fail);
     delete r;
 }
@@ -575,21 +577,24 @@ TokenRun *token_acquire(InferenceState *s, int pos)
     if (!ok) { s->steps_in_launches = true; return nullptr; }
     if (!s->one_launch) {
         TokenRun *r = new TokenRun();
-        if (hipHostMalloc((void **)&r->fail, sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        const size_t n = token_words(shape, nullptr, nullptr), bytes = n * 8 + s->NL * sizeof(TokenLayer);
+        // (a state that fills the device goes on in launches, which need none of this)
+        bool there = bytes <= s->step_bytes;
+        if (there && hipMalloc((void **)&r->words, bytes) != hipSuccess) { r->words = nullptr; there = false; }
+        if (there && hipHostMalloc((void **)&r->fail, sizeof(int), hipHostMallocDefault) != hipSuccess) { r->fail = nullptr; there = false; }
+        if (!there) {
             (void)hipGetLastError();
-            delete r;
+            token_release(r);
             s->steps_in_launches = true;
             return nullptr;
         }
         *r->fail = 0;
         r->shape = shape; r->tag = 1; r->pause = PAUSE;
-        const size_t n = token_words(shape, nullptr, nullptr);
-        r->words = metal_buf_create(n * 8);
-        hipLaunchKernelGGL(k_clear_words, dim3((unsigned)((n + TB - 1) / TB)), dim3(TB), 0, stream(), dptr_as<unsigned long long>(r->words), n);
-        r->table = metal_buf_create(s->NL * sizeof(TokenLayer));
+        r->table = (uint64_t *)(r->words + n);
+        hipLaunchKernelGGL(k_clear_words, dim3((unsigned)((n + TB - 1) / TB)), dim3(TB), 0, stream(), r->words, n);
         TokenArgs &a = r->args;
-        token_words(shape, &a, dptr_as<unsigned long long>(r->words));
-        a.layers = dptr_as<uint64_t>(r->table);
+        token_words(shape, &a, r->words);
+        a.layers = r->table;
         a.fail = r->fail;
         a.NL = s->NL; a.D = s->D; a.IS = s->IS; a.Hq = s->Hq; a.Hkv = s->Hkv; a.hd = s->hd; a.max_seq = s->max_seq; a.V = s->V;
         a.gemma = gemma; a.emb_scale = s->emb_scale; a.eps = s->eps; a.scale = 1.0f / sqrtf((float)s->hd);
@@ -598,7 +603,7 @@ TokenRun *token_acquire(InferenceState *s, int pos)
     TokenRun &r = *s->one_launch;
     if (r.layers.size() != now.size() || memcmp(r.layers.data(), now.data(), now.size() * sizeof(TokenLayer)) != 0) {
         r.layers = now;
-        HIP_CHECK(hipMemcpyAsync(dptr(r.table), r.layers.data(), now.size() * sizeof(TokenLayer), hipMemcpyHostToDevice, stream()));
+        HIP_CHECK(hipMemcpyAsync(r.table, r.layers.data(), now.size() * sizeof(TokenLayer), hipMemcpyHostToDevice, stream()));
         HIP_CHECK(hipStreamSynchronize(stream()));
     }
     r.args.head = (const void *)head; r.args.head_d = (const void *)head_d;
@@ -649,7 +654,7 @@ InferenceState *base_state(ModelType mt, int D, int V, int NL, int max_seq, Laye
     s->D = D; s->V = V; s->NL = NL;
     s->max_seq = max_seq; s->cur_len = 0; s->model_type = mt;
     s->stack = stack;
-    s->step_ticks = STEP_TICKS;
+    s->step_ticks = STEP_TICKS; s->step_bytes = SIZE_MAX;
     default_eos(s);
     HIP_CHECK(hipHostMalloc((void **)&s->logits_host, (size_t)V * 4, hipHostMallocDefault));
     HIP_CHECK(hipHostMalloc((void **)&s->best_host, sizeof(int), hipHostMallocDefault));
@@ -964,6 +969,7 @@ int inference_state_vocab_size(InferenceState *s) { return s->V; }
 void inference_state_reset(InferenceState *s) { s->cur_len = 0; }
 long hip_inference_steps_in_one_launch(InferenceState *s) { return s && s->one_launch ? s->one_launch->steps : 0; }
 void hip_inference_step_wait(InferenceState *s, long long ticks) { if (s && ticks >= 0) s->step_ticks = (uint64_t)ticks; }
+void hip_inference_step_memory(InferenceState *s, size_t bytes) { if (s) s->step_bytes = bytes; }
 int inference_state_position(InferenceState *s) { return s->cur_len; }
 
 static bool token_ok(InferenceState *s, int token)

@@ -111,6 +111,20 @@ def test_steps_are_one_launch_again_some_steps_after_a_wait_that_ran_out():
         assert np.linalg.norm(got - want) < 200 * 2.0 ** -24 * np.linalg.norm(want)
 
 
+def test_without_memory_for_its_words_a_state_decodes_in_launches():
+    c = SHAPES["gemma_320"].with_(weight_format="f16")
+    model = make_model(c, seed=49, gamma_jitter=0.1)
+    with InferenceState(c, model, max_seq=16, use_fp16=True) as inf:
+        inf.L.hip_gemm_profile_enable(1)
+        want = np.stack([inf.forward_token(t) for t in (1, 2, 3)])
+        inf.L.hip_gemm_profile_enable(0)
+        inf.reset()
+        inf.L.hip_inference_step_memory(inf.h, 1000)
+        got = np.stack([inf.forward_token(t) for t in (1, 2, 3)])
+        assert one_launch(inf) == 0 and np.array_equal(got, want)
+        assert inf.forward_token_argmax(4) >= 0 and one_launch(inf) == 0
+
+
 @pytest.mark.parametrize("kw", [dict(D=1120), dict(IS=6880), dict(V=1002), dict(hd=64, Hq=16), dict(D=2624), dict(IS=10304)], ids=str)
 def test_shapes_that_stay_with_the_launches(kw):
     base = dict(NL=1, D=1152, Hq=4, Hkv=1, hd=256, IS=2048, V=1000)
