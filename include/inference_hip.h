@@ -105,6 +105,9 @@ void hip_inference_step_wait(InferenceState *state, long long ticks);
 /* Such steps take some 200 KB of device memory per state, asked for by the first one; where the device has them no more, or a limit of `bytes` set
  * before it forbids them, the state's steps go in launches. */
 void hip_inference_step_memory(InferenceState *state, size_t bytes);
+/* The number that tells the words of the state's next such step from those before (0: it has taken none); `set` > 0 makes it that one, for tests of
+ * what happens where 32 bits end. */
+long long hip_inference_step_tag(InferenceState *state, long long set);
 /* how many steps of the state have been one launch */
 long hip_inference_steps_in_one_launch(InferenceState *state);
 

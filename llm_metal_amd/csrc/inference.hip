@@ -516,7 +516,8 @@ struct TokenRun {
     uint64_t *table;                     // the layers' addresses
     std::vector<TokenLayer> layers;      // as the table holds them
     int *fail;                           // pinned: a wait ran out
-    uint32_t tag;
+    size_t n_words;
+    uint64_t tag;                        // the next step's first; a step's NL + 1 fit 32 bits (next_tags)
     long steps;
     int rest, pause, good;               // steps that go in launches yet; as many after the next wait that runs out; taken since the last one
 };
@@ -534,6 +535,22 @@ __global__ __launch_bounds__(TB) void k_clear_words(unsigned long long *w, size_
 {
     const size_t i = (size_t)blockIdx.x * TB + threadIdx.x;
     if (i < n) w[i] = 0;
+}
+
+void clear_words(TokenRun &r)
+{
+    hipLaunchKernelGGL(k_clear_words, dim3((unsigned)((r.n_words + TB - 1) / TB)), dim3(TB), 0, stream(), r.words, r.n_words);
+    HIP_CHECK(hipGetLastError());
+}
+
+// Tags of a step: one per layer and one behind them, for all kinds of words alike, none of which a word may hold.  Every step writes all words but those
+// of the argmax, so only these could keep a tag until it is given out again: before that the words are cleared.
+uint32_t next_tags(TokenRun &r)
+{
+    if (r.tag + r.args.NL > UINT32_MAX) { clear_words(r); r.tag = 1; }
+    const uint32_t first = (uint32_t)r.tag;
+    r.tag += r.args.NL + 1;
+    return first;
 }
 
 // addresses of a weight's rows; false where they do not stay with the buffer or are not aligned
@@ -590,8 +607,9 @@ TokenRun *token_acquire(InferenceState *s, int pos)
         }
         *r->fail = 0;
         r->shape = shape; r->tag = 1; r->pause = PAUSE;
+        r->n_words = n;
         r->table = (uint64_t *)(r->words + n);
-        hipLaunchKernelGGL(k_clear_words, dim3((unsigned)((n + TB - 1) / TB)), dim3(TB), 0, stream(), r->words, n);
+        clear_words(*r);
         TokenArgs &a = r->args;
         token_words(shape, &a, r->words);
         a.layers = r->table;
@@ -623,8 +641,7 @@ bool token_in_one_launch(InferenceState *s, int token, int pos, bool logits)
     a.emb_row = dptr_as<float>(s->emb) + (size_t)token * s->D;
     a.logits_host = logits ? s->logits_host : nullptr;
     a.best_host = logits ? nullptr : s->best_host;
-    a.ticks = s->step_ticks; a.tag = r->tag; a.pos = pos;
-    r->tag += s->NL + 1;
+    a.ticks = s->step_ticks; a.tag = next_tags(*r); a.pos = pos;
     launch_token(a, r->shape, s->use_fp16 ? 0 : 1);
     for (int L = 0; L < s->NL; L++) { mark_written(s->kc[L]); mark_written(s->vc[L]); }
     mark_written(s->logits);
@@ -970,6 +987,12 @@ void inference_state_reset(InferenceState *s) { s->cur_len = 0; }
 long hip_inference_steps_in_one_launch(InferenceState *s) { return s && s->one_launch ? s->one_launch->steps : 0; }
 void hip_inference_step_wait(InferenceState *s, long long ticks) { if (s && ticks >= 0) s->step_ticks = (uint64_t)ticks; }
 void hip_inference_step_memory(InferenceState *s, size_t bytes) { if (s) s->step_bytes = bytes; }
+long long hip_inference_step_tag(InferenceState *s, long long set)
+{
+    if (!s || !s->one_launch) return 0;
+    if (set > 0) { clear_words(*s->one_launch); s->one_launch->tag = (uint64_t)set; }
+    return (long long)s->one_launch->tag;
+}
 int inference_state_position(InferenceState *s) { return s->cur_len; }
 
 static bool token_ok(InferenceState *s, int token)

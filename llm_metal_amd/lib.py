@@ -151,6 +151,7 @@ def load():
         "inference_state_model_type": (i, [vp]), "inference_state_vocab_size": (i, [vp]),
         "inference_state_reset": (None, [vp]), "inference_forward_token": (C.POINTER(C.c_float), [vp, i]),
         "inference_forward_token_argmax": (i, [vp, i]), "hip_inference_step_wait": (None, [vp, C.c_longlong]), "hip_inference_step_memory": (None, [vp, sz]),
+        "hip_inference_step_tag": (C.c_longlong, [vp, C.c_longlong]),
         "hip_inference_steps_in_one_launch": (C.c_long, [vp]), "inference_state_set_lora": (None, [vp, vp]),
         "inference_state_set_eos": (None, [vp, vp, i]), "inference_state_load_eos": (None, [vp, C.c_char_p]),
         "inference_state_position": (i, [vp]), "inference_forward_tokens": (i, [vp, vp, i, vp, i, vp]),

@@ -111,6 +111,27 @@ def test_steps_are_one_launch_again_some_steps_after_a_wait_that_ran_out():
         assert np.linalg.norm(got - want) < 200 * 2.0 ** -24 * np.linalg.norm(want)
 
 
+def test_tags_begin_anew_before_32_bits_end():
+    """A step's tags are NL + 1 numbers; zero, which words hold before they are first written, is none of them."""
+    c = SHAPES["gemma_320"].with_(weight_format="f16")
+    model = make_model(c, seed=50, gamma_jitter=0.1)
+    toks = list(range(1, 9))
+    with InferenceState(c, model, max_seq=16, use_fp16=True) as inf:
+        want = [inf.forward_token(t) for t in toks]
+        first = inf.L.hip_inference_step_tag(inf.h, 0)
+        for below in range(4 * c.NL + 8):
+            inf.reset()
+            assert inf.L.hip_inference_step_tag(inf.h, 2 ** 32 - below) == 2 ** 32 - below
+            for i, t in enumerate(toks[:6]):
+                assert np.array_equal(inf.forward_token(t), want[i]), (below, i)
+            # (nothing but these reads the words of the argmax)
+            assert [inf.forward_token_argmax(t) for t in toks[6:]] == [int(w.argmax()) for w in want[6:]], below
+            left = below // (c.NL + 1)                     # steps whose tags all lie below the end
+            if left < 8:
+                assert inf.L.hip_inference_step_tag(inf.h, 0) == 1 + (8 - left) * (c.NL + 1), below
+        assert first == 1 + 8 * (c.NL + 1) and one_launch(inf) == 8 * (4 * c.NL + 9)
+
+
 def test_without_memory_for_its_words_a_state_decodes_in_launches():
     c = SHAPES["gemma_320"].with_(weight_format="f16")
     model = make_model(c, seed=49, gamma_jitter=0.1)
