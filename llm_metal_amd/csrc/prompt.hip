@@ -643,7 +643,7 @@ bool prompt_attention_supported(int hd) { return hd == 32 || hd == 64 || hd == 1
 
 void launch_prompt_attention(const float *q, const float *kc, const float *vc, float *out, int M, int pos, int Hq, int Hkv, int hd, int max_seq)
 {
-    if (M <= 0 || pos < 0 || pos + M > max_seq || Hkv <= 0 || Hq % Hkv || (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)out) & 15)) {
+    if (M <= 0 || pos < 0 || pos + M > max_seq || Hkv <= 0 || Hq % Hkv || (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)(hd >= 128 ? vc : kc) | (uintptr_t)out) & 15)) {
         fprintf(stderr, "[fast_hip] prompt_attention: unsupported shape\n"); abort();
     }
     const int G = Hq / Hkv;
@@ -655,10 +655,10 @@ void launch_prompt_attention(const float *q, const float *kc, const float *vc, f
         else hipLaunchKernelGGL(k_prompt_attn_short<256>, waves, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale);
         return;
     }
-    // longest first; where all workgroups are resident at once, two to a CU, those that come second to one are the shortest first: 16 + 1 tiles
-    // meet, 15 + 2 .., where 16 + 8 to 8 + 1 did
+    // longest first; where all workgroups are resident at once, two to a CU, those that come second to one are the shortest first: of 512 on 256 CUs
+    // 16 + 1 tiles meet, 15 + 2 .., where 16 + 8 to 8 + 1 did
     const dim3 tall(Hkv, grid.x);
-    const int down = hd <= 128 && grid.x * grid.y <= 512 ? std::min<int>(grid.x, (256 + Hkv - 1) / Hkv) : (int)grid.x;
+    const int cus = num_cus(), down = hd <= 128 && (int)(grid.x * grid.y) <= 2 * cus ? std::min<int>(grid.x, (cus + Hkv - 1) / Hkv) : (int)grid.x;
 #define PA(HD_) hipLaunchKernelGGL(k_prompt_attn<HD_>, grid, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale)
 #define PS(HD_) hipLaunchKernelGGL(k_prompt_attn_split<HD_>, tall, dim3(TB), 0, stream(), q, kc, vc, out, M, pos, Hq, G, max_seq, scale, down)
     if (hd == 32) PA(32); else if (hd == 64) PA(64); else if (hd == 128) PS(128); else if (hd == 256) PS(256);
