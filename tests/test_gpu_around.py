@@ -96,6 +96,24 @@ def test_steps_of_one_token_on_few_and_many_keys(heads, kv_heads, dims, batch, t
 
 
 @FMT
+@pytest.mark.parametrize("n_bad", [3, 70])
+def test_a_token_that_is_not_finite_stays_in_its_chunk(n_bad, fmt, tmp_path):
+    """Steps of one token with heads of 128: keys and values that are not finite reach the later tokens of their chunk and no others, also
+    where a workgroup asks for a key again because it has no further one, and where they still lie in the ring."""
+    chunk, bad = 80, 7
+    cfg = around([(grouped(4, 2, 128, 128, chunk=chunk, dims=128), None)], width=64)
+    m = Model(cfg, tmp_path, edit=lambda name, a: np.where(np.arange(a.shape[0])[:, None] == bad, np.float32(np.inf), a) if name == "embed" else a)
+    toks = [t if t != bad else t + 1 for t in m.tokens(2 * chunk + 5, seed=9)]
+    want = so.run(cfg, m.W, toks)
+    toks[n_bad] = bad
+    with state(m, fmt, max_seq=len(toks)) as inf:
+        got = np.stack([inf.forward_token(t) for t in toks])
+        assert not np.isfinite(got[n_bad:chunk]).any()
+        for part in (slice(0, n_bad), slice(chunk, None)):           # (the head is the embedding: but for that row's logit)
+            assert logit_error(np.delete(got[part], bad, 1), np.delete(want[part], bad, 1)) < TOL[fmt]
+
+
+@FMT
 def test_a_reader_with_longer_chunks_than_the_keys_owner(fmt, tmp_path):
     """Keys that the layer which wrote them no longer sees are there for the layer that borrows them, in prompts longer than a
     step's portion would keep for the owner alone, and in decoding."""

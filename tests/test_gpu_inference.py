@@ -546,15 +546,22 @@ def test_logits_of_an_odd_vocabulary_behind_the_last_norm(D, V, model_type, fmt)
                                SFTConfig("q128", QWEN3, NL=1, D=128, Hq=8, Hkv=2, hd=128, IS=128, V=512),
                                SFTConfig("g256", GEMMA3, NL=1, D=128, Hq=8, Hkv=2, hd=256, IS=128, V=512, tied=True)], ids=lambda c: c.name)
 def test_attention_of_short_contexts_is_as_exact_as_that_of_long_ones(c):
-    """Against 64 bits over 60 tokens: the attention up to 256 keys and, with adapters of zeros attached, the one that takes any
-    number of keys.  They round 30000 logits differently: equal within 2 % (sums of sixteen columns in one were 3.4 % worse)."""
+    """Against 64 bits over 60 tokens: the attention up to 256 keys (heads of 128: inside the one launch of a step, and in a launch of its own)
+    and, with adapters of zeros attached, the one that takes any number of keys.  They round 30000 logits differently: equal
+    within 2 % (sums of sixteen columns in one were 3.4 % worse)."""
     model = make_model(c, seed=71, gamma_jitter=0.1)
     toks = [int(t) for t in np.random.default_rng(60).integers(0, c.V, 60)]
     want = oracle_decode(c, model, "f16", toks, 60, precision="f64")
     with InferenceState(c, model, max_seq=60) as inf:
         short = np.stack([inf.forward_token(t) for t in toks])
+        assert inf.L.hip_inference_steps_in_one_launch(inf.h) == (60 if c.hd == 128 else 0)
+        inf.reset()
+        inf.L.hip_gemm_profile_enable(1)                   # a profile counts launches
+        launches = np.stack([inf.forward_token(t) for t in toks])
+        inf.L.hip_gemm_profile_enable(0)
     with SFTState(c, model) as sft, InferenceState(c, model, max_seq=60) as inf:
         sft.set_lora(np.zeros_like(sft.lora()))
         inf.attach_lora(sft)
         other = np.stack([inf.forward_token(t) for t in toks])
     assert rel(short, want) < 1.02 * rel(other, want)
+    assert rel(launches, want) < 1.02 * rel(other, want)

@@ -1,5 +1,5 @@
-"""Steps of one sequence as one launch (token.hip) against the same steps in launches, which the oracle's decode chain is compared with
-elsewhere (test_gpu_inference.py): the largest and smallest widths that the one launch takes, shares of rows that do not come out even, columns
+"""Steps of one sequence as one launch (token.hip) against the same steps in launches; either way is compared with the oracle's decode chain
+elsewhere (test_gpu_inference.py).  The largest and smallest widths that the one launch takes, shares of rows that do not come out even, columns
 behind whole steps of 512, contexts up to and over its last key, and what it leaves to the launches."""
 import sys
 
@@ -58,7 +58,7 @@ def test_a_step_as_one_launch_is_the_step_in_launches(shape, fmt):
         srt = np.sort(want, axis=1)
         clear = srt[:, -1] - srt[:, -2] > 1e-4 * np.abs(srt[:, -1])
         assert clear.mean() > 0.9 and (np.asarray(best)[clear] == want.argmax(1)[clear]).all()
-        # the first of equal maxima is the argmax of what the call beside it hands out
+        # the argmax is that of what the call beside it hands out
         inf.reset()
         assert best[0] == int(got[0].argmax()) == inf.forward_token_argmax(toks[0])
 
@@ -111,6 +111,58 @@ def test_steps_are_one_launch_again_some_steps_after_a_wait_that_ran_out():
         assert np.linalg.norm(got - want) < 200 * 2.0 ** -24 * np.linalg.norm(want)
 
 
+# pairs of rows of a head that 80 workgroups share, 200 rows each, 80 at a time: neighbours of a unit, another wave's, another part of the workgroup's,
+# another workgroup's, the first and the last
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+@pytest.mark.parametrize("rows", [(8000, 8001), (8003, 8075), (8003, 8150), (8199, 8200), (3, 12007), (0, 15999)], ids=str)
+def test_the_first_of_equal_maxima(rows, fmt):
+    c = SHAPES["gemma_320"].with_(weight_format=fmt, V=16000, NL=2)
+    model = make_model(c, seed=51, gamma_jitter=0.1)
+    toks = [5, 6, 7]                                       # (the head is the embedding: rows that no token reads are changed)
+    def steps():
+        with InferenceState(c, model, max_seq=8, use_fp16=fmt == "f16") as inf:
+            logits = [inf.forward_token(t) for t in toks]
+            inf.reset()
+            best = [inf.forward_token_argmax(t) for t in toks]
+            assert one_launch(inf) == 2 * len(toks)
+            return logits, best
+    logits, _ = steps()
+    emb = model["token_emb"]
+    at = 20 + int(logits[2][20:].argmax())
+    emb[list(rows)] = 4 * emb[at]
+    logits, best = steps()
+    assert logits[2][rows[0]] == logits[2][rows[1]] == logits[2].max()       # (one step of columns: a row's sum does not depend on its place)
+    assert best == [int(l.argmax()) for l in logits] and best[2] == rows[0]
+
+
+def test_values_that_are_not_finite():
+    """Against the steps in launches: a token whose embedding is infinite, one whose embedding overflows on the way, and rows of the head that
+    are not finite.  An argmax passes over logits that are no number, and is zero where all are."""
+    c = SHAPES["qwen_1344"].with_(weight_format="f16")
+    model = make_model(c, seed=52, gamma_jitter=0.1)
+    model["token_emb"][9] = np.inf
+    model["token_emb"][10] = 1e30
+    model["lm_head"][7, 3], model["lm_head"][600, 5], model["lm_head"][601] = np.inf, -np.inf, np.nan
+    def steps(inf, toks):
+        inf.reset()
+        logits = np.stack([inf.forward_token(t) for t in toks])
+        inf.reset()
+        return logits, [inf.forward_token_argmax(t) for t in toks]
+    for toks in ([1, 2, 3, 4], [1, 2, 9, 3, 4], [9, 1], [1, 10, 2] + list(range(11, 80))):
+        with InferenceState(c, model, max_seq=80, use_fp16=True) as inf:
+            got, best = steps(inf, toks)
+            assert one_launch(inf) == 2 * len(toks)
+            inf.L.hip_gemm_profile_enable(1)
+            want, want_best = steps(inf, toks)
+            inf.L.hip_gemm_profile_enable(0)
+        assert best == want_best, toks
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got) * np.sign(got), np.isinf(want) * np.sign(want), equal_nan=True), toks
+        ok = np.isfinite(want)
+        assert np.linalg.norm(got[ok] - want[ok]) <= 200 * 2.0 ** -24 * np.linalg.norm(want[ok])
+        if 9 in toks:
+            assert np.isnan(got[toks.index(9):]).all() and set(best[toks.index(9):]) == {0}
+
+
 def test_tags_begin_anew_before_32_bits_end():
     """A step's tags are NL + 1 numbers; zero, which words hold before they are first written, is none of them."""
     c = SHAPES["gemma_320"].with_(weight_format="f16")
@@ -155,6 +207,29 @@ def test_shapes_that_stay_with_the_launches(kw):
         for t in (1, 2, 3):
             assert np.isfinite(inf.forward_token(t)).all()
         assert one_launch(inf) == 0
+
+
+# the last that fit and the first that do not, in turn: products of heads and their size, layers, a workgroup's rows where few of them share a product,
+# heads beside workgroups for the O product
+@pytest.mark.parametrize("kw,taken", [
+    (dict(D=1152, hd=256, Hq=4, Hkv=1), True), (dict(D=1152, hd=256, Hq=5, Hkv=1), False),
+    (dict(D=1152, hd=128, Hq=32, Hkv=8), True), (dict(D=1152, hd=128, Hq=33, Hkv=11), False),
+    (dict(NL=48), True), (dict(NL=49), False),
+    (dict(D=64, IS=640), True), (dict(D=64, IS=704), False),
+    (dict(D=64, Hq=8), True), (dict(D=64, Hq=9), False)], ids=str)
+def test_on_either_side_of_what_fits(kw, taken):
+    c = SFTConfig("t", QWEN3, **{**dict(NL=1, D=128, Hq=2, Hkv=1, hd=128, IS=384, V=260), **kw}).with_(weight_format="f16")
+    model = make_model(c, seed=53, gamma_jitter=0.1)
+    toks = list(range(8))
+    with InferenceState(c, model, max_seq=8, use_fp16=True) as inf:
+        got = np.stack([inf.forward_token(t) for t in toks])
+        assert one_launch(inf) == (len(toks) if taken else 0)
+        inf.L.hip_gemm_profile_enable(1)
+        inf.reset()
+        want = np.stack([inf.forward_token(t) for t in toks])
+        inf.L.hip_gemm_profile_enable(0)
+    # (roundings in a row grow with the layers: some 40 of each)
+    assert np.linalg.norm(got - want) <= max(200, 40 * c.NL) * 2.0 ** -24 * np.linalg.norm(want)
 
 
 # either side of the line: vocabularies that few workgroups read too slowly, layers of narrow Q8_0 models with heads of 128, which cost more than

@@ -144,8 +144,8 @@ def test_widths_of_decoded_rows(width, tmp_path):
 @pytest.mark.parametrize("vocab", [3, 161, 4098, 140003])
 @pytest.mark.parametrize("around_layers", [False, True])
 def test_logits_that_go_to_the_host_as_they_are_formed(around_layers, vocab, tmp_path):
-    """A wave of the head writes its rows 64 at a time: fewer rows than waves, odd ones, and 70 per wave.  What a step hands out is
-    what the same step leaves on the device, from where a portion's wanted rows are copied."""
+    """A wave of the head writes its rows 64 at a time: fewer rows than waves, odd ones, and 70 per wave.  A portion of one token hands
+    out the same bits, a longer one's rows are other sums."""
     say("host logits", around_layers, vocab)
     cfg = around([(grouped(2, 1, 16, 16, 9), dense(40))], width=64, vocab=vocab) if around_layers else config([(delta(2, 1, 16, 16, 2), None)], width=64, vocab=vocab)
     m = Model(cfg, tmp_path)
@@ -162,6 +162,34 @@ def test_logits_that_go_to_the_host_as_they_are_formed(around_layers, vocab, tmp
         inf.reset()
         one = [inf.forward_tokens(toks[:2], [1])[0], inf.forward_tokens(toks[2:], [1])[0]]
         assert logit_error(np.stack(one), several) < TOL["f16"] and logit_error(np.stack(one), want[1::2]) < TOL["f16"]
+
+
+@pytest.mark.parametrize("vocab", [3, 161, 4098, 140003])
+@pytest.mark.parametrize("around_layers", [False, True])
+def test_the_largest_logit_is_found_in_every_row(around_layers, vocab, tmp_path):
+    """The argmax reads the rows that the head leaves on the device beside those it writes to the host: the largest in turn in the
+    first, the last and rows on either side of a wave's 64, behind a step that left the largest elsewhere."""
+    say("argmax rows", around_layers, vocab)
+    cfg = around([(grouped(2, 1, 16, 16, 9), dense(40))], width=64, vocab=vocab) if around_layers else config([(delta(2, 1, 16, 16, 2), None)], width=64, vocab=vocab)
+    toks = [0, 2, 1, 0]
+    m = Model(cfg, tmp_path / "as drawn")
+    with state(m, "f16") as inf:
+        base = np.stack([inf.forward_token(t) for t in toks])
+    for row in sorted({r for r in (0, 1, 62, 63, 64, 69, 70, vocab // 2, vocab - 2, vocab - 1) if 0 <= r < vocab}):
+        best = int(base[1].argmax())
+
+        def place(name, a):
+            if name != ("embed" if around_layers else "head"):
+                return a
+            a = a.copy()
+            a[row] = a[best] * np.float32(4 if base[1][best] > 0 else 0.25)
+            return a
+        m = Model(cfg, tmp_path / str(row), edit=place)
+        with state(m, "f16") as inf:
+            got = np.stack([inf.forward_token(t) for t in toks])
+            assert int(got[1].argmax()) == row or around_layers and row in toks          # (there the head is the embedding)
+            inf.reset()
+            assert [inf.forward_token_argmax(t) for t in toks] == [int(g.argmax()) for g in got], row
 
 
 @pytest.mark.parametrize("window", [1, 2, 15, 16, 17, 63, 64, 65, 100])
