@@ -142,8 +142,9 @@ def decode_cpu_baseline(cfg):
 
 
 def decode_bench(args, cfg, L):
-    """Greedy generation, one token per step; the matrix-vector kernel is the dominant kernel and every one of its
-    launches is timed with HIP events on the library's stream in a second pass."""
+    """Greedy generation, one token per step.  A step that is one launch is its own dominant kernel, timed by the steps themselves (the host's
+    wait included); otherwise the matrix-vector kernel is, and every one of its launches is timed with HIP events on the library's stream in
+    a second pass, which counts the weights' bytes for either."""
     import ctypes as C
     from llm_metal_amd.sft import InferenceState, SFTState
     f16 = cfg.weight_format == "f16"
@@ -166,11 +167,13 @@ def decode_bench(args, cfg, L):
     for _ in range(args.warmup):
         tok = inf.forward_token_argmax(tok)
     L.metal_flush()
+    whole = L.hip_inference_steps_in_one_launch(inf.h)
     t1 = time.perf_counter()
     for _ in range(args.steps):
         tok = inf.forward_token_argmax(tok)
     L.metal_flush()
     dt = time.perf_counter() - t1
+    whole = L.hip_inference_steps_in_one_launch(inf.h) - whole == args.steps
     prof_steps = max(1, min(5, args.steps))
     L.hip_gemm_profile_enable(1)
     for _ in range(prof_steps):
@@ -199,7 +202,10 @@ def decode_bench(args, cfg, L):
     inf.free()
     if sft is not None:
         sft.free()
-    gbs = wb.value / (tms.value * 1e-3) / 1e9 if tms.value > 0 else 0.0
+    kernel, launches, kernel_ms = "k_matvec" if sft is None else "gemm_ring", n // prof_steps, tms.value / prof_steps
+    if whole:
+        kernel, launches, kernel_ms = "k_token", 1, dt / args.steps * 1e3
+    gbs = wb.value / prof_steps / (kernel_ms * 1e-3) / 1e9 if kernel_ms > 0 else 0.0
     out = {"metric": "greedy decode tokens/s, batch 1", "value": round(args.steps / dt, 1), "unit": "tokens/s", "n_gpus": 1,
            "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(dt / args.steps * 1e3, 3), "higher_is_better": True,
            "scaling": "weak", "vs_baseline": None, "dtype": "f16 weights x f32 activations, f32 accumulate" if f16 else
@@ -209,9 +215,9 @@ def decode_bench(args, cfg, L):
                       "weights": "own row-major matrices" if sft is None else "the training state's tiles, read in place"},
            "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
-                        "kernel": "k_matvec" if sft is None else "gemm_ring",
-                        "launches_per_step": n // prof_steps, "avg_launch_us": round(tms.value * 1e3 / max(n, 1), 2),
-                        "weight_bytes_per_step": wb.value / prof_steps, "matvec_ms_per_step": round(tms.value / prof_steps, 3)},
+                        "kernel": kernel,
+                        "launches_per_step": launches, "avg_launch_us": round(kernel_ms * 1e3 / max(launches, 1), 2),
+                        "weight_bytes_per_step": wb.value / prof_steps, "matvec_ms_per_step": round(kernel_ms, 3)},
            "setup_s": {"generate_weights": round(t_gen, 1), "upload_convert": round(t_init, 1)}}
     if batch:
         out["batched"] = batch

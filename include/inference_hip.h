@@ -97,8 +97,11 @@ const float *inference_forward_token(InferenceState *state, int token);
 int  inference_forward_token_argmax(InferenceState *state, int token);
 
 /* A step that the host waits for (the two calls above, inference_generate, places of inference_forward_tokens taken one by one) is one launch in
- * which all CUs take part, where the state has its own weights without adapters, up to 256 keys, heads of 128 or 256, and widths of whole 64 columns (d_model
- * <= 2560, FFN <= 10240, vocabulary a multiple of 4); otherwise five launches per layer.  Its workgroups wait for each other; should some be kept off
+ * which all CUs take part, where the state has its own weights without adapters, up to 256 keys, at most 48 layers, heads of 128 (all query heads
+ * together up to 4096 columns) or of 256 (up to 1024), widths of whole 64 columns (d_model <= 2560, FFN <= 10240), a vocabulary that is a multiple of 4, and
+ * enough workgroups -- a quarter of d_model, half of the FFN, at most one per CU -- that these are twice the query heads and none has more than 80 rows of
+ * a layer's product (of the O product without a workgroup per query head); and where it is the faster way, which long vocabularies over narrow models
+ * and narrow Q8_0 models of many layers with heads of 128 are not.  Otherwise five launches per layer.  Its workgroups wait for each other; should some be kept off
  * the device for longer than `ticks` of 10 ns (20 ms unless set), the step is taken again in launches, and the state's next 64 steps go so too (twice
  * as many each further time, up to 4096).  No counterpart in the reference. */
 void hip_inference_step_wait(InferenceState *state, long long ticks);

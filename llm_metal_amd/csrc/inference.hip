@@ -566,8 +566,12 @@ bool token_rows(InferenceState *s, const WMat *w, int rows, int cols, uint64_t *
 }
 
 // The run, with the layers' addresses as they are now; NULL: the step goes in launches.  Those it is for: the matrix-vector pipeline's own
-// weights without adapters, contexts of up to TOKEN_KEYS keys (what its attention is made for; k_attn_short's line too), shapes that the kernel holds
-// (token_fits) and for which it is the faster way (token_pays).  A profile of the products wants launches to count.
+// weights without adapters, contexts of up to TOKEN_KEYS keys, shapes that the kernel holds (token_fits) and for which it is the faster way (token_pays).
+// A profile of the products wants launches to count.
+// TOKEN_KEYS is where k_attn_short ends, up to which launches and one launch were compared, and not where the one launch falls behind.  Microseconds of
+// a greedy token at 200 / 300 / 1000 / 2000 keys, launches -> its attention's loop carried on: eight Gemma3-1B layers F16 273 -> 245 / 573 -> 271 /
+// 579 -> 428 / 588 -> 657, Q8_0 261 -> 211 / 557 -> 227 / 576 -> 351 / 577 -> 534; six 4B layers F16 340 -> 319 / 518 -> 328 / 531 -> 390 / 537 -> 479, Q8_0 267 ->
+// 250 / 448 -> 259 / 459 -> 321 / 462 -> 411; twelve of width 1024 F16 288 -> 272 / 541 -> 293 / 556 -> 448 / 570 -> 669.
 TokenRun *token_acquire(InferenceState *s, int pos)
 {
     if (s->steps_in_launches || steps_on_run(s) || !s->lora.empty() || pos >= TOKEN_KEYS || gemm_profiling()) return nullptr;

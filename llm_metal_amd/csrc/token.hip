@@ -5,7 +5,7 @@
 // one workgroup for the whole token, and what a product leaves passes from CU to CU as words of (value, tag): 64-bit device-scope
 // atomics, relaxed, each of which carries its own proof of arrival, so no flag, no fence and no write-back of caches stands between
 // the workgroup that wrote a value and the one that multiplies it.  A hand-over between all 256 workgroups takes 1.9 us for 1152 values
-// and 2.5 for 6912, with its barrier and LDS trip.
+// and 2.4 for 6912, with its barrier and LDS trip.
 //
 // Workgroup: sixteen waves.  The weights that a wave multiplies, product after product from the first layer to the head, come into a ring
 // in LDS of its own, RING slots ahead -- across products and layers, since weights depend on nothing.  A slot is 512 columns of R rows
@@ -18,8 +18,8 @@
 // of code for the slots of all products (with a copy per product, unrolled over stages in registers, the kernel was 118 KB, twice the instruction
 // cache: 30 us per layer of Gemma3-1B), all waves at the slots (with eight that multiply and eight that form vectors 38 us; a slot is a chain of 0.5 us) and
 // no more waves than it takes at everything else (sixteen share four issue slots).
-// Per token, greedy, contexts of 100, in five launches per layer -> so: Gemma3-1B Q8_0 735 -> 618 us, nine layers of Qwen3-4B F16 with a head of
-// 32 768 rows 487 -> 435.  Bound by the hand-overs and, Q8_0, by instructions (two per weight); F16 by the stream (5.5 TB/s while it flows).
+// Per token, greedy, contexts of up to 128, in five launches per layer -> so: Gemma3-1B Q8_0 734 -> 617 us, nine layers of Qwen3-4B F16 with a head of
+// 32 768 rows 480 -> 437.  Bound by the hand-overs and, Q8_0, by instructions (two per weight); F16 by the stream (5.5 TB/s while it flows).
 //
 // Words are reused layer after layer without a wait for readers: whoever writes one of a kind again has, through the vectors
 // between, seen a word from every workgroup that it wrote after its last look at the kind (all workgroups have rows of gate|up and
