@@ -17,6 +17,7 @@
 #include "devutil.h"
 #include "gemm.h"
 #include "gemm_kernel.h"
+#include "acc_tiles.h"
 #include <hip/hip_ext.h>
 #include <algorithm>
 
@@ -252,26 +253,12 @@ __global__ __launch_bounds__(256) void gemm_big(GemmKArgs g)
 }
 
 
-// F16 weight tiles need no unpacking, so their steps go from L2/HBM straight into LDS (global_load_lds_dwordx4: a
-// wave-uniform LDS base in M0, lane i's 16 bytes land at base + 16 i -- the [j][lane] order of the tiles) and never
-// pass through registers or ds_write.  K goes in half steps of 32 (two of a tile's four 1 KB slices per row block)
-// through six 24 KB LDS buffers, distinct objects: half step h is multiplied out of buffer h % 6 while h + 1 .. h + 5
-// are in LDS or on their way.  The copies are issued as assembly right after the barrier, so the compiler does not count
-// them among its own loads (it cannot tell which LDS bytes a pending copy writes and would wait for all of them before
-// every LDS read); the wait before the barrier is written by hand: the barrier that ends half step h - 1 finds h and
-// h + 1 in LDS -- every wave has waited for its own copies of them -- so slice 0 of h + 1 is read under the MFMAs of
-// slice 1 of h and no half step starts by waiting out an LDS round trip; h + 5 is requested into the buffer h - 1 left.
-//
-// GROUPED: the 128-row blocks of A belong to different weights of one shape, laid group.stride halves apart: block mt is
-// multiplied with number group.of[mt]; only the first group.of[M / 128] blocks have rows.
-//
-// SHORT: no sum of more than twelve MFMAs in one accumulator.  The matrix cores round an accumulator at every instruction, so a
-// sum over K = 2560 in one is 2.5 times as far from the exact one as a matrix-vector product's (units of 2^-24 of the result's
-// norm, 64 rows: 5.5 against 2.2; K = 9728: 10.5 against 3.9).  Two of the eight accumulators of a wave are added to sums of their own
-// in each of four half steps out of six, under the MFMAs of the others, and start again from zero.
-struct GroupArgs { const int *of; size_t stride; };
-template <bool GROUPED, bool SHORT = false>
-__global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group)
+// The product of operands that hold more than fp16 (value and residual rows): no sum of more than twelve MFMAs in one accumulator.  The
+// matrix cores round an accumulator at every instruction, so a sum over K = 2560 in one is 2.5 times as far from the exact one as a
+// matrix-vector product's (units of 2^-24 of the result's norm, 64 rows: 5.5 against 2.2; K = 9728: 10.5 against 3.9).  Two of the
+// eight accumulators of a wave are added to sums of their own in each of four half steps out of six, under the MFMAs of the
+// others, and start again from zero.  The walk through K is that of gemm_big_f16, below, in 32x32x16 instructions.
+__global__ __launch_bounds__(256) void gemm_big_short(GemmKArgs g)
 {
     constexpr int HB = 12 * 2 * 64;                       // half8 per buffer: [4 A + 8 W row blocks][2 slices][64 lanes]
     __shared__ half8 lb0[HB], lb1[HB], lb2[HB], lb3[HB], lb4[HB], lb5[HB];
@@ -280,13 +267,7 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
     const int MT = (g.M + 127) >> 7, NT = (g.N + 255) >> 8;
     const int m_patches = (MT + 7) >> 3;
     int mt, nt, chunk = 0;
-    if (GROUPED) {
-        // the blocks that have rows, column blocks first, dealt to the XCDs in contiguous shares: the row blocks of a weight
-        // meet in one L2, and few column blocks leave no XCD without work
-        const int total = group.of[MT] * NT, share = (total + 7) >> 3, seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * share + seq;
-        if (seq >= share || t >= total) return;
-        mt = t / NT; nt = t % NT;
-    } else if (g.m_tiles) {
+    if (g.m_tiles) {
         // few row blocks: those of one (column block, chunk) are consecutive workgroups of one XCD, so a weight tile comes
         // from memory once; the pairs are dealt to the XCDs in turn
         const int slot = blockIdx.x >> 3, pair = (slot / MT) * 8 + (blockIdx.x & 7);
@@ -302,10 +283,6 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
         if (mt >= MT || nt >= NT) return;
     }
     const int nb0 = nt * 8, mb0 = mt * 4;
-    if (GROUPED) {
-        const int e = __builtin_amdgcn_readfirstlane(group.of[mt]);
-        g.W.w16 += (size_t)e * group.stride;
-    }
     const int wm = wave >> 1, wn = wave & 1;
     const int k_beg = chunk * g.steps_per_chunk, nsteps = min(g.Kb, k_beg + g.steps_per_chunk) - k_beg;
     const int nhalf = 2 * nsteps, last = nhalf - 1;
@@ -354,13 +331,13 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                if (SHORT && k == out) {
+                if (k == out) {
                     sum[i][k] += acc[i][k];
                     acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], float16v{}, 0, 0, 0);
                 } else acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], acc[i][k], 0, 0, 0);
             }
     };
-    // (out: SHORT's column of accumulators to add to the sums)
+    // (out: the column of accumulators to add to the sums)
     auto step = [&](int hs, int out, const half8 (&cur)[HB], const half8 (&nxt)[HB], half8 (&free_buf)[HB]) __attribute__((always_inline)) {
         request(free_buf, min(hs + 5, last));
         half8 a1[2], w1[4];
@@ -396,12 +373,10 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
     if (full + 3 < nhalf) step(full + 3, 3, lb3, lb4, lb2);
     if (full + 4 < nhalf) step(full + 4, 4, lb4, lb5, lb3);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (SHORT) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) acc[i][k] += sum[i][k];
-    }
+        for (int k = 0; k < 4; k++) acc[i][k] += sum[i][k];
 
     if (mb0 * 32 + 128 <= g.M && (nb0 + 8) * 32 <= g.N) {
         float sc[2][16];
@@ -441,26 +416,43 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
 }
 
 
-// The same product on a 256 x 256 block: four waves of 128 x 128 (sixteen accumulator tiles each, in the accumulation
-// registers), so that a wave reads 0.5 KB of LDS per MFMA instead of 0.75 and a block fetches half as many operand bytes
-// per flop.  K goes in half steps of 32 (two of a tile's four 1 KB slices per row block) through five 32 KB LDS buffers
-// (all 160 KB of a CU): half step h is multiplied out of buffer h % 5 while h + 1 .. h + 4 are in LDS or on their way.
-// The copies are LDS-direct loads issued as assembly, right after the barrier: the compiler does not count them among
-// its own loads (it cannot tell which LDS bytes a pending copy writes and would wait for all of them before every LDS
-// read); the wait before the barrier is written by hand.
-// 8192 x 8192 x 8192 on random operands: 1 227 TFLOP/s against 1 083 for 128 x 256 (constant operands, which toggle few
-// bits and let the GPU hold a higher clock, give 1 667 and 1 387).  There are half as many blocks: launch_gemm_big picks
-// the shape that loses less to partial rounds and partial tiles.
-__global__ __launch_bounds__(256) void gemm_big_f16_256(GemmKArgs g)
+// F16 weight tiles need no unpacking, so their steps go from L2/HBM straight into LDS (global_load_lds_dwordx4: a
+// wave-uniform LDS base in M0, lane i's 16 bytes land at base + 16 i -- the [j][lane] order of the tiles) and never
+// pass through registers or ds_write.  BM x 256 outputs per workgroup, four waves of BM / 2 x 128.  K goes in half steps of
+// 32 (two of a tile's four 1 KB slices per row block) through a ring of LDS buffers (256 rows: five of 32 KB, all of a CU's
+// 160 KB; 128 rows: six of 24 KB): half step h is multiplied out of buffer h % NB while h + 1 .. h + NB - 1 are in LDS or on
+// their way.  The barrier that ends half step h - 1 finds h and h + 1 in LDS (every wave has waited for its own copies of
+// them), so the fragments of h + 1 are read under the MFMAs of h; h + NB - 1 is requested into the buffer that h - 1 left.
+//
+// What bounds it: the matrix cores' power.  On random operands the clock settles where the power limit is -- 1.5 to 1.75 GHz
+// under this loop, 2.4 on constant operands -- so what counts is energy per flop as much as idle cycles.  v_mfma_f32_16x16x32
+// takes the K = 32 of a half step at once and moves half the accumulator bytes per flop that 32x32x16 does; its sums are the same, bit for
+// bit.  A half step's two slices hold exactly the two fragments of a row block: lane l of the fragment of rows 16 s .. 16 s + 15
+// reads slice l >> 5, column half (l >> 4) & 1, row 16 s + (l & 15), conflict-free.  The MFMAs are assembly on accumulators in place (acc_tiles.h). With them pinned, one LDS read
+// or one copy goes under every second or third MFMA instead of all copies behind the barrier, where the matrix cores waited for them (a
+// K step of 64 took 2 800 cycles for 2 048 of MFMAs, now 2 370).  Random operands, alone: 2048 x 8192 x 9728 312 -> 241 us (1 045 -> 1 354 TFLOP/s), 2048 x 16384 x 2560 188 -> 148,
+// 8192^3 988 -> 799 us (1 113 -> 1 375); 16x16x32 with the copies in one burst 264, 174 and 850 us, 32x32x16 with them spread 261, 151, 848.
+//
+// GROUPED: the row blocks of A belong to different weights of one shape, laid group.stride halves apart: block mt is
+// multiplied with number group.of[mt]; only the first group.of[M / BM] blocks have rows.
+struct GroupArgs { const int *of; size_t stride; };
+template <int BM, bool GROUPED = false>
+__global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group)
 {
-    constexpr int HB = 16 * 2 * 64;                       // half8 per buffer: [16 row blocks][2 slices][64 lanes]
-    __shared__ half8 lb0[HB], lb1[HB], lb2[HB], lb3[HB], lb4[HB];
+    constexpr int AB = BM / 32, MI = BM / 32, AU = AB / 4;    // A row blocks of the block; 16-row tiles of a wave; A row blocks a wave fetches
+    constexpr int HB = (AB + 8) * 128, NB = BM == 256 ? 5 : 6;   // half8 per buffer: [AB A + 8 W row blocks][2 slices][64]; buffers
+    __shared__ half8 lds[NB * HB];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r = lane & 31, h = lane >> 5;
-    const int MT = (g.M + 255) >> 8, NT = (g.N + 255) >> 8;
+    const int MT = (g.M + BM - 1) / BM, NT = (g.N + 255) >> 8;
     const int m_patches = (MT + 7) >> 3;
     int mt, nt, chunk = 0;
-    if (g.m_tiles) {
+    if (GROUPED) {
+        // the blocks that have rows, column blocks first, dealt to the XCDs in contiguous shares: the row blocks of a weight
+        // meet in one L2, and few column blocks leave no XCD without work
+        const int total = group.of[MT] * NT, share = (total + 7) >> 3, seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * share + seq;
+        if (seq >= share || t >= total) return;
+        mt = t / NT; nt = t % NT;
+    } else if (g.m_tiles) {
         // few row blocks: those of one (column block, chunk) are consecutive workgroups of one XCD, so a weight tile comes
         // from memory once; the pairs are dealt to the XCDs in turn
         const int slot = blockIdx.x >> 3, pair = (slot / MT) * 8 + (blockIdx.x & 7);
@@ -475,130 +467,136 @@ __global__ __launch_bounds__(256) void gemm_big_f16_256(GemmKArgs g)
         nt = ((patch / m_patches) * 4 + (in_patch >> 3)) * 8 + xcd;
         if (mt >= MT || nt >= NT) return;
     }
-    const int nb0 = nt * 8, mb0 = mt * 8;
+    const int nb0 = nt * 8, mb0 = mt * AB;
+    if (GROUPED) g.W.w16 += (size_t)__builtin_amdgcn_readfirstlane(group.of[mt]) * group.stride;
     const int wm = wave >> 1, wn = wave & 1;
-    const int k_beg = chunk * g.steps_per_chunk, nsteps = min(g.Kb, k_beg + g.steps_per_chunk) - k_beg;
-    const int nhalf = 2 * nsteps, last = nhalf - 1;
-    // this wave's share of a half step: both slices of A row blocks w, 4 + w and of W row blocks w, 4 + w
-    const half8 *src[4];
-    src[0] = g.A + ((size_t)min(mb0 + wave, g.Mb - 1) * g.Kb + k_beg) * 256 + a_lane(lane);
-    src[1] = g.A + ((size_t)min(mb0 + 4 + wave, g.Mb - 1) * g.Kb + k_beg) * 256 + a_lane(lane);
-    src[2] = reinterpret_cast<const half8 *>(g.W.w16) + ((size_t)min(nb0 + wave, g.Nb - 1) * g.Kb + k_beg) * 256 + lane;
-    src[3] = reinterpret_cast<const half8 *>(g.W.w16) + ((size_t)min(nb0 + 4 + wave, g.Nb - 1) * g.Kb + k_beg) * 256 + lane;
-    const int dst[4] = {wave, 4 + wave, 8 + wave, 12 + wave};
+    const int k_beg = chunk * g.steps_per_chunk, nhalf = 2 * (min(g.Kb, k_beg + g.steps_per_chunk) - k_beg), last = nhalf - 1;
     float *const Cp = g.P + (size_t)chunk * g.plane_stride;
-
-    float16v acc[4][4];
+    // this wave's rows of C from m0 on, of which a lane ends with 16 j + mq .. + 3 and their factors; its columns from n0 on, 16 i + nr
+    const int m0 = mb0 * 32 + wm * (BM / 2), n0 = (nb0 + 4 * wn) * 32, mq = 4 * (lane >> 4), nr = lane & 15;
+    float sc[MI][4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int j = 0; j < MI; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int v = 0; v < 4; v++) sc[j][v] = 1.0f;
+    if (g.a_inv_scale) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-
-    typedef __attribute__((address_space(3))) void lds_void;
-    uint32_t loff[4][2];                                   // byte offsets inside a buffer of this wave's eight 1 KB pieces
+        for (int j = 0; j < MI; j++)
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) loff[u][j] = __builtin_amdgcn_readfirstlane((uint32_t)((dst[u] * 2 + j) * 64 * 16));
-    auto request = [&](half8 (&buf)[HB], int hs) __attribute__((always_inline)) {
-        const size_t o = (size_t)(hs >> 1) * 256 + (hs & 1) * 128;
-        const uint32_t base = (uint32_t)(uintptr_t)(lds_void *)buf;
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(src[u] + o + j * 64), "s"(base + loff[u][j]) : "m0");
-    };
-    constexpr int LOADS = 4 * 2, AHEAD = 4, LANDED = 2;    // copies per request and wave; requests in flight after a request; how many a barrier needs
-    constexpr int WAIT = (AHEAD - LANDED) * LOADS;
-    static_assert(WAIT == 16 && AHEAD * LOADS < 64, "the hand-written waits count this wave's LDS-direct loads; vmcnt has six bits");
-    half8 a0[4], w0[4];                                    // fragments of slice 0 of the half step about to be multiplied
-    auto read = [&](half8 (&a)[4], half8 (&w)[4], const half8 (&cur)[HB], int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) a[i] = cur[((4 * wm + i) * 2 + j) * 64 + lane];
-#pragma unroll
-        for (int k = 0; k < 4; k++) w[k] = cur[((8 + 4 * wn + k) * 2 + j) * 64 + lane];
-    };
-    auto multiply = [&](const half8 (&a)[4], const half8 (&w)[4]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], acc[i][k], 0, 0, 0);
-    };
-    // Half step hs is multiplied out of buffer hs % 5.  The barrier that ends half step hs - 1 has found hs and hs + 1 in
-    // LDS (every wave waited for its own copies of them), so slice 0 of hs + 1 is read while slice 1 of hs is multiplied
-    // and no half step starts by waiting out an LDS round trip; hs + 4 is requested into the buffer hs - 1 left.
-    auto step = [&](int hs, const half8 (&cur)[HB], const half8 (&nxt)[HB], half8 (&free_buf)[HB]) __attribute__((always_inline)) {
-        request(free_buf, min(hs + 4, last));
-        half8 a1[4], w1[4];
-        read(a1, w1, cur, 1);
-        multiply(a0, w0);
-        read(a0, w0, nxt, 0);
-        multiply(a1, w1);
-        // issue order: under each MFMA of slice 0 one LDS read of slice 1, under each of slice 1 one of the next slice 0
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i < 6 || (i >= 16 && i < 24)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        // in flight: this wave's copies of hs + 1 .. hs + 4, 8 each (4 pieces x 2 slices); hs + 1 and hs + 2 must have landed
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(WAIT) : "memory");
-    };
-    request(lb0, 0); request(lb1, min(1, last)); request(lb2, min(2, last)); request(lb3, min(3, last));
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(WAIT) : "memory");   // four requests out: the first two have landed
-    read(a0, w0, lb0, 0);
-    const int full = nhalf / 5 * 5;
-    for (int h0 = 0; h0 < full; h0 += 5) {
-        step(h0, lb0, lb1, lb4);
-        step(h0 + 1, lb1, lb2, lb0);
-        step(h0 + 2, lb2, lb3, lb1);
-        step(h0 + 3, lb3, lb4, lb2);
-        step(h0 + 4, lb4, lb0, lb3);
+            for (int v = 0; v < 4; v++) sc[j][v] = g.a_inv_scale[min(m0 + 16 * j + mq + v, g.M - 1)];
     }
-    if (full < nhalf) step(full, lb0, lb1, lb4);
-    if (full + 1 < nhalf) step(full + 1, lb1, lb2, lb0);
-    if (full + 2 < nhalf) step(full + 2, lb2, lb3, lb1);
-    if (full + 3 < nhalf) step(full + 3, lb3, lb4, lb2);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-    if (mb0 * 32 + 256 <= g.M && (nb0 + 8) * 32 <= g.N) {  // a block inside the matrix: stores without tests, factors first
-        float sc[4][16];
+    // this wave's share of a half step: both slices of A row blocks w (, 4 + w) and of W row blocks w, 4 + w (clamped: rows past
+    // the end are computed and never stored), as uniform bases and one lane offset per operand
+    auto uniform = [](const half8 *p) __attribute__((always_inline)) {
+        const uint64_t x = reinterpret_cast<uint64_t>(p);
+        return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32;
+    };
+    uint64_t src[AU + 2];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+    for (int u = 0; u < AU; u++) src[u] = uniform(g.A + ((size_t)min(mb0 + 4 * u + wave, g.Mb - 1) * g.Kb + k_beg) * 256);
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                sc[i][v] = g.a_inv_scale ? g.a_inv_scale[(mb0 + 4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3)] : 1.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m = (mb0 + 4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-                float *row = Cp + (size_t)m * g.ldp + (nb0 + 4 * wn) * 32 + r;
-#pragma unroll
-                for (int k = 0; k < 4; k++) row[k * 32] = acc[i][k][v] * sc[i][v];
+    for (int u = 0; u < 2; u++)
+        src[AU + u] = uniform(reinterpret_cast<const half8 *>(g.W.w16) + ((size_t)min(nb0 + 4 * u + wave, g.Nb - 1) * g.Kb + k_beg) * 256);
+    const uint32_t a_off = a_lane(lane) * 16, w_off = lane * 16;
+    typedef __attribute__((address_space(3))) void lds_void;
+    const uint32_t place0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void *)lds + wave * 2048);
+    constexpr int COPIES = 2 * (AU + 2);                      // of 1 KB, per half step and wave
+    static_assert(NB * COPIES < 64, "the hand-written waits count this wave's LDS-direct loads; vmcnt has six bits");
+    // copy c of half step hs (koff = 2048 hs) into the buffer that this wave's first place `place` lies in
+    auto copy = [&](uint32_t place, uint32_t koff, int c) __attribute__((always_inline)) {
+        const int u = c >> 1;
+        const uint32_t off = (u < AU ? a_off : w_off) + koff;
+        if (c & 1) asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024" :: "v"(off), "s"(src[u]), "s"(place), "n"(u * 8192) : "m0", "scc");
+        else asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(src[u]), "s"(place), "n"(u * 8192) : "m0", "scc");
+    };
+    const half8 *const frag = lds + (lane >> 5) * 64 + ((lane >> 4) & 1) * 32 + (lane & 15);
+    const half8 *const fa = frag + MI / 2 * wm * 128, *const fw = frag + (AB + 4 * wn) * 128;
+    auto read = [&](const half8 *f, int t, int buf) __attribute__((always_inline)) { return f[buf + (t >> 1) * 128 + (t & 1) * 16]; };
+
+    half8 A0[MI], A1[MI], W0[8], W1[8];
+    // the wait and barrier of a half step behind which `open` requests may still be under way
+    auto meet = [&](int open) __attribute__((always_inline)) {
+        if (NB > 5 && open >= 4) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((NB - 2) * COPIES) : "memory");
+        else if (open >= 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(3 * COPIES) : "memory");
+        else if (open == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * COPIES) : "memory");
+        else if (open == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(COPIES) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    // Half step hs: its fragments are in A and W; the next one's come out of the buffer at `nxt`; MORE: hs + NB goes into the buffer of
+    // hs, at `place`.  (sched_barrier: the reads stay under the MFMAs where they are written.)
+    auto step = [&](auto more, const half8 (&A)[MI], const half8 (&W)[8], half8 (&An)[MI], half8 (&Wn)[8], int hs, int nxt, uint32_t place) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more)::value;
+        constexpr int READS = MI + 8, EVERY = MI == 8 ? 3 : 2;  // (256 rows: 16 reads under 48 of the 64 MFMAs; 128: 12 under 24 of 32)
+        unrolled<8 * MI>([&](auto X) __attribute__((always_inline)) {
+            constexpr int x = X, i = x / MI, j = x % MI, t = x / EVERY;
+            if constexpr (x % EVERY == 0 && t < READS) {
+                if constexpr (t < MI) An[t] = read(fa, t, nxt); else Wn[t - MI] = read(fw, t - MI, nxt);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (MORE && j == 3 && i < COPIES) copy(place, (uint32_t)(hs + NB) * 2048, i);
+            AccTile<x>::add(A[j], W[i]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        if (MORE) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((NB - 2) * COPIES) : "memory");
+        else meet(last - hs - 2);
+    };
+    auto request = [&](uint32_t place, int hs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < COPIES; c++) copy(place, (uint32_t)hs * 2048, c);
+    };
+    // (nothing is requested past the end: a block's last half steps would wait for it -- five buffers, 3 us where all CUs do)
+    request(place0, 0); request(place0 + HB * 16, 1);
+#pragma unroll
+    for (int h = 2; h < NB; h++) if (h <= last) request(place0 + h * HB * 16, h);
+    unrolled<8 * MI>([](auto X) __attribute__((always_inline)) { AccTile<X>::clear(); });
+    meet(min(NB, nhalf) - 2);                                 // the first two have landed
+#pragma unroll
+    for (int t = 0; t < MI; t++) A0[t] = read(fa, t, 0);
+#pragma unroll
+    for (int t = 0; t < 8; t++) W0[t] = read(fw, t, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // every wave has read buffer 0 before it is requested anew
+    int nxt = HB, hs = 0;
+    uint32_t place = place0;
+    auto advance = [&]() __attribute__((always_inline)) {
+        nxt = nxt == (NB - 1) * HB ? 0 : nxt + HB;
+        place = place == place0 + (NB - 1) * HB * 16 ? place0 : place + HB * 16;
+    };
+    constexpr std::true_type more{};
+    constexpr std::false_type done{};
+    for (; hs + 1 + NB <= last; hs += 2) {
+        step(more, A0, W0, A1, W1, hs, nxt, place); advance();
+        step(more, A1, W1, A0, W0, hs + 1, nxt, place); advance();
+    }
+    if (NB % 2 && hs + NB <= last) request(place, hs + NB);   // (an odd ring: the last half step, nhalf being even)
+    for (; hs < nhalf; hs += 2) {
+        step(done, A0, W0, A1, W1, hs, nxt, place); advance();
+        step(done, A1, W1, A0, W0, hs + 1, nxt, place); advance();
+    }
+    settle_tiles();
+
+    if (mb0 * 32 + BM <= g.M && (nb0 + 8) * 32 <= g.N) {      // a block inside the matrix: stores without tests
+        unrolled<MI>([&](auto J) __attribute__((always_inline)) {
+            float *const row = Cp + (size_t)(m0 + 16 * J + mq) * g.ldp + n0 + nr;
+            unrolled<8>([&](auto I) __attribute__((always_inline)) {
+                const float4v x = AccTile<I * MI + J>::take();
+#pragma unroll
+                for (int v = 0; v < 4; v++) row[(size_t)v * g.ldp + 16 * I] = x[v] * sc[J][v];
+            });
+        });
         return;
     }
     // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
-    uint32_t col[4];
+    unrolled<MI>([&](auto J) __attribute__((always_inline)) {
+        const EdgeStore edge(Cp, m0 + 16 * J, g.M, g.ldp, 16);
+        unrolled<8>([&](auto I) __attribute__((always_inline)) {
+            const int n = n0 + 16 * I + nr;
+            const uint32_t col = EdgeStore::column(n < g.N, n * 4);
+            const float4v x = AccTile<I * MI + J>::take();
 #pragma unroll
-    for (int k = 0; k < 4; k++) { const int n = (nb0 + 4 * wn + k) * 32 + r; col[k] = EdgeStore::column(n < g.N, n * 4); }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float sc[16];
-#pragma unroll
-        for (int v = 0; v < 16; v++)
-            sc[v] = g.a_inv_scale ? g.a_inv_scale[min((mb0 + 4 * wm + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), g.M - 1)] : 1.0f;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const EdgeStore edge(Cp, (mb0 + 4 * wm + i) * 32 + 8 * (v >> 2), g.M, g.ldp);
-#pragma unroll
-            for (int k = 0; k < 4; k++) edge.f32(4 * h + (v & 3), col[k], acc[i][k][v] * sc[v]);
-        }
-    }
+            for (int v = 0; v < 4; v++) edge.f32(mq + v, col, x[v] * sc[J][v]);
+        });
+    });
 }
 
 // The 256 x 256 block over Q8_0 weight tiles that stay quantised all the way into LDS: the dequant-fused product for
@@ -957,15 +955,11 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
         const int wide_cols = full * cus / MX * 256;
         auto launch = [&](const GemmKArgs &a, bool w, hipEvent_t e0, hipEvent_t e1) {
             const dim3 grid = w ? grid_of(a, 256, 256) : grid_of(a, 128, 128 * WPW);
-#define BIG_LAUNCH(KERNEL) do { if (prof) hipExtLaunchKernelGGL((KERNEL), grid, block, 0, stream(), e0, e1, 0, a); \
-                                else hipLaunchKernelGGL((KERNEL), grid, block, 0, stream(), a); } while (0)
-            if (W.fmt == 0) {
-                if (w) BIG_LAUNCH(gemm_big_f16_256);
-                else if (prof) hipExtLaunchKernelGGL((gemm_big_f16<false>), grid, block, 0, stream(), e0, e1, 0, a, GroupArgs{});
-                else hipLaunchKernelGGL((gemm_big_f16<false>), grid, block, 0, stream(), a, GroupArgs{});
-            }
-            else if (W.fmt == 1) { if (a.W.nbq < a.Nb) BIG_LAUNCH((gemm_big_q8<1, 256, true>)); else BIG_LAUNCH((gemm_big_q8<1, 256>)); }
-            else BIG_LAUNCH((gemm_big_q8<2, 256>));
+#define BIG_LAUNCH(KERNEL, ...) do { if (prof) hipExtLaunchKernelGGL(KERNEL, grid, block, 0, stream(), e0, e1, 0, __VA_ARGS__); \
+                                     else hipLaunchKernelGGL(KERNEL, grid, block, 0, stream(), __VA_ARGS__); } while (0)
+            if (W.fmt == 0) { if (w) BIG_LAUNCH((gemm_big_f16<256>), a, GroupArgs{}); else BIG_LAUNCH((gemm_big_f16<128>), a, GroupArgs{}); }
+            else if (W.fmt == 1) { if (a.W.nbq < a.Nb) BIG_LAUNCH((gemm_big_q8<1, 256, true>), a); else BIG_LAUNCH((gemm_big_q8<1, 256>), a); }
+            else BIG_LAUNCH((gemm_big_q8<2, 256>), a);
 #undef BIG_LAUNCH
         };
         if (g_big_block == 0 && !wide && !mid && deep && g.S == 1 && full >= 1 && rest > 0 && rest * 2 <= cus && wide_cols < N) {
@@ -1035,8 +1029,8 @@ int launch_short_sums(const half_t *A, const WeightOp &W, float *P, size_t plane
     const dim3 grid(8 * ((M + 127) / 128) * (((N + 255) / 256 * g.S + 7) / 8));
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     if (gemm_prof_begin(weight_stream_bytes(W, N, K), 2.0 * M * N * K, &ev_a, &ev_b))
-        hipExtLaunchKernelGGL((gemm_big_f16<false, true>), grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g, GroupArgs{});
-    else hipLaunchKernelGGL((gemm_big_f16<false, true>), grid, dim3(256), 0, stream(), g, GroupArgs{});
+        hipExtLaunchKernelGGL(gemm_big_short, grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g);
+    else hipLaunchKernelGGL(gemm_big_short, grid, dim3(256), 0, stream(), g);
     HIP_CHECK(hipGetLastError());
     return g.S;
 }
@@ -1057,8 +1051,8 @@ void launch_gemm_groups(const half_t *A, const float *a_inv_scale, const half_t 
     const dim3 grid(8 * ((mt * nt + 7) / 8));
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     if (gemm_prof_begin(2.0 * groups * N * K, 2.0 * M * N * K, &ev_a, &ev_b))
-        hipExtLaunchKernelGGL((gemm_big_f16<true>), grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g, GroupArgs{group_of, group_stride});
-    else hipLaunchKernelGGL((gemm_big_f16<true>), grid, dim3(256), 0, stream(), g, GroupArgs{group_of, group_stride});
+        hipExtLaunchKernelGGL((gemm_big_f16<128, true>), grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g, GroupArgs{group_of, group_stride});
+    else hipLaunchKernelGGL((gemm_big_f16<128, true>), grid, dim3(256), 0, stream(), g, GroupArgs{group_of, group_stride});
     HIP_CHECK(hipGetLastError());
 }
 

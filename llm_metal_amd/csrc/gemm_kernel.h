@@ -93,16 +93,16 @@ __device__ __forceinline__ void load_w_q8_cols(half8 (&w)[4], const WeightOp &W,
 // the queue before it -- 12 to 15 us per launch of the large-M kernels (250 rows: 33 us on 6176 x 2560 against 18 at 256,
 // whose tiles lie inside).  Here nothing branches: the stores go through buffer descriptors that end with the matrix's last
 // row, and an element in a column past the end gets an offset past that end; the hardware drops what lies outside.  A descriptor
-// covers eight rows: offsets have 31 bits, which 256 rows of 2^21 floats would pass (eight: of 2^26).
+// covers eight rows (`span`: sixteen): offsets have 31 bits, which 256 rows of 2^21 floats would pass (sixteen: of 2^25).
 struct EdgeStore {
     __amdgpu_buffer_rsrc_t window;
     int row_bytes;
-    // base: the matrix's first row; row: the first of the eight (uniform); rows: of the matrix; ld: row stride
-    template <typename T> __device__ __forceinline__ EdgeStore(T *base, int row, int rows, int ld)
+    // base: the matrix's first row; row: the first of the span (uniform); rows: of the matrix; ld: row stride
+    template <typename T> __device__ __forceinline__ EdgeStore(T *base, int row, int rows, int ld, int span = 8)
     {
         row = __builtin_amdgcn_readfirstlane(row);
         row_bytes = ld * (int)sizeof(T);
-        const int n = __builtin_amdgcn_readfirstlane(min(max(rows - row, 0), 8));      // (a descriptor the compiler takes for divergent costs a loop per store)
+        const int n = __builtin_amdgcn_readfirstlane(min(max(rows - row, 0), span));      // (a descriptor the compiler takes for divergent costs a loop per store)
         window = __builtin_amdgcn_make_buffer_rsrc((void *)(base + (size_t)row * ld), 0, n * row_bytes, 0x00020000);
     }
     static __device__ __forceinline__ uint32_t column(bool in, int bytes) { return in ? (uint32_t)bytes : 0x80000000u; }
