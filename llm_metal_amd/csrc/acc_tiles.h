@@ -32,6 +32,16 @@ template <int T> struct AccTile;
         { \
             asm volatile("v_mfma_f32_16x16x32_f16 a[" #R0 ":" #R3 "], %0, %1, 0" :: "v"(a), "v"(w) : "a" #R0, "a" #R1, "a" #R2, "a" #R3); \
         } \
+        /* register R of the tile */ \
+        template <int R> static __device__ __forceinline__ float take_one() \
+        { \
+            float x; \
+            if constexpr (R == 0) asm volatile("v_accvgpr_read_b32 %0, a" #R0 : "=v"(x)); \
+            else if constexpr (R == 1) asm volatile("v_accvgpr_read_b32 %0, a" #R1 : "=v"(x)); \
+            else if constexpr (R == 2) asm volatile("v_accvgpr_read_b32 %0, a" #R2 : "=v"(x)); \
+            else asm volatile("v_accvgpr_read_b32 %0, a" #R3 : "=v"(x)); \
+            return x; \
+        } \
         static __device__ __forceinline__ float4v take() \
         { \
             float4v x; \

@@ -130,16 +130,38 @@ void set_big_gemm_block(int mode);     // F16 tiles: 0 block shape by the measur
 // Returns the number of planes written (fewer than `chunks` when K has too few steps for that many).
 int launch_gemm_big(const half_t *A_tiled, const float *a_inv_scale, const WeightOp &W, float *C, int ldc, int M, int N, int K,
                     int chunks = 1, size_t plane_stride = 0);
+// How gemm_big_pair's teams share the K steps (Kb per column block of 256): team t takes `steps` of them from t * steps on.
+struct PairWalk {
+    int steps, Kb;
+    __host__ __device__ int first(int block) const { return block * Kb / steps; }                        // the first team with a part of a column block
+    __host__ __device__ int piece(int team, int block) const { return team - first(block); }             // the plane it writes
+    __host__ __device__ int count(int n) const { const int b = n >> 8; return ((b + 1) * Kb - 1) / steps - first(b) + 1; }   // planes of column n
+    int planes() const { return Kb % steps == 0 ? Kb / steps : (Kb + steps - 2) / steps + 1; }         // at most
+    int pieces() const { return Kb % steps == 0 || steps % Kb == 0 ? (steps + Kb - 1) / Kb : 1 + (steps + Kb - 2) / Kb; }   // of a team, at most
+};
+constexpr float PAIR_RESIDUAL_SCALE = 2048.f;   // residual rows: this many times what a value row's rounding lost, in units of the value row's factor
 // A product whose operand rows hold more than fp16 does (value and residual rows): planes [M, N] whose sums are formed from parts
 // of at most sixteen MFMAs each, so that rounding the accumulators costs no more than the fp32 matrix-vector kernels lose.
 struct ShortPlan {
     int big, chunks;                   // the large-M kernel with that many K chunks, else t
     GemmPlan t;
+    int steps;                         // plan_short_pair: K steps per team of the pair kernel, at most `chunks` planes
     int planes() const { return big ? chunks : t.S; }
 };
 ShortPlan plan_short_sums(int M, int N, int K, int nbq, int fmt);
 // P: planes() planes; returns how many of them were written.  W: F16 tiles (f16_image_of) where the plan says big.
 int launch_short_sums(const half_t *A_tiled, const WeightOp &W, float *P, size_t plane_stride, int M, int N, int K, const ShortPlan &p);
+ShortPlan plan_short_pair(int M, int lo, int N, int K, int nbq, int fmt);
+// Rows 0 .. M - 1 values and lo .. lo + M - 1 their residuals, `inv` the factors of both (lo a multiple of 32 for the pair kernel).  What was written:
+// S planes of the whole product [M, N], or (whole false) of [lo + M, N] for the consumer to put together; P has room for either.
+// (whole: planes 0 .. walk.count(n) - 1 hold column n)
+struct PairPlanes { size_t plane; int S; bool whole; PairWalk walk; };
+inline size_t pair_plane_floats(const ShortPlan &p, int M, int lo, int N)
+{
+    const size_t apart = (size_t)(p.big ? 1 : p.t.S) * (lo + M), whole = p.big ? (size_t)p.chunks * M : 0;
+    return (apart > whole ? apart : whole) * N;
+}
+PairPlanes launch_short_pair(const half_t *A_tiled, const float *inv, const WeightOp &W, float *P, int M, int lo, int N, int K, const ShortPlan &p);
 int big_gemm_policy();                 // hip_gemm_force_large_m's choice
 // The same with F16 tiles for rows that belong to different weights [N, K] of one shape (the experts of a mixture), their
 // tiled images group_stride halves apart: row block i of 128 rows is multiplied with weight group_of[i] (device), and only the
@@ -163,16 +185,18 @@ void launch_rows_to_f16(const float *X, int ldx, half_t *out_tiled, float *inv_s
 // image and as the fp16 image of the rounding residual.  W: row-major F16 [N, K] buffer (its tiled image is cached).
 void gemm_f32a_exact(const float *A, struct ::MetalBuf *W, float *C, int M, int N, int K);
 // Its three parts, for callers that fold the first or the last into kernels of their own: the cached tiled image of W;
-// rows m and M + m of the tiled operand a16 [2M, K] and their factors inv [2M] from A [M, K]; launch_gemm over
+// rows m and M + m of the tiled operand a16 [2M, K] and their factors inv [2M] from A [M, K] (a residual row's factor is its value
+// row's over PAIR_RESIDUAL_SCALE); launch_gemm over
 // plan_gemm(2M, N, K) into planes of [2M, N]; C [M, N] from the planes.
 const half_t *tiled_weight_of(struct ::MetalBuf *W, int N, int K);
-void launch_rows_to_f16_split(const float *A, half_t *a16, float *inv, int M, int K);
+// (lo: where the residual rows begin, 0: at M)
+void launch_rows_to_f16_split(const float *A, half_t *a16, float *inv, int M, int K, int lo = 0);
 void launch_reduce_planes_split(const float *P, int S, size_t plane_stride, int ldp, const float *inv, float *C, int M, int N, int ldc = 0);   // (ldc 0: N)
-// element (m, n) of such a product: the planes of row m and of row M + m summed, each sum times its row's factor
+// element (m, n) of such a product: the planes of row m and of row lo + m summed, each sum times its row's factor
 __device__ __forceinline__ float split_planes_value(const float *__restrict__ P, int S, size_t plane_stride, int ldp,
-                                                    const float *__restrict__ inv, int M, int m, int n)
+                                                    const float *__restrict__ inv, int lo_row, int m, int n)
 {
-    const float *ph = P + (size_t)m * ldp + n, *pl = P + (size_t)(M + m) * ldp + n;
+    const float *ph = P + (size_t)m * ldp + n, *pl = P + (size_t)(lo_row + m) * ldp + n;
     float hi = 0.f, lo = 0.f;
     int p = 0;
     for (; p + 8 <= S; p += 8) {                          // eight planes' loads in flight; summed in plane order
@@ -183,7 +207,7 @@ __device__ __forceinline__ float split_planes_value(const float *__restrict__ P,
         for (int q = 0; q < 8; q++) { hi += h[q]; lo += l[q]; }
     }
     for (; p < S; p++) { hi += ph[p * plane_stride]; lo += pl[p * plane_stride]; }
-    return fmaf(lo, inv[M + m], hi * inv[m]);
+    return fmaf(lo, inv[lo_row + m], hi * inv[m]);
 }
 void launch_reduce_planes(const float *P, int S, size_t plane_stride, int ldp, const float *row_scale, float *C, int M, int N);
 // dst (tiled, Kb_dst K blocks) <- src row-major F16 [rows, cols]:

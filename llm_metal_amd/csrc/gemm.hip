@@ -47,10 +47,10 @@ __global__ __launch_bounds__(256) void rows_to_f16_scaled(
     if (threadIdx.x == 0) inv_scale[row] = 1.0f / s;
 }
 
-// The same, keeping 22 bits of every element: row m of the tiled operand holds the fp16 image of x, row M + m the
-// fp16 image of what that rounding lost (x - fp16(x s) / s is exact in fp32), each with its own power-of-two scale.
+// The same, keeping 22 bits of every element: row m of the tiled operand holds the fp16 image of x s, row lo + m that of
+// PAIR_RESIDUAL_SCALE times what that rounding lost, which is exact in fp32: half a unit in the last place of at most 2^13, so at most 2^12.
 __global__ __launch_bounds__(256) void rows_to_f16_split(
-    const float *__restrict__ X, int ldx, half_t *__restrict__ out, float *__restrict__ inv_scale, int M, int K, int Kb)
+    const float *__restrict__ X, int ldx, half_t *__restrict__ out, float *__restrict__ inv_scale, int lo, int K, int Kb)
 {
     __shared__ float sm[16];
     const int row = blockIdx.x;
@@ -59,20 +59,13 @@ __global__ __launch_bounds__(256) void rows_to_f16_split(
     for (int i = threadIdx.x; i < K; i += blockDim.x) amax = fmaxf(amax, fabsf(x[i]));
     amax = block_max(amax, sm);
     const float s = row_scale_for(amax), inv = 1.0f / s;
-    float lmax = 0.f;
     for (int i = threadIdx.x; i < Kb * 64; i += blockDim.x) {
-        const half_t h = (i < K) ? f2h(x[i] * s) : (half_t)0;
+        const float v = i < K ? x[i] * s : 0.f;
+        const half_t h = f2h(v);
         out[lmhip::tiled_a_index(row, i, Kb)] = h;
-        if (i < K) lmax = fmaxf(lmax, fabsf(x[i] - h2f(h) * inv));
+        out[lmhip::tiled_a_index(lo + row, i, Kb)] = f2h((v - h2f(h)) * lmhip::PAIR_RESIDUAL_SCALE);
     }
-    lmax = block_max(lmax, sm);
-    const float s2 = row_scale_for(lmax);
-    for (int i = threadIdx.x; i < Kb * 64; i += blockDim.x) {
-        half_t l = (half_t)0;
-        if (i < K) { const half_t h = f2h(x[i] * s); l = f2h((x[i] - h2f(h) * inv) * s2); }
-        out[lmhip::tiled_a_index(M + row, i, Kb)] = l;
-    }
-    if (threadIdx.x == 0) { inv_scale[row] = inv; inv_scale[M + row] = 1.0f / s2; }
+    if (threadIdx.x == 0) { inv_scale[row] = inv; inv_scale[lo + row] = inv / lmhip::PAIR_RESIDUAL_SCALE; }
 }
 
 // The same for rows a workgroup of 1024 threads can hold in registers (K <= 8192 * CPT, K % 4 == 0, X 16-byte aligned):
@@ -80,7 +73,7 @@ __global__ __launch_bounds__(256) void rows_to_f16_split(
 // once.  Same values as rows_to_f16_split.
 template <int CPT>
 __global__ __launch_bounds__(1024) void rows_to_f16_split_vec(
-    const float *__restrict__ X, int ldx, half_t *__restrict__ out, float *__restrict__ inv_scale, int M, int K, int Kb)
+    const float *__restrict__ X, int ldx, half_t *__restrict__ out, float *__restrict__ inv_scale, int lo, int K, int Kb)
 {
     __shared__ float sm[16];
     typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -100,30 +93,21 @@ __global__ __launch_bounds__(1024) void rows_to_f16_split_vec(
     }
     amax = block_max(amax, sm);
     const float s = row_scale_for(amax), inv = 1.0f / s;
-    float lmax = 0.f;
 #pragma unroll
     for (int u = 0; u < CPT; u++) {
         const int k0 = (threadIdx.x + 1024 * u) * 8;
-        half8 h;
+        half8 h, l;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             h[e] = f2h(v[u][e] * s);
-            v[u][e] = v[u][e] - h2f(h[e]) * inv;                            // what the rounding lost, exact in fp32
-            lmax = fmaxf(lmax, fabsf(v[u][e]));
+            l[e] = f2h((v[u][e] * s - h2f(h[e])) * lmhip::PAIR_RESIDUAL_SCALE);
         }
-        if (k0 < Kb * 64) *reinterpret_cast<half8 *>(out + lmhip::tiled_a_index(row, k0, Kb)) = h;
+        if (k0 < Kb * 64) {
+            *reinterpret_cast<half8 *>(out + lmhip::tiled_a_index(row, k0, Kb)) = h;
+            *reinterpret_cast<half8 *>(out + lmhip::tiled_a_index(lo + row, k0, Kb)) = l;
+        }
     }
-    lmax = block_max(lmax, sm);
-    const float s2 = row_scale_for(lmax);
-#pragma unroll
-    for (int u = 0; u < CPT; u++) {
-        const int k0 = (threadIdx.x + 1024 * u) * 8;
-        half8 l;
-#pragma unroll
-        for (int e = 0; e < 8; e++) l[e] = f2h(v[u][e] * s2);
-        if (k0 < Kb * 64) *reinterpret_cast<half8 *>(out + lmhip::tiled_a_index(M + row, k0, Kb)) = l;
-    }
-    if (threadIdx.x == 0) { inv_scale[row] = inv; inv_scale[M + row] = 1.0f / s2; }
+    if (threadIdx.x == 0) { inv_scale[row] = inv; inv_scale[lo + row] = inv / lmhip::PAIR_RESIDUAL_SCALE; }
 }
 
 // pseudo-random fp16 values in (-1, 1) for the timing entry points: constant operands would flatter the matrix cores,
@@ -758,12 +742,13 @@ namespace lmhip {
 
 const half_t *tiled_weight_of(MetalBuf *W, int N, int K) { return tiled_copy_of(W, N, K, 0); }
 
-void launch_rows_to_f16_split(const float *A, half_t *a16, float *inv, int M, int K)
+void launch_rows_to_f16_split(const float *A, half_t *a16, float *inv, int M, int K, int lo)
 {
+    if (!lo) lo = M;
     const bool vec = K % 4 == 0 && ((uintptr_t)A & 15) == 0;
-    if (vec && K <= 8192) hipLaunchKernelGGL(rows_to_f16_split_vec<1>, dim3(M), dim3(1024), 0, stream(), A, K, a16, inv, M, K, tiled_kb(K));
-    else if (vec && K <= 16384) hipLaunchKernelGGL(rows_to_f16_split_vec<2>, dim3(M), dim3(1024), 0, stream(), A, K, a16, inv, M, K, tiled_kb(K));
-    else hipLaunchKernelGGL(rows_to_f16_split, dim3(M), dim3(256), 0, stream(), A, K, a16, inv, M, K, tiled_kb(K));
+    if (vec && K <= 8192) hipLaunchKernelGGL(rows_to_f16_split_vec<1>, dim3(M), dim3(1024), 0, stream(), A, K, a16, inv, lo, K, tiled_kb(K));
+    else if (vec && K <= 16384) hipLaunchKernelGGL(rows_to_f16_split_vec<2>, dim3(M), dim3(1024), 0, stream(), A, K, a16, inv, lo, K, tiled_kb(K));
+    else hipLaunchKernelGGL(rows_to_f16_split, dim3(M), dim3(256), 0, stream(), A, K, a16, inv, lo, K, tiled_kb(K));
 }
 
 void launch_reduce_planes_split(const float *P, int S, size_t plane_stride, int ldp, const float *inv, float *C, int M, int N, int ldc)

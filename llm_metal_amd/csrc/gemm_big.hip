@@ -599,6 +599,186 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
     });
 }
 
+// The product of operands that hold more than fp16: row m of A as a value row m and a residual row lo + m that holds 2^11 times what
+// rounding the value row lost, in units of the same factor (lo a multiple of 32).  A block of 128 rows and 256 columns is a 256 x 256
+// block of gemm_big_f16 whose lower rows are the upper ones' residuals, so one wave ends with both products of an element and stores their
+// sum times the row's factor: one value where two rows' planes went to memory and came back.
+//
+// The matrix cores round an accumulator at every instruction of K = 16 (this one rounds twice), so no sum of more than twelve such steps stays
+// in one: in each of six half steps one or two of the eight columns of a wave's value tiles are added to sums in vector
+// registers -- two instructions an entry, under the MFMAs before the tile begins anew -- and the residual's tiles, 2^-11 of the result, stay.
+// (K = 2560, 64 rows, units of 2^-24 of the result's norm: 5.5 in one sum, 2.2 as a matrix-vector product forms it; K = 9728 10.5 and 3.9.)
+// The K steps of all column blocks stand in one row, and each team of workgroups (one per row block) takes an equal run of them, so no last round
+// of blocks is half empty: 304 blocks of 40 steps on 256 CUs are 48 steps for each instead of 80.  What a run holds of a column block is a piece
+// of it, and the n-th piece goes to plane n (PairWalk): a column block has as many planes as teams had a part in it.
+// The sums leave 96 registers for fragments: W is read in place behind the last MFMA that takes it, which keeps a half step's buffer in use
+// while it is multiplied, so the ring runs a half step less ahead than gemm_big_f16's.
+constexpr int PAIR_PERIOD = 6;
+constexpr int pair_flush(int phase, int n) { constexpr int f[6][2] = {{0, -1}, {2, 4}, {1, -1}, {3, 6}, {5, -1}, {7, -1}}; return f[phase][n]; }
+// the slot (MFMA of 64) ahead of which register u of the sixteen of a column's four value tiles is added to its sum: column f's tiles begin anew in
+// the slots 8 f + 4 ..
+constexpr int pair_slot(int f, int u) { return f == 0 ? u * 7 / 16 : (8 * f - 12 + u > 0 ? 8 * f - 12 + u : 0); }
+__global__ __launch_bounds__(256) void gemm_big_pair(GemmKArgs g, int lo)
+{
+    constexpr int HB = 16 * 128, NB = 5;                      // half8 per buffer: [4 value A + 4 residual A + 8 W row blocks][2 slices][64]; buffers
+    __shared__ half8 lds[NB * HB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // the row blocks of a team are consecutive workgroups of one XCD and walk K together, so a weight tile comes from memory once; the
+    // teams are dealt to the XCDs in turn
+    const int MT = (g.M + 127) >> 7, slot = blockIdx.x >> 3, team = (slot / MT) * 8 + (blockIdx.x & 7);
+    const int mb0 = (slot % MT) * 4, wm = wave >> 1, wn = wave & 1;
+    const int m0 = mb0 * 32 + wm * 64, mq = 4 * (lane >> 4), nr = lane & 15;
+    const PairWalk walk{g.steps_per_chunk, g.Kb};
+    const int begin = team * walk.steps;                      // of the K steps of all column blocks, one behind the other
+    int at = begin;
+    const int end = min(begin + walk.steps, ((g.N + 255) >> 8) * g.Kb);
+    if (at >= end) return;
+
+    // this wave's share of a half step: both slices of a value, its residual and two W row blocks (clamped: rows past the end
+    // are computed and never stored), as uniform bases and one lane offset per operand
+    auto uniform = [](const half8 *p) __attribute__((always_inline)) {
+        const uint64_t x = reinterpret_cast<uint64_t>(p);
+        return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32;
+    };
+    const int ab = min(mb0 + wave, g.Mb - 1);
+    const half8 *const w16 = reinterpret_cast<const half8 *>(g.W.w16);
+    uint64_t src[4];
+    const uint32_t a_off = a_lane(lane) * 16, w_off = lane * 16;
+    typedef __attribute__((address_space(3))) void lds_void;
+    const uint32_t place0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void *)lds + wave * 2048);
+    constexpr int COPIES = 8;                                 // of 1 KB, per half step and wave
+    constexpr int WAIT = (NB - 3) * COPIES;                   // all requests but the newest NB - 3 have landed (loads retire in order)
+    static_assert((NB - 1) * COPIES < 64, "the hand-written waits count this wave's LDS-direct loads; vmcnt has six bits");
+    auto copy = [&](uint32_t place, uint32_t koff, int c) __attribute__((always_inline)) {
+        const int u = c >> 1;
+        const uint32_t off = (u < 2 ? a_off : w_off) + koff;
+        if (c & 1) asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024" :: "v"(off), "s"(src[u]), "s"(place), "n"(u * 8192) : "m0", "scc");
+        else asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(src[u]), "s"(place), "n"(u * 8192) : "m0", "scc");
+    };
+    const half8 *const frag = lds + (lane >> 5) * 64 + ((lane >> 4) & 1) * 32 + (lane & 15);
+    const half8 *const fa = frag + 2 * wm * 128, *const fw = frag + (8 + 4 * wn) * 128;
+    auto read_a = [&](int t, int buf) __attribute__((always_inline)) { return fa[buf + (t >> 2) * 512 + ((t & 3) >> 1) * 128 + (t & 1) * 16]; };   // t < 4: values
+    auto read_w = [&](int t, int buf) __attribute__((always_inline)) { return fw[buf + (t >> 1) * 128 + (t & 1) * 16]; };
+
+    // the piece that begins at step `p`: column block, first step of it, half steps less one
+    int nt = 0, k_beg = 0, last = 0;
+    auto enter = [&](int p) __attribute__((always_inline)) {
+        nt = p / g.Kb; k_beg = p - nt * g.Kb;
+        last = 2 * min(g.Kb - k_beg, end - p) - 1;
+        src[0] = uniform(g.A + ((size_t)ab * g.Kb + k_beg) * 256);
+        src[1] = uniform(g.A + ((size_t)(ab + (lo >> 5)) * g.Kb + k_beg) * 256);
+#pragma unroll
+        for (int u = 0; u < 2; u++) src[2 + u] = uniform(w16 + ((size_t)min(nt * 8 + 4 * u + wave, g.Nb - 1) * g.Kb + k_beg) * 256);
+#pragma unroll
+        for (int h = 0; h < NB - 1; h++)
+#pragma unroll
+            for (int c = 0; c < COPIES; c++) copy(place0 + h * HB * 16, (uint32_t)min(h, last) * 2048, c);
+    };
+    float sum[8][4][4];
+    half8 A0[8], A1[8], W[8];
+    // Half step hs out of the buffer at `cur` (A in A, W but its last in W), the next one's fragments out of `nxt`; hs + NB - 1 goes to
+    // `place`, the buffer of hs - 1.  Tile 8 i + j: value rows 16 j, W rows 16 i; 8 i + 4 + j: their residuals.
+    auto step = [&](auto phase, const half8 (&A)[8], half8 (&An)[8], int hs, int cur, int nxt, uint32_t place) __attribute__((always_inline)) {
+        constexpr int P = decltype(phase)::value;
+        const uint32_t koff = (uint32_t)min(hs + NB - 1, last) * 2048;
+        unrolled<64>([&](auto X) __attribute__((always_inline)) {
+            constexpr int x = X, i = x / 8, jj = x % 8, j = jj % 4;
+            if constexpr (jj == 1) { if constexpr (i > 0) W[i - 1] = read_w(i - 1, nxt); else W[7] = read_w(7, cur); __builtin_amdgcn_sched_barrier(0); }
+            if constexpr (jj == 3) copy(place, koff, i);
+            if constexpr (jj == 5) { An[i] = read_a(i, nxt); __builtin_amdgcn_sched_barrier(0); }
+            unrolled<32>([&](auto U) __attribute__((always_inline)) {
+                constexpr int f = pair_flush(P, U / 16), u = U % 16;
+                if constexpr (f >= 0 && pair_slot(f, u) == x) sum[f][u / 4][u % 4] += AccTile<8 * f + u / 4>::template take_one<u % 4>();
+            });
+            if constexpr (jj < 4) AccTile<8 * i + 4 + j>::add(A[4 + j], W[i]);
+            else if constexpr (i == pair_flush(P, 0) || i == pair_flush(P, 1)) AccTile<8 * i + j>::begin(A[j], W[i]);
+            else AccTile<8 * i + j>::add(A[j], W[i]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(WAIT) : "memory");   // (what was read of the buffer that goes next has been multiplied)
+    };
+    enter(at);
+    for (;;) {
+        const int nhalf = last + 1;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) sum[i][j][v] = 0.f;
+        unrolled<64>([](auto X) __attribute__((always_inline)) { AccTile<X>::clear(); });
+        // NB - 1 requests are out and the first two have landed: in a later piece they are older than the 128 stores of the one before
+        if (at == begin) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(WAIT) : "memory");
+        else asm volatile("s_waitcnt vmcnt(63)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < 8; t++) A0[t] = read_a(t, 0);
+#pragma unroll
+        for (int t = 0; t < 7; t++) W[t] = read_w(t, 0);
+        int cur = 0, nxt = HB, hs = 0;
+        uint32_t place = place0 + (NB - 1) * HB * 16;
+        auto two = [&](auto phase) __attribute__((always_inline)) {
+            auto advance = [&]() __attribute__((always_inline)) {
+                cur = nxt;
+                nxt = nxt == (NB - 1) * HB ? 0 : nxt + HB;
+                place = place == place0 + (NB - 1) * HB * 16 ? place0 : place + HB * 16;
+            };
+            step(phase, A0, A1, hs, cur, nxt, place); advance();
+            step(std::integral_constant<int, decltype(phase)::value + 1>{}, A1, A0, hs + 1, cur, nxt, place); advance();
+            hs += 2;
+        };
+        const int full = nhalf / PAIR_PERIOD * PAIR_PERIOD;
+        while (hs < full) { two(std::integral_constant<int, 0>{}); two(std::integral_constant<int, 2>{}); two(std::integral_constant<int, 4>{}); }
+        if (hs < nhalf) two(std::integral_constant<int, 0>{});
+        if (hs < nhalf) two(std::integral_constant<int, 2>{});
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        settle_tiles();
+
+        float *const Cp = g.P + (size_t)walk.piece(team, nt) * g.plane_stride;
+        const int nb0 = nt * 8, n0 = (nb0 + 4 * wn) * 32;
+        int ld = g.ldp, mr = m0 + mq;
+        asm volatile("" : "+s"(ld), "+v"(mr));                // (the addresses are formed here, not kept in registers that the loop has no room for)
+        float sc[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) sc[j][v] = g.a_inv_scale[min(mr + 16 * j + v, g.M - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; j++) asm volatile("" : "+v"(sc[j][0]), "+v"(sc[j][1]), "+v"(sc[j][2]), "+v"(sc[j][3]));   // (here, ahead of the copies, which the compiler would wait for with them)
+        // the next piece's operands come while this one's sums leave (every wave is behind the last barrier: the buffers are free)
+        at += nhalf / 2;
+        if (at < end) enter(at);
+        auto value = [&](auto J, auto I, float (&y)[4]) __attribute__((always_inline)) {
+            const float4v h = AccTile<8 * I + J>::take(), l = AccTile<8 * I + 4 + J>::take();
+#pragma unroll
+            for (int v = 0; v < 4; v++) y[v] = fmaf(l[v], 1.0f / PAIR_RESIDUAL_SCALE, sum[I][J][v] + h[v]) * sc[J][v];
+        };
+        if (mb0 * 32 + 128 <= g.M && (nb0 + 8) * 32 <= g.N) { // a block inside the matrix: stores without tests
+            unrolled<4>([&](auto J) __attribute__((always_inline)) {
+                float *const row = Cp + (size_t)(mr + 16 * J) * ld + n0 + nr;
+                unrolled<8>([&](auto I) __attribute__((always_inline)) {
+                    float y[4];
+                    value(J, I, y);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) row[(size_t)v * ld + 16 * I] = y[v];
+                });
+            });
+        } else {                                              // a block that reaches past the matrix (EdgeStore): the same stores, without a branch
+            unrolled<4>([&](auto J) __attribute__((always_inline)) {
+                const EdgeStore edge(Cp, m0 + 16 * J, g.M, ld, 16);
+                unrolled<8>([&](auto I) __attribute__((always_inline)) {
+                    const int n = n0 + 16 * I + nr;
+                    const uint32_t col = EdgeStore::column(n < g.N, n * 4);
+                    float y[4];
+                    value(J, I, y);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) edge.f32(mq + v, col, y[v]);
+                });
+            });
+        }
+        if (at >= end) return;
+    }
+}
+
 // The 256 x 256 block over Q8_0 weight tiles that stay quantised all the way into LDS: the dequant-fused product for
 // many activation rows.  A half step of a weight row block is ONE 1 KB piece (16 int8 per lane: both 8-value slices), its
 // 64 fp16 scales another 128 bytes, so a block's half step is 16 KB of activations + 8 KB of weights instead of 32 KB and
@@ -840,6 +1020,14 @@ double mid_big_us(int wide, int M, int N, int K, int S, int cus)
     if (wide) return 1.6 + rounds * (7.5 + steps * (1.04 + 0.65 * busy)) + (0.144 + 0.2) * plane_mb;
     return 3.9 + rounds * (2.6 + steps * (0.73 + 0.23 * busy)) + (0.23 + 0.2) * plane_mb;
 }
+// the pair kernel with `steps` K steps per team: a step 1.0 to 1.5 us by how many CUs work, 6 us per piece of a team
+double pair_us(int M, int N, int K, int steps, int cus)
+{
+    const int Kb = tiled_kb(K), mt = (M + 127) / 128, nt = (N + 255) / 256;
+    const long teams = ((long)nt * Kb + steps - 1) / steps;
+    const double busy = (double)teams * mt / cus, plane_mb = ((double)Kb / steps + (Kb % steps ? 1.0 : 0.0)) * M * N * 4e-6;
+    return 1.6 + 6.0 * PairWalk{steps, Kb}.pieces() + steps * (1.04 + 0.45 * busy) + (0.144 + 0.2) * plane_mb;
+}
 MidPlan mid_plan(int M, int N, int K, bool one_plane)
 {
     const int cus = num_cus() > 0 ? num_cus() : 256, Kb = tiled_kb(K);
@@ -1033,6 +1221,56 @@ int launch_short_sums(const half_t *A, const WeightOp &W, float *P, size_t plane
     else hipLaunchKernelGGL(gemm_big_short, grid, dim3(256), 0, stream(), g);
     HIP_CHECK(hipGetLastError());
     return g.S;
+}
+
+// Value and residual rows: the pair kernel or the streaming kernel over all 2 M rows, by the same times; a block of 128 rows costs the pair kernel
+// what one of 256 costs gemm_big_f16.
+ShortPlan plan_short_pair(int M, int lo, int N, int K, int nbq, int fmt)
+{
+    ShortPlan p = plan_short_sums(lo + M, N, K, nbq, fmt);
+    if (fmt != 0 || big_gemm_policy() < 0) return p;
+    if (lo + M <= 64 && !big_gemm_policy()) return p;
+    const GemmPlan &t = p.t;
+    p.big = 0;
+    const int cus = num_cus() > 0 ? num_cus() : 256, Kb = tiled_kb(K);
+    double best = big_gemm_policy() ? 1e30 : 5.1 + 0.152 * (2e-6 * N * K) + 1.65 * (2e-9 * (lo + M) * N * K) + (0.115 + 0.2) * (4e-6 * t.S * (lo + M) * N);
+    // one round: as many teams as the CUs of every XCD hold, or teams of a K-th part of a column block each, without pieces that share a team
+    const int mt = (M + 127) / 128, nt = (N + 255) / 256, teams = 8 * std::max(1, cus / 8 / mt), least = std::max(1, (nt * Kb + teams - 1) / teams);
+    for (int S = 0; S <= 20 && (S <= 1 || S * 4 <= Kb); S++) {
+        const int steps = S ? std::max(least, (Kb + S - 1) / S) : least;
+        const double us = pair_us(M, N, K, steps, cus);
+        if (us < best) { best = us; p.big = 1; p.steps = steps; }
+    }
+    if (!p.big) return p;
+    if (g_big_split != 1) p.steps = std::max(1, Kb / std::max(1, g_big_split));
+    p.chunks = PairWalk{p.steps, Kb}.planes();
+    return p;
+}
+
+PairPlanes launch_short_pair(const half_t *A, const float *inv, const WeightOp &W, float *P, int M, int lo, int N, int K, const ShortPlan &p)
+{
+    PairPlanes out{(size_t)(lo + M) * N, 0, false, {}};
+    if (M <= 0 || N <= 0 || K <= 0) return out;
+    if (lo < M || !inv) { fprintf(stderr, "[fast_hip] gemm_pair: bad rows M=%d lo=%d\n", M, lo); abort(); }
+    if (!p.big || W.fmt != 0) { out.S = launch_short_sums(A, W, P, out.plane, lo + M, N, K, p); return out; }
+    if (!W.w16 || p.steps < 1 || (lo & 31)) { fprintf(stderr, "[fast_hip] gemm_pair: bad launch M=%d lo=%d N=%d K=%d chunks=%d\n", M, lo, N, K, p.chunks); abort(); }
+    GemmKArgs g{};
+    g.A = reinterpret_cast<const half8 *>(A); g.W = W; g.a_inv_scale = inv;
+    out.plane = (size_t)M * N;
+    g.P = P; g.ldp = N; g.plane_stride = out.plane;
+    g.M = M; g.N = N; g.Mb = tiled_rb(M); g.Nb = tiled_rb(N); g.Kb = tiled_kb(K);
+    g.steps_per_chunk = p.steps;
+    const int teams = ((N + 255) / 256 * g.Kb + p.steps - 1) / p.steps;
+    const dim3 grid(8 * ((M + 127) / 128) * ((teams + 7) / 8));
+    hipEvent_t ev_a = nullptr, ev_b = nullptr;
+    if (gemm_prof_begin(weight_stream_bytes(W, N, K), 4.0 * M * N * K, &ev_a, &ev_b))
+        hipExtLaunchKernelGGL(gemm_big_pair, grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g, lo);
+    else hipLaunchKernelGGL(gemm_big_pair, grid, dim3(256), 0, stream(), g, lo);
+    HIP_CHECK(hipGetLastError());
+    out.S = p.chunks;
+    out.walk = PairWalk{p.steps, g.Kb};
+    out.whole = true;
+    return out;
 }
 
 void launch_gemm_groups(const half_t *A, const float *a_inv_scale, const half_t *W, size_t group_stride, const int *group_of, float *C, int ldc,

@@ -211,11 +211,11 @@ __global__ __launch_bounds__(64) void k_lora_down(const float *__restrict__ ln, 
 }
 
 // act[b][i] = silu | gelu (gate) * up from the planes of the [gate | up] product of a batch
-__global__ __launch_bounds__(TB) void k_glu_planes(SplitPlanes gu, float *__restrict__ act, int B, int IS, int gelu)
+__global__ __launch_bounds__(TB) void k_glu_planes(SplitPlanes gu, float *__restrict__ act, int IS, int gelu)
 {
     const int b = blockIdx.y, i = blockIdx.x * TB + threadIdx.x;
     if (i >= IS) return;
-    const float g = planes_at(gu, B, b, i), u = planes_at(gu, B, b, IS + i);
+    const float g = planes_at(gu, b, i), u = planes_at(gu, b, IS + i);
     float a;
     if (gelu) {                                                           // shaders/q8_kernels.metal:349-362
         float t = 0.7978845608f * (g + 0.044715f * g * g * g);
@@ -226,13 +226,13 @@ __global__ __launch_bounds__(TB) void k_glu_planes(SplitPlanes gu, float *__rest
 }
 
 // k_add_norm for row blockIdx.x of a batch, with the branch taken from a product's planes (br.P) or absent, and with
-// ln also written as the next product's operand: rows b and B + b of the tiled fp16 image a16 [2B, D] and their factors
+// ln also written as the next product's operand: rows b and lo + b of the tiled fp16 image a16 [lo + B, D] and their factors
 // (what rows_to_f16_split makes of ln, element for element).  A thread holds elements tid + 1024 u, u < EPT, so
 // 1024 EPT >= the padded row; the sums run in k_add_norm's order.
 template <int EPT>
 __global__ __launch_bounds__(1024) void k_add_norm_split(float *__restrict__ x, SplitPlanes br, const float *__restrict__ g_branch,
                                                          const float *__restrict__ g, float *__restrict__ ln,
-                                                         half_t *__restrict__ a16, float *__restrict__ inv_out, int B, int D, float eps)
+                                                         half_t *__restrict__ a16, float *__restrict__ inv_out, int lo, int D, float eps)
 {
     __shared__ float sm[32];
     const int b = blockIdx.x, Kb = tiled_kb(D);
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(1024) void k_add_norm_split(float *__restrict__ x, 
     }
     if (br.P) {
 #pragma unroll
-        for (int u = 0; u < EPT; u++) { const int i = threadIdx.x + 1024 * u; bv[u] = i < D ? planes_at(br, B, b, i) : 0.f; }
+        for (int u = 0; u < EPT; u++) { const int i = threadIdx.x + 1024 * u; bv[u] = i < D ? planes_at(br, b, i) : 0.f; }
         if (g_branch) {
             float ss = 0.f;
 #pragma unroll
@@ -282,23 +282,16 @@ __global__ __launch_bounds__(1024) void k_add_norm_split(float *__restrict__ x, 
         if (ln && i < D) ln[(size_t)b * D + i] = v[u];
     }
     const float s = row_scale_for(mxg * inv), is = 1.0f / s;
-    float lmax = 0.f;
 #pragma unroll
     for (int u = 0; u < EPT; u++) {
         const int i = threadIdx.x + 1024 * u;
         const half_t h = f2h(v[u] * s);
-        if (i < Kb * 64) a16[tiled_a_index(b, i, Kb)] = h;
-        v[u] = v[u] - h2f(h) * is;
-        lmax = fmaxf(lmax, fabsf(v[u]));
+        if (i < Kb * 64) {
+            a16[tiled_a_index(b, i, Kb)] = h;
+            a16[tiled_a_index(lo + b, i, Kb)] = f2h((v[u] * s - h2f(h)) * PAIR_RESIDUAL_SCALE);
+        }
     }
-    lmax = block_max(lmax, sm);
-    const float s2 = row_scale_for(lmax);
-#pragma unroll
-    for (int u = 0; u < EPT; u++) {
-        const int i = threadIdx.x + 1024 * u;
-        if (i < Kb * 64) a16[tiled_a_index(B + b, i, Kb)] = f2h(v[u] * s2);
-    }
-    if (threadIdx.x == 0) { inv_out[b] = is; inv_out[B + b] = 1.0f / s2; }
+    if (threadIdx.x == 0) { inv_out[b] = is; inv_out[lo + b] = is / PAIR_RESIDUAL_SCALE; }
 }
 
 // The same with four neighbouring columns per piece, C pieces per thread (D and the product's strides multiples of four): the
@@ -307,7 +300,7 @@ __global__ __launch_bounds__(1024) void k_add_norm_split(float *__restrict__ x, 
 template <int NT, int C>
 __global__ __launch_bounds__(NT) void k_add_norm_split4(float *__restrict__ x, SplitPlanes br, const float *__restrict__ g_branch,
                                                         const float *__restrict__ g, float *__restrict__ ln,
-                                                        half_t *__restrict__ a16, float *__restrict__ inv_out, int B, int D, float eps)
+                                                        half_t *__restrict__ a16, float *__restrict__ inv_out, int lo, int D, float eps)
 {
     __shared__ float sm[32];
     const int b = blockIdx.x, Kb = tiled_kb(D);
@@ -327,7 +320,7 @@ __global__ __launch_bounds__(NT) void k_add_norm_split4(float *__restrict__ x, S
 #pragma unroll
         for (int u = 0; u < C; u++) {
             const int i = 4 * (threadIdx.x + NT * u);
-            if (i < D) bv[u] = planes4_at(br, B, b, i);
+            if (i < D) bv[u] = planes4_at(br, b, i);
         }
         if (g_branch) {
 #pragma unroll
@@ -351,42 +344,33 @@ __global__ __launch_bounds__(NT) void k_add_norm_split4(float *__restrict__ x, S
     }
     block_sum_max(ss, mxg, sm);
     const float inv = rsqrtf(ss / (float)D + eps), s = row_scale_for(mxg * inv), is = 1.0f / s;
-    float lmax = 0.f;
 #pragma unroll
     for (int u = 0; u < C; u++) {
         const int i = 4 * (threadIdx.x + NT * u);
         v[u] = v[u] * inv * gv[u];
         if (ln && i < D) *reinterpret_cast<float4v *>(ln + (size_t)b * D + i) = v[u];
-        half4 h;
+        half4 h, l;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             h[e] = f2h(v[u][e] * s);
-            v[u][e] -= h2f(h[e]) * is;
-            lmax = fmaxf(lmax, fabsf(v[u][e]));
+            l[e] = f2h((v[u][e] * s - h2f(h[e])) * PAIR_RESIDUAL_SCALE);
         }
-        if (i < Kb * 64) *reinterpret_cast<half4 *>(a16 + tiled_a_index(b, i, Kb)) = h;
+        if (i < Kb * 64) {
+            *reinterpret_cast<half4 *>(a16 + tiled_a_index(b, i, Kb)) = h;
+            *reinterpret_cast<half4 *>(a16 + tiled_a_index(lo + b, i, Kb)) = l;
+        }
     }
-    lmax = block_max(lmax, sm);
-    const float s2 = row_scale_for(lmax);
-#pragma unroll
-    for (int u = 0; u < C; u++) {
-        const int i = 4 * (threadIdx.x + NT * u);
-        half4 h;
-#pragma unroll
-        for (int e = 0; e < 4; e++) h[e] = f2h(v[u][e] * s2);
-        if (i < Kb * 64) *reinterpret_cast<half4 *>(a16 + tiled_a_index(B + b, i, Kb)) = h;
-    }
-    if (threadIdx.x == 0) { inv_out[b] = is; inv_out[B + b] = 1.0f / s2; }
+    if (threadIdx.x == 0) { inv_out[b] = is; inv_out[lo + b] = is / PAIR_RESIDUAL_SCALE; }
 }
 
 // rows x[0 .. M) of a step: one workgroup each, of 1024 threads while there are fewer rows than CUs and latency is what counts,
 // of 256 beyond
-void launch_add_norm_split(float *x, const SplitPlanes &br, const float *g_branch, const float *g, float *ln, half_t *a16, float *inv, int M, int D, float eps)
+void launch_add_norm_split(float *x, const SplitPlanes &br, const float *g_branch, const float *g, float *ln, half_t *a16, float *inv, int M, int lo, int D, float eps)
 {
     const int pad = tiled_kb(D) * 64;
     const bool four = D % 4 == 0 && br.N % 4 == 0 && (br.plane | br.plane2) % 4 == 0 &&
                       !(((uintptr_t)x | (uintptr_t)br.P | (uintptr_t)br.P2 | (uintptr_t)g_branch | (uintptr_t)g | (uintptr_t)ln) & 15);
-#define NORM_SPLIT(KERNEL, NT_) hipLaunchKernelGGL((KERNEL), dim3(M), dim3(NT_), 0, stream(), x, br, g_branch, g, ln, a16, inv, M, D, eps)
+#define NORM_SPLIT(KERNEL, NT_) hipLaunchKernelGGL((KERNEL), dim3(M), dim3(NT_), 0, stream(), x, br, g_branch, g, ln, a16, inv, lo, D, eps)
     if (four && M < 192) { if (pad <= 4096) NORM_SPLIT((k_add_norm_split4<1024, 1>), 1024); else NORM_SPLIT((k_add_norm_split4<1024, 2>), 1024); }
     else if (four) {
         if (pad <= 2048) NORM_SPLIT((k_add_norm_split4<256, 2>), 256);
@@ -1196,7 +1180,7 @@ bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
         float *ln = (s->lora.empty() || s->borrows_tiles) ? nullptr : dptr_as<float>(r.ln);      // fp32 copy: only k_lora_down reads it
         const float *gb = g_branch ? dptr_as<float>(g_branch) : nullptr;
         if constexpr (std::is_same_v<std::decay_t<decltype(br)>, FewPlanes>) launch_few_norm(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, B, D, s->eps);
-        else launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, B, D, s->eps);
+        else launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, B, B, D, s->eps);
     };
     // planes of (the operand in a16) x w^T; `inv`: the factors that operand's rows were split with.  The weight: the
     // tiled image of the state's own row-major matrix (made on first use), or the training state's tiles
@@ -1206,7 +1190,7 @@ bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
         const GemmPlan p = plan_gemm(2 * B, rows, cols, op.fmt ? op.nbq : 0, op.fmt);
         const size_t plane = (size_t)2 * B * rows;
         launch_gemm(a16, nullptr, op, P, rows, plane, 2 * B, rows, cols, p);
-        return SplitPlanes{P, inv, plane, p.S, rows};
+        return SplitPlanes{P, inv, plane, p.S, rows, B};
     };
     const bool bt = s->borrows_tiles;
     auto split = [&](MetalBuf *in, int K) { launch_rows_to_f16_split(dptr_as<float>(in), a16, inv_br, B, K); };
@@ -1255,7 +1239,7 @@ bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
             const SplitPlanes o = product(lw.o, bt ? &bl->o : nullptr, D, qd, inv_br);
             add_norm_b(o, g_post, g_ff);
             const SplitPlanes gu = product(&lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln);
-            hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, B), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), B, IS, gemma ? 1 : 0);
+            hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, B), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), IS, gemma ? 1 : 0);
             split(r.act, IS);
             pending = product(lw.down, bt ? &bl->down : nullptr, D, IS, inv_br);
         }
@@ -1421,21 +1405,24 @@ bool memory_for(size_t bytes, bool settled)
     return before >= bytes;
 }
 
+// the row of a step's operands where the residuals of its M rows begin: a row block of the tiles of its own
+int residual_row(int M) { return (M + 31) & ~31; }
+
 // What the products of a step of up to `cap` tokens need: planes, and the F16 images of the largest matrix where none is kept
 size_t prompt_product_bytes(const InferenceState *s, int cap)
 {
     const bool q8 = !s->use_fp16 && !s->borrows_tiles;
     const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
     const int shapes[4][2] = {{qd + 2 * kd + (s->borrows_tiles ? 2 * s->R : 0), s->D}, {s->D, qd}, {2 * s->IS, s->D}, {s->D, s->IS}};
-    const int head = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V), want = 2 * std::min(PROMPT_WANT, cap);
-    size_t planes = (size_t)plan_short_sums(want, head, s->D, 0, 0).planes() * want * head * sizeof(float), planes2 = 0, image = tiled_elems(head, s->D) * sizeof(half_t);
+    const int head = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V), want = std::min(PROMPT_WANT, cap);
+    auto pair_bytes = [](int M, int N, int K) { const int lo = residual_row(M); return pair_plane_floats(plan_short_pair(M, lo, N, K, 0, 0), M, lo, N) * sizeof(float); };
+    size_t planes = pair_bytes(want, head, s->D), planes2 = 0, image = tiled_elems(head, s->D) * sizeof(half_t);
     for (const auto &sh : shapes) {
         image = std::max(image, tiled_elems(sh[0], sh[1]) * sizeof(half_t));
-        for (int m = 64; m - 64 < 2 * cap; m += 64) {
-            const int M = std::min(m, 2 * cap);
-            const size_t n = (size_t)plan_short_sums(M, sh[0], sh[1], 0, 0).planes() * M * sh[0] * sizeof(float);
-            planes = std::max(planes, n);
-            if (M <= cap) planes2 = std::max(planes2, n);
+        for (int m = 32; m - 32 < cap; m += 32) {
+            const int M = std::min(m, cap);
+            planes = std::max(planes, pair_bytes(M, sh[0], sh[1]));
+            planes2 = std::max(planes2, (size_t)plan_short_sums(M, sh[0], sh[1], 0, 0).planes() * M * sh[0] * sizeof(float));
         }
     }
     return planes + (q8 ? planes2 + 2 * image : image);
@@ -1478,7 +1465,7 @@ bool prompt_takes(InferenceState *s, int n)
     if (s->prompt) return true;
     const int qd = s->Hq * s->hd, cap = std::min(PROMPT_ROWS, s->max_seq);
     size_t a16 = 0;
-    for (int K : {s->D, qd, s->IS}) a16 = std::max(a16, tiled_elems(2 * cap, K));
+    for (int K : {s->D, qd, s->IS}) a16 = std::max(a16, tiled_elems(2 * residual_row(cap), K));
     const size_t rows = (size_t)cap * (2 * (size_t)s->D + 2 * (size_t)qd + (prompt_glu_supported(s->IS) ? 0 : s->IS) + 4 + 2 * s->R) + s->max_seq + (size_t)PROMPT_WANT * s->D;
     if (!memory_for(rows * sizeof(float) + a16 * sizeof(half_t) + prompt_product_bytes(s, cap), true)) { s->prompt_refused = true; return false; }
     s->prompt = new PromptRun{};
@@ -1488,7 +1475,7 @@ bool prompt_takes(InferenceState *s, int n)
     r.q = fbuf((size_t)cap * qd); r.att = fbuf((size_t)cap * qd);
     if (!prompt_glu_supported(s->IS)) r.act = fbuf((size_t)cap * s->IS);
     r.a16 = metal_buf_create(a16 * sizeof(half_t));
-    r.inv_ln = fbuf((size_t)2 * cap); r.inv_br = fbuf((size_t)2 * cap);
+    r.inv_ln = fbuf((size_t)2 * residual_row(cap)); r.inv_br = fbuf((size_t)2 * residual_row(cap));
     r.ids = metal_buf_create((size_t)s->max_seq * sizeof(int));
     r.sel = fbuf((size_t)PROMPT_WANT * s->D);
     HIP_CHECK(hipHostMalloc((void **)&r.ids_host, (size_t)s->max_seq * sizeof(int), hipHostMallocDefault));
@@ -1521,22 +1508,24 @@ float *at_least(MetalBuf *&b, size_t n)
 SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv, int M, int row0 = 0)
 {
     const half_t *a16 = dptr_as<half_t>(r.a16);
-    auto planes = [&](const WeightOp &op, int m, MetalBuf *&buf, size_t &stride) {
-        stride = (size_t)m * rows;
-        const ShortPlan p = plan_short_sums(m, rows, cols, (op.fmt == 1 && op.nbq < tiled_rb(rows)) ? op.nbq : 0, op.fmt);
-        float *P = at_least(buf, stride * p.planes());
-        return launch_short_sums(a16, p.big ? f16_image_of(op, rows, cols) : op, P, stride, m, rows, cols, p);
-    };
     SplitPlanes out{};
-    out.inv = inv; out.N = rows;
-    if (tiles) out.S = planes(*tiles, 2 * M, r.planes, out.plane);
-    else if (s->use_fp16) out.S = planes(weight_f16(prompt_tiles(w, row0, rows)), 2 * M, r.planes, out.plane);
+    out.inv = inv; out.N = rows; out.lo = residual_row(M);
+    auto pairs = [&](const WeightOp &op) {
+        const ShortPlan p = plan_short_pair(M, out.lo, rows, cols, (op.fmt == 1 && op.nbq < tiled_rb(rows)) ? op.nbq : 0, op.fmt);
+        float *P = at_least(r.planes, pair_plane_floats(p, M, out.lo, rows));
+        const PairPlanes q = launch_short_pair(a16, inv, p.big ? f16_image_of(op, rows, cols) : op, P, M, out.lo, rows, cols, p);
+        out.S = q.S; out.plane = q.plane; out.whole = q.whole; out.walk = q.walk;
+    };
+    if (tiles) pairs(*tiles);
+    else if (s->use_fp16) pairs(weight_f16(prompt_tiles(w, row0, rows)));
     else {
         const size_t n = tiled_elems(rows, cols);
         half_t *hi = (half_t *)scratch(SCR_WF16, 2 * n * sizeof(half_t)), *lo = hi + n;
         q8_to_tiled_pair(w->mbuf, rows, cols, hi, lo);
-        out.S = planes(weight_f16(hi), 2 * M, r.planes, out.plane);
-        out.S2 = planes(weight_f16(lo), M, r.planes2, out.plane2);
+        pairs(weight_f16(hi));
+        out.plane2 = (size_t)M * rows;
+        const ShortPlan p = plan_short_sums(M, rows, cols, 0, 0);
+        out.S2 = launch_short_sums(a16, weight_f16(lo), at_least(r.planes2, out.plane2 * p.planes()), out.plane2, M, rows, cols, p);
         out.P2 = dptr_as<float>(r.planes2);
     }
     out.P = dptr_as<float>(r.planes);
@@ -1554,6 +1543,7 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
 {
     const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd, IS = s->IS, qd = Hq * hd, nqkv = qd + 2 * Hkv * hd;
     const bool gemma = s->model_type == MODEL_GEMMA3, bt = s->borrows_tiles, adapters = !s->lora.empty();
+    const int lo = residual_row(M);
     const int *ids = dptr_as<int>(r.ids) + pos;
     HIP_CHECK(hipMemcpyAsync((void *)ids, r.ids_host + pos, (size_t)M * sizeof(int), hipMemcpyHostToDevice, stream()));
     launch_embed_ids(dptr_as<float>(s->emb), ids, s->emb_scale, dptr_as<float>(r.x), M, D);
@@ -1562,7 +1552,7 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
     auto norm = [&](const SplitPlanes &br, MetalBuf *g_branch, MetalBuf *g, bool keep) {
         float *ln = keep ? dptr_as<float>(r.ln) : nullptr;
         const float *gb = g_branch ? dptr_as<float>(g_branch) : nullptr;
-        launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, M, D, s->eps);
+        launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, M, lo, D, s->eps);
     };
     const bool few = prompt_few(s, M), q8 = !s->use_fp16 && !bt;
     const int nq_rows = nqkv + (bt && adapters ? 2 * s->R : 0);               // (a training state's fused matrix continues with the rows of A_q and A_v)
@@ -1591,7 +1581,7 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
             few_norm(pending_few, pending_g, lw.g_in, adapters && !bt);
             if (q8) launch_few_full_q8(a16, inv_ln, few_q8_of(lw.qkv.mbuf, nq_rows, D), P, nq_rows, M, nq_rows, D);
             else launch_few_full(a16, inv_ln, tiles(&lw.qkv, bt ? &bl->qkv : nullptr, nq_rows), P, nq_rows, M, nq_rows, D);
-            h.qkv.P = P; h.qkv.S = 1; h.qkv.N = nq_rows;
+            h.qkv.P = P; h.qkv.S = 1; h.qkv.N = nq_rows; h.qkv.whole = true;
         } else {
             norm(pending, pending_g, lw.g_in, adapters && !bt);
             h.qkv = prompt_product(s, r, &lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D, inv_ln, M);
@@ -1620,14 +1610,14 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
             pending_g = gemma ? lw.g_post_ff : nullptr;
             continue;
         }
-        launch_rows_to_f16_split(dptr_as<float>(r.att), a16, inv_br, M, qd);
+        launch_rows_to_f16_split(dptr_as<float>(r.att), a16, inv_br, M, qd, lo);
         const SplitPlanes o = prompt_product(s, r, lw.o, bt ? &bl->o : nullptr, D, qd, inv_br, M);
         norm(o, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, false);
         const SplitPlanes gu = prompt_product(s, r, &lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln, M);
-        if (prompt_glu_supported(IS)) launch_prompt_glu(gu, a16, inv_br, M, IS, gemma ? 1 : 0);
+        if (prompt_glu_supported(IS)) launch_prompt_glu(gu, a16, inv_br, M, lo, IS, gemma ? 1 : 0);
         else {
-            hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, M), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), M, IS, gemma ? 1 : 0);
-            launch_rows_to_f16_split(dptr_as<float>(r.act), a16, inv_br, M, IS);
+            hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, M), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), IS, gemma ? 1 : 0);
+            launch_rows_to_f16_split(dptr_as<float>(r.act), a16, inv_br, M, IS, lo);
         }
         pending = prompt_product(s, r, lw.down, bt ? &bl->down : nullptr, D, IS, inv_br, M);
         pending_g = gemma ? lw.g_post_ff : nullptr;
@@ -1657,11 +1647,11 @@ void prompt_logits(InferenceState *s, PromptRun &r, const int *m, int count, flo
         return;
     }
     for (int i = 0; i < count; i++) row(i, dptr_as<float>(r.sel) + (size_t)i * D);
-    launch_rows_to_f16_split(dptr_as<float>(r.sel), dptr_as<half_t>(r.a16), dptr_as<float>(r.inv_br), count, D);
+    launch_rows_to_f16_split(dptr_as<float>(r.sel), dptr_as<half_t>(r.a16), dptr_as<float>(r.inv_br), count, D, residual_row(count));
     for (int n0 = 0, n; n0 < s->V; n0 += n) {              // (own weights: in parts, for which there is room in scratch if not for the whole head's image)
         n = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V - n0);
         const SplitPlanes lg = prompt_product(s, r, s->lm_head, s->borrows_tiles ? &s->borrowed_lm : nullptr, n, D, dptr_as<float>(r.inv_br), count, n0);
-        launch_reduce_planes_split(lg.P, lg.S, lg.plane, lg.N, lg.inv, out + n0, count, n, s->V);
+        launch_planes_to_rows(lg, out + n0, count, n, s->V);
     }
 }
 

@@ -43,14 +43,14 @@ __global__ __launch_bounds__(TB) void k_prompt_heads(PromptHeads a)
     const bool adapters = a.R > 0 && kind != 1;
     if (adapters && lane < a.R) {
         const int r = (kind == 0 ? 0 : a.R) + lane;
-        t = a.t ? a.t[(size_t)m * 2 * a.R + r] : planes_at(a.qkv, a.M, m, nqkv + r);
+        t = a.t ? a.t[(size_t)m * 2 * a.R + r] : planes_at(a.qkv, m, nqkv + r);
     }
     float x0[2] = {0.f, 0.f}, x1[2] = {0.f, 0.f};
     float ss = 0.f;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int i = lane + 64 * u;
-        if (i < half) { x0[u] = planes_at(a.qkv, a.M, m, slot * hd + i); x1[u] = planes_at(a.qkv, a.M, m, slot * hd + i + half); }
+        if (i < half) { x0[u] = planes_at(a.qkv, m, slot * hd + i); x1[u] = planes_at(a.qkv, m, slot * hd + i + half); }
         if (adapters) {
             const float *B = (kind == 0 ? a.Bq : a.Bv) + (size_t)h * hd * a.R;
             float d0 = 0.f, d1 = 0.f;
@@ -563,12 +563,18 @@ __global__ __launch_bounds__(TB) void k_prompt_attn_short(const float *__restric
     }
 }
 
+__global__ __launch_bounds__(TB) void k_planes_to_rows(SplitPlanes p, float *__restrict__ out, int N, int ldc)
+{
+    const int n = blockIdx.x * TB + threadIdx.x, m = blockIdx.y;
+    if (n < N) out[(size_t)m * ldc + n] = planes_at(p, m, n);
+}
+
 // One workgroup per token, the gated row in registers (C chunks of four columns per thread): the planes are read once and the
 // next product's operand leaves as two fp16 rows, where a gate kernel and a split kernel wrote and read the fp32 row between them.
 // 500 rows of 9728: 20.7 us.  (A few rows leave most CUs without one: at eight, 11.8 us against 9.2 for the two kernels, which a
 // batch's steps therefore keep.)
 template <int C, int GELU>
-__global__ __launch_bounds__(1024) void k_prompt_glu(SplitPlanes gu, half_t *__restrict__ a16, float *__restrict__ inv, int M, int IS, int Kb)
+__global__ __launch_bounds__(1024) void k_prompt_glu(SplitPlanes gu, half_t *__restrict__ a16, float *__restrict__ inv, int lo, int IS, int Kb)
 {
     __shared__ float sm[16];
     const int m = blockIdx.x;
@@ -580,7 +586,7 @@ __global__ __launch_bounds__(1024) void k_prompt_glu(SplitPlanes gu, half_t *__r
 #pragma unroll
         for (int e = 0; e < 4; e++) v[u][e] = 0.f;
         if (n < IS) {
-            const float4v g = planes4_at(gu, M, m, n), up = planes4_at(gu, M, m, IS + n);
+            const float4v g = planes4_at(gu, m, n), up = planes4_at(gu, m, IS + n);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float act = GELU ? 0.5f * g[e] * (1.0f + tanhf(gelu_inner(g[e]))) : g[e] / (1.0f + expf(-g[e]));
@@ -591,30 +597,21 @@ __global__ __launch_bounds__(1024) void k_prompt_glu(SplitPlanes gu, half_t *__r
     }
     amax = block_max(amax, sm);
     const float s = row_scale_for(amax), is = 1.0f / s;
-    float lmax = 0.f;
 #pragma unroll
     for (int u = 0; u < C; u++) {
         const int n = (threadIdx.x + 1024 * u) * 4;
-        half4 h;
+        half4 h, l;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             h[e] = f2h(v[u][e] * s);
-            v[u][e] -= h2f(h[e]) * is;
-            lmax = fmaxf(lmax, fabsf(v[u][e]));
+            l[e] = f2h((v[u][e] * s - h2f(h[e])) * PAIR_RESIDUAL_SCALE);
         }
-        if (n < Kb * 64) *reinterpret_cast<half4 *>(a16 + tiled_a_index(m, n, Kb)) = h;
+        if (n < Kb * 64) {
+            *reinterpret_cast<half4 *>(a16 + tiled_a_index(m, n, Kb)) = h;
+            *reinterpret_cast<half4 *>(a16 + tiled_a_index(lo + m, n, Kb)) = l;
+        }
     }
-    lmax = block_max(lmax, sm);
-    const float s2 = row_scale_for(lmax);
-#pragma unroll
-    for (int u = 0; u < C; u++) {
-        const int n = (threadIdx.x + 1024 * u) * 4;
-        half4 h;
-#pragma unroll
-        for (int e = 0; e < 4; e++) h[e] = f2h(v[u][e] * s2);
-        if (n < Kb * 64) *reinterpret_cast<half4 *>(a16 + tiled_a_index(M + m, n, Kb)) = h;
-    }
-    if (threadIdx.x == 0) { inv[m] = is; inv[M + m] = 1.0f / s2; }
+    if (threadIdx.x == 0) { inv[m] = is; inv[lo + m] = is / PAIR_RESIDUAL_SCALE; }
 }
 
 }  // namespace
@@ -667,16 +664,21 @@ void launch_prompt_attention(const float *q, const float *kc, const float *vc, f
 #undef PS
 }
 
+void launch_planes_to_rows(const SplitPlanes &p, float *out, int M, int N, int ldc)
+{
+    hipLaunchKernelGGL(k_planes_to_rows, dim3((N + TB - 1) / TB, M), dim3(TB), 0, stream(), p, out, N, ldc);
+}
+
 bool prompt_glu_supported(int IS) { return IS % 4 == 0 && tiled_kb(IS) * 64 <= 16384; }
 
-void launch_prompt_glu(const SplitPlanes &gu, half_t *a16, float *inv, int M, int IS, int gelu)
+void launch_prompt_glu(const SplitPlanes &gu, half_t *a16, float *inv, int M, int lo, int IS, int gelu)
 {
-    if (!prompt_glu_supported(IS) || gu.N % 4 || gu.N < 2 * IS || (gu.plane | gu.plane2) % 4 || ((uintptr_t)gu.P | (uintptr_t)gu.P2) & 15) {
+    if (!prompt_glu_supported(IS) || lo < M || gu.N % 4 || gu.N < 2 * IS || (gu.plane | gu.plane2) % 4 || ((uintptr_t)gu.P | (uintptr_t)gu.P2) & 15) {
         fprintf(stderr, "[fast_hip] prompt_glu: unsupported shape %d\n", IS); abort();
     }
     const int Kb = tiled_kb(IS), C = (Kb * 16 + 1023) / 1024;
-#define PG(C_) do { if (gelu) hipLaunchKernelGGL((k_prompt_glu<C_, 1>), dim3(M), dim3(1024), 0, stream(), gu, a16, inv, M, IS, Kb); \
-                    else hipLaunchKernelGGL((k_prompt_glu<C_, 0>), dim3(M), dim3(1024), 0, stream(), gu, a16, inv, M, IS, Kb); } while (0)
+#define PG(C_) do { if (gelu) hipLaunchKernelGGL((k_prompt_glu<C_, 1>), dim3(M), dim3(1024), 0, stream(), gu, a16, inv, lo, IS, Kb); \
+                    else hipLaunchKernelGGL((k_prompt_glu<C_, 0>), dim3(M), dim3(1024), 0, stream(), gu, a16, inv, lo, IS, Kb); } while (0)
     if (C == 1) PG(1); else if (C == 2) PG(2); else if (C == 3) PG(3); else PG(4);
 #undef PG
 }
