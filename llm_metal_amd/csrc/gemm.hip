@@ -287,8 +287,13 @@ namespace lmhip {
 // (64 KB of LDS each) — and loses when some CUs have one more than others (320 workgroups: 9.2 us against 8.1 for 240
 // on 2560 x 4096) or when not all are resident at once (beyond 512).  Among equally balanced splits the one with fewer
 // planes wins: a plane costs the product its stores and the consumer its loads (the more the shorter K is).
+//
+// So few row tiles that even sixteen chunks leave CUs without work (outputs of up to 1024 columns): as many chunks as leave each four K
+// steps, two rounds of a workgroup.  A product of four workgroups is their walk through K, and its planes are nothing: 256 columns of K = 256 ..
+// 4096 (a tiny model's) 66 us for the ten of a step in one chunk each, 42 so; the step 268 -> 226 us, as near to 64 bits as before.
 static int ring_chunks(int n_tiles, int Kb, int K, int cus)
 {
+    if (n_tiles * 16 < cus) return std::min(16, std::max(1, Kb / 4));
     int best = 1;
     double best_score = -1e9;
     for (int S = 1; S <= 32 && S <= Kb; S++) {
