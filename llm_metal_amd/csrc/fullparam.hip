@@ -18,6 +18,7 @@
 #include "devutil.h"
 #include "gemm.h"
 #include "fused.h"
+#include "walk_k.h"
 #include <hip/hip_ext.h>
 
 using namespace lmhip;
@@ -323,6 +324,114 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradJobs js, int Kt, float lr)
     }
 }
 
+// The same on blocks of 256 rows (m) and 128 columns (n) of the target, for launches of enough of them to fill the chip.  k_wgrad is bound by
+// what its operands draw through L2 -- 40 KB per 64 x 256 outputs and token step, 7.4 GB for the head below -- with the target's bytes
+// behind it.  Here they come through LDS once per block (48 KB per 256 x 128), three buffers of 24 KB, so that two workgroups
+// share a CU and one's update runs under the other's products.  The products go X first, which leaves a lane with four columns of one row; two tiles
+// of sixteen rows then trade halves between neighbouring groups of sixteen lanes, and a lane has eight, one 16-byte piece of the tiled target.  The
+// turned block goes through the ring's LDS.  Same sums and same update, so the same weights, bit for bit.
+// Gemma3-1B, 640 tokens, MODE 2: head (302 M weights) 904 -> 569 us, a layer's four matrices (26.8 M) 81 -> 63.
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void k_wgrad_block(WgradJobs js, int Kt, float lr)
+{
+    constexpr int NB = 3, LDT = 136;                      // halves per column of the turned block: 16-byte reads, columns four banks apart
+    static_assert(NB * walk_buffer(128) * sizeof(half8) >= 4 * 64 * LDT * sizeof(half_t), "the turned block lies in the ring");
+    __shared__ half8 lds[NB * walk_buffer(128)];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
+    const int total = js.first[js.n], per_xcd = (total + 7) >> 3;
+    int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (item >= total || (int)(blockIdx.x >> 3) >= per_xcd) return;
+    int k = 0;
+#pragma unroll
+    for (int i = 1; i < 4; i++) if (i < js.n && item >= js.first[i]) k = i;                  // uniform per workgroup
+    item -= js.first[k];
+    const int M_out = js.j[k].M_out, N_in = js.j[k].N_in;
+    const int KbG = tiled_kb(N_in), MbG = tiled_rb(M_out), NbX = tiled_rb(N_in);
+    const int gx = (KbG + 1) >> 1, nb0 = (item % gx) * 4, mb0 = (item / gx) * 8;             // 32-row blocks of X^T and Y^T
+    uint64_t src[3];
+    src[0] = uniform_address(js.j[k].XT + (size_t)min(nb0 + wave, NbX - 1) * Kt * 256);
+#pragma unroll
+    for (int u = 0; u < 2; u++) src[1 + u] = uniform_address(js.j[k].YT + (size_t)min(mb0 + 4 * u + wave, MbG - 1) * Kt * 256);
+    walk_k<128, NB>(lds, src, lane * 16, 2 * Kt);
+
+    // this wave's 64 columns are column block nk of the target, its 128 rows the row blocks mb .. mb + 3; after the trade a lane has row
+    // `row` of a row block and columns 16 j + 8 c .. + 7 of the column block
+    const int nk = nb0 / 2 + wm, mb = mb0 + 4 * wn, row = lane & 31, c = lane >> 5;
+    if (nk >= KbG) return;
+    half8 *const target = reinterpret_cast<half8 *>(js.j[k].target) + (size_t)nk * 256 + row;
+    half_t *const turned = reinterpret_cast<half_t *>(lds) + wave * 64 * LDT;
+    const float *const x_inv = js.j[k].x_inv + nk * 64 + 8 * c, *const y_inv = js.j[k].y_inv;
+    half8 old[4][4];
+    float sy[4];
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const int b = min(mb + p, MbG - 1);
+        sy[p] = y_inv[b * 32 + row];
+#pragma unroll
+        for (int j = 0; j < 4; j++) old[p][j] = __builtin_nontemporal_load(target + (size_t)b * KbG * 256 + (2 * (j & 1) + c) * 64 + 32 * (j >> 1));
+    }
+    auto update = [&](half_t o, float a) __attribute__((always_inline)) {                    // contraction is off in this file
+        return MODE == 0 ? f2h(h2f(o) + a) : MODE == 1 ? f2h(h2f(o) - lr * a) : f2h(h2f(o) - lr * h2f(f2h(0.f + a)));
+    };
+    unrolled<4>([&](auto J) __attribute__((always_inline)) {
+        float xs[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) xs[e] = x_inv[16 * J + e];
+        unrolled<4>([&](auto P) __attribute__((always_inline)) {
+            float4v a = AccTile<(2 * P) * 4 + J>::take(), b = AccTile<(2 * P + 1) * 4 + J>::take();
+            // (the trade wants its operands some cycles old, which the compiler sees to only for instructions of its own)
+            asm volatile("s_nop 3" : "+v"(a), "+v"(b));
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+                const u2 t = __builtin_bit_cast(u2, __builtin_amdgcn_permlane16_swap(__float_as_uint(a[e]), __float_as_uint(b[e]), false, false));
+                v[e] = __uint_as_float(t[0]);
+                v[4 + e] = __uint_as_float(t[1]);
+            }
+            half8 o = old[P][J];
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = update(o[e], v[e] * sy[P] * xs[e]);
+            if (mb + P < MbG) __builtin_nontemporal_store(o, target + (size_t)(mb + P) * KbG * 256 + (2 * (J & 1) + c) * 64 + 32 * (J >> 1));
+            if (MODE == 2) {
+                // rows r and r + 1 (neighbouring lanes) of four columns each: the even lane takes the first four, the odd one the others.  (Rows past the
+                // last are the padding of the turned image's reduction: zeros.)
+                typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+                u4 mine = __builtin_bit_cast(u4, o);
+                if ((mb + P) * 32 + row >= M_out) mine = u4{0, 0, 0, 0};
+                const bool odd = lane & 1;
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const uint32_t keep = odd ? mine[2 + q] : mine[q], give = odd ? mine[q] : mine[2 + q];
+                    const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xF, 0xF, false);   // quad_perm [1, 0, 3, 2]
+                    const uint32_t lo = odd ? got : keep, hi = odd ? keep : got;                                       // row r's pair, row r + 1's
+                    const int n = 16 * J + 8 * c + 4 * odd + 2 * q;
+                    uint32_t *const to = reinterpret_cast<uint32_t *>(turned + n * LDT + P * 32 + (row & ~1));
+                    to[0] = (lo & 0xFFFFu) | hi << 16;
+                    to[LDT / 2] = lo >> 16 | (hi & 0xFFFF0000u);
+                }
+            }
+        });
+    });
+    if (MODE == 2) {                                      // (a wave's own block: no barrier)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        half8 *const to = reinterpret_cast<half8 *>(js.j[k].WT);
+        const int KbT = tiled_kb(M_out);
+#pragma unroll
+        for (int th = 0; th < 2; th++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int kt = mb / 2 + t;
+                if (nk * 2 + th >= NbX || kt >= KbT) continue;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    __builtin_nontemporal_store(*reinterpret_cast<const half8 *>(turned + (th * 32 + row) * LDT + t * 64 + 32 * c + 8 * j),
+                                                &to[((size_t)(nk * 2 + th) * KbT + kt) * 256 + j * 64 + lane]);
+            }
+    }
+}
+
 // 64 x 64 blocks of W (tiled [Mo, Ni]):  if G: W = half(W - lr * G), G = 0 (f16_sgd_apply);
 // then the block is written, transposed, into WT (tiled [Ni, Mo]).
 // grid: x = K blocks of W, y = ceil(row tiles / 2), z = matrices of this shape (the layers of an arena, st / stT half8
@@ -449,22 +558,27 @@ void launch_wgrads(const WgradOperands *w, int n, int T, int mode, float lr)
     if (n <= 0 || n > 4 || T <= 0) { fprintf(stderr, "[fast_hip] wgrads: %d matrices\n", n); abort(); }
     WgradJobs js{};
     js.n = n;
-    int total = 0;
+    int total = 0, blocks = 0;
+    for (int i = 0; i < n; i++) blocks += ((tiled_kb(w[i].N_in) + 1) / 2) * ((tiled_rb(w[i].M_out) + 7) / 8);
+    const bool big = blocks >= num_cus();                 // (fewer leave CUs without one, where k_wgrad's four times as many do not)
     for (int i = 0; i < n; i++) {
         if (w[i].M_out <= 0 || w[i].N_in <= 0) { fprintf(stderr, "[fast_hip] wgrads: empty matrix\n"); abort(); }
         js.j[i] = WgradJob{reinterpret_cast<const half8 *>(w[i].XT), w[i].x_inv, reinterpret_cast<const half8 *>(w[i].YT), w[i].y_inv,
                            w[i].target_tiled, w[i].transposed, w[i].M_out, w[i].N_in};
         js.first[i] = total;
-        total += ((tiled_kb(w[i].N_in) + 3) / 4) * ((tiled_rb(w[i].M_out) + 1) / 2);
+        total += big ? ((tiled_kb(w[i].N_in) + 1) / 2) * ((tiled_rb(w[i].M_out) + 7) / 8) : ((tiled_kb(w[i].N_in) + 3) / 4) * ((tiled_rb(w[i].M_out) + 1) / 2);
     }
     for (int i = n; i <= 4; i++) js.first[i] = total;
-    const dim3 grid((total + 7) / 8 * 8);                 // whole rounds of the eight XCDs; k_wgrad maps ids to tiles
+    const dim3 grid((total + 7) / 8 * 8);                 // whole rounds of the eight XCDs; the kernels map ids to tiles
     double weights = 0.0;
     for (int i = 0; i < n; i++) weights += (double)w[i].M_out * w[i].N_in;
     // the F16 target is read and written once: 4 bytes per weight, and with its transposed image 6
-    if (mode == 2) LAUNCH_TIMED(6.0 * weights, 2.0 * T * weights, k_wgrad<2>, grid, dim3(256), 0, js, tiled_kb(T), lr);
-    else if (mode == 1) LAUNCH_TIMED(4.0 * weights, 2.0 * T * weights, k_wgrad<1>, grid, dim3(256), 0, js, tiled_kb(T), lr);
-    else LAUNCH_TIMED(4.0 * weights, 2.0 * T * weights, k_wgrad<0>, grid, dim3(256), 0, js, tiled_kb(T), lr);
+#define WGRAD(MODE, BYTES) do { if (big) LAUNCH_TIMED(BYTES * weights, 2.0 * T * weights, k_wgrad_block<MODE>, grid, dim3(256), 0, js, tiled_kb(T), lr); \
+                                else LAUNCH_TIMED(BYTES * weights, 2.0 * T * weights, k_wgrad<MODE>, grid, dim3(256), 0, js, tiled_kb(T), lr); } while (0)
+    if (mode == 2) WGRAD(2, 6.0);
+    else if (mode == 1) WGRAD(1, 4.0);
+    else WGRAD(0, 4.0);
+#undef WGRAD
 }
 
 void launch_wgrad(const half_t *XT, const float *x_inv, const half_t *YT, const float *y_inv, half_t *target_tiled,

@@ -17,7 +17,7 @@
 #include "devutil.h"
 #include "gemm.h"
 #include "gemm_kernel.h"
-#include "acc_tiles.h"
+#include "walk_k.h"
 #include <hip/hip_ext.h>
 #include <algorithm>
 
@@ -416,13 +416,9 @@ __global__ __launch_bounds__(256) void gemm_big_short(GemmKArgs g)
 }
 
 
-// F16 weight tiles need no unpacking, so their steps go from L2/HBM straight into LDS (global_load_lds_dwordx4: a
-// wave-uniform LDS base in M0, lane i's 16 bytes land at base + 16 i -- the [j][lane] order of the tiles) and never
-// pass through registers or ds_write.  BM x 256 outputs per workgroup, four waves of BM / 2 x 128.  K goes in half steps of
-// 32 (two of a tile's four 1 KB slices per row block) through a ring of LDS buffers (256 rows: five of 32 KB, all of a CU's
-// 160 KB; 128 rows: six of 24 KB): half step h is multiplied out of buffer h % NB while h + 1 .. h + NB - 1 are in LDS or on
-// their way.  The barrier that ends half step h - 1 finds h and h + 1 in LDS (every wave has waited for its own copies of
-// them), so the fragments of h + 1 are read under the MFMAs of h; h + NB - 1 is requested into the buffer that h - 1 left.
+// F16 weight tiles need no unpacking, so their steps go from L2/HBM straight into LDS and never pass through registers or
+// ds_write (walk_k).  BM x 256 outputs per workgroup, four waves of BM / 2 x 128; 256 rows: five buffers of 32 KB, all of a CU's
+// 160 KB; 128 rows: six of 24 KB.
 //
 // What bounds it: the matrix cores' power.  On random operands the clock settles where the power limit is -- 1.5 to 1.75 GHz
 // under this loop, 2.4 on constant operands -- so what counts is energy per flop as much as idle cycles.  v_mfma_f32_16x16x32
@@ -440,8 +436,8 @@ template <int BM, bool GROUPED = false>
 __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group)
 {
     constexpr int AB = BM / 32, MI = BM / 32, AU = AB / 4;    // A row blocks of the block; 16-row tiles of a wave; A row blocks a wave fetches
-    constexpr int HB = (AB + 8) * 128, NB = BM == 256 ? 5 : 6;   // half8 per buffer: [AB A + 8 W row blocks][2 slices][64]; buffers
-    __shared__ half8 lds[NB * HB];
+    constexpr int NB = BM == 256 ? 5 : 6;                     // buffers
+    __shared__ half8 lds[NB * walk_buffer(BM)];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int MT = (g.M + BM - 1) / BM, NT = (g.N + 255) >> 8;
     const int m_patches = (MT + 7) >> 3;
@@ -470,7 +466,7 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
     const int nb0 = nt * 8, mb0 = mt * AB;
     if (GROUPED) g.W.w16 += (size_t)__builtin_amdgcn_readfirstlane(group.of[mt]) * group.stride;
     const int wm = wave >> 1, wn = wave & 1;
-    const int k_beg = chunk * g.steps_per_chunk, nhalf = 2 * (min(g.Kb, k_beg + g.steps_per_chunk) - k_beg), last = nhalf - 1;
+    const int k_beg = chunk * g.steps_per_chunk, nhalf = 2 * (min(g.Kb, k_beg + g.steps_per_chunk) - k_beg);
     float *const Cp = g.P + (size_t)chunk * g.plane_stride;
     // this wave's rows of C from m0 on, of which a lane ends with 16 j + mq .. + 3 and their factors; its columns from n0 on, 16 i + nr
     const int m0 = mb0 * 32 + wm * (BM / 2), n0 = (nb0 + 4 * wn) * 32, mq = 4 * (lane >> 4), nr = lane & 15;
@@ -488,92 +484,13 @@ __global__ __launch_bounds__(256) void gemm_big_f16(GemmKArgs g, GroupArgs group
 
     // this wave's share of a half step: both slices of A row blocks w (, 4 + w) and of W row blocks w, 4 + w (clamped: rows past
     // the end are computed and never stored), as uniform bases and one lane offset per operand
-    auto uniform = [](const half8 *p) __attribute__((always_inline)) {
-        const uint64_t x = reinterpret_cast<uint64_t>(p);
-        return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32;
-    };
     uint64_t src[AU + 2];
 #pragma unroll
-    for (int u = 0; u < AU; u++) src[u] = uniform(g.A + ((size_t)min(mb0 + 4 * u + wave, g.Mb - 1) * g.Kb + k_beg) * 256);
+    for (int u = 0; u < AU; u++) src[u] = uniform_address(g.A + ((size_t)min(mb0 + 4 * u + wave, g.Mb - 1) * g.Kb + k_beg) * 256);
 #pragma unroll
     for (int u = 0; u < 2; u++)
-        src[AU + u] = uniform(reinterpret_cast<const half8 *>(g.W.w16) + ((size_t)min(nb0 + 4 * u + wave, g.Nb - 1) * g.Kb + k_beg) * 256);
-    const uint32_t a_off = a_lane(lane) * 16, w_off = lane * 16;
-    typedef __attribute__((address_space(3))) void lds_void;
-    const uint32_t place0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void *)lds + wave * 2048);
-    constexpr int COPIES = 2 * (AU + 2);                      // of 1 KB, per half step and wave
-    static_assert(NB * COPIES < 64, "the hand-written waits count this wave's LDS-direct loads; vmcnt has six bits");
-    // copy c of half step hs (koff = 2048 hs) into the buffer that this wave's first place `place` lies in
-    auto copy = [&](uint32_t place, uint32_t koff, int c) __attribute__((always_inline)) {
-        const int u = c >> 1;
-        const uint32_t off = (u < AU ? a_off : w_off) + koff;
-        if (c & 1) asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024" :: "v"(off), "s"(src[u]), "s"(place), "n"(u * 8192) : "m0", "scc");
-        else asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(src[u]), "s"(place), "n"(u * 8192) : "m0", "scc");
-    };
-    const half8 *const frag = lds + (lane >> 5) * 64 + ((lane >> 4) & 1) * 32 + (lane & 15);
-    const half8 *const fa = frag + MI / 2 * wm * 128, *const fw = frag + (AB + 4 * wn) * 128;
-    auto read = [&](const half8 *f, int t, int buf) __attribute__((always_inline)) { return f[buf + (t >> 1) * 128 + (t & 1) * 16]; };
-
-    half8 A0[MI], A1[MI], W0[8], W1[8];
-    // the wait and barrier of a half step behind which `open` requests may still be under way
-    auto meet = [&](int open) __attribute__((always_inline)) {
-        if (NB > 5 && open >= 4) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((NB - 2) * COPIES) : "memory");
-        else if (open >= 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(3 * COPIES) : "memory");
-        else if (open == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * COPIES) : "memory");
-        else if (open == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(COPIES) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-    // Half step hs: its fragments are in A and W; the next one's come out of the buffer at `nxt`; MORE: hs + NB goes into the buffer of
-    // hs, at `place`.  (sched_barrier: the reads stay under the MFMAs where they are written.)
-    auto step = [&](auto more, const half8 (&A)[MI], const half8 (&W)[8], half8 (&An)[MI], half8 (&Wn)[8], int hs, int nxt, uint32_t place) __attribute__((always_inline)) {
-        constexpr bool MORE = decltype(more)::value;
-        constexpr int READS = MI + 8, EVERY = MI == 8 ? 3 : 2;  // (256 rows: 16 reads under 48 of the 64 MFMAs; 128: 12 under 24 of 32)
-        unrolled<8 * MI>([&](auto X) __attribute__((always_inline)) {
-            constexpr int x = X, i = x / MI, j = x % MI, t = x / EVERY;
-            if constexpr (x % EVERY == 0 && t < READS) {
-                if constexpr (t < MI) An[t] = read(fa, t, nxt); else Wn[t - MI] = read(fw, t - MI, nxt);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if constexpr (MORE && j == 3 && i < COPIES) copy(place, (uint32_t)(hs + NB) * 2048, i);
-            AccTile<x>::add(A[j], W[i]);
-        });
-        __builtin_amdgcn_sched_barrier(0);
-        if (MORE) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((NB - 2) * COPIES) : "memory");
-        else meet(last - hs - 2);
-    };
-    auto request = [&](uint32_t place, int hs) __attribute__((always_inline)) {
-#pragma unroll
-        for (int c = 0; c < COPIES; c++) copy(place, (uint32_t)hs * 2048, c);
-    };
-    // (nothing is requested past the end: a block's last half steps would wait for it -- five buffers, 3 us where all CUs do)
-    request(place0, 0); request(place0 + HB * 16, 1);
-#pragma unroll
-    for (int h = 2; h < NB; h++) if (h <= last) request(place0 + h * HB * 16, h);
-    unrolled<8 * MI>([](auto X) __attribute__((always_inline)) { AccTile<X>::clear(); });
-    meet(min(NB, nhalf) - 2);                                 // the first two have landed
-#pragma unroll
-    for (int t = 0; t < MI; t++) A0[t] = read(fa, t, 0);
-#pragma unroll
-    for (int t = 0; t < 8; t++) W0[t] = read(fw, t, 0);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // every wave has read buffer 0 before it is requested anew
-    int nxt = HB, hs = 0;
-    uint32_t place = place0;
-    auto advance = [&]() __attribute__((always_inline)) {
-        nxt = nxt == (NB - 1) * HB ? 0 : nxt + HB;
-        place = place == place0 + (NB - 1) * HB * 16 ? place0 : place + HB * 16;
-    };
-    constexpr std::true_type more{};
-    constexpr std::false_type done{};
-    for (; hs + 1 + NB <= last; hs += 2) {
-        step(more, A0, W0, A1, W1, hs, nxt, place); advance();
-        step(more, A1, W1, A0, W0, hs + 1, nxt, place); advance();
-    }
-    if (NB % 2 && hs + NB <= last) request(place, hs + NB);   // (an odd ring: the last half step, nhalf being even)
-    for (; hs < nhalf; hs += 2) {
-        step(done, A0, W0, A1, W1, hs, nxt, place); advance();
-        step(done, A1, W1, A0, W0, hs + 1, nxt, place); advance();
-    }
-    settle_tiles();
+        src[AU + u] = uniform_address(reinterpret_cast<const half8 *>(g.W.w16) + ((size_t)min(nb0 + 4 * u + wave, g.Nb - 1) * g.Kb + k_beg) * 256);
+    walk_k<BM, NB>(lds, src, a_lane(lane) * 16, nhalf);
 
     if (mb0 * 32 + BM <= g.M && (nb0 + 8) * 32 <= g.N) {      // a block inside the matrix: stores without tests
         unrolled<MI>([&](auto J) __attribute__((always_inline)) {
@@ -636,10 +553,6 @@ __global__ __launch_bounds__(256) void gemm_big_pair(GemmKArgs g, int lo)
 
     // this wave's share of a half step: both slices of a value, its residual and two W row blocks (clamped: rows past the end
     // are computed and never stored), as uniform bases and one lane offset per operand
-    auto uniform = [](const half8 *p) __attribute__((always_inline)) {
-        const uint64_t x = reinterpret_cast<uint64_t>(p);
-        return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32;
-    };
     const int ab = min(mb0 + wave, g.Mb - 1);
     const half8 *const w16 = reinterpret_cast<const half8 *>(g.W.w16);
     uint64_t src[4];
@@ -665,10 +578,10 @@ __global__ __launch_bounds__(256) void gemm_big_pair(GemmKArgs g, int lo)
     auto enter = [&](int p) __attribute__((always_inline)) {
         nt = p / g.Kb; k_beg = p - nt * g.Kb;
         last = 2 * min(g.Kb - k_beg, end - p) - 1;
-        src[0] = uniform(g.A + ((size_t)ab * g.Kb + k_beg) * 256);
-        src[1] = uniform(g.A + ((size_t)(ab + (lo >> 5)) * g.Kb + k_beg) * 256);
+        src[0] = uniform_address(g.A + ((size_t)ab * g.Kb + k_beg) * 256);
+        src[1] = uniform_address(g.A + ((size_t)(ab + (lo >> 5)) * g.Kb + k_beg) * 256);
 #pragma unroll
-        for (int u = 0; u < 2; u++) src[2 + u] = uniform(w16 + ((size_t)min(nt * 8 + 4 * u + wave, g.Nb - 1) * g.Kb + k_beg) * 256);
+        for (int u = 0; u < 2; u++) src[2 + u] = uniform_address(w16 + ((size_t)min(nt * 8 + 4 * u + wave, g.Nb - 1) * g.Kb + k_beg) * 256);
 #pragma unroll
         for (int h = 0; h < NB - 1; h++)
 #pragma unroll
