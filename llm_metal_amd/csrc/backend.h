@@ -23,6 +23,12 @@ struct MetalBuf {
 namespace lmhip {
 
 hipStream_t stream();
+// A branch of the work beside the stream.  side_begin: a second stream of the library's, behind everything that stream() holds
+// so far; side_end: what is put into stream() from here on waits for the branch.  Every begin has its end before the call that
+// began it returns, so waiting for stream() waits for both.  A branch takes no scratch arena (they belong to stream()) and
+// writes nothing that stream() reads or writes before the end.
+hipStream_t side_begin();
+void side_end();
 int  initialized();
 int  num_cus();
 void die(const char *what, hipError_t e, const char *file, int line);

@@ -8,6 +8,8 @@
 namespace {
 int         g_refcount = 0;
 hipStream_t g_stream = nullptr;
+hipStream_t g_side = nullptr;             // made when first used
+hipEvent_t  g_side_from = nullptr, g_side_to = nullptr;
 int         g_num_cus = 0;
 struct Arena { void *p = nullptr; size_t cap = 0; };
 Arena       g_scratch[lmhip::SCR_COUNT];
@@ -16,6 +18,21 @@ Arena       g_scratch[lmhip::SCR_COUNT];
 namespace lmhip {
 
 hipStream_t stream() { return g_stream; }
+hipStream_t side_begin()
+{
+    if (!g_side) {
+        HIP_CHECK(hipStreamCreateWithFlags(&g_side, hipStreamNonBlocking));
+        for (hipEvent_t *e : {&g_side_from, &g_side_to}) HIP_CHECK(hipEventCreateWithFlags(e, hipEventDisableTiming | hipEventReleaseToDevice));
+    }
+    HIP_CHECK(hipEventRecord(g_side_from, g_stream));
+    HIP_CHECK(hipStreamWaitEvent(g_side, g_side_from, 0));
+    return g_side;
+}
+void side_end()
+{
+    HIP_CHECK(hipEventRecord(g_side_to, g_side));
+    HIP_CHECK(hipStreamWaitEvent(g_stream, g_side_to, 0));
+}
 int initialized() { return g_refcount > 0; }
 int num_cus() { return g_num_cus; }
 
@@ -81,6 +98,12 @@ void fast_metal_shutdown(void)
     for (auto &a : g_scratch) { if (a.p) hipFree(a.p); a.p = nullptr; a.cap = 0; }
     hipStreamDestroy(g_stream);
     g_stream = nullptr;
+    if (!g_side) return;
+    hipStreamSynchronize(g_side);
+    hipEventDestroy(g_side_from);
+    hipEventDestroy(g_side_to);
+    hipStreamDestroy(g_side);
+    g_side = nullptr; g_side_from = g_side_to = nullptr;
 }
 
 MetalBuf *metal_buf_create(size_t size)

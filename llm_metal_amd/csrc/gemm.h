@@ -167,7 +167,7 @@ int big_gemm_policy();                 // hip_gemm_force_large_m's choice
 // tiled images group_stride halves apart: row block i of 128 rows is multiplied with weight group_of[i] (device), and only the
 // first group_of[M / 128] blocks have rows (the rest of C is not written).  M is a multiple of 128; `groups`: how many weights.
 void launch_gemm_groups(const half_t *A_tiled, const float *a_inv_scale, const half_t *W_tiled, size_t group_stride, const int *group_of,
-                        float *C, int ldc, int M, int N, int K, int groups);
+                        float *C, int ldc, int M, int N, int K, int groups, hipStream_t s);
 // true when the large-M kernel is the faster one for this product; one_plane: its result is wanted in one plane
 bool use_big_gemm(int M, int N, int K, int fmt, bool one_plane = false);
 bool mid_takes_big(int M, int N, int K, bool one_plane);   // the part of that rule for 65 to 1023 rows on F16 tiles (gemm_big.hip)

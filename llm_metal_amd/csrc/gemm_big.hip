@@ -1187,7 +1187,7 @@ PairPlanes launch_short_pair(const half_t *A, const float *inv, const WeightOp &
 }
 
 void launch_gemm_groups(const half_t *A, const float *a_inv_scale, const half_t *W, size_t group_stride, const int *group_of, float *C, int ldc,
-                        int M, int N, int K, int groups)
+                        int M, int N, int K, int groups, hipStream_t s)
 {
     if (M <= 0 || N <= 0 || K <= 0) return;
     if (ldc < N || (M & 127) || !A || !W || !group_of || group_stride < tiled_elems(N, K)) {
@@ -1202,8 +1202,8 @@ void launch_gemm_groups(const half_t *A, const float *a_inv_scale, const half_t 
     const dim3 grid(8 * ((mt * nt + 7) / 8));
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
     if (gemm_prof_begin(2.0 * groups * N * K, 2.0 * M * N * K, &ev_a, &ev_b))
-        hipExtLaunchKernelGGL((gemm_big_f16<128, true>), grid, dim3(256), 0, stream(), ev_a, ev_b, 0, g, GroupArgs{group_of, group_stride});
-    else hipLaunchKernelGGL((gemm_big_f16<128, true>), grid, dim3(256), 0, stream(), g, GroupArgs{group_of, group_stride});
+        hipExtLaunchKernelGGL((gemm_big_f16<128, true>), grid, dim3(256), 0, s, ev_a, ev_b, 0, g, GroupArgs{group_of, group_stride});
+    else hipLaunchKernelGGL((gemm_big_f16<128, true>), grid, dim3(256), 0, s, g, GroupArgs{group_of, group_stride});
     HIP_CHECK(hipGetLastError());
 }
 

@@ -6,7 +6,7 @@ namespace lmhip {
 namespace {
 
 #define LAUNCH(kern, grid, block, lds, ...) do { \
-    hipLaunchKernelGGL(kern, grid, block, lds, stream(), __VA_ARGS__); HIP_CHECK(hipGetLastError()); } while (0)
+    hipLaunchKernelGGL(kern, grid, block, lds, s, __VA_ARGS__); HIP_CHECK(hipGetLastError()); } while (0)
 
 // One wave per row: its experts and their weights
 __global__ __launch_bounds__(256) void k_route(MoeRows a)
@@ -153,28 +153,29 @@ MoeGroups moe_groups_at(int *base, int rows, int top, int E)
     return g;
 }
 
-void launch_moe_groups(const MoeRows &a, const MoeGroups &g)
+void launch_moe_groups(const MoeRows &a, const MoeGroups &g, hipStream_t s)
 {
     const int n = a.rows * a.top;
     LAUNCH(k_moe_count, dim3(a.E), dim3(256), 0, a.idx, n, g.count);
     LAUNCH(k_moe_place, dim3(a.E), dim3(256), 0, a.idx, n, a.top, a.E, g);
 }
 
-void launch_moe_gather(const MoeGroups &g, const half_t *a16, const float *inv, half_t *out16, float *out_inv, int K)
+void launch_moe_gather(const MoeGroups &g, const half_t *a16, const float *inv, half_t *out16, float *out_inv, int K, hipStream_t s)
 {
     const int Kb = tiled_kb(K), per = 16;
     LAUNCH(k_moe_gather, dim3(g.tiles * 4, (Kb + per - 1) / per), dim3(256), 0, g, a16, inv, out16, out_inv, Kb, per);
 }
 
-void launch_moe_act(const MoeGroups &g, const float *up, int ld, int n, half_t *out16, float *out_inv, int K)
+void launch_moe_act(const MoeGroups &g, const float *up, int ld, int n, half_t *out16, float *out_inv, int K, hipStream_t s)
 {
     LAUNCH(k_moe_act, dim3(g.tiles * 128), dim3(256), (size_t)K * 4, g, up, ld, n, out16, out_inv, K);
 }
 
-void launch_route(const MoeRows &a) { LAUNCH(k_route, dim3((a.rows + 3) / 4), dim3(256), 0, a); }
+void launch_route(const MoeRows &a, hipStream_t s) { LAUNCH(k_route, dim3((a.rows + 3) / 4), dim3(256), 0, a); }
 
 void launch_experts_per_row(const MoeRows &a)
 {
+    hipStream_t s = stream();
     const dim3 up((a.ffp + 3) / 4, a.top, a.rows), down((a.Dp + 3) / 4, a.rows);
     if (a.f32) { LAUNCH(k_expert_up<float>, up, dim3(256), 0, a); LAUNCH(k_expert_down<float>, down, dim3(256), 0, a); }
     else { LAUNCH(k_expert_up<half_t>, up, dim3(256), 0, a); LAUNCH(k_expert_down<half_t>, down, dim3(256), 0, a); }

@@ -309,16 +309,17 @@ struct MoeRows {
     float *act;                                          // [rows][top][ffp]
     float *y;                                            // [rows][Dp]
 };
-void launch_route(const MoeRows &a);
+// (s: the stream, or a branch beside it)
+void launch_route(const MoeRows &a, hipStream_t s);
 void launch_experts_per_row(const MoeRows &a);           // each row reads its own experts
 
 int moe_group_tiles(int rows, int top, int E);
 size_t moe_group_ints(int rows, int top, int E);
 MoeGroups moe_groups_at(int *base, int rows, int top, int E);
-void launch_moe_groups(const MoeRows &a, const MoeGroups &g);
+void launch_moe_groups(const MoeRows &a, const MoeGroups &g, hipStream_t s);
 // rows of the tiled operand a16 (K columns, factors inv) gathered into the groups' order
-void launch_moe_gather(const MoeGroups &g, const half_t *a16, const float *inv, half_t *out16, float *out_inv, int K);
+void launch_moe_gather(const MoeGroups &g, const half_t *a16, const float *inv, half_t *out16, float *out_inv, int K, hipStream_t s);
 // squared ReLU of [tiles * 128][ld] as the next product's operand of K columns (n of them real)
-void launch_moe_act(const MoeGroups &g, const float *up, int ld, int n, half_t *out16, float *out_inv, int K);
+void launch_moe_act(const MoeGroups &g, const float *up, int ld, int n, half_t *out16, float *out_inv, int K, hipStream_t s);
 
 }  // namespace lmhip

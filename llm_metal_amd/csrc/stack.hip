@@ -620,6 +620,49 @@ void feed_forward(LayerStack *st, StackRun *r, StackLayer &L, int n)
     r->pending = 1; r->post_g = ptr<float>(L.g_ff_post); r->post_b = nullptr;
 }
 
+MoeRows moe_rows(const LayerStack *st, const StackRun *r, const StackLayer &L, int n)
+{
+    const LayerConfig &c = L.c;
+    MoeRows m{};
+    m.rows = n; m.E = c.experts; m.top = c.top; m.ff = c.ff; m.ffp = L.down.cols; m.D = st->D; m.Dp = st->Dp; m.f32 = st->f32;
+    m.up_rows = L.up_rows; m.down_rows = L.down_rows;
+    m.z = ptr<float>(r->cin) + L.o_router; m.ldz = L.in.rows; m.idx = ptr<int>(r->route_idx); m.w = ptr<float>(r->route_w);
+    m.h = ptr<float>(r->h); m.up = dptr(L.up.buf); m.down = dptr(L.down.buf); m.act = ptr<float>(r->act); m.y = ptr<float>(r->ymoe);
+    return m;
+}
+
+// The branch for a layer's experts, wherever they are grouped (16 rows and more): beside the mixer, both read the norm's rows
+// and what the first product made of them, and neither fills the chip (the delta rule's chunks are 64 workgroups for 103 us at
+// 2000 tokens, the experts' launches together 120 us).  Nevurax 1k, prompt and one token, in line -> beside: 16 tokens 724 -> 604 us,
+// 100 tokens 798 -> 660, 600 tokens 1025 -> 842, 2000 tokens 1641 -> 1344.
+// Their tiled images are made (once) in the stream, ahead of it.
+hipStream_t experts_begin(const StackLayer &L)
+{
+    tiled_weight_of(L.up.buf, L.up.rows, L.up.cols);
+    tiled_weight_of(L.down.buf, L.down.rows, L.down.cols);
+    return side_begin();
+}
+
+// the experts' part of a layer over all rows, sorted by expert; writes the run's route_* and moe_* buffers alone
+void grouped_experts(LayerStack *st, StackRun *r, const StackLayer &L, int n, hipStream_t s)
+{
+    const LayerConfig &c = L.c;
+    const MoeRows m = moe_rows(st, r, L, n);
+    launch_route(m, s);
+    const MoeGroups g = moe_groups_at(ptr<int>(r->moe_tab), n, c.top, c.experts);
+    const int M = g.tiles * 128;
+    float *up = ptr<float>(r->moe_up), *inv = ptr<float>(r->moe_inv), *inv_act = inv + r->moe_rows;
+    half_t *rows16 = ptr<half_t>(r->moe_a16), *act16 = ptr<half_t>(r->moe_act);
+    launch_moe_groups(m, g, s);
+    launch_moe_gather(g, ptr<half_t>(r->a16), ptr<float>(r->inv), rows16, inv, st->Dp, s);
+    launch_gemm_groups(rows16, inv, tiled_weight_of(L.up.buf, L.up.rows, L.up.cols), tiled_elems(L.up_rows, L.up.cols), g.of, up, L.up_rows,
+                       M, c.ff, L.up.cols, c.experts, s);
+    launch_moe_act(g, up, L.up_rows, c.ff, act16, inv_act, m.ffp, s);
+    launch_gemm_groups(act16, inv_act, tiled_weight_of(L.down.buf, L.down.rows, L.down.cols), tiled_elems(L.down_rows, L.down.cols), g.of,
+                       ptr<float>(r->moe_y), st->Dp, M, st->Dp, L.down.cols, c.experts, s);
+    r->groups = g; r->groups_top = c.top;
+}
+
 // decoding one sequence with F16 weights and norms around the sublayers: the vector of every product is the residual with
 // the sum before it, both normed inside the product's launch; the residual goes back and forth between two places.
 // emb: the token's row where it is the residual as it lies in the table, or null (r->x holds it)
@@ -735,37 +778,29 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
         const bool grouped = c.experts && !st->f32 && n >= 16 && n * c.top >= c.experts;
         norm(st, r, L.g_norm, n, 1, c.experts && !grouped);
         product(st, L.in, ptr<half_t>(r->a16), ptr<float>(r->inv), ptr<float>(r->h), st->Dp, ptr<float>(r->cin), n);
+        // (a dense feed-forward overwrites the rows that the experts read)
+        const bool beside = grouped && !c.dense_ff;
         CatRows cat = cat_rows(st, r, L);
+        const hipStream_t s = beside ? experts_begin(L) : stream();
         switch (c.mixer) {
         case MIX_LATENT: cat.o = mix_latent(st, r, L, r->layers[i], rows); break;
         case MIX_GROUPED: cat.o = mix_grouped(st, r, L, rows, cat); break;
         case MIX_MLSTM: cat.o = mix_mlstm(st, r, L, r->layers[i], rows, cat); break;
         default: cat.o = mix_delta(st, r, L, r->layers[i], rows, cat);
         }
+        if (beside) grouped_experts(st, r, L, n, s);
         launch_cat_rows(cat, n);
         product(st, L.out, cat.a16, cat.inv, cat.cat, cat.ldk, ptr<float>(r->cout), n);
-        r->pending = 1; r->post_g = ptr<float>(L.g_post); r->post_b = ptr<float>(L.b_out);
+        r->post_g = ptr<float>(L.g_post); r->post_b = ptr<float>(L.b_out);
+        if (beside) { side_end(); r->pending = 5; continue; }
+        r->pending = 1;
         if (c.dense_ff) feed_forward(st, r, L, n);
         if (!c.experts) continue;
-        MoeRows m{};
-        m.rows = n; m.E = c.experts; m.top = c.top; m.ff = c.ff; m.ffp = L.down.cols; m.D = st->D; m.Dp = st->Dp; m.f32 = st->f32;
-        m.up_rows = L.up_rows; m.down_rows = L.down_rows;
-        m.z = ptr<float>(r->cin) + L.o_router; m.ldz = L.in.rows; m.idx = ptr<int>(r->route_idx); m.w = ptr<float>(r->route_w);
-        m.h = ptr<float>(r->h); m.up = dptr(L.up.buf); m.down = dptr(L.down.buf); m.act = ptr<float>(r->act); m.y = ptr<float>(r->ymoe);
-        launch_route(m);
-        if (!grouped) { launch_experts_per_row(m); r->pending = 3; continue; }
-        const MoeGroups g = moe_groups_at(ptr<int>(r->moe_tab), n, c.top, c.experts);
-        const int M = g.tiles * 128;
-        float *up = ptr<float>(r->moe_up), *inv = ptr<float>(r->moe_inv), *inv_act = inv + r->moe_rows;
-        half_t *rows16 = ptr<half_t>(r->moe_a16), *act16 = ptr<half_t>(r->moe_act);
-        launch_moe_groups(m, g);
-        launch_moe_gather(g, ptr<half_t>(r->a16), ptr<float>(r->inv), rows16, inv, st->Dp);
-        launch_gemm_groups(rows16, inv, tiled_weight_of(L.up.buf, L.up.rows, L.up.cols), tiled_elems(L.up_rows, L.up.cols), g.of, up, L.up_rows,
-                           M, c.ff, L.up.cols, c.experts);
-        launch_moe_act(g, up, L.up_rows, c.ff, act16, inv_act, m.ffp);
-        launch_gemm_groups(act16, inv_act, tiled_weight_of(L.down.buf, L.down.rows, L.down.cols), tiled_elems(L.down_rows, L.down.cols), g.of,
-                           ptr<float>(r->moe_y), st->Dp, M, st->Dp, L.down.cols, c.experts);
-        r->pending = 5; r->groups = g; r->groups_top = c.top;
+        if (grouped) { grouped_experts(st, r, L, n, s); r->pending = 5; continue; }
+        const MoeRows m = moe_rows(st, r, L, n);
+        launch_route(m, s);
+        launch_experts_per_row(m);
+        r->pending = 3;
     }
 }
 

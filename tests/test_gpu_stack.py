@@ -97,6 +97,23 @@ def test_states_are_used_again(mixed, tmp_path):
                     assert np.array_equal(got, run_portions(fresh, p, [17, 2, 1]))
 
 
+@pytest.mark.parametrize("n", [15, 16, 17, 110])
+def test_experts_beside_the_mixer(n, tmp_path):
+    """From 16 rows on the experts run beside the mixer: against the oracle, and passes that follow one another without a wait
+    between their launches give the same bits."""
+    cfg, ra, rg = MODELS["mixed"]
+    m = Model(cfg, tmp_path, ra, rg)
+    toks = m.tokens(n, seed=3)
+    want = so.run(cfg, m.W, toks)
+    with state(m, "f16") as inf, state(m, "f16") as other:
+        first = inf.forward_tokens(toks, [n - 1])
+        for _ in range(5):
+            for st in (inf, other):
+                st.reset()
+                assert np.array_equal(st.forward_tokens(toks, [n - 1]), first)
+        assert logit_error(first, want[n - 1:]) < TOL["f16"]
+
+
 @MIXED
 @pytest.mark.parametrize("fmt", ["f32", "f16"])
 def test_lock_step_batches_against_each_alone(fmt, mixed, tmp_path):
