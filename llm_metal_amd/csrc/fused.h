@@ -282,5 +282,9 @@ void launch_wgrads(const WgradOperands *w, int n, int T, int mode, float lr);
 void launch_apply_retile(half_t *W_tiled, half_t *G_tiled, half_t *WT_tiled, int M_out, int N_in, float lr,
                          int matrices = 1, size_t stride = 0, size_t strideT = 0);
 void launch_untile_f16(const half_t *src_tiled, int Kb, int row_off, int k_off, int transpose, int rows, int cols, half_t *dst);
+// the same for whole columns from row block rb0 on, many matrices to a launch (UNTILE_JOBS a power of two)
+struct UntileJob { const half_t *src; half_t *dst; int Kb, rb0, rows, cols; };
+constexpr int UNTILE_JOBS = 64;
+void launch_untile_jobs(const UntileJob *jobs, int n);
 
 }  // namespace lmhip

@@ -1316,20 +1316,25 @@ LayerW *sft_get_layers(SFTState *s)
                                       view(s->g_q, s->hd), view(s->g_k, s->hd)};
         }
     }
+    std::vector<UntileJob> jobs;                          // all matrices in one launch (or a few)
     for (int L = 0; L < NL; L++) {
         struct Src { MetalBuf *W; size_t st; int N, row_off, kind; };
         const Src src[7] = {{s->wqkv, s->st_qkv, D, 0, W_QKV}, {s->wqkv, s->st_qkv, D, qd, W_QKV}, {s->wqkv, s->st_qkv, D, qd + kd, W_QKV},
                             {s->wo, s->st_o, qd, 0, W_O}, {s->wgu, s->st_gu, D, 0, W_GU}, {s->wgu, s->st_gu, D, IS, W_GU}, {s->wd, s->st_d, IS, 0, W_D}};
         for (int w = 0; w < 7; w++) {
             half_t *out = at<half_t>(s->wmats_out[(size_t)L * 7 + w].mbuf);
+            const int Kb = tiled_kb(src[w].N);
             if (s->q8_native) {
                 const WeightOp op = wop(s, src[w].kind, L, false);
-                launch_untile_q8(op.q, op.d, 1, tiled_kb(src[w].N), src[w].row_off, 0, 0, rows[w], cols[w], out);
+                launch_untile_q8(op.q, op.d, 1, Kb, src[w].row_off, 0, 0, rows[w], cols[w], out);
+            } else if (src[w].row_off % 32 == 0) {
+                jobs.push_back(UntileJob{at<half_t>(src[w].W, L * src[w].st), out, Kb, src[w].row_off / 32, rows[w], cols[w]});
             } else {
-                launch_untile_f16(at<half_t>(src[w].W, L * src[w].st), tiled_kb(src[w].N), src[w].row_off, 0, 0, rows[w], cols[w], out);
+                launch_untile_f16(at<half_t>(src[w].W, L * src[w].st), Kb, src[w].row_off, 0, 0, rows[w], cols[w], out);
             }
         }
     }
+    launch_untile_jobs(jobs.data(), (int)jobs.size());
     return s->layers_out.data();
 }
 

@@ -285,3 +285,22 @@ def test_full_checkpoint_file_and_layer_accessors():
         lm = st.L.sft_get_lm_head(st.h).contents
         got = Buf(st.L, lm.mbuf, lm.rows * lm.cols * 2, owned=False).read(np.uint16, (lm.rows, lm.cols))
         assert np.array_equal(got, oracle.f32_to_f16_bits(used["lm_head"]))
+
+
+@pytest.mark.parametrize("change", [dict(NL=1), dict(NL=9, V=1000, D=192, Hq=3, Hkv=1, IS=416), dict(NL=10, V=4100), dict(NL=19)],
+                         ids=lambda d: f"{d['NL']} layers, V {d.get('V', C1.V)}")
+def test_matrices_handed_out(change):
+    """Every matrix of sft_get_layers / sft_get_lm_head, bit for bit: widths that end inside a tile of 64, row counts that end inside
+    one of 32, and layer counts on both sides of what one launch takes (64 matrices)."""
+    from llm_metal_amd.sft import Buf
+    cfg = C1.with_(name="handed_out", R=0, **change)
+    model = make_model(cfg, seed=5)
+    used = oracle.weights_as_used(model)
+    fields = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
+    with SFTState(cfg, model) as st:
+        layers = st.L.sft_get_layers(st.h)
+        mats = [(getattr(layers[i], f).contents, used[k][i]) for i in range(cfg.NL) for f, k in zip(fields, MATS)]
+        mats.append((st.L.sft_get_lm_head(st.h).contents, used["lm_head"]))
+        for wm, want in mats:
+            got = Buf(st.L, wm.mbuf, wm.rows * wm.cols * 2, owned=False).read(np.uint16, (wm.rows, wm.cols))
+            assert np.array_equal(got, oracle.f32_to_f16_bits(want))
