@@ -1152,6 +1152,15 @@ bool few_rows_fit(const InferenceState *s)
     return true;
 }
 
+// Logits that the head's kernel stores into pinned memory leave it in parts of the vocabulary (whole row blocks of the weight, enough of them to fill the
+// chip), so that the caller's copy of one part is made while the next one is formed.
+int batch_parts(const InferenceState *s, const BatchRun &r)
+{
+    const size_t bytes = (size_t)r.B * s->V * sizeof(float);
+    return bytes < ((size_t)512 << 10) || s->V < 16384 ? 1 : bytes < ((size_t)4 << 20) || s->V < 32768 ? 2 : 4;
+}
+int batch_part(const InferenceState *s, int i, int parts) { return i < parts ? (int)((long)s->V * i / parts / 32 * 32) : s->V; }   // its first column
+
 // One step for B tokens at the same position: forward_token_batch, src/nn/fast_inference.c:808-893.  Every product
 // reads its weight once for all B vectors (matrix cores over the tiled image, 22 bits of every activation); what
 // is per sequence -- adapter terms, per-head RMSNorm, RoPE, cache store, attention -- has the sequence as a grid
@@ -1159,7 +1168,8 @@ bool few_rows_fit(const InferenceState *s)
 // product's planes are summed by the kernel that consumes them and the norm kernel writes the next product's operand itself,
 // where a row is one workgroup's.
 // host: pinned memory for the logits of a single sequence besides, or null; true: they go there as they are formed.
-bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int pos, float *host = nullptr)
+// to_host (r.few, r.logits_host there): the logits go to r.logits_host instead of r.logits, an event behind each part of batch_parts.
+bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int pos, float *host = nullptr, bool to_host = false)
 {
     if (s->stack) {
         stack_forward(s->stack, r.stk, tokens, 1, pos);
@@ -1247,7 +1257,13 @@ bool forward_token_batch(InferenceState *s, BatchRun &r, const int *tokens, int 
     }
     if (r.few) {
         add_norm_b(pending_few, pending_g, s->g_final);
-        launch_few_full(a16, inv_ln, weight(s->lm_head, bt ? &s->borrowed_lm : nullptr, s->V, D).w16, dptr_as<float>(r.logits), s->V, B, s->V, D);
+        const half_t *W = weight(s->lm_head, bt ? &s->borrowed_lm : nullptr, s->V, D).w16;
+        if (!to_host) launch_few_full(a16, inv_ln, W, dptr_as<float>(r.logits), s->V, B, s->V, D);
+        for (int i = 0, n = to_host ? batch_parts(s, r) : 0; i < n; i++) {
+            const int c0 = batch_part(s, i, n), cols = batch_part(s, i + 1, n) - c0;
+            launch_few_full(a16, inv_ln, W + (size_t)c0 * tiled_kb(D) * 64, r.logits_host + c0, s->V, B, cols, D);
+            HIP_CHECK(hipEventRecord(r.part_there[i], stream()));
+        }
     }
     else {
         add_norm_b(pending, pending_g, s->g_final);
@@ -1321,27 +1337,52 @@ BatchRun &batch_acquire(InferenceState *s, BatchRun *&slot, int B)
     return r;
 }
 
+// pinned memory and events for the run's logits; false: none left
+bool batch_logits_room(InferenceState *s, BatchRun &r)
+{
+    if (!r.logits_host && hipHostMalloc((void **)&r.logits_host, (size_t)r.B * s->V * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        r.logits_host = nullptr;
+        return false;
+    }
+    for (hipEvent_t &e : r.part_there) if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return true;
+}
+
 // The run's logits to the caller's memory, through pinned memory of the run's own.  While the step runs, the pages of `out` are made
 // present (new ones cost a fault each, half of what the runtime's copy takes); then a part is copied while the next one arrives.
+// formed: the head's kernel has stored them there (forward_token_batch, to_host); else they are copied there first.
 // us a step, of which the kernels / with the runtime's copy / in one / two / four parts: 8 sequences of a vocabulary of 32 768 (1 MB,
 // nine layers of the 4B shape) 662 / 910 / 750 / 718 / 738, 32 of 16 384 (2 MB) 278 / 405 / 395 / 364 / 368, 20 of 70 000 (5.6 MB,
 // nine layers of Gemma3-1B's) 1130 with the runtime's, 850 / 800 / 770; 2 of 9 000 (72 KB) 28 more in four parts than in one.
-void batch_logits_to(InferenceState *s, BatchRun &r, float *out)
+// Stored by the head's kernel, a copy in pinned memory ahead of that -> so: 8 sequences of 32 768 722 -> 701 us in two parts (716 / 705 / 699 in one / three /
+// four), 2 of 9 000 with three layers 239 -> 222 in one (225 in two), 4 of 30 000 402 -> 387, 32 of 16 384 463 -> 457, 20 of 70 000 833 -> 815 in four (853 in one).
+void batch_logits_to(InferenceState *s, BatchRun &r, float *out, bool formed)
 {
-    const size_t bytes = (size_t)r.B * s->V * sizeof(float), parts = bytes < ((size_t)512 << 10) ? 1 : bytes < ((size_t)4 << 20) ? 2 : 4;
-    if (!r.logits_host && hipHostMalloc((void **)&r.logits_host, bytes, hipHostMallocDefault) != hipSuccess) { (void)hipGetLastError(); r.logits_host = nullptr; }
-    if (!r.logits_host) {                                                // (no pinned memory left)
+    const size_t V = s->V, bytes = (size_t)r.B * V * sizeof(float);
+    auto pages = [&] { for (size_t at = 0; at < bytes; at += 4096) ((volatile char *)out)[at] = 0; };
+    if (formed) {
+        pages();
+        for (int i = 0, n = batch_parts(s, r); i < n; i++) {
+            const size_t c0 = batch_part(s, i, n), cols = batch_part(s, i + 1, n) - c0;
+            HIP_CHECK(hipEventSynchronize(r.part_there[i]));
+            if (cols == V) memcpy(out, r.logits_host, bytes);
+            else for (int b = 0; b < r.B; b++) memcpy(out + b * V + c0, r.logits_host + b * V + c0, cols * sizeof(float));
+        }
+        return;
+    }
+    if (!batch_logits_room(s, r)) {
         HIP_CHECK(hipMemcpyAsync(out, dptr(r.logits), bytes, hipMemcpyDeviceToHost, stream()));
         HIP_CHECK(hipStreamSynchronize(stream()));
         return;
     }
+    const size_t parts = bytes < ((size_t)512 << 10) ? 1 : bytes < ((size_t)4 << 20) ? 2 : 4;
     auto from = [&](size_t i) { return i < parts ? bytes / 64 * i / parts * 64 : bytes; };
     for (size_t i = 0; i < parts; i++) {
-        if (!r.part_there[i]) HIP_CHECK(hipEventCreateWithFlags(&r.part_there[i], hipEventDisableTiming));
         HIP_CHECK(hipMemcpyAsync((char *)r.logits_host + from(i), (const char *)dptr(r.logits) + from(i), from(i + 1) - from(i), hipMemcpyDeviceToHost, stream()));
         HIP_CHECK(hipEventRecord(r.part_there[i], stream()));
     }
-    for (size_t at = 0; at < bytes; at += 4096) ((volatile char *)out)[at] = 0;
+    pages();
     for (size_t i = 0; i < parts; i++) {
         HIP_CHECK(hipEventSynchronize(r.part_there[i]));
         memcpy((char *)out + from(i), (const char *)r.logits_host + from(i), from(i + 1) - from(i));
@@ -1854,9 +1895,10 @@ int inference_step_batch(InferenceState *s, const int *tokens, int batch_size, i
         if (tokens[b] < 0 || tokens[b] >= s->V) { fprintf(stderr, "[BatchGen] token %d outside the vocabulary (%d)\n", tokens[b], s->V); return -1; }
     BatchRun &r = batch_acquire(s, s->batch, B);
     if (pos != 0 && pos != r.len) { fprintf(stderr, "[BatchGen] step at position %d, but the batch's caches hold %d\n", pos, r.len); return -1; }
-    forward_token_batch(s, r, tokens, pos);
+    const bool formed = logits && r.few && batch_logits_room(s, r);
+    forward_token_batch(s, r, tokens, pos, nullptr, formed);
     r.len = pos + 1;
-    if (logits) batch_logits_to(s, r, logits);
+    if (logits) batch_logits_to(s, r, logits, formed);
     return 0;
 }
 

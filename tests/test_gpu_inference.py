@@ -193,6 +193,23 @@ def test_batch_steps_over_shapes_that_fill_no_tile(kw, batches, model_type):
                 assert maxrel(got[b], single) < 1e-4, (B, b, maxrel(got[b], single))
 
 
+@pytest.mark.parametrize("V,B", [(260, 3), (16380, 9), (16388, 9), (16388, 7), (32772, 31), (32772, 32)])
+def test_parts_of_a_batch_steps_logits(V, B):
+    """Logits that reach the host in parts of the vocabulary (one, two or four by V and B) which end inside a tile of 32 columns: every
+    column of every sequence against the single-sequence path, as in the test above."""
+    say("parts of logits", V, B)
+    c = C1.with_(name="parts", NL=1, seq=8, V=V, tied=True)
+    model = make_model(c, seed=43, gamma_jitter=0.1)
+    seqs = np.random.default_rng(B).integers(1, V, (B, 2))
+    with InferenceState(c, model, max_seq=8, use_fp16=True) as inf:
+        got = np.stack([inf.step_batch(seqs[:, i], i) for i in range(2)], axis=1)
+        assert np.array_equal(got[:, 0], inf.step_batch(seqs[:, 0], 0))
+        for b in sorted({0, 1 % B, B // 2, B - 1}):
+            inf.reset()
+            single = np.stack([inf.forward_token(int(t)) for t in seqs[b]])
+            assert maxrel(got[b], single) < 1e-4, (b, maxrel(got[b], single))
+
+
 @pytest.mark.parametrize("V", [260, 50004, 400004], ids=["one_part", "two_parts", "four_parts"])
 def test_logits_of_batch_steps_are_the_callers_own(V):
     """Ordinary arrays, as numpy's own are: each owns its memory, may be resized, and keeps what it holds when further steps and the end
