@@ -75,6 +75,7 @@ struct GemmPlan {
     int rotate;    // start each workgroup at a different K step of its chunk
     int ring;      // gemm_ring (one 64-row tile of activations; F16 or Q8_0 weights): kg K groups of four waves per workgroup
     int kg;
+    int whole;     // planes stay fp32: cut more often than for balance, where a half per part would round more than one of the sum
     int wide;      // ring plans: gemm_ring_wide, four weight row blocks per workgroup (nb = 4), one K group
 };
 

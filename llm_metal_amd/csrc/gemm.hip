@@ -291,9 +291,10 @@ namespace lmhip {
 // So few row tiles that even sixteen chunks leave CUs without work (outputs of up to 1024 columns): as many chunks as leave each four K
 // steps, two rounds of a workgroup.  A product of four workgroups is their walk through K, and its planes are nothing: 256 columns of K = 256 ..
 // 4096 (a tiny model's) 66 us for the ten of a step in one chunk each, 42 so; the step 268 -> 226 us, as near to 64 bits as before.
+static bool few_row_tiles(int n_tiles, int cus) { return n_tiles * 16 < cus; }
 static int ring_chunks(int n_tiles, int Kb, int K, int cus)
 {
-    if (n_tiles * 16 < cus) return std::min(16, std::max(1, Kb / 4));
+    if (few_row_tiles(n_tiles, cus)) return std::min(16, std::max(1, Kb / 4));
     int best = 1;
     double best_score = -1e9;
     for (int S = 1; S <= 32 && S <= Kb; S++) {
@@ -323,6 +324,7 @@ GemmPlan plan_gemm(int M, int N, int K, int nbq, int fmt)
         p.steps = (Kb + S - 1) / S;
         p.S = (Kb + p.steps - 1) / p.steps;
         p.rotate = 0;
+        p.whole = p.S > 1 && few_row_tiles(p.n_tiles, cus);
         // four weight row blocks per workgroup (up to three workgroups per CU) with the same K chunks, when every CU
         // still gets such a workgroup (with 0.9 of them -- 9728 x 2560 and 6176 x 2560 in three and five chunks -- the
         // products alone gain 2-7 %, the step nothing with F16 weights and it loses 1 % with Q8_0); more than 32 rows: with one

@@ -350,7 +350,7 @@ Planes gemm(SFTState *s, const half_t *A, const float *inv, const WeightOp &W, i
     if (!out && (size_t)p.S * stride > s->planes_cap) { fprintf(stderr, "[fast_sft] plane buffer too small\n"); abort(); }
     if (out && p.S != 1) { fprintf(stderr, "[fast_sft] direct GEMM output needs S == 1\n"); abort(); }
     // a direct (final) output gets its row factors in the GEMM epilogue; planes leave them to the consumer
-    if (out || !p.ring) hscale = 0.f;
+    if (out || !p.ring || p.whole) hscale = 0.f;
     launch_gemm(A, out ? inv : nullptr, W, P, N, stride, s->BN, N, K, p, hscale);
     const float unscale = hscale != 0.f ? 1.0f / hscale : 0.f;
     if (sg && sg->cols) {
