@@ -60,7 +60,7 @@ template <int MAXV, bool GROUPED, int NT = RB>
 __global__ __launch_bounds__(NT) void k_norm_rows(KARGS24)
 {
     KARGS_HOT(NormRowsArgs, a);                           // rows_launched, D, pf
-    __shared__ float sm[32];
+    __shared__ float sm[64];
     if (blockIdx.x >= a.rows_launched) {                  // workgroups beyond the rows fetch weights; they are the last
         prefetch_weight_tiles<NT>(a.pf, blockIdx.x - a.rows_launched);      // to finish and have nothing to wait for
         return;
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(NT) void k_norm_rows(KARGS24)
             float ss = 0.f;
 #pragma unroll
             for (int t = 0; t < MAXV; t++) ss += sumsq4(b[t]);
-            ss = block_sum(ss, sm);
+            ss = block_sum<NT, false>(ss, sm + 32);
             inv = rsqrtf(ss / (float)D + a.eps);
         }
 #pragma unroll
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(NT) void k_norm_rows(KARGS24)
 #pragma unroll
         for (int t = 0; t < MAXV; t++)
             mxg = fmaxf(mxg, amax4(make_float4(x[t].x * gn[t].x, x[t].y * gn[t].y, x[t].z * gn[t].z, x[t].w * gn[t].w)));
-        block_sum_max(ss, mxg, sm);
+        block_sum_max<NT, false>(ss, mxg, sm);
         inv = rsqrtf(ss / (float)D + a.eps);
         amax = mxg * inv;
 #pragma unroll
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(NT) void k_norm_rows(KARGS24)
             x[t].x = x[t].x * inv * g.x; x[t].y = x[t].y * inv * g.y; x[t].z = x[t].z * inv * g.z; x[t].w = x[t].w * inv * g.w;
         }
     } else {
-        ss = block_sum(ss, sm);
+        ss = block_sum<NT, false>(ss, sm);
         inv = rsqrtf(ss / (float)D + a.eps);
 #pragma unroll
         for (int t = 0; t < MAXV; t++) {
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(NT) void k_norm_rows(KARGS24)
             x[t].x = x[t].x * inv * g.x; x[t].y = x[t].y * inv * g.y; x[t].z = x[t].z * inv * g.z; x[t].w = x[t].w * inv * g.w;
             amax = fmaxf(amax, amax4(x[t]));
         }
-        amax = block_max(amax, sm);
+        amax = block_max<NT, false>(amax, sm + 16);
     }
     const float s = row_scale_for(amax);
     const int Kb = tiled_kb(D);
@@ -773,7 +773,7 @@ __global__ __launch_bounds__(NT) void k_qkv_bwd_rows(QkvBwdArgs a)
         }
         __syncthreads();
     }
-    amax = block_max(amax, sm);                           // (every entry of the row was written by a thread that also took it into its maximum)
+    amax = block_max<NT, false>(amax, sm);                           // (every entry of the row was written by a thread that also took it into its maximum)
     const float s = row_scale_for(amax);
     write_f16_tiled(buf, n, a.out16, row, s);
     if (threadIdx.x == 0) a.inv_scale[row] = 1.0f / s;
@@ -999,7 +999,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
             amax = fmaxf(amax, amax4(act[t]));
         }
     }
-    amax = block_max(amax, sm);
+    amax = block_max<NT, false>(amax, sm);
     const float s = row_scale_for(amax);
     const int Kb = tiled_kb(IS);
 #pragma unroll
@@ -1048,7 +1048,7 @@ __global__ __launch_bounds__(GC) void k_glu_fwd_cols(KARGS16)
             amax = fmaxf(amax, amax4(act[t]));
         }
     }
-    amax = block_max(amax, sm);
+    amax = block_max<GC, false>(amax, sm);
     const float s = row_scale_for(amax);
     const int Kb = tiled_kb(IS);
 #pragma unroll
@@ -1104,7 +1104,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
             amax = fmaxf(amax, fmaxf(amax4(dg[t]), amax4(du[t])));
         }
     }
-    amax = block_max(amax, sm);
+    amax = block_max<NT, false>(amax, sm);
     const float s = row_scale_for(amax);
     const int Kb = tiled_kb(2 * IS);
 #pragma unroll
@@ -1155,7 +1155,7 @@ __global__ __launch_bounds__(GC) void k_glu_bwd_cols(KARGS16)
             amax = fmaxf(amax, amax4(o[t]));
         }
     }
-    amax = block_max(amax, sm);
+    amax = block_max<GC, false>(amax, sm);
     const float s = row_scale_for(amax);
     const int Kb = tiled_kb(2 * IS);
 #pragma unroll
@@ -1174,7 +1174,7 @@ template <int MAXV, bool GROUPED, int NT = RB>
 __global__ __launch_bounds__(NT) void k_norm_bwd_rows(KARGS24)
 {
     KARGS_HOT(NormBwdArgs, a);                            // rows_launched, D, pf
-    __shared__ float sm[32];
+    __shared__ float sm[80];
     if (blockIdx.x >= a.rows_launched) {                  // these set the kernel's duration: nothing to wait for
         prefetch_weight_tiles<NT>(a.pf, blockIdx.x - a.rows_launched);
         return;
@@ -1214,7 +1214,7 @@ __global__ __launch_bounds__(NT) void k_norm_bwd_rows(KARGS24)
         ss += sumsq4(x[t]);
         dot += dy[t].x * g[t].x * x[t].x + dy[t].y * g[t].y * x[t].y + dy[t].z * g[t].z * x[t].z + dy[t].w * g[t].w * x[t].w;
     }
-    block_sum2(ss, dot, sm);
+    block_sum2<NT, false>(ss, dot, sm);
     const float inv = rsqrtf(ss / (float)D + a.eps);
     const float coeff = dot * inv * inv / (float)D;
     float4 dx[MAXV];
@@ -1249,7 +1249,7 @@ __global__ __launch_bounds__(NT) void k_norm_bwd_rows(KARGS24)
             ssb += sumsq4(x[t]);
             dotb += dx[t].x * g[t].x * x[t].x + dx[t].y * g[t].y * x[t].y + dx[t].z * g[t].z * x[t].z + dx[t].w * g[t].w * x[t].w;
         }
-        block_sum2(ssb, dotb, sm);
+        block_sum2<NT, false>(ssb, dotb, sm + 32);
         const float invb = rsqrtf(ssb / (float)D + a.eps);
         const float cb = dotb * invb * invb / (float)D;
 #pragma unroll
@@ -1262,7 +1262,7 @@ __global__ __launch_bounds__(NT) void k_norm_bwd_rows(KARGS24)
     }
 #pragma unroll
     for (int t = 0; t < MAXV; t++) amax = fmaxf(amax, amax4(dx[t]));
-    amax = block_max(amax, sm);
+    amax = block_max<NT, false>(amax, sm + 64);
     const float s = row_scale_for(amax);
     const int Kb = tiled_kb(D);
 #pragma unroll
@@ -1289,7 +1289,7 @@ __device__ __forceinline__ void ce_chunk_range(int V, int chunk, int &c_beg, int
 
 __global__ __launch_bounds__(256) void k_ce_partial(CeArgs a)
 {
-    __shared__ float sm[16];
+    __shared__ float sm[32];
     const size_t r = blockIdx.y;
     const int chunk = blockIdx.x, V = a.V;
     const float *lg = a.logits + r * V;
@@ -1306,8 +1306,8 @@ __global__ __launch_bounds__(256) void k_ce_partial(CeArgs a)
         if (m4 > tm) { ts *= expf(tm - m4); tm = m4; }
         ts += expf(x.x - tm) + expf(x.y - tm) + expf(x.z - tm) + expf(x.w - tm);
     }
-    const float mx = block_max(tm, sm);
-    const float sum = block_sum_products(ts, expf(tm - mx), sm);   // a thread without elements: 0 * exp(-1e30 - mx) = 0
+    const float mx = block_max<256, false>(tm, sm);
+    const float sum = block_sum_products<256, false>(ts, expf(tm - mx), sm + 16);   // a thread without elements: 0 * exp(-1e30 - mx) = 0
     if (threadIdx.x == 0) a.partials[r * CE_CHUNKS + chunk] = make_float2(mx, sum);
 }
 
