@@ -132,6 +132,8 @@ struct StackRun {
     std::vector<Layer> layers;
     MetalBuf *x2 = nullptr;                              // the residual's other place (fused steps of NORMS_AROUND)
     const float *xr = nullptr;                                 // where the fused steps left it
+    struct Sum { const float *p = nullptr; int S = 1; size_t plane = 0; const float *inv = nullptr; };
+    Sum waiting;                                         // the output product's planes where the next norm adds them up (p null: cout holds the sum)
     const float *post_g = nullptr, *post_b = nullptr;    // NORMS_AROUND: norm weight and bias of the sum that waits in cout
     MetalBuf *tok = nullptr, *want = nullptr;
     int *tok_host = nullptr, *want_host = nullptr;       // pinned; tok_host [B * max_seq], each portion in its own place
@@ -173,6 +175,7 @@ struct Rows { int B, T, pos; int n() const { return B * T; } };
 // src = want[m] when `want`, else m * step + first.
 struct NormRows {
     float *x; const float *cout, *ymoe;
+    int planes; size_t plane; const float *factor;       // cout: that many planes, `plane` floats apart, whose sum times factor[src] it is (one: as it is)
     const float *g; half_t *a16; float *inv, *h;
     const int *want;
     int step, first, D, Dp, keep; float eps;

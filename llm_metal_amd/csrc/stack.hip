@@ -320,8 +320,9 @@ MlstmAux mlstm_aux(Aux &x, const LayerConfig &c, int B, int T)
     return d;
 }
 
-// C [M][w.rows] = A x w^T; A as the run's F16 operand (a16, inv) or, in 32-bit, as fp32 rows
-void product(const LayerStack *st, const StackMat &w, const half_t *a16, const float *inv, const float *A, int lda, float *C, int M)
+// C [M][w.rows] = A x w^T; A as the run's F16 operand (a16, inv) or, in 32-bit, as fp32 rows.  leave: a product in several planes stays so (in
+// scratch, up to its next use), and they are described there.
+void product(const LayerStack *st, const StackMat &w, const half_t *a16, const float *inv, const float *A, int lda, float *C, int M, StackRun::Sum *leave = nullptr)
 {
     const int N = w.rows, K = w.cols;
     if (st->f32) { launch_gemm_f32(A, lda, dptr_as<float>(w.buf), K, C, N, M, N, K); return; }
@@ -332,6 +333,7 @@ void product(const LayerStack *st, const StackMat &w, const half_t *a16, const f
         if (chunks == 1) { launch_gemm_big(a16, inv, op, C, N, M, N, K); return; }
         float *P = (float *)scratch(SCR_PARTIAL, plane * chunks * sizeof(float));
         const int S = launch_gemm_big(a16, nullptr, op, P, N, M, N, K, chunks, plane);
+        if (leave && S > 1) { *leave = {P, S, plane, inv}; return; }
         launch_reduce_planes(P, S, plane, N, inv, C, M, N);
         return;
     }
@@ -339,6 +341,7 @@ void product(const LayerStack *st, const StackMat &w, const half_t *a16, const f
     if (p.S == 1) { launch_gemm(a16, inv, op, C, N, 0, M, N, K, p); return; }
     float *P = (float *)scratch(SCR_PARTIAL, plane * p.S * sizeof(float));
     launch_gemm(a16, nullptr, op, P, N, plane, M, N, K, p);
+    if (leave) { *leave = {P, p.S, plane, inv}; return; }
     launch_reduce_planes(P, p.S, plane, N, inv, C, M, N);
 }
 
@@ -474,7 +477,8 @@ void norm(LayerStack *st, StackRun *r, MetalBuf *g, int rows, int keep, bool nee
     }
     NormRows n{};
     n.x = ptr<float>(r->x);
-    if (r->pending & 1) n.cout = ptr<float>(r->cout);
+    if (r->pending & 1) n.cout = r->waiting.p ? r->waiting.p : ptr<float>(r->cout);
+    n.planes = r->waiting.S; n.plane = r->waiting.plane; n.factor = r->waiting.inv;
     if (r->pending & 2) n.ymoe = ptr<float>(r->ymoe);
     if (r->pending & 4) { n.moe_y = ptr<float>(r->moe_y); n.moe_pos = r->groups.pos; n.route_w = ptr<float>(r->route_w); n.top = r->groups_top; }
     n.g = ptr<float>(g); n.a16 = ptr<half_t>(r->a16); n.inv = ptr<float>(r->inv); n.h = need_h || st->f32 ? ptr<float>(r->h) : nullptr;
@@ -771,6 +775,10 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
         launch_embed_rows(ptr<float>(st->emb), ptr<int>(r->tok), st->cfg.emb_scale, ptr<float>(r->x), st->D, st->Dp, n);
     }
     if (r->one) { if (st->cfg.norms == NORMS_AROUND) decode_layers_around(st, r, pos, nullptr); else decode_layers(st, r, pos); return; }
+    // the next layer's norm adds up the planes of an output product (nothing between them uses scratch); the last one's sum is made at once:
+    // its norm comes with stack_logits, which other work may precede
+    const bool adds_planes = st->cfg.norms != NORMS_AROUND;
+    r->waiting = {};
     for (size_t i = 0; i < st->layers.size(); i++) {
         StackLayer &L = st->layers[i];
         const LayerConfig &c = L.c;
@@ -790,7 +798,8 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
         }
         if (beside) grouped_experts(st, r, L, n, s);
         launch_cat_rows(cat, n);
-        product(st, L.out, cat.a16, cat.inv, cat.cat, cat.ldk, ptr<float>(r->cout), n);
+        r->waiting = {};
+        product(st, L.out, cat.a16, cat.inv, cat.cat, cat.ldk, ptr<float>(r->cout), n, adds_planes && i + 1 < st->layers.size() ? &r->waiting : nullptr);
         r->post_g = ptr<float>(L.g_post); r->post_b = ptr<float>(L.b_out);
         if (beside) { side_end(); r->pending = 5; continue; }
         r->pending = 1;
