@@ -485,7 +485,7 @@ def _main():
                 "unit": "TFLOP/s" if compute_bound else "GB/s",
                 "frac": round(tfs / MFMA_PEAK_TFS if compute_bound else gbs / HBM_PEAK_GBS, 4), "traffic": None,
                 "kernel": ("gemm_big_q8<1>, gemm_big_q8<2>" if cfg.BN >= 1024 and cfg.weight_format != "f16" and args.q8_large_m == "unpack-in-lds" else
-                           "gemm_big_f16_256, gemm_big_f16" if cfg.BN >= 1024 else
+                           "gemm_big_f16<256>, gemm_big_f16<128>" if cfg.BN >= 1024 else
                            # full-parameter pass: the products, the weight gradients (F16 read-modify-write of the accumulators), the
                            # apply (W, G and the transposed image) and the operand transposes (time only) are timed together
                            "gemm_tiled, gemm_big_f16*, k_wgrad, k_apply_retile, k_transpose_scaled_jobs" if cfg.R == 0 else

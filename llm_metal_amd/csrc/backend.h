@@ -1,5 +1,5 @@
-// Internal header of the HIP backend: buffer handle layout, the library's one
-// stream, scratch arenas and launch-time checks shared by the translation units.
+// Internal header of the HIP backend: buffer handle layout, the library's
+// stream and the branch beside it, scratch arenas and launch-time checks shared by the translation units.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

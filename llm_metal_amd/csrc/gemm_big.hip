@@ -11,7 +11,7 @@
 // with conflict-free 16-byte loads.  LDS is double buffered and the operands travel three steps ahead in registers:
 // during the MFMAs of step k the loads of step k+3 are issued and step k+1 is written to the other buffer; one
 // barrier per step.  That is the kernel for Q8_0 tiles (gemm_big<1>, <2>); F16 tiles take gemm_big_f16 (the same block)
-// or gemm_big_f16_256 (a 256 x 256 block) below, whose operands reach LDS without passing through registers, and
+// or gemm_big_f16<256> (a 256 x 256 block) below, whose operands reach LDS without passing through registers, and
 // launch_gemm_big chooses between the two block shapes, or gives each a part of the columns.
 #include "backend.h"
 #include "devutil.h"
@@ -695,7 +695,7 @@ __global__ __launch_bounds__(256) void gemm_big_pair(GemmKArgs g, int lo)
 // The 256 x 256 block over Q8_0 weight tiles that stay quantised all the way into LDS: the dequant-fused product for
 // many activation rows.  A half step of a weight row block is ONE 1 KB piece (16 int8 per lane: both 8-value slices), its
 // 64 fp16 scales another 128 bytes, so a block's half step is 16 KB of activations + 8 KB of weights instead of 32 KB and
-// six buffers fit; the copies are LDS-direct loads as in gemm_big_f16_256 (the scales as one dword per lane, lanes 32-63
+// six buffers fit; the copies are LDS-direct loads as in gemm_big_f16<256> (the scales as one dword per lane, lanes 32-63
 // fetching the same 128 bytes again into the second half of a 256-byte slot, which keeps every lane active and inside
 // the array).  A wave unpacks its fragments on the way from LDS to the MFMA: bytes to exact fp16 integers with
 // v_perm_b32, times the scale with packed fp16 multiplies -- the values an F16 image of the dequantised weight holds.
@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256) void gemm_big_q8(GemmKArgs g)
 #pragma unroll
             for (int k = 0; k < 4; k++) acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], acc[i][k], 0, 0, 0);
     };
-    // Half step hs is multiplied out of buffer hs % 6 (see gemm_big_f16_256): the barrier that ends half step hs - 1 has
+    // Half step hs is multiplied out of buffer hs % 6 (see gemm_big_f16<256>): the barrier that ends half step hs - 1 has
     // found hs and hs + 1 in LDS, slice 0 of hs + 1 is read and unpacked while slice 1 of hs is multiplied, hs + 5 is
     // requested into the buffer hs - 1 left.  Eight copies per wave and half step.
     auto step = [&](int hs, const uint4v (&cur)[HB], int slot, const uint4v (&nxt)[HB], int nslot, uint4v (&free_buf)[HB], int fslot)
