@@ -1,6 +1,6 @@
 // Backend core: init / shutdown, buffers, flush, scratch arenas.
 // Replaces the buffer and queue half of the reference's src/nn/fast_metal.m
-// (:69-249): one device, one in-order stream, explicit HBM allocations.
+// (:69-249): one device, one in-order stream (and a branch that begins and ends within a call), explicit HBM allocations.
 #include "backend.h"
 #include <string.h>
 #include <vector>
