@@ -144,6 +144,26 @@ def test_prompt_with_adapters(fmt):
                 assert maxrel(inf.forward_token(toks[71]), want[71]) < TOL and inf.position() == 72
 
 
+def test_prompts_on_the_q8_tiles_of_a_training_state():
+    """Products of gate|up go through an F16 image of the tiles from 512 rows on (160 blocks of 128 x 256), and at any length where the
+    large-M kernel is asked for (1: on images, 2: on the tiles as they are); the image holds the values that a tile is unpacked to."""
+    c = C1.with_(name="q8_tiles", weight_format="q8_0", IS=2464)
+    model, toks, L = make_model(c, seed=9, gamma_jitter=0.1), tokens(c, 1024, 10), lib.load()
+    with SFTState(c, model) as sft:
+        sft.train_step(*make_batch(c, seed=8), 1e-3)
+        with InferenceState(sft=sft, max_seq=1024) as inf:
+            want = one_by_one(inf, toks)
+            for policy, n in ((0, 6), (0, 500), (0, 511), (0, 512), (0, 513), (0, 600), (0, 1024), (1, 40), (1, 100), (2, 100)):
+                print(policy, n, flush=True)
+                rows = sorted({0, n // 3, n - 2, n - 1})
+                L.hip_gemm_force_large_m(policy)
+                try:
+                    inf.reset()
+                    assert maxrel(inf.forward_tokens(toks[:n], rows), want[rows]) < TOL
+                finally:
+                    L.hip_gemm_force_large_m(0)
+
+
 def test_generation_from_prompts():
     c = C1
     model, prompt = make_model(c, seed=9, gamma_jitter=0.1), tokens(C1, 45, 10)
