@@ -147,22 +147,26 @@ struct ShortPlan {
     int big, chunks;                   // the large-M kernel with that many K chunks, else t
     GemmPlan t;
     int steps;                         // plan_short_pair: K steps per team of the pair kernel, at most `chunks` planes
+    int lo;                            // plan_short_pair: the operand's row where its residual rows begin
     int planes() const { return big ? chunks : t.S; }
 };
 ShortPlan plan_short_sums(int M, int N, int K, int nbq, int fmt);
 // P: planes() planes; returns how many of them were written.  W: F16 tiles (f16_image_of) where the plan says big.
 int launch_short_sums(const half_t *A_tiled, const WeightOp &W, float *P, size_t plane_stride, int M, int N, int K, const ShortPlan &p);
-ShortPlan plan_short_pair(int M, int lo, int N, int K, int nbq, int fmt);
-// Rows 0 .. M - 1 values and lo .. lo + M - 1 their residuals, `inv` the factors of both (lo a multiple of 32 for the pair kernel).  What was written:
-// S planes of the whole product [M, N], or (whole false) of [lo + M, N] for the consumer to put together; P has room for either.
+// The pair kernel takes the residuals from a row block of their own on, the others right behind the values (five tokens on Q8_0 tiles are ten rows and
+// not 37: two 4B layers 267 -> 261 us, Gemma3-1B's 206 -> 201): a plan is made ahead of its operand.
+constexpr int pair_row(int M) { return (M + 31) & ~31; }
+ShortPlan plan_short_pair(int M, int N, int K, int nbq, int fmt);
+// Rows 0 .. M - 1 values and p.lo .. p.lo + M - 1 their residuals, `inv` the factors of both.  What was written: S planes of the whole product
+// [M, N], or (whole false) of [p.lo + M, N] for the consumer to put together; P has room for either.
 // (whole: planes 0 .. walk.count(n) - 1 hold column n)
 struct PairPlanes { size_t plane; int S; bool whole; PairWalk walk; };
-inline size_t pair_plane_floats(const ShortPlan &p, int M, int lo, int N)
+inline size_t pair_plane_floats(const ShortPlan &p, int M, int N)
 {
-    const size_t apart = (size_t)(p.big ? 1 : p.t.S) * (lo + M), whole = p.big ? (size_t)p.chunks * M : 0;
+    const size_t apart = (size_t)(p.big ? 1 : p.t.S) * (p.lo + M), whole = p.big ? (size_t)p.chunks * M : 0;
     return (apart > whole ? apart : whole) * N;
 }
-PairPlanes launch_short_pair(const half_t *A_tiled, const float *inv, const WeightOp &W, float *P, int M, int lo, int N, int K, const ShortPlan &p);
+PairPlanes launch_short_pair(const half_t *A_tiled, const float *inv, const WeightOp &W, float *P, int M, int N, int K, const ShortPlan &p);
 int big_gemm_policy();                 // hip_gemm_force_large_m's choice
 // The same with F16 tiles for rows that belong to different weights [N, K] of one shape (the experts of a mixture), their
 // tiled images group_stride halves apart: row block i of 128 rows is multiplied with weight group_of[i] (device), and only the

@@ -1139,16 +1139,17 @@ int launch_short_sums(const half_t *A, const WeightOp &W, float *P, size_t plane
 // Value and residual rows: the pair kernel or the streaming kernel over all 2 M rows, by the same times; a block of 128 rows costs the pair kernel
 // what one of 256 costs gemm_big_f16.  Q8_0 tiles that go through their F16 image (plan_short_sums' rule, and not asked to stay quantised)
 // are the pair kernel's as well: a plan that says big for F16 tiles always has its steps.
-ShortPlan plan_short_pair(int M, int lo, int N, int K, int nbq, int fmt)
+ShortPlan plan_short_pair(int M, int N, int K, int nbq, int fmt)
 {
-    ShortPlan p = plan_short_sums(lo + M, N, K, nbq, fmt);
+    ShortPlan p = plan_short_sums(2 * M, N, K, nbq, fmt);
+    p.lo = M;
     const int policy = big_gemm_policy();
     if (policy < 0 || (fmt != 0 && (!p.big || large_m_unpacks_q8()))) return p;
-    if (lo + M <= 64 && !policy) return p;
+    if (M <= 32 && !policy) return p;
     const GemmPlan &t = p.t;
     p.big = 0;
     const int cus = num_cus() > 0 ? num_cus() : 256, Kb = tiled_kb(K);
-    double best = policy || fmt ? 1e30 : 5.1 + 0.152 * (2e-6 * N * K) + 1.65 * (2e-9 * (lo + M) * N * K) + (0.115 + 0.2) * (4e-6 * t.S * (lo + M) * N);
+    double best = policy || fmt ? 1e30 : 5.1 + 0.152 * (2e-6 * N * K) + 1.65 * (4e-9 * M * N * K) + (0.115 + 0.2) * (8e-6 * t.S * M * N);
     // one round: as many teams as the CUs of every XCD hold, or teams of a K-th part of a column block each, without pieces that share a team
     const int mt = (M + 127) / 128, nt = (N + 255) / 256, teams = 8 * std::max(1, cus / 8 / mt), least = std::max(1, (nt * Kb + teams - 1) / teams);
     for (int S = 0; S <= 20 && (S <= 1 || S * 4 <= Kb); S++) {
@@ -1159,11 +1160,13 @@ ShortPlan plan_short_pair(int M, int lo, int N, int K, int nbq, int fmt)
     if (!p.big) return p;
     if (g_big_split != 1) p.steps = std::max(1, Kb / std::max(1, g_big_split));
     p.chunks = PairWalk{p.steps, Kb}.planes();
+    p.lo = pair_row(M);
     return p;
 }
 
-PairPlanes launch_short_pair(const half_t *A, const float *inv, const WeightOp &W, float *P, int M, int lo, int N, int K, const ShortPlan &p)
+PairPlanes launch_short_pair(const half_t *A, const float *inv, const WeightOp &W, float *P, int M, int N, int K, const ShortPlan &p)
 {
+    const int lo = p.lo;
     PairPlanes out{(size_t)(lo + M) * N, 0, false, {}};
     if (M <= 0 || N <= 0 || K <= 0) return out;
     if (lo < M || !inv) { fprintf(stderr, "[fast_hip] gemm_pair: bad rows M=%d lo=%d\n", M, lo); abort(); }

@@ -1446,9 +1446,6 @@ bool memory_for(size_t bytes, bool settled)
     return before >= bytes;
 }
 
-// the row of a step's operands where the residuals of its M rows begin: a row block of the tiles of its own
-int residual_row(int M) { return (M + 31) & ~31; }
-
 // What the products of a step of up to `cap` tokens need: planes, and the F16 images of the largest matrix where none is kept
 size_t prompt_product_bytes(const InferenceState *s, int cap)
 {
@@ -1456,7 +1453,7 @@ size_t prompt_product_bytes(const InferenceState *s, int cap)
     const int qd = s->Hq * s->hd, kd = s->Hkv * s->hd;
     const int shapes[4][2] = {{qd + 2 * kd + (s->borrows_tiles ? 2 * s->R : 0), s->D}, {s->D, qd}, {2 * s->IS, s->D}, {s->D, s->IS}};
     const int head = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V), want = std::min(PROMPT_WANT, cap);
-    auto pair_bytes = [](int M, int N, int K) { const int lo = residual_row(M); return pair_plane_floats(plan_short_pair(M, lo, N, K, 0, 0), M, lo, N) * sizeof(float); };
+    auto pair_bytes = [](int M, int N, int K) { return pair_plane_floats(plan_short_pair(M, N, K, 0, 0), M, N) * sizeof(float); };
     size_t planes = pair_bytes(want, head, s->D), planes2 = 0, image = tiled_elems(head, s->D) * sizeof(half_t);
     for (const auto &sh : shapes) {
         image = std::max(image, tiled_elems(sh[0], sh[1]) * sizeof(half_t));
@@ -1506,7 +1503,7 @@ bool prompt_takes(InferenceState *s, int n)
     if (s->prompt) return true;
     const int qd = s->Hq * s->hd, cap = std::min(PROMPT_ROWS, s->max_seq);
     size_t a16 = 0;
-    for (int K : {s->D, qd, s->IS}) a16 = std::max(a16, tiled_elems(2 * residual_row(cap), K));
+    for (int K : {s->D, qd, s->IS}) a16 = std::max(a16, tiled_elems(2 * pair_row(cap), K));
     const size_t rows = (size_t)cap * (2 * (size_t)s->D + 2 * (size_t)qd + (prompt_glu_supported(s->IS) ? 0 : s->IS) + 4 + 2 * s->R) + s->max_seq + (size_t)PROMPT_WANT * s->D;
     if (!memory_for(rows * sizeof(float) + a16 * sizeof(half_t) + prompt_product_bytes(s, cap), true)) { s->prompt_refused = true; return false; }
     s->prompt = new PromptRun{};
@@ -1516,7 +1513,7 @@ bool prompt_takes(InferenceState *s, int n)
     r.q = fbuf((size_t)cap * qd); r.att = fbuf((size_t)cap * qd);
     if (!prompt_glu_supported(s->IS)) r.act = fbuf((size_t)cap * s->IS);
     r.a16 = metal_buf_create(a16 * sizeof(half_t));
-    r.inv_ln = fbuf((size_t)2 * residual_row(cap)); r.inv_br = fbuf((size_t)2 * residual_row(cap));
+    r.inv_ln = fbuf((size_t)2 * pair_row(cap)); r.inv_br = fbuf((size_t)2 * pair_row(cap));
     r.ids = metal_buf_create((size_t)s->max_seq * sizeof(int));
     r.sel = fbuf((size_t)PROMPT_WANT * s->D);
     HIP_CHECK(hipHostMalloc((void **)&r.ids_host, (size_t)s->max_seq * sizeof(int), hipHostMallocDefault));
@@ -1544,17 +1541,22 @@ float *at_least(MetalBuf *&b, size_t n)
     return dptr_as<float>(b);
 }
 
-// planes of (the operand in r.a16, rows split by `inv`) x w^T: w the state's own matrix (its tiled F16 image, or for Q8_0 the
+// the plan of a prompt's product with a matrix [rows, cols]: the state's own (F16 images in any case) or a training state's tiles
+ShortPlan prompt_plan(const WeightOp *tiles, int rows, int cols, int M)
+{
+    return tiles ? plan_short_pair(M, rows, cols, (tiles->fmt == 1 && tiles->nbq < tiled_rb(rows)) ? tiles->nbq : 0, tiles->fmt) : plan_short_pair(M, rows, cols, 0, 0);
+}
+
+// planes of (the operand in r.a16, rows split by `inv`, residuals from row p.lo on) x w^T: w the state's own matrix (its tiled F16 image, or for Q8_0 the
 // two images of d q and of what rounding that to F16 lost) or a training state's tiles
-SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv, int M, int row0 = 0)
+SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const WeightOp *tiles, int rows, int cols, const float *inv, int M, const ShortPlan &p, int row0 = 0)
 {
     const half_t *a16 = dptr_as<half_t>(r.a16);
     SplitPlanes out{};
-    out.inv = inv; out.N = rows; out.lo = residual_row(M);
+    out.inv = inv; out.N = rows; out.lo = p.lo;
     auto pairs = [&](const WeightOp &op) {
-        const ShortPlan p = plan_short_pair(M, out.lo, rows, cols, (op.fmt == 1 && op.nbq < tiled_rb(rows)) ? op.nbq : 0, op.fmt);
-        float *P = at_least(r.planes, pair_plane_floats(p, M, out.lo, rows));
-        const PairPlanes q = launch_short_pair(a16, inv, p.big ? f16_image_of(op, rows, cols) : op, P, M, out.lo, rows, cols, p);
+        float *P = at_least(r.planes, pair_plane_floats(p, M, rows));
+        const PairPlanes q = launch_short_pair(a16, inv, p.big ? f16_image_of(op, rows, cols) : op, P, M, rows, cols, p);
         out.S = q.S; out.plane = q.plane; out.whole = q.whole; out.walk = q.walk;
     };
     if (tiles) pairs(*tiles);
@@ -1565,8 +1567,8 @@ SplitPlanes prompt_product(InferenceState *s, PromptRun &r, const WMat *w, const
         q8_to_tiled_pair(w->mbuf, rows, cols, hi, lo);
         pairs(weight_f16(hi));
         out.plane2 = (size_t)M * rows;
-        const ShortPlan p = plan_short_sums(M, rows, cols, 0, 0);
-        out.S2 = launch_short_sums(a16, weight_f16(lo), at_least(r.planes2, out.plane2 * p.planes()), out.plane2, M, rows, cols, p);
+        const ShortPlan p2 = plan_short_sums(M, rows, cols, 0, 0);
+        out.S2 = launch_short_sums(a16, weight_f16(lo), at_least(r.planes2, out.plane2 * p2.planes()), out.plane2, M, rows, cols, p2);
         out.P2 = dptr_as<float>(r.planes2);
     }
     out.P = dptr_as<float>(r.planes);
@@ -1584,13 +1586,12 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
 {
     const int D = s->D, Hq = s->Hq, Hkv = s->Hkv, hd = s->hd, IS = s->IS, qd = Hq * hd, nqkv = qd + 2 * Hkv * hd;
     const bool gemma = s->model_type == MODEL_GEMMA3, bt = s->borrows_tiles, adapters = !s->lora.empty();
-    const int lo = residual_row(M);
     const int *ids = dptr_as<int>(r.ids) + pos;
     HIP_CHECK(hipMemcpyAsync((void *)ids, r.ids_host + pos, (size_t)M * sizeof(int), hipMemcpyHostToDevice, stream()));
     launch_embed_ids(dptr_as<float>(s->emb), ids, s->emb_scale, dptr_as<float>(r.x), M, D);
     half_t *a16 = dptr_as<half_t>(r.a16);
     float *inv_ln = dptr_as<float>(r.inv_ln), *inv_br = dptr_as<float>(r.inv_br);
-    auto norm = [&](const SplitPlanes &br, MetalBuf *g_branch, MetalBuf *g, bool keep) {
+    auto norm = [&](const SplitPlanes &br, MetalBuf *g_branch, MetalBuf *g, bool keep, int lo) {
         float *ln = keep ? dptr_as<float>(r.ln) : nullptr;
         const float *gb = g_branch ? dptr_as<float>(g_branch) : nullptr;
         launch_add_norm_split(dptr_as<float>(r.x), br, gb, dptr_as<float>(g), ln, a16, inv_ln, M, lo, D, s->eps);
@@ -1624,8 +1625,9 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
             else launch_few_full(a16, inv_ln, tiles(&lw.qkv, bt ? &bl->qkv : nullptr, nq_rows), P, nq_rows, M, nq_rows, D);
             h.qkv.P = P; h.qkv.S = 1; h.qkv.N = nq_rows; h.qkv.whole = true;
         } else {
-            norm(pending, pending_g, lw.g_in, adapters && !bt);
-            h.qkv = prompt_product(s, r, &lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D, inv_ln, M);
+            const ShortPlan p = prompt_plan(bt ? &bl->qkv : nullptr, nq_rows, D, M);
+            norm(pending, pending_g, lw.g_in, adapters && !bt, p.lo);
+            h.qkv = prompt_product(s, r, &lw.qkv, bt ? &bl->qkv : nullptr, nq_rows, D, inv_ln, M, p);
         }
         h.g_q = lw.g_q ? dptr_as<float>(lw.g_q) : nullptr; h.g_k = lw.g_k ? dptr_as<float>(lw.g_k) : nullptr;
         h.rope = dptr_as<float2>(s->rope_tabs) + ((size_t)s->theta_slot[L] * s->max_seq + pos) * (hd / 2);
@@ -1651,20 +1653,22 @@ void prompt_step(InferenceState *s, PromptRun &r, std::vector<MetalBuf *> &kc, s
             pending_g = gemma ? lw.g_post_ff : nullptr;
             continue;
         }
-        launch_rows_to_f16_split(dptr_as<float>(r.att), a16, inv_br, M, qd, lo);
-        const SplitPlanes o = prompt_product(s, r, lw.o, bt ? &bl->o : nullptr, D, qd, inv_br, M);
-        norm(o, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, false);
-        const SplitPlanes gu = prompt_product(s, r, &lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln, M);
-        if (prompt_glu_supported(IS)) launch_prompt_glu(gu, a16, inv_br, M, lo, IS, gemma ? 1 : 0);
+        const ShortPlan po = prompt_plan(bt ? &bl->o : nullptr, D, qd, M), pgu = prompt_plan(bt ? &bl->gu : nullptr, 2 * IS, D, M),
+                        pd = prompt_plan(bt ? &bl->down : nullptr, D, IS, M);
+        launch_rows_to_f16_split(dptr_as<float>(r.att), a16, inv_br, M, qd, po.lo);
+        const SplitPlanes o = prompt_product(s, r, lw.o, bt ? &bl->o : nullptr, D, qd, inv_br, M, po);
+        norm(o, gemma ? lw.g_post_attn : nullptr, gemma ? lw.g_pre_ff : lw.g_post_attn, false, pgu.lo);
+        const SplitPlanes gu = prompt_product(s, r, &lw.gu, bt ? &bl->gu : nullptr, 2 * IS, D, inv_ln, M, pgu);
+        if (prompt_glu_supported(IS)) launch_prompt_glu(gu, a16, inv_br, M, pd.lo, IS, gemma ? 1 : 0);
         else {
             hipLaunchKernelGGL(k_glu_planes, dim3((IS + TB - 1) / TB, M), dim3(TB), 0, stream(), gu, dptr_as<float>(r.act), IS, gemma ? 1 : 0);
-            launch_rows_to_f16_split(dptr_as<float>(r.act), a16, inv_br, M, IS, lo);
+            launch_rows_to_f16_split(dptr_as<float>(r.act), a16, inv_br, M, IS, pd.lo);
         }
-        pending = prompt_product(s, r, lw.down, bt ? &bl->down : nullptr, D, IS, inv_br, M);
+        pending = prompt_product(s, r, lw.down, bt ? &bl->down : nullptr, D, IS, inv_br, M, pd);
         pending_g = gemma ? lw.g_post_ff : nullptr;
     }
     if (few) few_norm(pending_few, pending_g, s->g_final, true);
-    else norm(pending, pending_g, s->g_final, true);
+    else norm(pending, pending_g, s->g_final, true, M);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1688,10 +1692,12 @@ void prompt_logits(InferenceState *s, PromptRun &r, const int *m, int count, flo
         return;
     }
     for (int i = 0; i < count; i++) row(i, dptr_as<float>(r.sel) + (size_t)i * D);
-    launch_rows_to_f16_split(dptr_as<float>(r.sel), dptr_as<half_t>(r.a16), dptr_as<float>(r.inv_br), count, D, residual_row(count));
-    for (int n0 = 0, n; n0 < s->V; n0 += n) {              // (own weights: in parts, for which there is room in scratch if not for the whole head's image)
+    const WeightOp *tiles = s->borrows_tiles ? &s->borrowed_lm : nullptr;
+    for (int n0 = 0, n, lo = 0; n0 < s->V; n0 += n) {      // (own weights: in parts, for which there is room in scratch if not for the whole head's image)
         n = s->borrows_tiles ? s->V : std::min(PROMPT_HEAD_ROWS, s->V - n0);
-        const SplitPlanes lg = prompt_product(s, r, s->lm_head, s->borrows_tiles ? &s->borrowed_lm : nullptr, n, D, dptr_as<float>(r.inv_br), count, n0);
+        const ShortPlan p = prompt_plan(tiles, n, D, count);
+        if (p.lo != lo) launch_rows_to_f16_split(dptr_as<float>(r.sel), dptr_as<half_t>(r.a16), dptr_as<float>(r.inv_br), count, D, lo = p.lo);
+        const SplitPlanes lg = prompt_product(s, r, s->lm_head, tiles, n, D, dptr_as<float>(r.inv_br), count, p, n0);
         launch_planes_to_rows(lg, out + n0, count, n, s->V);
     }
 }

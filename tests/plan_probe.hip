@@ -16,20 +16,23 @@ int main()
         for (const auto &sh : shapes)
             for (int M : rows)
                 for (int fmt : {0, 1, 2}) {
-                    const int N = sh[0], K = sh[1], Kb = tiled_kb(K), lo = (M + 31) & ~31;
-                    const ShortPlan p = plan_short_pair(M, lo, N, K, 0, fmt);
+                    const int N = sh[0], K = sh[1], Kb = tiled_kb(K);
+                    const ShortPlan p = plan_short_pair(M, N, K, 0, fmt);
                     asked++;
-                    if (!p.big) continue;
-                    big++;
-                    if (fmt != 0 && large_m_unpacks_q8()) continue;         // (tiles that stay quantised: not the pair kernel's)
-                    bool ok = p.steps >= 1 && (lo & 31) == 0;
-                    if (ok) {
+                    const bool pair = p.big && !(fmt != 0 && large_m_unpacks_q8());      // (tiles that stay quantised: not the pair kernel's)
+                    // residual rows in a row block of their own where the pair kernel reads them, else no row between them and the values
+                    bool ok = p.lo == (pair ? (M + 31) / 32 * 32 : M);
+                    if (pair) {
+                        big++;
+                        ok = ok && p.steps >= 1;
+                    }
+                    if (pair && ok) {
                         const PairWalk w{p.steps, Kb};
                         const int blocks = (N + 255) / 256, teams = (blocks * Kb + p.steps - 1) / p.steps;
                         ok = p.chunks == w.planes();
                         for (int b = 0; b < blocks && ok; b++) ok = w.count(b * 256) >= 1 && w.count(b * 256) <= p.chunks && w.first(b) + w.count(b * 256) <= teams;
                     }
-                    if (!ok && bad++ < 10) printf("FAIL policy %d fmt %d M %d lo %d N %d K %d: steps %d planes %d\n", policy, fmt, M, lo, N, K, p.steps, p.chunks);
+                    if (!ok && bad++ < 10) printf("FAIL policy %d fmt %d M %d N %d K %d: big %d lo %d steps %d planes %d\n", policy, fmt, M, N, K, p.big, p.lo, p.steps, p.chunks);
                 }
     }
     printf("asked %ld big %ld bad %ld\n", asked, big, bad);
