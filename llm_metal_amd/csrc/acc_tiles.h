@@ -4,9 +4,11 @@
 // a product's result other registers than its operand and copies whole tiles between the register files all through a loop (32x32
 // tiles, which it cannot move so freely, it leaves), and as "+a" operands of assembly it still moves one now and then, next to an
 // instruction whose result is not there yet -- it does not know what the assembly does.  Every instruction here names its tile
-// as overwritten, so no value of the compiler's own lives in these registers across one.  A kernel that uses them has to leave
-// 100 vector registers or more free: it is spilling that makes the compiler take accumulation registers for itself.
-// Who reads a tile (take) keeps it 18 cycles or more behind the last instruction that wrote it: settle().
+// as overwritten, so no value of the compiler's own lives in these registers across one; between them it takes them for free.  So a kernel that uses
+// them has to give it no reason to: check_acc.py reads the assembly of every build and stops it where the compiler names an accumulation
+// register, spills, or writes an MFMA's operand too short ahead of it (its hazard pass does not look inside assembly).  (Vector registers taken
+// today: gemm_big_pair 254 of 256, gemm_big_f16<256> 156, k_wgrad_block<2> 106 of the 128 beside its tiles.)
+// Who reads a tile (take) keeps it 18 cycles or more behind the last instruction that wrote it: settle_tiles().
 #pragma once
 #include "devutil.h"
 #include <type_traits>
