@@ -184,6 +184,9 @@ void hip_gemm_large_m_split(int mode);
  * as much of the GPU on useful work as 128 x 256 does, counting partial rounds of blocks and partial tiles), 1 = always
  * 128 x 256, 2 = always 256 x 256. */
 void hip_gemm_large_m_block(int mode);
+/* Weight gradients in blocks of 256 x 128 whose operands come through LDS: 0 = by the measured rule (where a launch has a
+ * block for every CU), 1 = always, -1 = never.  Same weights and accumulators, bit for bit. */
+void hip_wgrad_block(int mode);
 /* A training state with frozen Q8_0 weights whose products run on the large-M kernel keeps the F16 image of every
  * weight it has used (made once instead of once per product) while they fit this many MB per state (default 65536;
  * the 4B model needs 16 GB); weights beyond that, or all with 0, get an image per product.  With 0 the prompts of a

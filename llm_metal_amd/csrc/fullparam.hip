@@ -562,6 +562,9 @@ void launch_transpose_scaled_jobs(const TransposeOperand *ops, int n, int T)
     LAUNCH_TIMED(0.0, 0.0, k_transpose_scaled_jobs, dim3(total), dim3(256), 0, js, T);
 }
 
+static int g_wgrad_block = 0;                             // hip_wgrad_block's choice
+void set_wgrad_block(int mode) { g_wgrad_block = mode; }
+
 void launch_wgrads(const WgradOperands *w, int n, int T, int mode, float lr)
 {
     if (n <= 0 || n > 4 || T <= 0) { fprintf(stderr, "[fast_hip] wgrads: %d matrices\n", n); abort(); }
@@ -569,7 +572,7 @@ void launch_wgrads(const WgradOperands *w, int n, int T, int mode, float lr)
     js.n = n;
     int total = 0, blocks = 0;
     for (int i = 0; i < n; i++) blocks += ((tiled_kb(w[i].N_in) + 1) / 2) * ((tiled_rb(w[i].M_out) + 7) / 8);
-    const bool big = blocks >= num_cus();                 // (fewer leave CUs without one, where k_wgrad's four times as many do not)
+    const bool big = g_wgrad_block ? g_wgrad_block > 0 : blocks >= num_cus();             // (fewer leave CUs without one, where k_wgrad's four times as many do not)
     for (int i = 0; i < n; i++) {
         if (w[i].M_out <= 0 || w[i].N_in <= 0) { fprintf(stderr, "[fast_hip] wgrads: empty matrix\n"); abort(); }
         js.j[i] = WgradJob{reinterpret_cast<const half8 *>(w[i].XT), w[i].x_inv, reinterpret_cast<const half8 *>(w[i].YT), w[i].y_inv,

@@ -128,6 +128,7 @@ int big_gemm_chunks(int M, int N, int K, int fmt);
 int big_gemm_chunks_for(int M, int N, int K, const WeightOp &W);
 void set_big_gemm_split(int mode);     // 1 measured rule, 0 never, n > 1 always n chunks
 void set_big_gemm_block(int mode);     // F16 tiles: 0 block shape by the measured rule, 1 always 128 x 256, 2 always 256 x 256
+void set_wgrad_block(int mode);        // weight gradients (fullparam.hip): 0 by the measured rule, 1 always in blocks of 256 x 128, -1 never
 // Returns the number of planes written (fewer than `chunks` when K has too few steps for that many).
 int launch_gemm_big(const half_t *A_tiled, const float *a_inv_scale, const WeightOp &W, float *C, int ldc, int M, int N, int K,
                     int chunks = 1, size_t plane_stride = 0);

@@ -814,6 +814,7 @@ void hip_gemm_ring_wide(int on) { lmhip::set_gemm_ring_wide(on); }
 void hip_gemm_half_planes(int on) { lmhip::set_gemm_half_planes(on); }
 void hip_gemm_large_m_split(int mode) { set_big_gemm_split(mode); }
 void hip_gemm_large_m_block(int mode) { set_big_gemm_block(mode); }
+void hip_wgrad_block(int mode) { lmhip::set_wgrad_block(mode); }
 
 void hip_gemm_profile_enable(int on)
 {

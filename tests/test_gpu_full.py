@@ -13,6 +13,7 @@ import tempfile
 import numpy as np
 import pytest
 
+from llm_metal_amd import lib
 from llm_metal_amd.configs import C1, TINY_GEMMA3
 from llm_metal_amd.sft import SFTState
 from llm_metal_amd.synth import make_batch, make_model
@@ -304,3 +305,43 @@ def test_matrices_handed_out(change):
         for wm, want in mats:
             got = Buf(st.L, wm.mbuf, wm.rows * wm.cols * 2, owned=False).read(np.uint16, (wm.rows, wm.cols))
             assert np.array_equal(got, oracle.f32_to_f16_bits(want))
+
+
+# 32-row blocks of X^T that end a target's column blocks half way (D = 1312, IS = 2084 of 64), an even number of column blocks of 64 and an
+# odd one, row counts that end inside tiles of 32 and blocks of 256; fewer blocks than one workgroup's, and many
+EDGES = [C1.with_(name="edges", NL=1, R=0, D=1312, Hq=12, Hkv=4, IS=2084, V=2084), C1.with_(name="small", NL=2, R=0, D=96, Hq=3, Hkv=1, hd=32, IS=100, V=260)]
+
+
+@pytest.mark.parametrize("rows", [17, 64, 300])
+@pytest.mark.parametrize("cfg", EDGES, ids=lambda c: c.name)
+def test_weight_gradients_in_blocks_are_the_same_bits(cfg, rows):
+    """k_wgrad_block against k_wgrad, which the small models above hold to the oracle: accumulators, weights and their transposed images, from
+    one K step of tokens to five, in the three ways that gradients are used; each twice, so that what the padding holds takes part."""
+    c = cfg.with_(seq=rows)
+    model = make_model(c, seed=61, gamma_jitter=0.1)
+    tok, tgt = make_batch(c, seed=62)
+    rng, got = np.random.default_rng(63), {}
+    prompt, toks, adv = _completions(c, rng, 1, 4, [rows - 4])
+    old = [np.full(rows - 4, -5.0, np.float32)]
+    adv = np.ones(1, np.float32)
+    for mode in (-1, 1):
+        out = got[mode] = []
+        lib.load().hip_wgrad_block(mode)
+        for use in ("accumulate", "sgd", "apply"):
+            print(c.name, rows, mode, use, flush=True)
+            with SFTState(c, model) as st:
+                if use != "sgd":
+                    st.alloc_grad_accum()
+                for _ in range(2):
+                    if use == "apply":
+                        out.append(st.grpo_apply_completions(prompt, toks, old, adv, 0.2, 0.05))
+                    else:
+                        out.append(np.float64(st.train_step(tok, tgt, 0.05)))
+                out += [st.matrix_f16(L, k, source) for L, k in all_matrices(c) for source in ((2,) if use == "accumulate" else (0, 1))]
+                if use == "accumulate":
+                    st.apply_grad_sgd(0.05)
+                    out += [st.matrix_f16(L, k, source) for L, k in all_matrices(c) for source in (0, 1)]
+                out.append(np.float64(st.train_step(tok, tgt, 0.0)))
+    assert len(got[1]) == len(got[-1]) and all(np.isfinite(x).all() for x in got[1] if x.dtype.kind == "f")
+    for i, (a, b) in enumerate(zip(got[1], got[-1])):
+        assert np.array_equal(a, b), i
