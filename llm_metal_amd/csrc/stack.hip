@@ -635,10 +635,22 @@ MoeRows moe_rows(const LayerStack *st, const StackRun *r, const StackLayer &L, i
     return m;
 }
 
-// The branch for a layer's experts, wherever they are grouped (16 rows and more): beside the mixer, both read the norm's rows
-// and what the first product made of them, and neither fills the chip (the delta rule's chunks are 64 workgroups for 103 us at
-// 2000 tokens, the experts' launches together 120 us).  Nevurax 1k, prompt and one token, in line -> beside: 16 tokens 724 -> 604 us,
-// 100 tokens 798 -> 660, 600 tokens 1025 -> 842, 2000 tokens 1641 -> 1344.
+// The branch for a layer's experts: beside the mixer, both read the norm's rows and what the first product made of them, and neither fills the
+// chip (the delta rule's chunks are 64 workgroups for 103 us at 2000 tokens, the experts' launches together 120 us).  Prompt and one
+// token, in line -> beside, us: Nevurax 1k 16 / 100 / 2048 tokens 726 / 795 / 1612 -> 674 / 693 / 1349, 2k 16 / 256 / 2048 1123 / 1422 / 2791 -> 1007 /
+// 1245 / 2464, 4k 16 / 256 / 2048 1634 / 2095 / 5469 -> 1500 / 1855 / 5207.
+// It costs the host 28 us a layer (12 to 15 of them for each wait of a stream for an event), which a prompt pays once.  A step of a batch pays it
+// for every token, beside some 220 us of launches and the pages of 4 MB of logits: experts of 96 MB and more are worth it (16 / 32 sequences,
+// 2k 1055 / 1337 -> 919 / 1205, 4k 1520 / 1875 -> 1337 / 1725), those of the 1k model (64 MB) only while the host keeps ahead: 16 / 24 / 28 / 32
+// sequences 640 / 720 / 755 / 785 -> 575 / 645 / 675 / 710 with a fast one, 655 / 757 / 795 / 811 -> 733 / 989 / 984 / 904 with a slow one.  There
+// they stay in line.
+constexpr size_t BESIDE_BYTES = (size_t)96 << 20;
+bool experts_beside(const StackLayer &L, int T)
+{
+    const size_t weights = (size_t)L.up.rows * L.up.cols + (size_t)L.down.rows * L.down.cols;
+    return !L.c.dense_ff && (T > 1 || weights * sizeof(half_t) >= BESIDE_BYTES);      // (a dense feed-forward overwrites the rows that the experts read)
+}
+
 // Their tiled images are made (once) in the stream, ahead of it.
 hipStream_t experts_begin(const StackLayer &L)
 {
@@ -786,8 +798,7 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
         const bool grouped = c.experts && !st->f32 && n >= 16 && n * c.top >= c.experts;
         norm(st, r, L.g_norm, n, 1, c.experts && !grouped);
         product(st, L.in, ptr<half_t>(r->a16), ptr<float>(r->inv), ptr<float>(r->h), st->Dp, ptr<float>(r->cin), n);
-        // (a dense feed-forward overwrites the rows that the experts read)
-        const bool beside = grouped && !c.dense_ff;
+        const bool beside = grouped && experts_beside(L, T);
         CatRows cat = cat_rows(st, r, L);
         const hipStream_t s = beside ? experts_begin(L) : stream();
         switch (c.mixer) {

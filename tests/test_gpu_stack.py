@@ -99,8 +99,8 @@ def test_states_are_used_again(mixed, tmp_path):
 
 @pytest.mark.parametrize("n", [15, 16, 17, 110])
 def test_experts_beside_the_mixer(n, tmp_path):
-    """From 16 rows on the experts run beside the mixer: against the oracle, and passes that follow one another without a wait
-    between their launches give the same bits."""
+    """From 16 rows on the experts run beside the mixer: against the oracle, and every pass gives the same bits: passes that are waited for, of two
+    states in turn, and portions of one sequence that follow one another without a wait (only the last one's logits are asked for)."""
     cfg, ra, rg = MODELS["mixed"]
     m = Model(cfg, tmp_path, ra, rg)
     toks = m.tokens(n, seed=3)
@@ -112,6 +112,32 @@ def test_experts_beside_the_mixer(n, tmp_path):
                 st.reset()
                 assert np.array_equal(st.forward_tokens(toks, [n - 1]), first)
         assert logit_error(first, want[n - 1:]) < TOL["f16"]
+    toks = m.tokens(6 * n, seed=4)
+    with state(m, "f16", 6 * n) as inf, state(m, "f16", 6 * n) as other:
+        waited = [inf.forward_tokens(toks[i:i + n], [n - 1]) for i in range(0, 6 * n, n)]
+        for _ in range(3):
+            other.reset()
+            for i in range(0, 5 * n, n):
+                other.forward_tokens(toks[i:i + n])
+            assert np.array_equal(other.forward_tokens(toks[5 * n:], [n - 1]), waited[-1])
+
+
+# (two layers whose experts' weights are 96 MB, as few as run beside the mixer in a step of one token)
+@pytest.mark.parametrize("cfg", [MODELS["mixed"][0], config([(delta(2, 1, 8, 8, 2), moe(48, 4, 1024, 0)), (latent(2), moe(48, 4, 1024, 8))], width=512)],
+                         ids=["in_line", "beside"])
+def test_batches_with_grouped_experts(cfg, tmp_path):
+    """Batches of 16 sequences and more, a token each, whose experts are read once for all of them: each sequence against itself alone."""
+    m = Model(cfg, tmp_path, 12, 20)
+    for B in (16, 17, 31):
+        seqs = np.array([m.tokens(6, seed=70 + b) for b in range(B)])
+        with state(m, "f16", 8) as inf:
+            first = [inf.step_batch(seqs[:, t], t) for t in range(6)]
+            again = [inf.step_batch(seqs[:, t], t, want_logits=t == 5) for t in range(6)]
+            assert np.array_equal(again[5], first[5])
+            got = np.stack(first, axis=1)
+            for b in (0, B // 2, B - 1):
+                inf.reset()
+                assert logit_error(got[b], np.stack([inf.forward_token(int(t)) for t in seqs[b]])) < TOL["f16"], (B, b)
 
 
 @MIXED
