@@ -26,7 +26,9 @@ hipStream_t stream();
 // A branch of the work beside the stream.  side_begin: a second stream of the library's, behind everything that stream() holds
 // so far; side_end: what is put into stream() from here on waits for the branch.  Every begin has its end before the call that
 // began it returns, so waiting for stream() waits for both.  A branch takes no scratch arena (they belong to stream()) and
-// writes nothing that stream() reads or writes before the end.
+// writes nothing that stream() reads or writes before the end.  side_open: makes the second stream and its events, which
+// side_begin else does, and has both streams wait for each other once; for what is loaded ahead of the first call.
+void side_open();
 hipStream_t side_begin();
 void side_end();
 int  initialized();

@@ -8,7 +8,7 @@
 namespace {
 int         g_refcount = 0;
 hipStream_t g_stream = nullptr;
-hipStream_t g_side = nullptr;             // made when first used
+hipStream_t g_side = nullptr;             // side_open
 hipEvent_t  g_side_from = nullptr, g_side_to = nullptr;
 int         g_num_cus = 0;
 struct Arena { void *p = nullptr; size_t cap = 0; };
@@ -18,12 +18,17 @@ Arena       g_scratch[lmhip::SCR_COUNT];
 namespace lmhip {
 
 hipStream_t stream() { return g_stream; }
+void side_open()
+{
+    if (g_side) return;
+    HIP_CHECK(hipStreamCreateWithFlags(&g_side, hipStreamNonBlocking));
+    for (hipEvent_t *e : {&g_side_from, &g_side_to}) HIP_CHECK(hipEventCreateWithFlags(e, hipEventDisableTiming | hipEventReleaseToDevice));
+    side_begin();
+    side_end();
+}
 hipStream_t side_begin()
 {
-    if (!g_side) {
-        HIP_CHECK(hipStreamCreateWithFlags(&g_side, hipStreamNonBlocking));
-        for (hipEvent_t *e : {&g_side_from, &g_side_to}) HIP_CHECK(hipEventCreateWithFlags(e, hipEventDisableTiming | hipEventReleaseToDevice));
-    }
+    side_open();
     HIP_CHECK(hipEventRecord(g_side_from, g_stream));
     HIP_CHECK(hipStreamWaitEvent(g_side, g_side_from, 0));
     return g_side;

@@ -256,6 +256,7 @@ LayerStack *stack_load(ModelFile *f, const StackConfig &cfg, int f32, int max_se
     metal_buf_free(ld.overflow);
     if (over) { fprintf(stderr, "[FastGen] a weight lies outside the F16 range; load the model in 32-bit precision\n"); ld.ok = false; }
     if (!ld.ok) { stack_free(st); return nullptr; }
+    if (!f32 && std::any_of(st->layers.begin(), st->layers.end(), [](const StackLayer &L) { return L.c.experts > 0; })) side_open();
     return st;
 }
 
@@ -644,19 +645,14 @@ MoeRows moe_rows(const LayerStack *st, const StackRun *r, const StackLayer &L, i
 // 2k 1055 / 1337 -> 919 / 1205, 4k 1520 / 1875 -> 1337 / 1725), those of the 1k model (64 MB) only while the host keeps ahead: 16 / 24 / 28 / 32
 // sequences 640 / 720 / 755 / 785 -> 575 / 645 / 675 / 710 with a fast one, 655 / 757 / 795 / 811 -> 733 / 989 / 984 / 904 with a slow one.  There
 // they stay in line.
+// The pass that makes their tiled images makes them in line, behind the mixer: with the host's allocations ahead of it a state's first prompt of 100
+// tokens (1k) took 2.3 ms and not 1.8, on another machine 3.0.
 constexpr size_t BESIDE_BYTES = (size_t)96 << 20;
 bool experts_beside(const StackLayer &L, int T)
 {
+    for (const MetalBuf *b : {L.up.buf, L.down.buf}) if (!b->tiled[0].dev || b->tiled[0].version != b->version) return false;
     const size_t weights = (size_t)L.up.rows * L.up.cols + (size_t)L.down.rows * L.down.cols;
     return !L.c.dense_ff && (T > 1 || weights * sizeof(half_t) >= BESIDE_BYTES);      // (a dense feed-forward overwrites the rows that the experts read)
-}
-
-// Their tiled images are made (once) in the stream, ahead of it.
-hipStream_t experts_begin(const StackLayer &L)
-{
-    tiled_weight_of(L.up.buf, L.up.rows, L.up.cols);
-    tiled_weight_of(L.down.buf, L.down.rows, L.down.cols);
-    return side_begin();
 }
 
 // the experts' part of a layer over all rows, sorted by expert; writes the run's route_* and moe_* buffers alone
@@ -800,7 +796,7 @@ void stack_forward(LayerStack *st, StackRun *r, const int *tokens, int T, int po
         product(st, L.in, ptr<half_t>(r->a16), ptr<float>(r->inv), ptr<float>(r->h), st->Dp, ptr<float>(r->cin), n);
         const bool beside = grouped && experts_beside(L, T);
         CatRows cat = cat_rows(st, r, L);
-        const hipStream_t s = beside ? experts_begin(L) : stream();
+        const hipStream_t s = beside ? side_begin() : stream();
         switch (c.mixer) {
         case MIX_LATENT: cat.o = mix_latent(st, r, L, r->layers[i], rows); break;
         case MIX_GROUPED: cat.o = mix_grouped(st, r, L, rows, cat); break;
