@@ -506,6 +506,7 @@ __global__ __launch_bounds__(256) void k_untile_tiles(UntileJobs js)
     for (int i = 0; i < 4; i++) v[i] = __builtin_nontemporal_load(&p[i * 64]);
 #pragma unroll
     for (int i = 0; i < 4; i++) t[wave][lane & 31][(lane >> 5) * 4 + i] = v[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                 // (other lanes' pieces are read next)
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < 4; i++) {
