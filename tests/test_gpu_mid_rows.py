@@ -57,7 +57,7 @@ def test_full_parameter_pass_equals_streaming_kernel(rows):
         assert rel(b, a) < 5e-3                             # the accumulators themselves are F16
 
 
-@pytest.mark.parametrize("n", [33, 100, 400, 511])
+@pytest.mark.parametrize("n", [33, 100, 400, 511, 513, 1000, 1024])
 def test_prompt_equals_streaming_kernel(n):
     c = C1.with_(name="mid_prompt", D=1312, IS=2084, NL=2, Hq=12, Hkv=4, V=2052)
     model = make_model(c, seed=25, gamma_jitter=0.1)
