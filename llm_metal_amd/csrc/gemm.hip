@@ -288,9 +288,11 @@ namespace lmhip {
 // on 2560 x 4096) or when not all are resident at once (beyond 512).  Among equally balanced splits the one with fewer
 // planes wins: a plane costs the product its stores and the consumer its loads (the more the shorter K is).
 //
-// So few row tiles that even sixteen chunks leave CUs without work (outputs of up to 1024 columns): as many chunks as leave each four K
+// So few row tiles that even sixteen chunks leave CUs without work (outputs of up to 960 columns on 256 CUs): as many chunks as leave each four K
 // steps, two rounds of a workgroup.  A product of four workgroups is their walk through K, and its planes are nothing: 256 columns of K = 256 ..
-// 4096 (a tiny model's) 66 us for the ten of a step in one chunk each, 42 so; the step 268 -> 226 us, as near to 64 bits as before.
+// 4096 (a tiny model's) 66 us for the ten of a step in one chunk each, 42 so; the step 268 -> 226 us.  Four layers of width 384 / 512 / 640 / 768 / 896 /
+// 960, 64 rows: 481 / 516 / 494 / 509 / 485 / 466 -> 389 / 411 / 428 / 440 / 475 / 451 us.  The planes are fp32 (GemmPlan::whole); errors against
+// 64 bits over 18 tiny steps, F16 and Q8_0, times those of one chunk: losses 0.96, logits 0.98, adapters 0.96.
 static bool few_row_tiles(int n_tiles, int cus) { return n_tiles * 16 < cus; }
 static int ring_chunks(int n_tiles, int Kb, int K, int cus)
 {

@@ -1,8 +1,9 @@
 // Large-M GEMM: C[M, N] = inv_scale[m] * A16[M, K] * W[N, K]^T for M of several hundred rows and more
 // (batch * seq = 2048 in the Q8_0 configuration), where a weight tile is reused by enough activation rows
 // that the matrix cores, not HBM, bound the product.  Same operands as the weight-streaming kernel
-// (gemm.h: tiled fp16 activations with per-row power-of-two factors; F16 or Q8_0 weight tiles), same
-// arithmetic (v_mfma_f32_32x32x16_f16, fp32 accumulation), one launch; K chunks (planes) where the blocks leave CUs idle.
+// (gemm.h: tiled fp16 activations with per-row power-of-two factors; F16 or Q8_0 weight tiles), fp16 products
+// and fp32 accumulation, one launch; K chunks (planes) where the blocks leave CUs idle.  Q8_0 tiles and gemm_big_short multiply with
+// v_mfma_f32_32x32x16_f16, F16 tiles (gemm_big_f16, gemm_big_pair) with v_mfma_f32_16x16x32_f16 on accumulators in place (acc_tiles.h).
 //
 // A workgroup of four waves owns a 128 x 256 block of C and walks K in steps of 64.  Per step every wave
 // fetches one 32-row block of the activation tile and two of the weight tile from L2/HBM in the MFMA
@@ -253,11 +254,13 @@ __global__ __launch_bounds__(256) void gemm_big(GemmKArgs g)
 }
 
 
-// The product of operands that hold more than fp16 (value and residual rows): no sum of more than twelve MFMAs in one accumulator.  The
-// matrix cores round an accumulator at every instruction, so a sum over K = 2560 in one is 2.5 times as far from the exact one as a
+// The product whose sums are of short parts (of a prompt's rows with what rounding a Q8_0 weight to F16 lost; value and residual rows take
+// gemm_big_pair): no more than twelve MFMAs in one accumulator.  The matrix cores round an accumulator at every instruction, so a sum over K = 2560 in one is 2.5 times as far from the exact one as a
 // matrix-vector product's (units of 2^-24 of the result's norm, 64 rows: 5.5 against 2.2; K = 9728: 10.5 against 3.9).  Two of the
 // eight accumulators of a wave are added to sums of their own in each of four half steps out of six, under the MFMAs of the
-// others, and start again from zero.  The walk through K is that of gemm_big_f16, below, in 32x32x16 instructions.
+// others, and start again from zero.  K goes in half steps of 32 through six buffers: half step hs is multiplied out of buffer hs % 6, in two
+// slices of 16; the barrier that ends hs - 1 has found hs and hs + 1 in LDS, slice 0 of hs + 1 is read under the products of slice 1 of hs,
+// and hs + 5 is requested into the buffer that hs - 1 left.
 __global__ __launch_bounds__(256) void gemm_big_short(GemmKArgs g)
 {
     constexpr int HB = 12 * 2 * 64;                       // half8 per buffer: [4 A + 8 W row blocks][2 slices][64 lanes]
@@ -824,7 +827,7 @@ __global__ __launch_bounds__(256) void gemm_big_q8(GemmKArgs g)
 #pragma unroll
             for (int k = 0; k < 4; k++) acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[k], acc[i][k], 0, 0, 0);
     };
-    // Half step hs is multiplied out of buffer hs % 6 (see gemm_big_f16<256>): the barrier that ends half step hs - 1 has
+    // Half step hs is multiplied out of buffer hs % 6, as in gemm_big_short: the barrier that ends half step hs - 1 has
     // found hs and hs + 1 in LDS, slice 0 of hs + 1 is read and unpacked while slice 1 of hs is multiplied, hs + 5 is
     // requested into the buffer hs - 1 left.  Eight copies per wave and half step.
     auto step = [&](int hs, const uint4v (&cur)[HB], int slot, const uint4v (&nxt)[HB], int nslot, uint4v (&free_buf)[HB], int fslot)
@@ -1096,8 +1099,7 @@ int launch_gemm_big(const half_t *A, const float *a_inv_scale, const WeightOp &W
 }
 
 // The plan: the streaming kernel (its waves and planes in any case form short sums; at most four K steps per wave, sixteen MFMAs) or
-// the 128 x 256 block, by the times of mid_plan at any number of rows -- the 256 x 256 block has no registers for a second set of
-// sums.  Operands that are not F16 tiles: use_big_gemm's rule.
+// the 128 x 256 block, by the times of mid_plan at any number of rows.  Operands that are not F16 tiles: use_big_gemm's rule.
 ShortPlan plan_short_sums(int M, int N, int K, int nbq, int fmt)
 {
     ShortPlan p{0, 1, plan_gemm(M, N, K, nbq, fmt)};
