@@ -488,7 +488,7 @@ def _main():
                            "gemm_big_f16<256>, gemm_big_f16<128>" if cfg.BN >= 1024 else
                            # full-parameter pass: the products, the weight gradients (F16 read-modify-write of the accumulators), the
                            # apply (W, G and the transposed image) and the operand transposes (time only) are timed together
-                           "gemm_tiled, gemm_big_f16*, k_wgrad, k_apply_retile, k_transpose_scaled_jobs" if cfg.R == 0 else
+                           "gemm_tiled, gemm_big_f16*, k_wgrad, k_wgrad_block, k_apply_retile, k_transpose_scaled_jobs" if cfg.R == 0 else
                            "gemm_ring, gemm_ring_wide" if 32 < cfg.BN <= 64 and args.gemm_ring and args.gemm_ring_wide else
                            "gemm_ring" if cfg.BN <= 64 and args.gemm_ring else "gemm_tiled"),
                 "launches_per_step": n // prof_steps,
